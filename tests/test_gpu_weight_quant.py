@@ -158,3 +158,28 @@ def test_full_size_tensor_sampled_rows(oracle):
     wn = w[sample].cpu().numpy()
     want = oracle.quantize_rows_w(wn, hadamard=True)
     assert blocks_equal(blocks[sample], want), block_diff(blocks[sample], want)
+
+
+@pytest.mark.parametrize("K,wgroup", [(256, 0), (1536, 0), (1536, 64), (1280, 256)])
+def test_search_at_rounding_boundaries_and_extreme_scales(oracle, K, wgroup):
+    """The clip search takes the correctly rounded quotient only where x * (1 / s) is near a half-way point or 1 / s is
+    no normal number: rows full of exact ties and of values one step beside them, rows of denormals, of the largest
+    floats, with an infinity, and ordinary ones."""
+    rng = np.random.default_rng(K + wgroup)
+    half = rng.integers(-14, 15, size=(12, K)).astype(f32) * f32(0.5)     # k / 2: ties at scale 1
+    half[:, ::64] = 7.0                                                    # amax 7: the first ratio's scale is exactly 1
+    w = half.copy()
+    w[1] = np.nextafter(half[1], f32(np.inf))
+    w[2] = np.nextafter(half[2], f32(-np.inf))
+    w[3] = half[3] * f32(2.0 ** -140)
+    w[4] = half[4] * f32(2.0 ** -124)
+    w[5] = half[5] * f32(2.0 ** 124)
+    w[6] = half[6] * f32(0.1)
+    w[7] = half[7] * f32(1.0 / 3.0)
+    w[8] = (rng.standard_normal(K) * 2.0 ** -130).astype(f32)
+    w[9] = (rng.standard_normal(K) * 1e37).astype(f32)
+    w[10, 5] = np.inf
+    w[11] = rng.standard_normal(K).astype(f32)
+    got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4, wgroup=wgroup)
+    want = oracle.quantize_rows_w(w, wgroup=wgroup)
+    assert blocks_equal(got, want), block_diff(got, want)
