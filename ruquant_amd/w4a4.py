@@ -253,6 +253,61 @@ def quantize_act(x, clip, hadamard_=False, n_rot=None):
     return out.cpu().numpy().view(BLOCK_DTYPE).reshape(M, K // 256)
 
 
+# Blocks travel between the host's ordinary memory and the GPU through pinned buffers of this size, a few at a time: a
+# copy from or to pageable memory is staged by the runtime on one thread and waits for each stage (17.7 MB from the GPU
+# 950 us, of which the link needs 320; 12.5 MB to it 350 + 185 us for a private copy, the link 230), this way the
+# link, the host's copy (several threads) and the kernels run side by side. torch's pinned-memory cache hands the
+# buffers out and takes them back, so concurrent calls have their own and no call keeps any.
+_STAGE_BYTES = 4 << 20
+_STAGES = 3
+
+
+def _chunks(n, most):
+    """[0, n) in equal runs of at most `most`"""
+    k = max(1, -(-n // most))
+    return [(n * i // k, n * (i + 1) // k) for i in range(k)]
+
+
+def _stages(nbytes):
+    return [torch.empty(nbytes, dtype=torch.uint8, pin_memory=True) for _ in range(_STAGES)]
+
+
+def _copy_bytes(pinned, src):
+    """numpy bytes into the head of a pinned tensor (torch's copy uses several threads; it takes writable arrays only)"""
+    if src.flags.writeable:
+        pinned[:src.size].copy_(torch.from_numpy(src))
+    else:
+        np.copyto(pinned[:src.size].numpy(), src)
+
+
+def _fetch(dev, parts):
+    """Bytes of the device tensor `dev` as a new numpy array; parts: (first byte, one past the last byte, event behind
+    which they are ready), in the order in which they become ready."""
+    host = np.empty(dev.numel(), dtype=np.uint8)
+    to = torch.from_numpy(host)
+    copier = torch.cuda.Stream(dev.device)
+    runs = [(a0 + a, a0 + b, ready) for a0, b0, ready in parts for a, b in _chunks(b0 - a0, _STAGE_BYTES)]
+    stages = _stages(max(b - a for a, b, _ in runs))
+    done = [None] * len(runs)
+
+    def land(i):
+        a, b, _ = runs[i]
+        done[i].synchronize()
+        to[a:b].copy_(stages[i % _STAGES][:b - a])
+
+    with torch.cuda.stream(copier):
+        for i, (a, b, ready) in enumerate(runs):
+            if i >= _STAGES:
+                land(i - _STAGES)
+            copier.wait_event(ready)
+            stages[i % _STAGES][:b - a].copy_(dev[a:b], non_blocking=True)
+            done[i] = torch.cuda.Event()
+            done[i].record()
+    for i in range(max(0, len(runs) - _STAGES), len(runs)):
+        land(i)
+    return host
+
+
 def quantize_weights(w, type_, n_rot=None, wgroup=0):
     """w[N, K] fp32 on the GPU -> [N, K/256] weight blocks (numpy, host): the type's from_float_ref for whole
     tensors (quantize_row_w4a4_ref / quantize_row_w4a4h_ref, patch lines 2681-2710). wgroup 0 / 256 / 64 is the
@@ -261,16 +316,27 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
     assert w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and w.stride(1) == 1
     N, K = w.shape
     n_rot = int(n_rot or K)
-    nbytes = L.rq_w4a4_quantize_weights_workspace_bytes(int(type_), K, N, int(wgroup))
+    # With one scale per row the search has a wavefront for four rows: 4096 rows are one per SIMD, and as many more take
+    # as long again, so a tensor goes through in runs of that many and a run's blocks travel while the next one is
+    # searched. (Weight groups fill the GPU with any number of rows: the same runs serve.)
+    runs = [(a, min(a + 4096, N)) for a in range(0, N, 4096)]
+    nbytes = L.rq_w4a4_quantize_weights_workspace_bytes(int(type_), K, min(N, 4096), int(wgroup))
     if nbytes == 0:
         raise RqError("unsupported weight shape or group: K=%d N=%d wgroup=%d" % (K, N, wgroup))
     ws = _device_bytes(nbytes, w.device)
-    out = torch.zeros(N * (K // 256) * 144, dtype=torch.uint8, device=w.device)
+    row = (K // 256) * 144
+    out = torch.empty(N * row, dtype=torch.uint8, device=w.device)
+    ldw = w.stride(0) if N > 1 else K
+    parts = []
     with torch.cuda.device(w.device):
-        rc = L.rq_w4a4_quantize_weights(int(type_), w.data_ptr(), w.stride(0) if N > 1 else K, N, K, n_rot,
-                                        int(wgroup), out.data_ptr(), ws.data_ptr(), ws.numel(), _stream_ptr())
-    _check(rc, "rq_w4a4_quantize_weights")
-    return out.cpu().numpy().view(BLOCK_DTYPE).reshape(N, K // 256)
+        for a, b in runs:
+            rc = L.rq_w4a4_quantize_weights(int(type_), w.data_ptr() + 4 * ldw * a, ldw, b - a, K, n_rot, int(wgroup),
+                                            out.data_ptr() + row * a, ws.data_ptr(), ws.numel(), _stream_ptr())
+            _check(rc, "rq_w4a4_quantize_weights")
+            ready = torch.cuda.Event()
+            ready.record()
+            parts.append((row * a, row * b, ready))
+        return _fetch(out, parts).view(BLOCK_DTYPE).reshape(N, K // 256)
 
 
 def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
@@ -285,11 +351,32 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
     if n_rot is None:
         n_rot = int(blocks[0, 0]["pad"][0 if type_ in (TYPE_W4A4, TYPE_W4A4H) else 1]) if rows else K
     dev = torch.device(device)
-    raw = torch.from_numpy(blocks.view(np.uint8).reshape(-1).copy()).to(dev)
+    row = nb * 144
     out = torch.empty((rows, K), dtype=torch.float32, device=dev)
+    raw = torch.empty(rows * row, dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
-        rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr(), rows, K, int(n_rot), out.data_ptr(), K, _stream_ptr())
-    _check(rc, "rq_w4a4_dequantize")
+        # a run of rows is decoded while the next one travels
+        current = torch.cuda.current_stream()
+        copier = torch.cuda.Stream()
+        copier.wait_stream(current)   # (the memory of `raw` may still be in use by work in front of this call)
+        runs = _chunks(rows, max(1, _STAGE_BYTES // max(row, 1)))
+        host = blocks.view(np.uint8).reshape(-1)
+        stages = _stages(row * max(b - a for a, b in runs)) if rows else []
+        sent = [None] * _STAGES
+        for i, (a, b) in enumerate(runs):
+            n, k = row * (b - a), i % _STAGES
+            if sent[k] is not None:
+                sent[k].synchronize()
+            if n:
+                _copy_bytes(stages[k], host[row * a:row * b])
+                with torch.cuda.stream(copier):
+                    raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
+                    sent[k] = torch.cuda.Event()
+                    sent[k].record()
+                current.wait_event(sent[k])
+            rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot),
+                                      out.data_ptr() + 4 * K * a, K, _stream_ptr())
+            _check(rc, "rq_w4a4_dequantize")
     return out
 
 

@@ -183,3 +183,16 @@ def test_search_at_rounding_boundaries_and_extreme_scales(oracle, K, wgroup):
     got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4, wgroup=wgroup)
     want = oracle.quantize_rows_w(w, wgroup=wgroup)
     assert blocks_equal(got, want), block_diff(got, want)
+
+
+def test_conversions_in_several_runs(oracle):
+    """Tensors that go through in several runs of rows and more runs than there are pinned buffers; one row more than a
+    run; a read-only array."""
+    w = tensor(4097, 256, 3)
+    got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4)
+    want = oracle.quantize_rows_w(w)
+    assert blocks_equal(got, want), block_diff(got, want)
+    blocks = np.tile(want, (9, 4))[:30001]            # 17 MB of blocks: five runs
+    blocks.flags.writeable = False
+    got = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy()
+    assert bits_equal(got, rq.dequantize_rows(blocks))
