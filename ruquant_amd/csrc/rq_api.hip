@@ -307,7 +307,13 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     if (!(stages & 2)) return 0;
 
     // launches: one for all weights, or one per weight
-    const int n_launch = one_launch && path != kPathGemm ? 1 : n;
+    // (the fp6 GEMM's slabs do not depend on N, so it needs no room beyond the largest weight's. It runs weights with and
+    // without multipliers through different kernels: a set that has both kinds goes weight by weight. K = 5120, 2048
+    // tokens, N = 6144 + 1024 + 1024: the three launches leave 128, 64 and 64 tiles over to be cut along K, one launch is
+    // two whole rounds of tiles)
+    bool fuse_gemm = fp6 && G == kGroup;
+    for (int i = 1; i < n && fuse_gemm; ++i) fuse_gemm = multipliers_noted(prepared[i]) == multipliers_noted(prepared[0]);
+    const int n_launch = (path == kPathGemm ? fuse_gemm : one_launch) ? 1 : n;
     for (int l = 0; l < n_launch; ++l) {
         FusedWeights fw;
         memset(&fw, 0, sizeof fw);
@@ -333,6 +339,18 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
             g.panels = 0;
             e = launch_skinny(g, stream);
             if (e != hipSuccess) return (int) e;
+        } else if (fp6) {
+            Gemm6Args g;
+            g.w = fw;
+            g.act6 = wsb + W.off_i8;
+            g.u = q.u;
+            g.M = (int) M;
+            g.Mp = (int) W.Mp;
+            g.groups_per_fold = G / kGroup;
+            g.cells = have_slabs ? wsb + W.off_tot : nullptr;
+            g.weight_multipliers = multipliers_noted(fw.prepared[0]);
+            e = launch_gemm6(g, stream);
+            if (e != hipSuccess) return (int) e;
         } else if (gemm) {
             GemmArgs g;
             g.prepared = fw.prepared[0];
@@ -344,9 +362,7 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
             g.M = (int) M;
             g.Mp = (int) W.Mp;
             g.groups_per_fold = G / kGroup;
-            g.cells = have_slabs ? wsb + W.off_tot : nullptr;
-            g.weight_multipliers = multipliers_noted(fw.prepared[0]);
-            e = fp6 ? launch_gemm6(g, stream) : launch_gemm(g, stream);
+            e = launch_gemm(g, stream);
             if (e != hipSuccess) return (int) e;
         } else {
             for (int c = 0; c < W.chunks; ++c) {

@@ -271,12 +271,21 @@ struct GemmArgs {
     int64_t         ldy;
     int             M, Mp;
     int             groups_per_fold;   // 1; 2 or 4 when the activation groups are 128 or 256 wide
-    void           *cells;             // fp6 form: arrival counters (zero on entry, left zero) and slabs of the tiles cut along K
-    bool            weight_multipliers = false;   // fp6 form: the host has seen this weight's flag for multipliers set
 };
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream);
-// the fp6 form: act8 = the fp6 fragment plane with the multipliers behind it; the weight needs the fp6 plane
-hipError_t launch_gemm6(const GemmArgs &a, hipStream_t stream);
+
+// the fp6 form, up to three weights in one launch: the fp6 fragment plane with the multipliers behind it; every weight
+// needs its fp6 plane
+struct Gemm6Args {
+    FusedWeights    w;
+    const uint8_t  *act6;
+    const float    *u;      // [Mp]
+    int             M, Mp;
+    int             groups_per_fold;      // 1; 2 or 4 when the activation groups are 128 or 256 wide
+    void           *cells;                // arrival counters (zero on entry, left zero) and slabs of the tiles cut along K
+    bool            weight_multipliers;   // the host has seen these weights' flags for multipliers set
+};
+hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream);
 // How a launch of the fp6 form is cut: n_whole tiles (256 rows x 128 tokens) run whole, the rest in `parts` slices of
 // K each, which meet in cell_bytes of workspace: kGemm6CounterBytes of arrival counters (one int per cut tile: zero on
 // entry, left zero), then one slab of partial totals per slice (needs no clearing).
@@ -285,7 +294,7 @@ struct Gemm6Plan {
     int    n_tiles, n_whole, parts;
     size_t cell_bytes;
 };
-Gemm6Plan gemm6_plan(int64_t N, int64_t M, int ng, int groups_per_fold);
+Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold);
 
 // up to 64 tokens: MFMA arithmetic on a GEMV-shaped weight stream; same operands as the GEMM plus the split-K cells
 struct SkinnyArgs {

@@ -84,7 +84,9 @@ constexpr int kDeviceScope = 16;               // cache policy of a buffer acces
 
 // WITHK: the stage of the kernel form that folds with weight multipliers from LDS. (Two layouts, because the 512
 // bytes shift the stages' LDS offsets, and with them the plain kernel's loop needs base registers it does not have.)
-template <bool WITHK>
+// (SET is a tag that keeps the helpers of two kernels apart: a helper that both call no longer has constant LDS addresses
+// when the compiler simplifies it ahead of inlining, and the plain loop then spills 113 registers instead of 9.)
+template <bool WITHK, bool SET>
 struct StageT {
     static constexpr int kCells = WITHK ? kStageCellsK : kStageCellsPlain;
     static constexpr int kTailLanes = WITHK ? 44 : 40;   // lanes of a wavefront's fifth load
@@ -476,15 +478,30 @@ __device__ __forceinline__ void body64(Ctx &c, Stage &s0, Stage &s1, Stage &s2, 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the refetches of the last steps
 }
 
+// Up to three weights of one K in one launch: row tile r of the launch belongs to weight w with first[w] <= r <
+// first[w + 1]. (What a launch loses is its end: the tiles beyond whole rounds of the chip, cut along K, and the wait for
+// the last of them. One launch over q + k + v at K = 5120, N = 6144 + 1024 + 1024, 2048 tokens, has 512 tiles, two whole
+// rounds.)
+struct TileSet {
+    const float   *s_w[kMaxFused];
+    const uint8_t *kmul[kMaxFused];
+    const int32_t *flags[kMaxFused];
+    float         *y[kMaxFused];
+    int64_t        ldy[kMaxFused];
+    int64_t        N[kMaxFused];
+    int            n_panels[kMaxFused];
+    int            first[kMaxFused];   // unused slots hold the total, so no tile selects them
+};
+
 // KFMA (activation groups of 64 only): the form of the kernel for tensors with weight multipliers; see group_units
-template <int GS, bool KFMA>
+// SET: a launch over several weights (a form of its own: the loop has no register to spare for the selection, and a single
+// weight's launch would pay 1 % for it)
+template <int GS, bool KFMA, bool SET>
 __global__ void __launch_bounds__(kThreads)
-rq_gemm6_kernel(const float *__restrict__ s_w, const uint8_t *__restrict__ kmul,
-                const int32_t *__restrict__ flags, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
-                const float *__restrict__ u, float *__restrict__ y, int64_t ldy, int64_t N, int M, int Mp, int ng,
-                int n_panels, int n_tok_tiles, int n_tiles, int super_tiles, int n_whole, int parts,
-                int *__restrict__ counters, unsigned long long *__restrict__ slabs) {
-    using Stage = StageT<KFMA>;
+rq_gemm6_kernel(const TileSet ts, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
+                const float *__restrict__ u, int M, int Mp, int ng, int n_tok_tiles, int n_tiles, int super_tiles,
+                int n_whole, int parts, int *__restrict__ counters, unsigned long long *__restrict__ slabs) {
+    using Stage = StageT<KFMA, SET>;
     __shared__ Stage ring[kRing];
     Stage &s0 = ring[0], &s1 = ring[1], &s2 = ring[2], &s3 = ring[3];
     static_assert(8 * 32 * kXposeStride * 4 <= sizeof(Stage), "the epilogue's output blocks fit one stage");
@@ -524,6 +541,18 @@ rq_gemm6_kernel(const float *__restrict__ s_w, const uint8_t *__restrict__ kmul,
         }
         slot = v - n_whole;
     }
+    int wsel = 0;
+    if (SET) {
+        wsel = (row_tile >= ts.first[1]) + (row_tile >= ts.first[2]);
+        row_tile -= wsel == 0 ? 0 : wsel == 1 ? ts.first[1] : ts.first[2];   // now of its weight
+    }
+    const float *__restrict__ s_w = wsel == 0 ? ts.s_w[0] : wsel == 1 ? ts.s_w[1] : ts.s_w[2];
+    const uint8_t *__restrict__ kmul = wsel == 0 ? ts.kmul[0] : wsel == 1 ? ts.kmul[1] : ts.kmul[2];
+    const int32_t *__restrict__ flags = wsel == 0 ? ts.flags[0] : wsel == 1 ? ts.flags[1] : ts.flags[2];
+    float *__restrict__ y = wsel == 0 ? ts.y[0] : wsel == 1 ? ts.y[1] : ts.y[2];
+    const int64_t ldy = wsel == 0 ? ts.ldy[0] : wsel == 1 ? ts.ldy[1] : ts.ldy[2];
+    const int64_t N = wsel == 0 ? ts.N[0] : wsel == 1 ? ts.N[1] : ts.N[2];
+    const int n_panels = wsel == 0 ? ts.n_panels[0] : wsel == 1 ? ts.n_panels[1] : ts.n_panels[2];
     const bool sliced = (int) blockIdx.x >= n_whole;
     // this workgroup's steps (two groups each) of the tile's ng / 2
     const int s_begin = sliced ? (int) ((int64_t) (ng / 2) * part / parts) : 0;
@@ -740,9 +769,8 @@ rq_gemm6_kernel(const float *__restrict__ s_w, const uint8_t *__restrict__ kmul,
 
 }  // namespace
 
-Gemm6Plan gemm6_plan(int64_t N, int64_t M, int ng, int groups_per_fold) {
+Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold) {
     Gemm6Plan pl;
-    const int n_row_tiles = (int) ((N + kTileRows - 1) / kTileRows);
     const int n_tok_tiles = (int) ((M + kTileTok - 1) / kTileTok);
     pl.n_tiles = n_row_tiles * n_tok_tiles;
     pl.n_whole = pl.n_tiles;
@@ -777,11 +805,26 @@ Gemm6Plan gemm6_plan(int64_t N, int64_t M, int ng, int groups_per_fold) {
     return pl;
 }
 
-hipError_t launch_gemm6(const GemmArgs &a, hipStream_t stream) {
-    const uint8_t *p = a.prepared;
-    const int n_row_tiles = a.L.n_rtiles;
+hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
+    TileSet ts;
+    int n_row_tiles = 0;
+    for (int i = 0; i < kMaxFused; ++i) {
+        const int k = i < a.w.n ? i : a.w.n - 1;   // unused slots repeat the last weight (never selected)
+        const PreparedLayout &L = a.w.L[k];
+        const uint8_t *p = a.w.prepared[k];
+        ts.s_w[i] = reinterpret_cast<const float *>(p + L.off_sw);
+        ts.kmul[i] = p + L.off_kmul;
+        ts.flags[i] = reinterpret_cast<const int32_t *>(p + L.off_flags);
+        ts.y[i] = a.w.y[k];
+        ts.ldy[i] = a.w.ldy[k];
+        ts.N[i] = L.N;
+        ts.n_panels[i] = L.n_panels;
+        ts.first[i] = n_row_tiles;
+        if (i < a.w.n) n_row_tiles += L.n_rtiles;
+    }
+    const int ng = a.w.L[0].ng;
     const int n_tok_tiles = a.Mp / kTileTok;
-    Gemm6Plan pl = gemm6_plan(a.L.N, a.M, a.L.ng, a.groups_per_fold);
+    Gemm6Plan pl = gemm6_plan(n_row_tiles, a.M, ng, a.groups_per_fold);
     if (pl.n_tiles != n_row_tiles * n_tok_tiles) return hipErrorInvalidValue;
     if (a.cells == nullptr) {   // a workspace without slabs: every tile whole
         pl.n_whole = pl.n_tiles;
@@ -789,20 +832,26 @@ hipError_t launch_gemm6(const GemmArgs &a, hipStream_t stream) {
     }
     const int super_tiles = n_tok_tiles % 4 == 0 && n_row_tiles % 8 == 0;
     const int grid = pl.n_whole + (pl.n_tiles - pl.n_whole) * pl.parts;
-    const float *m4 = reinterpret_cast<const float *>(a.act8 + act6_plane_bytes(a.L.ng, a.Mp));
-#define RQ_LAUNCH6(GS, KFMA)                                                                                        \
-    hipLaunchKernelGGL((rq_gemm6_kernel<GS, KFMA>), dim3(grid), dim3(kThreads), 0, stream,                            \
-                       reinterpret_cast<const float *>(p + a.L.off_sw), p + a.L.off_kmul,                           \
-                       reinterpret_cast<const int32_t *>(p + a.L.off_flags), a.act8, m4, a.u, a.y, a.ldy, a.L.N, a.M, \
-                       a.Mp, a.L.ng, a.L.n_panels, n_tok_tiles, pl.n_tiles, super_tiles, pl.n_whole, pl.parts,      \
+    const float *m4 = reinterpret_cast<const float *>(a.act6 + act6_plane_bytes(ng, a.Mp));
+#define RQ_LAUNCH6(GS, KFMA, SET)                                                                                      \
+    hipLaunchKernelGGL((rq_gemm6_kernel<GS, KFMA, SET>), dim3(grid), dim3(kThreads), 0, stream, ts, a.act6, m4, a.u, a.M,  \
+                       a.Mp, ng, n_tok_tiles, pl.n_tiles, super_tiles, pl.n_whole, pl.parts,                         \
                        reinterpret_cast<int *>(a.cells),                                                             \
                        reinterpret_cast<unsigned long long *>(reinterpret_cast<uint8_t *>(a.cells) + kGemm6CounterBytes))
     // (a.weight_multipliers: what the host knows about the tensor; only a choice between two kernels that are both
     // right for every tensor)
-    if (a.groups_per_fold == 1 && a.weight_multipliers) RQ_LAUNCH6(1, true);
-    else if (a.groups_per_fold == 1) RQ_LAUNCH6(1, false);
-    else if (a.groups_per_fold == 2) RQ_LAUNCH6(2, false);
-    else RQ_LAUNCH6(4, false);
+    if (a.w.n > 1) {
+        if (a.groups_per_fold != 1) return hipErrorInvalidValue;   // (wider groups go weight by weight)
+        if (a.weight_multipliers) RQ_LAUNCH6(1, true, true);
+        else RQ_LAUNCH6(1, false, true);
+    } else if (a.groups_per_fold == 1) {
+        if (a.weight_multipliers) RQ_LAUNCH6(1, true, false);
+        else RQ_LAUNCH6(1, false, false);
+    } else if (a.groups_per_fold == 2) {
+        RQ_LAUNCH6(2, false, false);
+    } else {
+        RQ_LAUNCH6(4, false, false);
+    }
 #undef RQ_LAUNCH6
     return hipGetLastError();
 }

@@ -173,3 +173,31 @@ def test_int8_gemm_under_rq_gemm_fp6_0():
     out = subprocess.run([sys.executable, "-u", os.path.join(HERE, "gemm_i8_case.py")], env=env, capture_output=True,
                          text=True, timeout=600)
     assert out.returncode == 0 and "ALL OK" in out.stdout, out.stdout[-3000:] + out.stderr[-2000:]
+
+
+@pytest.mark.parametrize("wgroup", [0, 64], ids=["legacy", "wgroup64"])
+@pytest.mark.parametrize("M,slabs", [(65, True), (200, True), (200, False), (4700, True)])
+def test_several_weights_in_one_launch(oracle, M, slabs, wgroup):
+    """Three weights of one kind whose row tiles (2 + 1 + 4, ragged) are counted through in one launch: all tiles cut
+    along K, the same on a workspace without slabs (whole tiles), and whole rounds with tiles left over (7 x 37 tiles).
+    Outputs with row strides of their own; what lies beside them stays."""
+    K, type_ = 512, rq.TYPE_W4A4
+    ws, bl = [], []
+    for i, N in enumerate([384, 98, 1000]):
+        b, wf = adversarial_weights(oracle, N, K, type_, seed=30 + i, wgroup=wgroup)
+        bl.append(b)
+        ws.append(rq.W4A4Weight(b, type_, DEV))
+    x = adversarial_activations(M, K, type_, wf, seed=M)
+    xd = torch.from_numpy(x).to(DEV)
+    outs = [torch.full((M, w.N + 3 * i), -7.0, dtype=torch.float32, device=DEV) for i, w in enumerate(ws)]
+    # (without slabs: only the cells for 64 tokens' rows behind the activations, as for a call of the fewest bytes)
+    nbytes = rq.fused_workspace_bytes(ws, M) - (0 if slabs else 30 << 20)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    for rep in range(2):   # the second call meets the counters the first one left
+        rq.mul_mat_fused(ws, xd, outs=[o[:, :w.N] for o, w in zip(outs, ws)], workspace=work)
+        torch.cuda.synchronize()
+        for b, w, o in zip(bl, ws, outs):
+            want = oracle.mul_mat(type_, b, x, w.clip)
+            got = o.cpu().numpy()
+            assert bits_equal(got[:, :w.N], want), first_mismatch(got[:, :w.N], want)
+            assert (got[:, w.N:] == -7.0).all()
