@@ -260,6 +260,8 @@ def quantize_act(x, clip, hadamard_=False, n_rot=None):
 # buffers out and takes them back, so concurrent calls have their own and no call keeps any.
 _STAGE_BYTES = 4 << 20
 _STAGES = 3
+# Blocks that fit one buffer have nothing to run beside: they cross through one buffer on the caller's own stream. (The
+# second stream, its events and two more buffers cost 40 us, more than a small tensor's whole conversion.)
 
 
 def _chunks(n, most):
@@ -285,6 +287,12 @@ def _fetch(dev, parts):
     which they are ready), in the order in which they become ready."""
     host = np.empty(dev.numel(), dtype=np.uint8)
     to = torch.from_numpy(host)
+    if len(parts) == 1 and dev.numel() <= _STAGE_BYTES:
+        stage = torch.empty(dev.numel(), dtype=torch.uint8, pin_memory=True)
+        stage.copy_(dev, non_blocking=True)
+        torch.cuda.current_stream().synchronize()
+        to.copy_(stage)
+        return host
     copier = torch.cuda.Stream(dev.device)
     runs = [(a0 + a, a0 + b, ready) for a0, b0, ready in parts for a, b in _chunks(b0 - a0, _STAGE_BYTES)]
     stages = _stages(max(b - a for a, b, _ in runs))
@@ -355,6 +363,14 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
     out = torch.empty((rows, K), dtype=torch.float32, device=dev)
     raw = torch.empty(rows * row, dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
+        if rows * row <= _STAGE_BYTES:
+            if rows:
+                stage = torch.empty(rows * row, dtype=torch.uint8, pin_memory=True)
+                _copy_bytes(stage, blocks.view(np.uint8).reshape(-1))
+                raw.copy_(stage, non_blocking=True)
+            rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr(), rows, K, int(n_rot), out.data_ptr(), K, _stream_ptr())
+            _check(rc, "rq_w4a4_dequantize")
+            return out
         # a run of rows is decoded while the next one travels
         current = torch.cuda.current_stream()
         copier = torch.cuda.Stream()

@@ -196,3 +196,18 @@ def test_conversions_in_several_runs(oracle):
     blocks.flags.writeable = False
     got = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy()
     assert bits_equal(got, rq.dequantize_rows(blocks))
+
+
+@pytest.mark.parametrize("rows", [1, 3639, 3640, 3641])
+def test_conversions_around_one_buffer(oracle, rows):
+    """A tensor whose blocks fit one pinned buffer (3640 rows of 8 blocks, 4 MiB) goes through without the second stream;
+    the last that fits and the first that does not; a read-only array and a writable one."""
+    w = tensor(rows, 2048, 5)
+    got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4)
+    want = oracle.quantize_rows_w(w)
+    assert blocks_equal(got, want), block_diff(got, want)
+    for writable in (True, False):
+        blocks = want.copy()
+        blocks.flags.writeable = writable
+        out = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy()
+        assert bits_equal(out, rq.dequantize_rows(blocks))
