@@ -482,15 +482,18 @@ __device__ __forceinline__ void body64(Ctx &c, Stage &s0, Stage &s1, Stage &s2, 
 // first[w + 1]. (What a launch loses is its end: the tiles beyond whole rounds of the chip, cut along K, and the wait for
 // the last of them. One launch over q + k + v at K = 5120, N = 6144 + 1024 + 1024, 2048 tokens, has 512 tiles, two whole
 // rounds.)
+// (a single weight's launch, SET = false, carries one entry)
+template <bool SET>
 struct TileSet {
-    const float   *s_w[kMaxFused];
-    const uint8_t *kmul[kMaxFused];
-    const int32_t *flags[kMaxFused];
-    float         *y[kMaxFused];
-    int64_t        ldy[kMaxFused];
-    int64_t        N[kMaxFused];
-    int            n_panels[kMaxFused];
-    int            first[kMaxFused];   // unused slots hold the total, so no tile selects them
+    static constexpr int kN = SET ? kMaxFused : 1;
+    const float   *s_w[kN];
+    const uint8_t *kmul[kN];
+    const int32_t *flags[kN];
+    float         *y[kN];
+    int64_t        ldy[kN];
+    int64_t        N[kN];
+    int            n_panels[kN];
+    int            first[kN];   // unused slots hold the total, so no tile selects them
 };
 
 // KFMA (activation groups of 64 only): the form of the kernel for tensors with weight multipliers; see group_units
@@ -498,7 +501,7 @@ struct TileSet {
 // weight's launch would pay 1 % for it)
 template <int GS, bool KFMA, bool SET>
 __global__ void __launch_bounds__(kThreads)
-rq_gemm6_kernel(const TileSet ts, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
+rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
                 const float *__restrict__ u, int M, int Mp, int ng, int n_tok_tiles, int n_tiles, int super_tiles,
                 int n_whole, int parts, int *__restrict__ counters, unsigned long long *__restrict__ slabs) {
     using Stage = StageT<KFMA, SET>;
@@ -542,17 +545,21 @@ rq_gemm6_kernel(const TileSet ts, const uint8_t *__restrict__ act6, const float 
         slot = v - n_whole;
     }
     int wsel = 0;
-    if (SET) {
+    if constexpr (SET) {
         wsel = (row_tile >= ts.first[1]) + (row_tile >= ts.first[2]);
         row_tile -= wsel == 0 ? 0 : wsel == 1 ? ts.first[1] : ts.first[2];   // now of its weight
     }
-    const float *__restrict__ s_w = wsel == 0 ? ts.s_w[0] : wsel == 1 ? ts.s_w[1] : ts.s_w[2];
-    const uint8_t *__restrict__ kmul = wsel == 0 ? ts.kmul[0] : wsel == 1 ? ts.kmul[1] : ts.kmul[2];
-    const int32_t *__restrict__ flags = wsel == 0 ? ts.flags[0] : wsel == 1 ? ts.flags[1] : ts.flags[2];
-    float *__restrict__ y = wsel == 0 ? ts.y[0] : wsel == 1 ? ts.y[1] : ts.y[2];
-    const int64_t ldy = wsel == 0 ? ts.ldy[0] : wsel == 1 ? ts.ldy[1] : ts.ldy[2];
-    const int64_t N = wsel == 0 ? ts.N[0] : wsel == 1 ? ts.N[1] : ts.N[2];
-    const int n_panels = wsel == 0 ? ts.n_panels[0] : wsel == 1 ? ts.n_panels[1] : ts.n_panels[2];
+    auto of_weight = [&](const auto &v) {
+        if constexpr (SET) return wsel == 0 ? v[0] : wsel == 1 ? v[1] : v[2];
+        else return v[0];
+    };
+    const float *__restrict__ s_w = of_weight(ts.s_w);
+    const uint8_t *__restrict__ kmul = of_weight(ts.kmul);
+    const int32_t *__restrict__ flags = of_weight(ts.flags);
+    float *__restrict__ y = of_weight(ts.y);
+    const int64_t ldy = of_weight(ts.ldy);
+    const int64_t N = of_weight(ts.N);
+    const int n_panels = of_weight(ts.n_panels);
     const bool sliced = (int) blockIdx.x >= n_whole;
     // this workgroup's steps (two groups each) of the tile's ng / 2
     const int s_begin = sliced ? (int) ((int64_t) (ng / 2) * part / parts) : 0;
@@ -561,6 +568,10 @@ rq_gemm6_kernel(const TileSet ts, const uint8_t *__restrict__ act6, const float 
     // the fp6 plane's address stands beside the flag word (it is inside the prepared buffer, or, for a weight that was
     // prepared in place, a buffer of its own)
     const uint8_t *w6 = reinterpret_cast<const uint8_t *>((uintptr_t) *reinterpret_cast<const unsigned long long *>(flags + 2));
+    // (read up here, in front of the assembly statements: behind them the compiler takes the word as possibly overwritten
+    // and fetches it with a vector load, whose wait stands for a trip to memory between the set-up and the first group, 0.4
+    // to 1 us of every launch)
+    const bool hask = flags[0] & 1;
     Ctx c;
     c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     c.wr = c.wave & 3;
@@ -627,7 +638,6 @@ rq_gemm6_kernel(const TileSet ts, const uint8_t *__restrict__ act6, const float 
             }
         }
     }
-    const bool hask = flags[0] & 1;
     // fp32 rounding toward minus infinity for the folds (MODE bits 1:0); the MFMA sums are exact in any mode
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2" ::: "memory");
     if (KFMA || hask) {   // (the form for weight multipliers takes every tensor that way: multipliers of 1 where there are none)
@@ -767,6 +777,20 @@ rq_gemm6_kernel(const TileSet ts, const uint8_t *__restrict__ act6, const float 
     }
 }
 
+template <bool SET>
+void set_weight(TileSet<SET> &ts, int slot, const FusedWeights &w, int k, int first) {
+    const PreparedLayout &L = w.L[k];
+    const uint8_t *p = w.prepared[k];
+    ts.s_w[slot] = reinterpret_cast<const float *>(p + L.off_sw);
+    ts.kmul[slot] = p + L.off_kmul;
+    ts.flags[slot] = reinterpret_cast<const int32_t *>(p + L.off_flags);
+    ts.y[slot] = w.y[k];
+    ts.ldy[slot] = w.ldy[k];
+    ts.N[slot] = L.N;
+    ts.n_panels[slot] = L.n_panels;
+    ts.first[slot] = first;
+}
+
 }  // namespace
 
 Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold) {
@@ -806,21 +830,14 @@ Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold) {
 }
 
 hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
-    TileSet ts;
+    TileSet<true> ts;
+    TileSet<false> t1;
     int n_row_tiles = 0;
     for (int i = 0; i < kMaxFused; ++i) {
         const int k = i < a.w.n ? i : a.w.n - 1;   // unused slots repeat the last weight (never selected)
-        const PreparedLayout &L = a.w.L[k];
-        const uint8_t *p = a.w.prepared[k];
-        ts.s_w[i] = reinterpret_cast<const float *>(p + L.off_sw);
-        ts.kmul[i] = p + L.off_kmul;
-        ts.flags[i] = reinterpret_cast<const int32_t *>(p + L.off_flags);
-        ts.y[i] = a.w.y[k];
-        ts.ldy[i] = a.w.ldy[k];
-        ts.N[i] = L.N;
-        ts.n_panels[i] = L.n_panels;
-        ts.first[i] = n_row_tiles;
-        if (i < a.w.n) n_row_tiles += L.n_rtiles;
+        set_weight(ts, i, a.w, k, n_row_tiles);
+        if (i == 0) set_weight(t1, 0, a.w, 0, 0);
+        if (i < a.w.n) n_row_tiles += a.w.L[k].n_rtiles;
     }
     const int ng = a.w.L[0].ng;
     const int n_tok_tiles = a.Mp / kTileTok;
@@ -833,8 +850,8 @@ hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
     const int super_tiles = n_tok_tiles % 4 == 0 && n_row_tiles % 8 == 0;
     const int grid = pl.n_whole + (pl.n_tiles - pl.n_whole) * pl.parts;
     const float *m4 = reinterpret_cast<const float *>(a.act6 + act6_plane_bytes(ng, a.Mp));
-#define RQ_LAUNCH6(GS, KFMA, SET)                                                                                      \
-    hipLaunchKernelGGL((rq_gemm6_kernel<GS, KFMA, SET>), dim3(grid), dim3(kThreads), 0, stream, ts, a.act6, m4, a.u, a.M,  \
+#define RQ_LAUNCH6(GS, KFMA, SET, TS)                                                                                      \
+    hipLaunchKernelGGL((rq_gemm6_kernel<GS, KFMA, SET>), dim3(grid), dim3(kThreads), 0, stream, TS, a.act6, m4, a.u, a.M,  \
                        a.Mp, ng, n_tok_tiles, pl.n_tiles, super_tiles, pl.n_whole, pl.parts,                         \
                        reinterpret_cast<int *>(a.cells),                                                             \
                        reinterpret_cast<unsigned long long *>(reinterpret_cast<uint8_t *>(a.cells) + kGemm6CounterBytes))
@@ -842,15 +859,15 @@ hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
     // right for every tensor)
     if (a.w.n > 1) {
         if (a.groups_per_fold != 1) return hipErrorInvalidValue;   // (wider groups go weight by weight)
-        if (a.weight_multipliers) RQ_LAUNCH6(1, true, true);
-        else RQ_LAUNCH6(1, false, true);
+        if (a.weight_multipliers) RQ_LAUNCH6(1, true, true, ts);
+        else RQ_LAUNCH6(1, false, true, ts);
     } else if (a.groups_per_fold == 1) {
-        if (a.weight_multipliers) RQ_LAUNCH6(1, true, false);
-        else RQ_LAUNCH6(1, false, false);
+        if (a.weight_multipliers) RQ_LAUNCH6(1, true, false, t1);
+        else RQ_LAUNCH6(1, false, false, t1);
     } else if (a.groups_per_fold == 2) {
-        RQ_LAUNCH6(2, false, false);
+        RQ_LAUNCH6(2, false, false, t1);
     } else {
-        RQ_LAUNCH6(4, false, false);
+        RQ_LAUNCH6(4, false, false, t1);
     }
 #undef RQ_LAUNCH6
     return hipGetLastError();
