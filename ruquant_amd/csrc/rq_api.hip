@@ -172,7 +172,7 @@ Path path_of(int64_t M) {
 
 int run_products(int type, int n, const void *const *prepared, int64_t K, const int64_t *N, const float *x,
                  int64_t ldx, int64_t M, float *const *y, const int64_t *ldy, float clip, int64_t n_rot, void *ws,
-                 size_t ws_bytes, hipStream_t stream, int stages = 3) {
+                 size_t ws_bytes, hipStream_t stream, int stages = 3, bool shared = false) {
     if (n < 1 || n > 3 || !prepared || !N || !y || !ldy || !x || !ws) return RQ_E_ARGUMENT;
     int64_t Nmax = 0;
     for (int i = 0; i < n; ++i) {
@@ -269,6 +269,34 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     q.single = fp6 ? 2 : single;
     q.m4 = reinterpret_cast<float *>(wsb + W.off_i8 + act6_plane_bytes((int) (K / kGroup), W.Mp));
     q.mvals = reinterpret_cast<uint8_t *>(wsb + W.off_i8) + (size_t) (K / kGroup) * act_mp * 64;
+    // the weights of launch l of n_launch (1: all of them, n: one each)
+    auto weights_of = [&](int l, int n_launch) {
+        FusedWeights fw;
+        memset(&fw, 0, sizeof fw);
+        fw.n = n_launch == 1 ? n : 1;
+        for (int j = 0; j < fw.n; ++j) {
+            const int i = n_launch == 1 ? j : l;
+            fw.prepared[j] = reinterpret_cast<const uint8_t *>(prepared[i]);
+            fw.L[j] = prepared_layout(K, N[i]);
+            fw.y[j] = y[i];
+            fw.ldy[j] = ldy[i];
+        }
+        return fw;
+    };
+    auto skinny_args = [&](const FusedWeights &fw) {
+        SkinnyArgs g;
+        g.w = fw;
+        g.act8 = wsb + W.off_i8;
+        g.mvals = single ? q.mvals : nullptr;
+        g.u = q.u;
+        g.M = (int) M;
+        g.Mp = act_mp;
+        g.runs_per_group = G / kGroup;
+        g.tot = reinterpret_cast<int32_t *>(wsb + W.off_tot);
+        g.panel0 = 0;
+        g.panels = 0;
+        return g;
+    };
     const float *gemv_x = x;      // what the GEMV quantizes from: the rotated rows, or x itself for W4A4
     int64_t gemv_ldx = ldx;
     if (!gemm) q.G = kGroup;
@@ -289,7 +317,20 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         q.zero_ints = 2 * slots * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
     } else if (path == kPathSkinny) {
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
-        q.zero_ints = 2 * M * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
+        // The cells of the panels that are cut along K. (A shared activation's products come in calls of their own,
+        // with any weight of at most N rows: cells for all of them. One 64-token call, K = 5120, N = 17408, with all
+        // cells cleared: 8.9 MB, by workgroups of which a compute unit holds one or two; 34.5 us, now 33.7.)
+        int64_t cells = 0;
+        if (shared) {
+            cells = M * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
+        } else {
+            const int n_launch = one_launch ? 1 : n;
+            for (int l = 0; l < n_launch; ++l) {
+                const int64_t c = skinny_cells(skinny_args(weights_of(l, n_launch)));
+                if (c > cells) cells = c;
+            }
+        }
+        q.zero_ints = 2 * cells;
     } else if (fp6) {
         // the arrival counters of the tiles the fp6 GEMM cuts along K
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
@@ -315,28 +356,9 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     for (int i = 1; i < n && fuse_gemm; ++i) fuse_gemm = multipliers_noted(prepared[i]) == multipliers_noted(prepared[0]);
     const int n_launch = (path == kPathGemm ? fuse_gemm : one_launch) ? 1 : n;
     for (int l = 0; l < n_launch; ++l) {
-        FusedWeights fw;
-        memset(&fw, 0, sizeof fw);
-        fw.n = n_launch == 1 ? n : 1;
-        for (int j = 0; j < fw.n; ++j) {
-            const int i = n_launch == 1 ? j : l;
-            fw.prepared[j] = reinterpret_cast<const uint8_t *>(prepared[i]);
-            fw.L[j] = prepared_layout(K, N[i]);
-            fw.y[j] = y[i];
-            fw.ldy[j] = ldy[i];
-        }
+        const FusedWeights fw = weights_of(l, n_launch);
         if (path == kPathSkinny) {
-            SkinnyArgs g;
-            g.w = fw;
-            g.act8 = wsb + W.off_i8;
-            g.mvals = single ? q.mvals : nullptr;
-            g.u = q.u;
-            g.M = (int) M;
-            g.Mp = act_mp;
-            g.runs_per_group = G / kGroup;
-            g.tot = reinterpret_cast<int32_t *>(wsb + W.off_tot);
-            g.panel0 = 0;
-            g.panels = 0;
+            const SkinnyArgs g = skinny_args(fw);
             e = launch_skinny(g, stream);
             if (e != hipSuccess) return (int) e;
         } else if (fp6) {
@@ -546,7 +568,7 @@ int rq_w4a4_mul_mat_stages(int type, const void *prepared_dev, int64_t K, int64_
                            size_t workspace_bytes, rq_stream_t stream, int stages) {
     if (stages < 1 || stages > 3) return RQ_E_ARGUMENT;
     return run_products(type, 1, &prepared_dev, K, &N, x_dev, ldx, M, &y_dev, &ldy, clip, n_rot, workspace_dev,
-                        workspace_bytes, (hipStream_t) stream, stages);
+                        workspace_bytes, (hipStream_t) stream, stages, true);
 }
 
 int rq_w4a4_stage_mask(int type, int64_t K, int64_t M, int64_t n_rot) {

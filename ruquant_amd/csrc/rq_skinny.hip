@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(kThreads, TT == 1 ? 4 : (SINGLE && TT == 2) ? 
 rq_skinny_kernel(const WeightSet ws, const uint4 *__restrict__ act8, const uint8_t *__restrict__ mvals,
                  const float *__restrict__ u, int M, int Mp, int gsh,
                  int n_units, int nz,
-                 unsigned long long *__restrict__ cells, int n_rows_pad, int main_panels, int tail_split,
+                 unsigned long long *__restrict__ cells, int cell_rows, int main_panels, int tail_split,
                  int slice_base, int slice_extra, int panel0) {
     constexpr int kTok = TT * 16;
     constexpr int kStride = kTok + 1;             // padded: the epilogue reads a column of this array
@@ -316,7 +316,8 @@ rq_skinny_kernel(const WeightSet ws, const uint4 *__restrict__ act8, const uint8
     // What the epilogue needs from memory is asked for first: loads return in order, so by the time the first group
     // of weights is here these are too, and the tail of the kernel has no trip to memory left but its own stores.
     const int64_t nrow = (int64_t) wpanel * kPanelRows + lane;      // row of its weight
-    const int64_t cell_row = (int64_t) panel * kPanelRows + lane;   // row of the launch (split-K cell)
+    // split-K cell: only the panels that are cut have cells
+    const int64_t cell_row = (int64_t) (panel - main_panels) * kPanelRows + lane;
     const float sw_row = s_w[nrow];                 // rows past N are stored as zero
     float u_tok[kTok / kWaves];
 #pragma unroll
@@ -364,7 +365,7 @@ rq_skinny_kernel(const WeightSet ws, const uint4 *__restrict__ act8, const uint8
         if (t >= M) break;
         int32_t sum = s_tot[lane * kStride + tl];
         if (nks > 1) {
-            unsigned long long *cell = cells + (size_t) t * n_rows_pad + cell_row;
+            unsigned long long *cell = cells + (size_t) t * cell_rows + cell_row;
             const unsigned long long mine = (1ull << 48) + (unsigned long long) (long long) sum;
             const unsigned long long now =
                 __hip_atomic_fetch_add(cell, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine;
@@ -376,25 +377,26 @@ rq_skinny_kernel(const WeightSet ws, const uint4 *__restrict__ act8, const uint8
     }
 }
 
+int token_blocks(int M, int tt) { return (M + tt * 16 - 1) / (tt * 16); }
+
+SkinnyPlan plan_of(const SkinnyArgs &a, int n_panels, int ng, int nz, int gf) {
+    if (a.panels > 0) return SkinnyPlan{ n_panels, 1 };   // whole K per workgroup: no arrival cells
+    return skinny_plan(n_panels, ng, a.M, nz, gf);
+}
+
 template <int TT, bool SINGLE, bool WIDE = false>
 hipError_t launch_tt(const SkinnyArgs &a, hipStream_t stream) {
     const WeightSet ws = make_weight_set(a.w);
     const int n_panels = a.panels > 0 ? a.panels : ws.first[kMaxFused];
-    const int nz = (a.M + TT * 16 - 1) / (TT * 16);
+    const int nz = token_blocks(a.M, TT);
     const int gf = WIDE ? a.runs_per_group : 1, gsh = gf == 4 ? 2 : gf == 2 ? 1 : 0;
     const int n_groups = ws.ng / gf;   // what a slice of K is counted in
-    SkinnyPlan plan;
-    if (a.panels > 0) {   // whole K per workgroup: no arrival cells
-        plan.main_panels = n_panels;
-        plan.tail_split = 1;
-    } else {
-        plan = skinny_plan(n_panels, ws.ng, a.M, nz, gf);
-    }
+    const SkinnyPlan plan = plan_of(a, n_panels, ws.ng, nz, gf);
     const int n_units = plan.main_panels + (n_panels - plan.main_panels) * plan.tail_split;
     const int blocks = (n_units + 7) / 8 * 8 * nz;
     hipLaunchKernelGGL((rq_skinny_kernel<TT, SINGLE, WIDE>), dim3(blocks), dim3(kThreads), 0, stream, ws,
                        reinterpret_cast<const uint4 *>(a.act8), a.mvals, a.u, a.M, a.Mp, gsh, n_units, nz,
-                       reinterpret_cast<unsigned long long *>(a.tot), ws.first[kMaxFused] * kPanelRows,
+                       reinterpret_cast<unsigned long long *>(a.tot), (n_panels - plan.main_panels) * kPanelRows,
                        plan.main_panels, plan.tail_split, n_groups / plan.tail_split, n_groups % plan.tail_split,
                        a.panels > 0 ? a.panel0 : 0);
     return hipGetLastError();
@@ -436,28 +438,47 @@ SkinnyPlan skinny_plan(int n_panels, int ng, int M, int nz, int runs_per_group) 
     return plan;
 }
 
+namespace {
+
+int panels_of(const FusedWeights &w) {
+    int n = 0;
+    for (int i = 0; i < w.n; ++i) n += w.L[i].n_panels;
+    return n;
+}
+
+// token tiles of 16 per wavefront
+int token_tiles(const SkinnyArgs &a) {
+    if (a.panels > 0) return 2;   // the tail of a GEMM launch: blocks of 32 tokens
+    if (a.M <= 16) return 1;
+    // activation groups of 128 / 256 (and the two-plane form): more tokens as blocks of 32
+    if (a.mvals == nullptr || a.runs_per_group > 1) return 2;
+    // 33..64 tokens: one workgroup with four token tiles per wavefront reads the weights once and halves the
+    // workgroup count, two blocks of 32 tokens give twice the workgroups. The former wins on long rows and on
+    // weights with a whole round of panels (K=17408, N=5120, M=64: 22.7 against 26.9 us; K=5120, N=17408: 27.1
+    // against 27.9), the latter on small weights (K=5120, N=5120: 10.9 against 15.8 us).
+    const bool wide = a.w.L[0].ng >= 160 || panels_of(a.w) >= device_compute_units();
+    return a.M > 32 && wide ? 4 : 2;
+}
+
+}  // namespace
+
+// What the activation launch has to clear: every cell a launch over all rows could have is 8.9 MB at N = 17408 and
+// 64 tokens, more than the activations themselves; only the panels beyond whole rounds (16 of 272 there, 0.5 MB) meet
+// in cells.
+int64_t skinny_cells(const SkinnyArgs &a) {
+    const int tt = token_tiles(a), n_panels = panels_of(a.w);
+    const SkinnyPlan plan = plan_of(a, n_panels, a.w.L[0].ng, token_blocks(a.M, tt), a.runs_per_group);
+    return plan.tail_split > 1 ? (int64_t) a.M * (n_panels - plan.main_panels) * kPanelRows : 0;
+}
+
 hipError_t launch_skinny(const SkinnyArgs &a, hipStream_t stream) {
-    constexpr int tt1_max = 16;   // most tokens served with one token tile of 16 per wavefront
-    if (a.panels > 0) return launch_tt<2, false>(a, stream);   // the tail of a GEMM launch: blocks of 32 tokens
-    if (a.mvals != nullptr && a.runs_per_group > 1) {
-        // activation groups of 128 / 256: one or two token tiles per wavefront, more tokens as blocks of 32
-        if (a.M <= 16) return launch_tt<1, true, true>(a, stream);
-        return launch_tt<2, true, true>(a, stream);
+    const int tt = token_tiles(a);
+    if (a.panels > 0 || a.mvals == nullptr) {   // the digit planes
+        return tt == 1 ? launch_tt<1, false>(a, stream) : launch_tt<2, false>(a, stream);
     }
-    if (a.mvals != nullptr) {   // the caller wrote single-plane activations
-        // 33..64 tokens: one workgroup with four token tiles per wavefront reads the weights once and halves the
-        // workgroup count, two blocks of 32 tokens give twice the workgroups. The former wins on long rows and on
-        // weights with a whole round of panels (K=17408, N=5120, M=64: 22.7 against 26.9 us; K=5120, N=17408: 27.1
-        // against 27.9), the latter on small weights (K=5120, N=5120: 10.9 against 15.8 us).
-        int n_panels = 0;
-        for (int i = 0; i < a.w.n; ++i) n_panels += a.w.L[i].n_panels;
-        const bool wide = a.w.L[0].ng >= 160 || n_panels >= device_compute_units();
-        if (a.M > 32 && wide) return launch_tt<4, true>(a, stream);
-        if (a.M <= 16) return launch_tt<1, true>(a, stream);
-        return launch_tt<2, true>(a, stream);
-    }
-    if (a.M <= (tt1_max > 64 ? 64 : tt1_max)) return launch_tt<1, false>(a, stream);
-    return launch_tt<2, false>(a, stream);
+    if (a.runs_per_group > 1) return tt == 1 ? launch_tt<1, true, true>(a, stream) : launch_tt<2, true, true>(a, stream);
+    if (tt == 4) return launch_tt<4, true>(a, stream);
+    return tt == 1 ? launch_tt<1, true>(a, stream) : launch_tt<2, true>(a, stream);
 }
 
 }  // namespace rq

@@ -616,3 +616,29 @@ def test_rows_are_independent_and_calls_repeatable(oracle):
         assert torch.equal(one[0], big[t]), t
     five = rq.mul_mat(W, xd[10:15], workspace=ws)
     assert torch.equal(five, big[10:15])
+
+
+@pytest.mark.parametrize("M,Ns", [(5, [16449]), (33, [16449]), (64, [16384]), (16, [16320, 70]), (40, [4000, 300, 900])])
+@pytest.mark.parametrize("one_launch", [True, False], ids=["one_launch", "launch_each"])
+def test_split_k_cells_in_a_dirty_workspace(oracle, M, Ns, one_launch):
+    """Up to 64 tokens the panels beyond whole rounds of the chip meet in cells of the workspace, and the call clears
+    the cells of those panels only: one such panel, none, a few behind a round, all of them; the weights of a call in one
+    launch, or (cells for the largest alone) in launches that take turns on the same cells. The workspace holds other
+    bytes before each call."""
+    K, type_ = 1024, rq.TYPE_W4A4
+    ws, bl = [], []
+    for i, N in enumerate(Ns):
+        b, wf = adversarial_weights(oracle, N, K, type_, seed=50 + i)
+        bl.append(b)
+        ws.append(rq.W4A4Weight(b, type_, DEV))
+    x = adversarial_activations(M, K, type_, wf, seed=M)
+    xd = torch.from_numpy(x).to(DEV)
+    nbytes = rq.fused_workspace_bytes(ws, M) if one_launch else max(rq.fused_workspace_bytes([w], M) for w in ws)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    for fill in (0xA5, 0x01):
+        work.fill_(fill)
+        outs = rq.mul_mat_fused(ws, xd, workspace=work)
+        torch.cuda.synchronize()
+        for b, w, o in zip(bl, ws, outs):
+            want = oracle.mul_mat(type_, b, x, w.clip)
+            assert bits_equal(o.cpu().numpy(), want), first_mismatch(o.cpu().numpy(), want)
