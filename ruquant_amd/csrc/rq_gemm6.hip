@@ -34,21 +34,9 @@
 
 #pragma clang fp contract(off)
 
-// Timing-only builds (-DRQ6_VARIANT=n, results are wrong): the loop with one ingredient left out, to see what each
-// costs. 1: no fetches; 2: no MFMAs or folds (groups of 128 / 256 only); 3: operands made up in registers instead of
-// read from LDS; 4: no barrier; 5: MFMAs and folds alone (1 + 3 + 4).
-#ifndef RQ6_VARIANT
-#define RQ6_VARIANT 0
-#endif
-
 namespace rq {
 
 namespace {
-
-constexpr bool kWithFetch = RQ6_VARIANT != 1 && RQ6_VARIANT != 5;
-constexpr bool kWithCompute = RQ6_VARIANT != 2;
-constexpr bool kWithLdsReads = RQ6_VARIANT != 3 && RQ6_VARIANT != 5;
-constexpr bool kWithBarrier = RQ6_VARIANT != 4 && RQ6_VARIANT != 5;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -230,12 +218,6 @@ __device__ __forceinline__ void compute(const Ctx &c, const Stage &s, int st, fl
     for (int gi = 0; gi < 2; ++gi) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-#if RQ6_VARIANT == 3 || RQ6_VARIANT == 5
-            for (int e = 0; e < 6; ++e) { A[gi][i][e] = c.lane * (e + gi + 1) + st; B[gi][i][e] = c.lane * (e + i + 3) + st; }
-            m4[gi][i] = 4.0f;
-            asm volatile("" : "+v"(A[gi][i]), "+v"(B[gi][i]));
-            continue;
-#endif
             A[gi][i] = fragment(s, kOffA + gi * kCellsA + (2 * c.wr + i) * (kFrag6 / 16), c.lane);
             B[gi][i] = fragment(s, kOffB + gi * kCellsB + (2 * c.wc + i) * (kFrag6 / 16), c.lane);
             m4[gi][i] = reinterpret_cast<const float *>(&s.cell[kOffM + gi * kCellsM])[64 * c.wc + 32 * i + (c.lane & 31)];
@@ -296,10 +278,10 @@ __device__ __forceinline__ void step(Ctx &c, const Stage &cur, Stage &refill, in
                                      int32_t (&tot)[2][2][16], v16f (&carry)[2][2]) {
     // the loads of steps st + 1 and st + 2 may still be in flight
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoadsPerStep) : "memory");
-    if (kWithBarrier) __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (kWithFetch) fetch(c, refill, st + 3);
-    if (kWithCompute) compute<HASK, GS>(c, cur, st, acc, tot, carry);
+    fetch(c, refill, st + 3);
+    compute<HASK, GS>(c, cur, st, acc, tot, carry);
 }
 
 __device__ __forceinline__ void flush(float (&acc)[2][2][16], int32_t (&tot)[2][2][16]) {
@@ -410,10 +392,6 @@ __device__ __forceinline__ void body64(Ctx &c, Stage &s0, Stage &s1, Stage &s2, 
                                        int32_t (&tot)[2][2][16]) {
     Stage *ring[kRing] = { &s0, &s1, &s2, &s3 };
     Operands X, Y;
-    if (!kWithLdsReads) {
-        for (int i = 0; i < 2; ++i) for (int e = 0; e < 6; ++e) { X.A[i][e] = c.lane * (e + 1); X.B[i][e] = c.lane * (e + i + 3); Y.A[i][e] = c.lane * (e + 7); Y.B[i][e] = c.lane * (e + i + 2); }
-        X.m4[0] = X.m4[1] = Y.m4[0] = Y.m4[1] = 4.0f;
-    }
     v16f P = {};
     float pm = 0.0f;
     // stages 0 and 1 whole, of stage 2 the first three runs: its other two loads and everything after them is dealt
@@ -436,22 +414,20 @@ __device__ __forceinline__ void body64(Ctx &c, Stage &s0, Stage &s1, Stage &s2, 
             const Stage &next = *ring[(j + 1) % kRing];
             Stage &refill2 = *ring[(j + 2) % kRing];
             Stage &refill3 = *ring[(j + 3) % kRing];
-            if (kWithLdsReads) read_operands(c, cur, 1, Y);
+            read_operands(c, cur, 1, Y);
             __builtin_amdgcn_sched_barrier(0);
             group_units<HASK, KFMA>(c, X, c.g0 + 2 * st, *ring[(j + 3) % kRing], 1, cur, 0, P, pm, acc, tot, [&](int un) {
-                if (!kWithFetch) return;
                 if (un == 0) fetch_run(c, refill2, st + 2, 3);
                 if (un == 2) fetch_tail(c, refill2, st + 2);
             });
             // stage st + 1 is whole once every wavefront has seen its own loads of it arrive (those of step st + 2
             // may still be in flight); stage st - 1 is then free for step st + 3
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoadsPerStep) : "memory");
-            if (kWithBarrier) __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            if (kWithLdsReads) read_operands(c, next, 0, X);   // (past the last step: stale cells, never used)
+            read_operands(c, next, 0, X);   // (past the last step: stale cells, never used)
             __builtin_amdgcn_sched_barrier(0);
             group_units<HASK, KFMA>(c, Y, c.g0 + 2 * st + 1, cur, 0, cur, 1, P, pm, acc, tot, [&](int un) {
-                if (!kWithFetch) return;
                 if (un < 3) fetch_run(c, refill3, st + 3, un);
             });
             if (HASK && KFMA) flush(acc, tot);   // (every accumulator has taken two groups' terms since the last one)
