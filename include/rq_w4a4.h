@@ -123,6 +123,16 @@ int rq_w4a4_mul_mat(int type, const void *prepared_dev, int64_t K, int64_t N,
                     float clip, int64_t n_rot,
                     void *workspace_dev, size_t workspace_bytes, rq_stream_t stream);
 
+/* rq_w4a4_mul_mat for a caller that will not run stage 2 of rq_w4a4_mul_mat_stages on this workspace afterwards: same
+ * arguments and results. rq_w4a4_mul_mat clears the split-K cells of all N rows, so that a later stage-2 call finds them
+ * clear whichever of them its plan uses; this call clears only those that it uses itself (5 to 64 tokens; K = 5120,
+ * N = 17408 at 64 tokens: 0.5 instead of 8.9 MB). No counterpart in the reference. */
+int rq_w4a4_mul_mat_once(int type, const void *prepared_dev, int64_t K, int64_t N,
+                         const float *x_dev, int64_t ldx, int64_t M,
+                         float *y_dev, int64_t ldy,
+                         float clip, int64_t n_rot,
+                         void *workspace_dev, size_t workspace_bytes, rq_stream_t stream);
+
 /* rq_w4a4_mul_mat for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): no counterpart in the reference, which takes its scratch from the backend pool.
  * Same arguments and results as rq_w4a4_mul_mat without the workspace: the scratch is a 16 MiB array inside the
@@ -141,8 +151,10 @@ int rq_w4a4_mul_mat_static(int type, const void *prepared_dev, int64_t K, int64_
 /* rq_w4a4_mul_mat in its two stages, for the reference's shared quantized activation (rq_act_cache, P:1996-2023,
  * P:2160-2172): consecutive MUL_MATs of one x (q / k / v, gate / up) that were not fused rotate and quantize x once.
  * stages = 1: activation transform only (Hadamard + quantizer; also clears the split-K cells of N rows);
- * stages = 2: product + epilogue only, on a workspace that a stages-1 or stages-3 call filled for the same type, K, M,
- *             x, clip and n_rot and for at least as many weight rows (cells of more rows were not cleared);
+ * stages = 2: product + epilogue only, on a workspace that an earlier call filled for the same type, K, M, x, clip and
+ *             n_rot and for at least as many weight rows (cells of more rows were not cleared; of a fused call, the
+ *             rows of its largest weight count). Stages 1 and 3, rq_w4a4_mul_mat and rq_w4a4_mul_mat_fused fill;
+ *             rq_w4a4_mul_mat_once and rq_w4a4_mul_mat_fused_once do not;
  * stages = 3: both (identical to rq_w4a4_mul_mat). The workspace must have been zero-filled once when it was
  * allocated if stage 2 is ever used on it with a different N than the filling call. One token on the one-launch
  * decode path has no separate activation stage: stage 1 does nothing there and stage 2 is the whole operator.
@@ -163,6 +175,13 @@ int rq_w4a4_mul_mat_fused(int type, int n, const void *const *prepared_dev, int6
                           float *const *y_dev, const int64_t *ldy,
                           float clip, int64_t n_rot,
                           void *workspace_dev, size_t workspace_bytes, rq_stream_t stream);
+
+/* rq_w4a4_mul_mat_fused with the promise of rq_w4a4_mul_mat_once: no stage-2 call follows on this workspace. */
+int rq_w4a4_mul_mat_fused_once(int type, int n, const void *const *prepared_dev, int64_t K, const int64_t *N,
+                               const float *x_dev, int64_t ldx, int64_t M,
+                               float *const *y_dev, const int64_t *ldy,
+                               float clip, int64_t n_rot,
+                               void *workspace_dev, size_t workspace_bytes, rq_stream_t stream);
 
 /* ---- the activation side on its own (the A4 / A4H from_float of the CPU type traits, P:71-88) ------- */
 
@@ -224,7 +243,9 @@ int rq_w4a4_dequantize(int type, const void *blocks_dev, int64_t rows, int64_t K
 int rq_w4a4_stage_mask(int type, int64_t K, int64_t M, int64_t n_rot);
 
 /* Library version, for the host binding to check: bumped whenever an entry point, an error code or the meaning of an
- * argument changes. A binding built against this header refuses a library that reports another number. */
+ * argument changes. A binding built against this header refuses a library that reports another number. (An entry point
+ * that is only added leaves the number: everything an older binding calls is as it was, and a binding that needs it finds
+ * its symbol missing from an older library.) */
 #define RQ_ABI_VERSION 3
 int rq_w4a4_abi_version(void);
 

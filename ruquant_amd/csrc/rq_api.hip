@@ -170,9 +170,10 @@ Path path_of(int64_t M) {
     return M <= kGemvMax ? kPathGemv : kPathSkinny;
 }
 
+// once: no stage-2 call will use what this call leaves in the workspace
 int run_products(int type, int n, const void *const *prepared, int64_t K, const int64_t *N, const float *x,
                  int64_t ldx, int64_t M, float *const *y, const int64_t *ldy, float clip, int64_t n_rot, void *ws,
-                 size_t ws_bytes, hipStream_t stream, int stages = 3, bool shared = false) {
+                 size_t ws_bytes, hipStream_t stream, int stages = 3, bool once = false) {
     if (n < 1 || n > 3 || !prepared || !N || !y || !ldy || !x || !ws) return RQ_E_ARGUMENT;
     int64_t Nmax = 0;
     for (int i = 0; i < n; ++i) {
@@ -317,11 +318,12 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         q.zero_ints = 2 * slots * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
     } else if (path == kPathSkinny) {
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
-        // The cells of the panels that are cut along K. (A shared activation's products come in calls of their own,
-        // with any weight of at most N rows: cells for all of them. One 64-token call, K = 5120, N = 17408, with all
-        // cells cleared: 8.9 MB, by workgroups of which a compute unit holds one or two; 34.5 us, now 33.7.)
+        // A stage-2 call may follow with any weight of at most N rows, whose plan cuts other panels than this call's:
+        // cells for all rows. A call that is said to be the workspace's only one clears the cells of the panels that it
+        // cuts itself. (One 64-token call, K = 5120, N = 17408: all cells are 8.9 MB, cleared by workgroups of which a
+        // compute unit holds one or two; 34.5 us, 33.7 with the cells of the 16 cut panels alone.)
         int64_t cells = 0;
-        if (shared) {
+        if (!once) {
             cells = M * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
         } else {
             const int n_launch = one_launch ? 1 : n;
@@ -552,6 +554,13 @@ int rq_w4a4_mul_mat(int type, const void *prepared_dev, int64_t K, int64_t N, co
                         workspace_bytes, (hipStream_t) stream);
 }
 
+int rq_w4a4_mul_mat_once(int type, const void *prepared_dev, int64_t K, int64_t N, const float *x_dev, int64_t ldx,
+                         int64_t M, float *y_dev, int64_t ldy, float clip, int64_t n_rot, void *workspace_dev,
+                         size_t workspace_bytes, rq_stream_t stream) {
+    return run_products(type, 1, &prepared_dev, K, &N, x_dev, ldx, M, &y_dev, &ldy, clip, n_rot, workspace_dev,
+                        workspace_bytes, (hipStream_t) stream, 3, true);
+}
+
 int rq_w4a4_mul_mat_static(int type, const void *prepared_dev, int64_t K, int64_t N, const float *x_dev, int64_t ldx,
                            int64_t M, float *y_dev, int64_t ldy, float clip, int64_t n_rot, rq_stream_t stream) {
     if (!shape_ok(type, K, N, M)) return RQ_E_UNSUPPORTED;
@@ -560,7 +569,7 @@ int rq_w4a4_mul_mat_static(int type, const void *prepared_dev, int64_t K, int64_
     void *ws = static_scratch(&e);   // resolved by rq_w4a4_prepare on this device; here only looked up
     if (!ws) return (int) e;
     return run_products(type, 1, &prepared_dev, K, &N, x_dev, ldx, M, &y_dev, &ldy, clip, n_rot, ws,
-                        (size_t) RQ_STATIC_SCRATCH_BYTES, (hipStream_t) stream);
+                        (size_t) RQ_STATIC_SCRATCH_BYTES, (hipStream_t) stream, 3, true);
 }
 
 int rq_w4a4_mul_mat_stages(int type, const void *prepared_dev, int64_t K, int64_t N, const float *x_dev, int64_t ldx,
@@ -568,7 +577,7 @@ int rq_w4a4_mul_mat_stages(int type, const void *prepared_dev, int64_t K, int64_
                            size_t workspace_bytes, rq_stream_t stream, int stages) {
     if (stages < 1 || stages > 3) return RQ_E_ARGUMENT;
     return run_products(type, 1, &prepared_dev, K, &N, x_dev, ldx, M, &y_dev, &ldy, clip, n_rot, workspace_dev,
-                        workspace_bytes, (hipStream_t) stream, stages, true);
+                        workspace_bytes, (hipStream_t) stream, stages);
 }
 
 int rq_w4a4_stage_mask(int type, int64_t K, int64_t M, int64_t n_rot) {
@@ -586,6 +595,14 @@ int rq_w4a4_mul_mat_fused(int type, int n, const void *const *prepared_dev, int6
                           rq_stream_t stream) {
     return run_products(type, n, prepared_dev, K, N, x_dev, ldx, M, y_dev, ldy, clip, n_rot, workspace_dev,
                         workspace_bytes, (hipStream_t) stream);
+}
+
+int rq_w4a4_mul_mat_fused_once(int type, int n, const void *const *prepared_dev, int64_t K, const int64_t *N,
+                               const float *x_dev, int64_t ldx, int64_t M, float *const *y_dev, const int64_t *ldy,
+                               float clip, int64_t n_rot, void *workspace_dev, size_t workspace_bytes,
+                               rq_stream_t stream) {
+    return run_products(type, n, prepared_dev, K, N, x_dev, ldx, M, y_dev, ldy, clip, n_rot, workspace_dev,
+                        workspace_bytes, (hipStream_t) stream, 3, true);
 }
 
 int rq_w4a4_hadamard(const float *x_dev, int64_t ldx, int64_t M, int64_t K, int64_t n_rot, float *out_dev,

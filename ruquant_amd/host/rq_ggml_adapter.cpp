@@ -205,7 +205,7 @@ void ggml_cuda_mul_mat_rq_w4a4_fused(rq_backend_context &ctx, const rq_tensor *c
         c.n_rot = fu0->n_rot;
         c.K = K;
         c.M = M;
-        // (a fused call may have cleared the cells of all its weights; the largest one is what it surely cleared)
+        // (a fused call clears the cells of all its weights' rows, or, on a workspace for the largest, of that one's)
         c.rows_cleared = (Nmax + 63) / 64 * 64;
         c.valid = rc == 0;
     }

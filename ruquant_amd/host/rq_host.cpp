@@ -8,7 +8,9 @@
 // the same x goes through ggml_cuda_rq_w4a4_can_fuse / _fused. With "cache <weights2.bin> <N2> <y2.bin>" the two
 // weights run as separate calls inside one graph evaluation (the second reuses the first's quantized activation),
 // then x is negated in place and a new evaluation runs both again: y.bin / y2.bin hold the results for -x, and
-// <y2.bin>.first the second weight's result of the first evaluation; the JSON carries the hit / miss counts.
+// <y2.bin>.first the second weight's result of the first evaluation; the JSON carries the hit / miss counts. With a
+// fifth extra argument the scratch holds other bytes before each of these evaluations, as after other products ("dirty"),
+// and the first weight's call may be a fused one over both weights ("dirty_fused", the second weight then once more alone).
 #include "rq_ggml_adapter.h"
 
 #include <hip/hip_runtime.h>
@@ -64,7 +66,8 @@ static rq_tensor f32_tensor(int64_t cols, int64_t rows, void *dev) {
 
 int main(int argc, char **argv) {
     if (argc < 8) {
-        fprintf(stderr, "usage: %s type K N M weights.bin x.bin y.bin [iters] [fuse weights2.bin N2 y2.bin]\n", argv[0]);
+        fprintf(stderr, "usage: %s type K N M weights.bin x.bin y.bin [iters] "
+                        "[fuse|cache weights2.bin N2 y2.bin [dirty|dirty_fused]]\n", argv[0]);
         return 2;
     }
     const int type = atoi(argv[1]);
@@ -74,6 +77,8 @@ int main(int argc, char **argv) {
     if (argc > argi && strcmp(argv[argi], "fuse") != 0) iters = atoi(argv[argi++]);
     const bool cache = argc > argi + 3 && strcmp(argv[argi], "cache") == 0;
     const bool fuse = argc > argi + 3 && (strcmp(argv[argi], "fuse") == 0 || cache);
+    const bool dirty_fused = cache && argc > argi + 4 && strcmp(argv[argi + 4], "dirty_fused") == 0;
+    const bool dirty = dirty_fused || (cache && argc > argi + 4 && strcmp(argv[argi + 4], "dirty") == 0);
     const int64_t N2 = fuse ? atoll(argv[argi + 2]) : 0;
 
     int n_dev = 0;
@@ -151,11 +156,28 @@ int main(int argc, char **argv) {
     long long hits_first = 0, misses_first = 0, hits_again = 0, misses_again = 0;
     if (cache) {
         // one graph evaluation, two separate calls of the same x: the second finds x already rotated and quantized
-        ctx.act_hits = ctx.act_misses = 0;
-        ggml_cuda_rq_graph_begin(ctx);
-        ggml_cuda_mul_mat_rq_w4a4(ctx, &w, &x, &y);
-        ggml_cuda_mul_mat_rq_w4a4(ctx, &w2, &x, &y2);
-        CK(hipStreamSynchronize(stream));
+        auto evaluate = [&]() {
+            ctx.act_hits = ctx.act_misses = 0;
+            if (dirty) {
+                CK(hipMemset(ctx.scratch, 0xA5, ctx.scratch_bytes));
+                CK(hipDeviceSynchronize());
+            }
+            ggml_cuda_rq_graph_begin(ctx);
+            if (dirty_fused) {
+                const rq_tensor *ws[2] = { &w, &w2 };
+                rq_tensor *ds[2] = { &y, &y2 };
+                ggml_cuda_mul_mat_rq_w4a4_fused(ctx, ws, ds, 2, &x);
+                CK(hipStreamSynchronize(stream));
+                CK(hipMemset(y2d, 0xFF, (size_t) M * N2 * 4));   // what the second call leaves out shows
+                CK(hipDeviceSynchronize());
+            } else {
+                ggml_cuda_mul_mat_rq_w4a4(ctx, &w, &x, &y);
+            }
+            ggml_cuda_mul_mat_rq_w4a4(ctx, &w2, &x, &y2);
+            CK(hipStreamSynchronize(stream));
+            return 0;
+        };
+        if (evaluate()) return 1;
         hits_first = ctx.act_hits;
         misses_first = ctx.act_misses;
         {
@@ -170,11 +192,7 @@ int main(int argc, char **argv) {
         float *xf = reinterpret_cast<float *>(xh.data());
         for (size_t i = 0; i < (size_t) M * K; ++i) xf[i] = -xf[i];
         CK(hipMemcpy(xd, xh.data(), x_bytes, hipMemcpyHostToDevice));
-        ctx.act_hits = ctx.act_misses = 0;
-        ggml_cuda_rq_graph_begin(ctx);
-        ggml_cuda_mul_mat_rq_w4a4(ctx, &w, &x, &y);
-        ggml_cuda_mul_mat_rq_w4a4(ctx, &w2, &x, &y2);
-        CK(hipStreamSynchronize(stream));
+        if (evaluate()) return 1;
         hits_again = ctx.act_hits;
         misses_again = ctx.act_misses;
         iters = 0;

@@ -82,6 +82,9 @@ PROTOTYPES = {
                                             ctypes.c_void_p]),
 }
 
+for _name in ("rq_w4a4_mul_mat", "rq_w4a4_mul_mat_fused"):
+    PROTOTYPES[_name + "_once"] = PROTOTYPES[_name]   # the same arguments
+
 
 def load_library():
     """Returns the ctypes handle of librq_w4a4.so; raises LibraryMissing when it has not been built."""
@@ -101,7 +104,10 @@ def load_library():
             raise LibraryMissing("%s reports ABI version %s, this binding is written for %d: rebuild it with `make -C %s`"
                                  % (LIB_PATH, version, ABI_VERSION, CSRC))
         for name, (res, args) in PROTOTYPES.items():
-            fn = getattr(L, name)
+            try:
+                fn = getattr(L, name)
+            except AttributeError:
+                raise LibraryMissing("%s has no %s: rebuild it with `make -C %s`" % (LIB_PATH, name, CSRC)) from None
             fn.restype = res
             fn.argtypes = args
         _lib = L

@@ -134,7 +134,8 @@ class W4A4Weight:
 
 
 def mul_mat(weight, x, out=None, workspace=None, clip=None):
-    """y[M, N] = x[M, K] . W^T, bit-identical to the ggml-cpu W4A4 / W4A4H MUL_MAT."""
+    """y[M, N] = x[M, K] . W^T, bit-identical to the ggml-cpu W4A4 / W4A4H MUL_MAT. The workspace holds nothing for later
+    calls afterwards (SharedActivation fills one that does)."""
     # (the single product's own entry point: no argument arrays to build. With the device and stream handled as in
     # _on_device_of the host takes 5 us for a one-token call instead of 11.7 us, less than the kernel)
     L = load_library()
@@ -148,7 +149,7 @@ def mul_mat(weight, x, out=None, workspace=None, clip=None):
         workspace = _device_bytes(fused_workspace_bytes([weight], M), x.device)
     ldx = x.stride(0) if M > 1 else K
     ldy = out.stride(0) if out.shape[0] > 1 else out.shape[1]
-    rc = _on_device_of(x, L.rq_w4a4_mul_mat, weight.type, weight.prepared.data_ptr(), K, N, x.data_ptr(), ldx, M,
+    rc = _on_device_of(x, L.rq_w4a4_mul_mat_once, weight.type, weight.prepared.data_ptr(), K, N, x.data_ptr(), ldx, M,
                        out.data_ptr(), ldy, weight.clip if clip is None else clip, max(weight.n_rot, 0),
                        workspace.data_ptr(), workspace.numel())
     if rc != 0:
@@ -166,7 +167,8 @@ def fused_workspace_bytes(weights, M):
 
 
 def mul_mat_fused(weights, x, outs=None, workspace=None, clip=None):
-    """Up to three weights of one type, K, clip and rotation length against the same activations."""
+    """Up to three weights of one type, K, clip and rotation length against the same activations. As after mul_mat, the
+    workspace holds nothing for later calls."""
     L = load_library()
     w0 = weights[0]
     assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and x.stride(1) == 1
@@ -185,7 +187,7 @@ def mul_mat_fused(weights, x, outs=None, workspace=None, clip=None):
     Ns = (ctypes.c_int64 * n)(*[w.N for w in weights])
     ldys = (ctypes.c_int64 * n)(*[o.stride(0) if o.shape[0] > 1 else o.shape[1] for o in outs])
     ldx = x.stride(0) if M > 1 else K
-    rc = _on_device_of(x, L.rq_w4a4_mul_mat_fused, w0.type, n, prepared, K, Ns, x.data_ptr(), ldx, M, ys, ldys,
+    rc = _on_device_of(x, L.rq_w4a4_mul_mat_fused_once, w0.type, n, prepared, K, Ns, x.data_ptr(), ldx, M, ys, ldys,
                        w0.clip if clip is None else clip, max(w0.n_rot, 0), workspace.data_ptr(), workspace.numel())
     _check(rc, "rq_w4a4_mul_mat")
     return outs

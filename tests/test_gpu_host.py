@@ -86,6 +86,75 @@ def test_host_shares_the_quantized_activation_between_separate_calls(oracle, tmp
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,N2,first", [(64, 6144, 1024, "dirty"), (16, 10240, 6144, "dirty"), (5, 16384, 1024, "dirty"),
+                                          (40, 6144, 1024, "dirty_fused"), (16, 17408, 10240, "dirty_fused")])
+def test_host_shares_the_activation_in_a_used_scratch(oracle, tmp_path, M, N, N2, first):
+    """The scratch is shared by all products, so where the split-K cells of one lie, another has left its activations:
+    the call that makes the activation must clear the cells of every weight that may use it, not only those of the panels
+    it cuts itself. q -> k at 64 tokens (q cuts no panel, k all of them), feed-forward widths, a fused call first."""
+    type_, K = rq.TYPE_W4A4H, 5120
+    b1 = synth.random_weight_blocks(N, K, 61, type_, clip=0.9)
+    b2 = synth.random_weight_blocks(N2, K, 62, type_, clip=0.9)
+    x = synth.activations("outlier_channels", M, K, 63)
+    b2.tofile(tmp_path / "w2.bin")
+    r, y = _run(tmp_path, type_, K, N, M, b1, x, extra=("cache", tmp_path / "w2.bin", N2, tmp_path / "y2.bin", first))
+    assert r.returncode == 0, r.stderr
+    info = json.loads(r.stdout.strip().splitlines()[-1])
+    assert (info["act_hits_first"], info["act_misses_first"]) == (1, 1)
+    assert (info["act_hits_again"], info["act_misses_again"]) == (1, 1)
+    c = float(np.float32(0.9))
+    y2_first = np.fromfile(str(tmp_path / "y2.bin") + ".first", dtype=np.float32).reshape(M, N2)
+    y2 = np.fromfile(tmp_path / "y2.bin", dtype=np.float32).reshape(M, N2)
+    for got, w, xs in ((y2_first, b2, x), (y, b1, -x), (y2, b2, -x)):
+        want = oracle.mul_mat(type_, w, xs, c, n_rot=K)
+        assert bits_equal(got, want), first_mismatch(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fill", ["mul_mat", "fused", "stage 1", "stage 3"])
+@pytest.mark.parametrize("type_,K,M,N,N2", [(rq.TYPE_W4A4H, 5120, 64, 6144, 1024), (rq.TYPE_W4A4, 5120, 33, 4096, 300),
+                                            (rq.TYPE_W4A4H, 17408, 16, 4096, 1024), (rq.TYPE_W4A4, 1024, 5, 16449, 70),
+                                            (rq.TYPE_W4A4, 1024, 4, 2000, 70), (rq.TYPE_W4A4, 1024, 70, 2000, 70)])
+def test_every_filling_call_clears_for_stage_2(oracle, type_, K, M, N, N2, fill):
+    """Stage 2 of rq_w4a4_mul_mat_stages runs on the workspace of any earlier call of the same x with at least as many
+    weight rows: a plain product, a fused one, stage 1 or both stages. The workspace holds other bytes before that."""
+    import ctypes
+    import torch
+    dev = "cuda:0"
+    n_rot = K if type_ == rq.TYPE_W4A4H else 0
+    b, x = {}, synth.activations("student_t4", M, K, 70 + M)
+    W = {}
+    for n in (N, N2):
+        b[n] = synth.random_weight_blocks(n, K, n, type_)
+        W[n] = rq.W4A4Weight(b[n], type_, dev)
+    L = rq.load_library()
+    xd = torch.from_numpy(x).to(dev)
+    work = torch.full((rq.fused_workspace_bytes([W[N], W[N2]], M),), 0xA5, dtype=torch.uint8, device=dev)
+    y = {n: torch.full((M, n), float("nan"), dtype=torch.float32, device=dev) for n in (N, N2)}
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    tail = (1.0, n_rot, work.data_ptr(), work.numel(), st)
+    one = (type_, W[N].prepared.data_ptr(), K, N, xd.data_ptr(), K, M, y[N].data_ptr(), N) + tail
+    if fill == "mul_mat":
+        rc = L.rq_w4a4_mul_mat(*one)
+    elif fill == "fused":
+        rc = L.rq_w4a4_mul_mat_fused(type_, 2, (ctypes.c_void_p * 2)(*[W[n].prepared.data_ptr() for n in (N, N2)]), K,
+                                     (ctypes.c_int64 * 2)(N, N2), xd.data_ptr(), K, M,
+                                     (ctypes.c_void_p * 2)(*[y[n].data_ptr() for n in (N, N2)]),
+                                     (ctypes.c_int64 * 2)(N, N2), *tail)
+    else:
+        rc = L.rq_w4a4_mul_mat_stages(*one, int(fill[-1]))
+    assert rc == 0
+    y[N2].fill_(float("nan"))
+    again = (type_, W[N2].prepared.data_ptr(), K, N2, xd.data_ptr(), K, M, y[N2].data_ptr(), N2) + tail
+    assert L.rq_w4a4_mul_mat_stages(*again, 2) == 0
+    assert L.rq_w4a4_mul_mat_stages(*one, 2) == 0     # (the filling weight once more: the cells were left zero)
+    torch.cuda.synchronize()
+    for n in (N2, N):
+        got, want = y[n].cpu().numpy(), oracle.mul_mat(type_, b[n], x, 1.0, n_rot=n_rot)
+        assert bits_equal(got, want), first_mismatch(got, want)
+
+
+@pytest.mark.gpu
 def test_host_reports_unsupported_shape(tmp_path):
     # K with no Hadamard factorization: the backend declines, ggml would fall back to the CPU
     type_, K, N, M = rq.TYPE_W4A4H, 7 * 256, 64, 1
