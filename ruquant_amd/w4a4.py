@@ -272,8 +272,13 @@ def _chunks(n, most):
     return [(n * i // k, n * (i + 1) // k) for i in range(k)]
 
 
+def _pinned(nbytes):
+    # (host memory whatever torch's default device is)
+    return torch.empty(nbytes, dtype=torch.uint8, device="cpu", pin_memory=True)
+
+
 def _stages(nbytes):
-    return [torch.empty(nbytes, dtype=torch.uint8, pin_memory=True) for _ in range(_STAGES)]
+    return [_pinned(nbytes) for _ in range(_STAGES)]
 
 
 def _copy_bytes(pinned, src):
@@ -290,7 +295,7 @@ def _fetch(dev, parts):
     host = np.empty(dev.numel(), dtype=np.uint8)
     to = torch.from_numpy(host)
     if len(parts) == 1 and dev.numel() <= _STAGE_BYTES:
-        stage = torch.empty(dev.numel(), dtype=torch.uint8, pin_memory=True)
+        stage = _pinned(dev.numel())
         stage.copy_(dev, non_blocking=True)
         torch.cuda.current_stream().synchronize()
         to.copy_(stage)
@@ -367,7 +372,7 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
     with torch.cuda.device(dev):
         if rows * row <= _STAGE_BYTES:
             if rows:
-                stage = torch.empty(rows * row, dtype=torch.uint8, pin_memory=True)
+                stage = _pinned(rows * row)
                 _copy_bytes(stage, blocks.view(np.uint8).reshape(-1))
                 raw.copy_(stage, non_blocking=True)
             rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr(), rows, K, int(n_rot), out.data_ptr(), K, _stream_ptr())

@@ -211,3 +211,17 @@ def test_conversions_around_one_buffer(oracle, rows):
         blocks.flags.writeable = writable
         out = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy()
         assert bits_equal(out, rq.dequantize_rows(blocks))
+
+
+@pytest.mark.parametrize("rows", [200, 30001])
+def test_conversions_under_a_default_device(oracle, rows):
+    """A program may have made the GPU torch's default device: the conversions' host buffers stay on the host (one
+    buffer; several)."""
+    w = tensor(200, 256, 9)
+    want = oracle.quantize_rows_w(w)
+    blocks = np.tile(want, (rows // 200 + 1, 4))[:rows]
+    with torch.device(DEV):
+        got = rq.quantize_weights(torch.from_numpy(np.tile(w, (rows // 200 + 1, 1))[:rows]).to(DEV), rq.TYPE_W4A4)
+        out = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV)
+    assert blocks_equal(got, np.tile(want, (rows // 200 + 1, 1))[:rows])
+    assert bits_equal(out.cpu().numpy(), rq.dequantize_rows(blocks))
