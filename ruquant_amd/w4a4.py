@@ -281,6 +281,12 @@ def _stages(nbytes):
     return [_pinned(nbytes) for _ in range(_STAGES)]
 
 
+def _refuse_capture():
+    """A graph replays a copy from the pinned buffer's address, and the buffer is another call's by then."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RqError("conversions read and write host memory: not under graph capture")
+
+
 def _copy_bytes(pinned, src):
     """numpy bytes into the head of a pinned tensor (torch's copy uses several threads; it takes writable arrays only)"""
     if src.flags.writeable:
@@ -344,6 +350,7 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
     ldw = w.stride(0) if N > 1 else K
     parts = []
     with torch.cuda.device(w.device):
+        _refuse_capture()
         for a, b in runs:
             rc = L.rq_w4a4_quantize_weights(int(type_), w.data_ptr() + 4 * ldw * a, ldw, b - a, K, n_rot, int(wgroup),
                                             out.data_ptr() + row * a, ws.data_ptr(), ws.numel(), _stream_ptr())
@@ -370,6 +377,7 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
     out = torch.empty((rows, K), dtype=torch.float32, device=dev)
     raw = torch.empty(rows * row, dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
+        _refuse_capture()
         if rows * row <= _STAGE_BYTES:
             if rows:
                 stage = _pinned(rows * row)

@@ -225,3 +225,18 @@ def test_conversions_under_a_default_device(oracle, rows):
         out = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV)
     assert blocks_equal(got, np.tile(want, (rows // 200 + 1, 1))[:rows])
     assert bits_equal(out.cpu().numpy(), rq.dequantize_rows(blocks))
+
+
+@pytest.mark.parametrize("rows", [200, 9000])
+def test_conversions_are_refused_under_capture(rows):
+    """A captured conversion would replay a copy of whatever its host buffer holds by then: it is refused (one buffer;
+    several), and works again outside."""
+    w = torch.randn((rows, 1024), dtype=torch.float32, device=DEV)
+    blocks = rq.quantize_weights(w, rq.TYPE_W4A4)
+    want = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV)
+    torch.cuda.synchronize()
+    for convert in (lambda: rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV), lambda: rq.quantize_weights(w, rq.TYPE_W4A4)):
+        with pytest.raises(rq.RqError, match="capture"):
+            with torch.cuda.graph(torch.cuda.CUDAGraph()):
+                convert()
+    assert torch.equal(rq.dequantize(rq.quantize_weights(w, rq.TYPE_W4A4), rq.TYPE_W4A4, device=DEV), want)
