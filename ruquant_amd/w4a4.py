@@ -9,6 +9,7 @@ ggml_cuda_mul_mat_rq_w4a4_fused. A ``W4A4Weight`` plays the part of the ggml wei
 torch owns device memory and the stream; every computation happens inside librq_w4a4.so.
 """
 import ctypes
+import threading
 
 import numpy as np
 import torch
@@ -281,6 +282,26 @@ def _stages(nbytes):
     return [_pinned(nbytes) for _ in range(_STAGES)]
 
 
+# A stream's first work costs 0.2 ms, and 2.9 ms while it gets a hardware queue of its own (a few per process), so a
+# conversion in several runs does not take another of torch's streams each time but keeps the one that its thread used
+# beside the same current stream. (Not one for all: copies wait for the work in front of them on the current stream,
+# and would make another stream's conversion wait for it too.)
+_copiers = threading.local()
+_COPIERS = 8   # per thread, the latest ones
+
+
+def _copier(current):
+    kept = _copiers.__dict__.setdefault("streams", {})
+    key = (current.device_index, current.cuda_stream)
+    stream = kept.pop(key, None)
+    if stream is None:
+        stream = torch.cuda.Stream(current.device)
+        if len(kept) >= _COPIERS:
+            del kept[next(iter(kept))]
+    kept[key] = stream   # (the latest at the end)
+    return stream
+
+
 def _refuse_capture():
     """A graph replays a copy from the pinned buffer's address, and the buffer is another call's by then."""
     if torch.cuda.is_current_stream_capturing():
@@ -306,7 +327,7 @@ def _fetch(dev, parts):
         torch.cuda.current_stream().synchronize()
         to.copy_(stage)
         return host
-    copier = torch.cuda.Stream(dev.device)
+    copier = _copier(torch.cuda.current_stream(dev.device))
     runs = [(a0 + a, a0 + b, ready) for a0, b0, ready in parts for a, b in _chunks(b0 - a0, _STAGE_BYTES)]
     stages = _stages(max(b - a for a, b, _ in runs))
     done = [None] * len(runs)
@@ -388,7 +409,7 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
             return out
         # a run of rows is decoded while the next one travels
         current = torch.cuda.current_stream()
-        copier = torch.cuda.Stream()
+        copier = _copier(current)
         copier.wait_stream(current)   # (the memory of `raw` may still be in use by work in front of this call)
         runs = _chunks(rows, max(1, _STAGE_BYTES // max(row, 1)))
         host = blocks.view(np.uint8).reshape(-1)

@@ -1,10 +1,13 @@
 """GPU parity of the weight-side quantizer and the dequantizers (the types' from_float_ref / to_float, patch lines
 2507-2580, 2681-2710, 2738-2773) against the CPU oracle: every byte of every block, every bit of every float."""
+import threading
+
 import numpy as np
 import pytest
 import torch
 
 import ruquant_amd as rq
+from ruquant_amd import w4a4
 from tests.gpu_util import bits_equal, first_mismatch
 
 pytestmark = pytest.mark.gpu
@@ -240,3 +243,39 @@ def test_conversions_are_refused_under_capture(rows):
             with torch.cuda.graph(torch.cuda.CUDAGraph()):
                 convert()
     assert torch.equal(rq.dequantize(rq.quantize_weights(w, rq.TYPE_W4A4), rq.TYPE_W4A4, device=DEV), want)
+
+
+def test_conversions_keep_their_second_stream():
+    """Conversions in several runs keep the stream that their copies go to (a new one costs milliseconds at its first
+    work): one per thread and current stream, a bounded number of them; the blocks are right on all of them."""
+    w = torch.randn((9000, 1024), dtype=torch.float32, device=DEV)   # 5.2 MB of blocks
+    blocks = rq.quantize_weights(w, rq.TYPE_W4A4)
+    want = rq.dequantize_rows(blocks)
+    kept = w4a4._copiers.streams
+    n = len(kept)
+    before = dict(kept)
+    for _ in range(3):
+        assert blocks_equal(rq.quantize_weights(w, rq.TYPE_W4A4), blocks)
+        assert bits_equal(rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy(), want)
+    assert w4a4._copiers.streams == before and len(kept) == n
+    torch.cuda.synchronize()
+    for _ in range(2 * w4a4._COPIERS):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            assert bits_equal(rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy(), want)
+    assert len(w4a4._copiers.streams) == w4a4._COPIERS
+
+    seen, ok = [], []
+
+    def other():
+        for _ in range(5):
+            ok.append(blocks_equal(rq.quantize_weights(w, rq.TYPE_W4A4), blocks))
+            ok.append(bits_equal(rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy(), want))
+        seen.append(list(w4a4._copiers.streams.values()))
+
+    threads = [threading.Thread(target=other) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(ok) == 20 and all(ok)
+    assert [len(s) for s in seen] == [1, 1] and seen[0][0] is not seen[1][0]
