@@ -37,7 +37,10 @@ def _stream_ptr():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# the current stream's handle as a number (a torch without a GPU backend does not have the call, and runs this package's
+# tools for block files all the same)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _on_device_of(x, fn, *args):

@@ -54,6 +54,22 @@ def test_stage_mask_is_a_host_query():
     assert L.rq_w4a4_stage_mask(rq.TYPE_W4A4H, 5120, 1, 1000) == 0
 
 
+def test_package_imports_without_torch_gpu_internals():
+    """The call that reads a stream's handle as a number is one of torch's internals: without it the package imports and
+    its host functions work, and the handle comes from the Stream object."""
+    code = ("import torch\n"
+            "torch.randn(2)\n"
+            "del torch._C._cuda_getCurrentRawStream\n"
+            "import ruquant_amd as rq\n"
+            "from ruquant_amd import w4a4\n"
+            "torch.cuda.current_stream = lambda index: type('S', (), {'cuda_stream': 40 + index})\n"
+            "assert w4a4._raw_stream(2) == 42\n"
+            "assert rq.hadamard_factor(5120) == (20, 256)\n"
+            "print('ok')\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stderr[-2000:]
+
+
 def test_library_is_in_tree():
     assert os.path.exists(LIB_PATH) and LIB_PATH.startswith(ROOT)
 
