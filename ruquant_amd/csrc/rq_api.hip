@@ -356,6 +356,8 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     // two whole rounds of tiles)
     bool fuse_gemm = fp6 && G == kGroup;
     for (int i = 1; i < n && fuse_gemm; ++i) fuse_gemm = multipliers_noted(prepared[i]) == multipliers_noted(prepared[0]);
+    // (without room for slabs no tile is cut, and one launch never has more rounds)
+    if (fuse_gemm && n > 1 && have_slabs) fuse_gemm = gemm6_one_launch(weights_of(0, 1), M, multipliers_noted(prepared[0]));
     const int n_launch = (path == kPathGemm ? fuse_gemm : one_launch) ? 1 : n;
     for (int l = 0; l < n_launch; ++l) {
         const FusedWeights fw = weights_of(l, n_launch);

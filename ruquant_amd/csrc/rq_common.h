@@ -295,6 +295,8 @@ struct Gemm6Plan {
     size_t cell_bytes;
 };
 Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold);
+// whether one launch over all these weights (activation groups of 64) is not slower than one each
+bool gemm6_one_launch(const FusedWeights &w, int64_t M, bool weight_multipliers);
 
 // up to 64 tokens: MFMA arithmetic on a GEMV-shaped weight stream; same operands as the GEMM plus the split-K cells
 struct SkinnyArgs {

@@ -805,6 +805,37 @@ Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold) {
     return pl;
 }
 
+namespace {
+
+// Microseconds of a launch by its plan: a round of whole tiles and, behind it, the slices of the tiles that are cut, by
+// steps of two groups. Fitted to 112 sets of two and three weights (K = 2560 to 32768, 5 to 750 tiles), in one launch and
+// in one each; it gives the ratio of the two within 7 % where that is near 1.
+double launch_price(int n_row_tiles, int64_t M, int ng, bool weight_multipliers) {
+    const Gemm6Plan pl = gemm6_plan(n_row_tiles, M, ng, 1);
+    const int steps = ng / 2;
+    const int rounds = (pl.n_whole + kPlanUnits - 1) / kPlanUnits;
+    const double whole = weight_multipliers ? 5.8 + 1.53 * steps : 7.4 + 0.72 * steps;
+    const int slice = (steps + pl.parts - 1) / pl.parts;
+    const double cut = weight_multipliers ? 11.5 + 1.56 * slice + 0.8 * (pl.parts - 1) : 12.3 + 0.85 * slice + 1.1 * (pl.parts - 1);
+    return rounds * whole + (pl.parts > 1 ? cut : 0.0);
+}
+
+}  // namespace
+
+// One launch has at most the rounds of all the separate ones, but what it has left over may be too many tiles to cut (more
+// than half a round), where each weight's own tiles can be. With long rows that is the greater loss: K = 17408,
+// N = 4134 + 2216, 525 tokens (85 + 45 tiles) 123.4 us in one launch, 116.4 in two; K = 32768, 66 + 82 tiles 204 and 196.
+// The other way round K = 5120, N = 6144 + 1024 + 1024, 512 tokens is 40 and 79 us. (3 % apart is what the prices tell.)
+bool gemm6_one_launch(const FusedWeights &w, int64_t M, bool weight_multipliers) {
+    int n_row_tiles = 0;
+    double each = 0.0;
+    for (int i = 0; i < w.n; ++i) {
+        n_row_tiles += w.L[i].n_rtiles;
+        each += launch_price(w.L[i].n_rtiles, M, w.L[i].ng, weight_multipliers);
+    }
+    return launch_price(n_row_tiles, M, w.L[0].ng, weight_multipliers) <= 1.03 * each;
+}
+
 hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
     TileSet<true> ts;
     TileSet<false> t1;

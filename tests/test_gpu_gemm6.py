@@ -1,6 +1,7 @@
 """The wide-batch product kernel on the fp6 MFMA (rq_gemm6.hip): launches made of whole tiles and of tiles cut along
 K, compared bit for bit with the oracle; and the int8 MFMA kernel it replaced, which RQ_GEMM_FP6=0 still selects, in a
 child process (the variable is read once per process)."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -201,3 +202,33 @@ def test_several_weights_in_one_launch(oracle, M, slabs, wgroup):
             got = o.cpu().numpy()
             assert bits_equal(got[:, :w.N], want), first_mismatch(got[:, :w.N], want)
             assert (got[:, w.N:] == -7.0).all()
+
+
+def _graph_nodes(call):
+    """kernel launches of one call: nodes of the graph that captures it"""
+    call()
+    torch.cuda.synchronize()
+    with open("/proc/self/maps") as f:   # (the copy that torch runs on)
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        call()
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("K,Ns,M,launches", [(17408, (4134, 2216), 525, 2), (17408, (10029, 6404), 234, 2),
+                                             (17408, (8192, 16384), 256, 1), (5120, (4134, 2216), 525, 1),
+                                             (5120, (6144, 1024, 1024), 512, 1)])
+def test_one_launch_only_where_it_is_not_slower(K, Ns, M, launches):
+    """Weights whose tiles can each be cut along K but not together (85 + 45 of 256, long rows) keep their own launches;
+    either way the bits are those of the separate products."""
+    type_ = rq.TYPE_W4A4
+    ws = [rq.W4A4Weight(synth.random_weight_blocks(N, K, i, type_), type_, DEV) for i, N in enumerate(Ns)]
+    x = torch.from_numpy(synth.activations("student_t4", M, K, 5)).to(DEV)
+    outs = [torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV) for N in Ns]
+    work = torch.empty(rq.fused_workspace_bytes(ws, M), dtype=torch.uint8, device=DEV)
+    assert _graph_nodes(lambda: rq.mul_mat_fused(ws, x, outs=outs, workspace=work)) == 1 + launches
+    for w, o in zip(ws, outs):
+        assert torch.equal(o, rq.mul_mat(w, x))
