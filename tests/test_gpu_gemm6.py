@@ -179,9 +179,9 @@ def test_int8_gemm_under_rq_gemm_fp6_0():
 @pytest.mark.parametrize("wgroup", [0, 64], ids=["legacy", "wgroup64"])
 @pytest.mark.parametrize("M,slabs", [(65, True), (200, True), (200, False), (4700, True)])
 def test_several_weights_in_one_launch(oracle, M, slabs, wgroup):
-    """Three weights of one kind whose row tiles (2 + 1 + 4, ragged) are counted through in one launch: all tiles cut
-    along K, the same on a workspace without slabs (whole tiles), and whole rounds with tiles left over (7 x 37 tiles).
-    Outputs with row strides of their own; what lies beside them stays."""
+    """Three weights of one kind whose row tiles (2 + 1 + 4, ragged) are counted through in one launch, rows too short to
+    be cut along K: one and two token tiles, a workspace without slabs, and a whole round with tiles left over (7 x 37
+    tiles). Outputs with row strides of their own; what lies beside them stays."""
     K, type_ = 512, rq.TYPE_W4A4
     ws, bl = [], []
     for i, N in enumerate([384, 98, 1000]):
@@ -232,3 +232,38 @@ def test_one_launch_only_where_it_is_not_slower(K, Ns, M, launches):
     assert _graph_nodes(lambda: rq.mul_mat_fused(ws, x, outs=outs, workspace=work)) == 1 + launches
     for w, o in zip(ws, outs):
         assert torch.equal(o, rq.mul_mat(w, x))
+
+
+@pytest.mark.parametrize("K,M,Ns,wgroups,moved,launches", [
+    (2560, 512, (500, 200, 1200), (0, 0, 0), False, 1),        # 2 + 1 + 5 row tiles: super-tiles over weights, all cut
+    (512, 4096, (500, 200, 1200), (256, 256, 256), False, 1),  # the same, one whole round
+    (2560, 200, (1000, 700), (64, 64), False, 1),              # two weights: the third slot selects nothing
+    (2560, 200, (384, 98, 1000), (64, 0, 64), False, 3),       # with and without multipliers: a launch each
+    (2560, 200, (384, 98, 1000), (64, 256, 0), True, 1)],      # copies the launcher knows nothing of: folds per tile
+    ids=["super_tiles_cut", "super_tiles_whole", "two_weights", "both_kinds", "unknown_addresses"])
+def test_sets_of_weights(oracle, K, M, Ns, wgroups, moved, launches):
+    """Sets whose tiles are cut, whole and in super-tiles that straddle weights, against the oracle, with outputs of their
+    own row strides."""
+    type_ = rq.TYPE_W4A4
+    ws, bl, kept = [], [], []
+    for i, (N, g) in enumerate(zip(Ns, wgroups)):
+        b, wf = adversarial_weights(oracle, N, K, type_, seed=60 + i, wgroup=g)
+        w = rq.W4A4Weight(b, type_, DEV)
+        if moved:
+            copy = torch.empty(w.prepared.numel() + 4096, dtype=torch.uint8, device=DEV)[2048:2048 + w.prepared.numel()]
+            copy.copy_(w.prepared)
+            kept.append(w.prepared)   # (the copy's fp6 plane is the original's)
+            w.prepared = copy
+        bl.append(b)
+        ws.append(w)
+    x = adversarial_activations(M, K, type_, wf, seed=M)
+    xd = torch.from_numpy(x).to(DEV)
+    outs = [torch.full((M, N + 3 * i), -7.0, dtype=torch.float32, device=DEV) for i, N in enumerate(Ns)]
+    work = torch.full((rq.fused_workspace_bytes(ws, M),), 0xA5, dtype=torch.uint8, device=DEV)
+    views = [o[:, :N] for o, N in zip(outs, Ns)]
+    assert _graph_nodes(lambda: rq.mul_mat_fused(ws, xd, outs=views, workspace=work)) == 1 + launches
+    for b, w, o in zip(bl, ws, outs):
+        want = oracle.mul_mat(type_, b, x, w.clip)
+        got = o.cpu().numpy()
+        assert bits_equal(got[:, :w.N], want), first_mismatch(got[:, :w.N], want)
+        assert (got[:, w.N:] == -7.0).all()

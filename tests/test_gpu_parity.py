@@ -622,7 +622,7 @@ def test_rows_are_independent_and_calls_repeatable(oracle):
 @pytest.mark.parametrize("one_launch", [True, False], ids=["one_launch", "launch_each"])
 def test_split_k_cells_in_a_dirty_workspace(oracle, M, Ns, one_launch):
     """Up to 64 tokens the panels beyond whole rounds of the chip meet in cells of the workspace, and the call clears
-    the cells of those panels only: one such panel, none, a few behind a round, all of them; the weights of a call in one
+    the cells of those panels only: two such panels, one, none, or all the panels of a small weight; the weights of a call in one
     launch, or (cells for the largest alone) in launches that take turns on the same cells. The workspace holds other
     bytes before each call."""
     K, type_ = 1024, rq.TYPE_W4A4
@@ -642,3 +642,20 @@ def test_split_k_cells_in_a_dirty_workspace(oracle, M, Ns, one_launch):
         for b, w, o in zip(bl, ws, outs):
             want = oracle.mul_mat(type_, b, x, w.clip)
             assert bits_equal(o.cpu().numpy(), want), first_mismatch(o.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("M,Ns", [(40, [16384]), (5, [16449]), (16, [16384, 70])])
+def test_split_k_cells_behind_the_two_step_rotation(oracle, M, Ns):
+    """Up to 40 tokens of a long Paley stage (K = 4352 = 68 x 64) the rotation's launch clears the cells: with no panel cut
+    it has nothing to clear; two panels cut; a second weight whose panels are all behind the round."""
+    K, type_ = 4352, rq.TYPE_W4A4H
+    ws, bl = [], []
+    for i, N in enumerate(Ns):
+        bl.append(synth.random_weight_blocks(N, K, 80 + i, type_))
+        ws.append(rq.W4A4Weight(bl[-1], type_, DEV))
+    x = synth.activations("student_t4", M, K, M)
+    work = torch.full((rq.fused_workspace_bytes(ws, M),), 0xA5, dtype=torch.uint8, device=DEV)
+    outs = rq.mul_mat_fused(ws, torch.from_numpy(x).to(DEV), workspace=work)
+    for b, w, o in zip(bl, ws, outs):
+        want = oracle.mul_mat(type_, b, x, w.clip, n_rot=K)
+        assert bits_equal(o.cpu().numpy(), want), first_mismatch(o.cpu().numpy(), want)

@@ -189,8 +189,8 @@ def test_search_at_rounding_boundaries_and_extreme_scales(oracle, K, wgroup):
 
 
 def test_conversions_in_several_runs(oracle):
-    """Tensors that go through in several runs of rows and more runs than there are pinned buffers; one row more than a
-    run; a read-only array."""
+    """Tensors that go through in several runs of rows; one row more than a run; on the way to the GPU more runs than there
+    are pinned buffers; a read-only array."""
     w = tensor(4097, 256, 3)
     got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4)
     want = oracle.quantize_rows_w(w)
@@ -199,6 +199,25 @@ def test_conversions_in_several_runs(oracle):
     blocks.flags.writeable = False
     got = rq.dequantize(blocks, rq.TYPE_W4A4, device=DEV).cpu().numpy()
     assert bits_equal(got, rq.dequantize_rows(blocks))
+
+
+@pytest.mark.parametrize("type_,wgroup", [(rq.TYPE_W4A4H, 0), (rq.TYPE_W4A4, 64)])
+def test_blocks_fetched_in_more_runs_than_buffers(type_, wgroup):
+    """9000 rows of 4096: three runs of rows, seven copies (20.7 MB) through three buffers, which are used again while the
+    next run is searched. The bytes are those of one call of the C entry point."""
+    N, K = 9000, 4096
+    g = torch.Generator(device=DEV)
+    g.manual_seed(4)
+    w = torch.randn((N, K), dtype=torch.float32, device=DEV, generator=g) * 0.02
+    L = rq.load_library()
+    ws = torch.empty(L.rq_w4a4_quantize_weights_workspace_bytes(type_, K, N, wgroup), dtype=torch.uint8, device=DEV)
+    out = torch.full((N * (K // 256) * 144,), 0xA5, dtype=torch.uint8, device=DEV)
+    assert L.rq_w4a4_quantize_weights(type_, w.data_ptr(), K, N, K, K, wgroup, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                                      torch.cuda.current_stream().cuda_stream) == 0
+    want = out.cpu().numpy().view(rq.BLOCK_DTYPE).reshape(N, K // 256)
+    for _ in range(2):
+        got = rq.quantize_weights(w, type_, wgroup=wgroup)
+        assert blocks_equal(got, want), block_diff(got, want)
 
 
 @pytest.mark.parametrize("rows", [1, 3639, 3640, 3641])
