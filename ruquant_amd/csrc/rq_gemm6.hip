@@ -864,17 +864,19 @@ hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
                        reinterpret_cast<unsigned long long *>(reinterpret_cast<uint8_t *>(a.cells) + kGemm6CounterBytes))
     // (a.weight_multipliers: what the host knows about the tensor; only a choice between two kernels that are both
     // right for every tensor)
-    if (a.w.n > 1) {
+    // (The kernels lie in the code object in the order in which they stand here. Behind the 57 KB of the H68 rotation a
+    // launch starts with a cold instruction cache, and how much of it the two share depends on the place: with the sets'
+    // kernels first, K = 17408, N = 5120 takes 60.1 us at 256 tokens and 77.9 at 512, with the single weights' first 58.7
+    // and 76.9; each kernel by itself takes the same time either way.)
+    if (a.w.n == 1) {
+        if (a.groups_per_fold == 1 && a.weight_multipliers) RQ_LAUNCH6(1, true, false, t1);
+        else if (a.groups_per_fold == 1) RQ_LAUNCH6(1, false, false, t1);
+        else if (a.groups_per_fold == 2) RQ_LAUNCH6(2, false, false, t1);
+        else RQ_LAUNCH6(4, false, false, t1);
+    } else {
         if (a.groups_per_fold != 1) return hipErrorInvalidValue;   // (wider groups go weight by weight)
         if (a.weight_multipliers) RQ_LAUNCH6(1, true, true, ts);
         else RQ_LAUNCH6(1, false, true, ts);
-    } else if (a.groups_per_fold == 1) {
-        if (a.weight_multipliers) RQ_LAUNCH6(1, true, false, t1);
-        else RQ_LAUNCH6(1, false, false, t1);
-    } else if (a.groups_per_fold == 2) {
-        RQ_LAUNCH6(2, false, false, t1);
-    } else {
-        RQ_LAUNCH6(4, false, false, t1);
     }
 #undef RQ_LAUNCH6
     return hipGetLastError();
