@@ -169,7 +169,9 @@ int rq_w4a4_mul_mat_stages(int type, const void *prepared_dev, int64_t K, int64_
  * length against the same x (q/k/v, gate/up): one activation transform, then the products.
  * workspace: rq_w4a4_workspace_bytes for N = the sum of the weights' row counts, each rounded up to 64: the streaming
  * kernels (M <= 64) then serve all the weights from one launch, as the reference's skinny kernel does. A workspace
- * sized for the largest N alone is also accepted; the products are then launched one per weight. */
+ * sized for the largest N alone is also accepted; the products are then launched one per weight. From M = 65 either
+ * size does: the products go in one launch unless some of the weights have multipliers and others not, the activation
+ * groups are wider than 64, or one launch would be the slower way (long rows whose tiles only fit cut one by one). */
 int rq_w4a4_mul_mat_fused(int type, int n, const void *const *prepared_dev, int64_t K, const int64_t *N,
                           const float *x_dev, int64_t ldx, int64_t M,
                           float *const *y_dev, const int64_t *ldy,

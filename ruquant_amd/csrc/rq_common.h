@@ -312,7 +312,7 @@ struct SkinnyArgs {
     int             panel0, panels;
 };
 hipError_t launch_skinny(const SkinnyArgs &a, hipStream_t stream);
-int64_t skinny_cells(const SkinnyArgs &a);   // split-K cells of that launch (8 bytes each, from a.tot on)
+int64_t skinny_cells(const SkinnyArgs &a);   // split-K cells that launch uses (8 bytes each, from a.tot on)
 struct SkinnyPlan {
     int main_panels;   // leading panels that run as one whole-K workgroup each
     int tail_split;    // K slices (workgroups) per remaining panel

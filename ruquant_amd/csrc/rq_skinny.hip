@@ -462,9 +462,9 @@ int token_tiles(const SkinnyArgs &a) {
 
 }  // namespace
 
-// What the activation launch has to clear: every cell a launch over all rows could have is 8.9 MB at N = 17408 and
-// 64 tokens, more than the activations themselves; only the panels beyond whole rounds (16 of 272 there, 0.5 MB) meet
-// in cells.
+// What the activation launch has to clear for this product launch alone: the cells of all rows, which a later product of
+// another weight may use, are 8.9 MB at N = 17408 and 64 tokens, more than the activations themselves; only the panels
+// beyond whole rounds (16 of 272 there, 0.5 MB) meet in cells.
 int64_t skinny_cells(const SkinnyArgs &a) {
     const int tt = token_tiles(a), n_panels = panels_of(a.w);
     const SkinnyPlan plan = plan_of(a, n_panels, a.w.L[0].ng, token_blocks(a.M, tt), a.runs_per_group);

@@ -141,7 +141,8 @@ def mul_mat(weight, x, out=None, workspace=None, clip=None):
     """y[M, N] = x[M, K] . W^T, bit-identical to the ggml-cpu W4A4 / W4A4H MUL_MAT. The workspace holds nothing for later
     calls afterwards (SharedActivation fills one that does)."""
     # (the single product's own entry point: no argument arrays to build. With the device and stream handled as in
-    # _on_device_of the host takes 5 us for a one-token call instead of 11.7 us, less than the kernel)
+    # _on_device_of the host takes 5 us for a one-token call instead of 11.7: less than the kernel from K = 5120,
+    # N = 5120 on (6.3 us), about as long as the smallest ones (K = 4096, N = 1024: 5.3))
     L = load_library()
     assert x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and x.stride(1) == 1
     M, K = x.shape
@@ -164,7 +165,8 @@ def mul_mat(weight, x, out=None, workspace=None, clip=None):
 def fused_workspace_bytes(weights, M):
     """Workspace for a fused call that serves all its weights from one launch of the streaming kernels: split-K
     cells for the rows of every weight (each padded to 64). With room for the largest weight only
-    (rq_w4a4_workspace_bytes of the largest N) the call still works, one product launch per weight."""
+    (rq_w4a4_workspace_bytes of the largest N) the call still works, one product launch per weight up to 64 tokens.
+    Above 64 tokens the room per weight does not count, and how many launches there are does not depend on it."""
     w0 = weights[0]
     N = w0.N if len(weights) == 1 else sum((w.N + 63) // 64 * 64 for w in weights)
     return load_library().rq_w4a4_workspace_bytes(w0.type, w0.K, N, M)
@@ -414,21 +416,20 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
         current = torch.cuda.current_stream()
         copier = _copier(current)
         copier.wait_stream(current)   # (the memory of `raw` may still be in use by work in front of this call)
-        runs = _chunks(rows, max(1, _STAGE_BYTES // max(row, 1)))
+        runs = _chunks(rows, max(1, _STAGE_BYTES // row))   # (a row too long for the library is refused by it)
         host = blocks.view(np.uint8).reshape(-1)
-        stages = _stages(row * max(b - a for a, b in runs)) if rows else []
+        stages = _stages(row * max(b - a for a, b in runs))
         sent = [None] * _STAGES
         for i, (a, b) in enumerate(runs):
             n, k = row * (b - a), i % _STAGES
             if sent[k] is not None:
                 sent[k].synchronize()
-            if n:
-                _copy_bytes(stages[k], host[row * a:row * b])
-                with torch.cuda.stream(copier):
-                    raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
-                    sent[k] = torch.cuda.Event()
-                    sent[k].record()
-                current.wait_event(sent[k])
+            _copy_bytes(stages[k], host[row * a:row * b])
+            with torch.cuda.stream(copier):
+                raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
+                sent[k] = torch.cuda.Event()
+                sent[k].record()
+            current.wait_event(sent[k])
             rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot),
                                       out.data_ptr() + 4 * K * a, K, _stream_ptr())
             _check(rc, "rq_w4a4_dequantize")
