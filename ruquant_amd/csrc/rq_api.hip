@@ -259,14 +259,22 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     q.mode = gemm && !two_step ? kActI8 : kActStats;
     q.u = reinterpret_cast<float *>(wsb + W.off_u);
     q.act = reinterpret_cast<uint32_t *>(wsb + W.off_i8);
+    // 33 .. 64 tokens of a call that shares its activation with no other: the small units of the fp6 product where they are
+    // the faster ones (block6_takes); they read the activations as the fp6 GEMM does
+    bool small6 = false;
+    if (path == kPathSkinny && once && G == kGroup && gemm_fp6_enabled() && !two_step) {
+        int64_t panels = 0;
+        for (int i = 0; i < n; ++i) panels += (N[i] + kPanelRows - 1) / kPanelRows;
+        small6 = block6_takes(panels, M);
+    }
     // token stride of the digit planes: the GEMM pads to its tile; the skinny kernel wants them dense (a padded
     // plane would put all of its reads on the few L2 channels that the used 256 bytes of every 2 KB map to)
-    const int act_mp = path == kPathSkinny ? (int) ((M + 15) / 16 * 16) : (int) W.Mp;
+    const int act_mp = path == kPathSkinny && !small6 ? (int) ((M + 15) / 16 * 16) : (int) W.Mp;
     q.Mp = act_mp;
     // the skinny path: one plane of q - z and the multipliers beside it (half the activation bytes per group, which
     // count against the weight bytes a compute unit can have in flight)
-    const bool single = path == kPathSkinny;
-    const bool fp6 = path == kPathGemm && gemm_fp6_enabled();
+    const bool fp6 = small6 || (path == kPathGemm && gemm_fp6_enabled());
+    const bool single = path == kPathSkinny && !small6;
     q.single = fp6 ? 2 : single;
     q.m4 = reinterpret_cast<float *>(wsb + W.off_i8 + act6_plane_bytes((int) (K / kGroup), W.Mp));
     q.mvals = reinterpret_cast<uint8_t *>(wsb + W.off_i8) + (size_t) (K / kGroup) * act_mp * 64;
@@ -316,7 +324,7 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         // only the token slots this call can touch: [min(M, 8)][padded rows] cells of two ints
         const int64_t slots = M < kGemvTokens ? M : kGemvTokens;
         q.zero_ints = 2 * slots * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
-    } else if (path == kPathSkinny) {
+    } else if (path == kPathSkinny && !small6) {
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
         // A stage-2 call may follow with any weight of at most N rows, whose plan cuts other panels than this call's:
         // cells for all rows. A call that is said to be the workspace's only one clears the cells of the panels that it
@@ -333,7 +341,7 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
             }
         }
         q.zero_ints = 2 * cells;
-    } else if (fp6) {
+    } else if (fp6 && !small6) {
         // the arrival counters of the tiles the fp6 GEMM cuts along K
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
         q.zero_ints = (int64_t) (kGemm6CounterBytes / sizeof(int32_t));
@@ -357,11 +365,12 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     bool fuse_gemm = fp6 && G == kGroup;
     for (int i = 1; i < n && fuse_gemm; ++i) fuse_gemm = multipliers_noted(prepared[i]) == multipliers_noted(prepared[0]);
     // (without room for slabs no tile is cut, and one launch never has more rounds)
-    if (fuse_gemm && n > 1 && have_slabs) fuse_gemm = gemm6_one_launch(weights_of(0, 1), M, multipliers_noted(prepared[0]));
-    const int n_launch = (path == kPathGemm ? fuse_gemm : one_launch) ? 1 : n;
+    if (fuse_gemm && n > 1 && have_slabs && !small6) fuse_gemm = gemm6_one_launch(weights_of(0, 1), M, multipliers_noted(prepared[0]));
+    if (small6) fuse_gemm = one_launch;
+    const int n_launch = (fp6 || path == kPathGemm ? fuse_gemm : one_launch) ? 1 : n;
     for (int l = 0; l < n_launch; ++l) {
         const FusedWeights fw = weights_of(l, n_launch);
-        if (path == kPathSkinny) {
+        if (path == kPathSkinny && !small6) {
             const SkinnyArgs g = skinny_args(fw);
             e = launch_skinny(g, stream);
             if (e != hipSuccess) return (int) e;
@@ -375,7 +384,7 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
             g.groups_per_fold = G / kGroup;
             g.cells = have_slabs ? wsb + W.off_tot : nullptr;
             g.weight_multipliers = multipliers_noted(fw.prepared[0]);
-            e = launch_gemm6(g, stream);
+            e = small6 ? launch_block6(g, stream) : launch_gemm6(g, stream);
             if (e != hipSuccess) return (int) e;
         } else if (gemm) {
             GemmArgs g;

@@ -1,0 +1,394 @@
+// The fp6 product (rq_gemm6.hip) for launches that are small for the chip: few tokens above 64, few rows, or the tiles
+// that are left over behind whole rounds of the tiled kernel.
+//
+// The tiled kernel's unit of work is 256 rows x 128 tokens, 200 us of one compute unit at long rows; a launch of few tiles
+// has to cut them along K across workgroups, whose partial totals meet in memory one after the other, and takes 19 us at
+// K = 5120 however little there is to do. Here the unit is one panel of 64 rows x 64 tokens, an eighth of a tile, with its
+// whole K: the eight wavefronts of a workgroup take the activation groups in turn (each all 64 x 64 outputs of its groups),
+// and their totals meet in LDS. No workspace, no arrival counts, nothing that waits for another workgroup.
+//
+// Arithmetic and operands are the tiled kernel's: one v_mfma_f32_32x32x64_f8f6f4 on fp6 fragments per 32 x 32 outputs and
+// group, and the floor as one FMA rounded toward minus infinity (see there for why both are exact; reference patch lines
+// 148-177). The fragments go from memory (L2, after the first reader) straight into registers, four groups of a wavefront
+// in flight (non-temporal hints and deeper or shallower rings change nothing). Measured: 4.2 us + 0.52 us per group of a
+// wavefront (K = 5120: ten of them, 9.3 us; the tiled kernel 19.5), of which the loads, 6 KB per group through the
+// compute unit's 64 bytes per cycle, take 0.32 and the vector ALU and the MFMAs 0.33. Beyond two rounds of the chip the tiled
+// kernel's twofold reuse out of LDS wins.
+#include "rq_common.h"
+
+#pragma clang fp contract(off)
+
+namespace rq {
+
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+constexpr int kWaves = 8, kThreads = kWaves * 64;
+constexpr int kTok = 64;                       // tokens of a unit
+constexpr int kUnitsPerTile = 8;               // 4 panels x 2 runs of 64 tokens of a tile of 256 x 128
+// groups of a wavefront whose operands are on their way (with weight multipliers the registers end there)
+constexpr int depth_of(bool hask) { return hask ? 2 : 4; }
+constexpr int kTokStride = kPanelRows + 4;     // ints between tokens of a wavefront's totals in LDS
+constexpr float kBias = 12582912.0f;           // 1.5 x 2^23
+constexpr int kBiasBits = 0x4B400000;
+constexpr int kFlushGroups = 28;               // (and the tile of one more that is folded late): less than 2^22
+
+template <bool HASK>
+struct Frag {
+    v8i A[2], B[2];       // this lane's parts of the two fragments of rows and the two of tokens (six registers each)
+    float m4[2];          // 4 m of this lane's two tokens
+    uint32_t kw[HASK ? 8 : 1];   // weight multipliers of the lane's rows (32 a + 8 q + 4 (lane / 32) + 0 .. 3), a byte each
+};
+
+// (global memory, said so: the plane's address comes out of memory, and the loads the compiler makes for a pointer of unknown
+// kind may be LDS accesses too, which it waits out whole, everything in flight behind them included)
+typedef const __attribute__((address_space(1))) uint8_t gbyte;
+typedef const __attribute__((address_space(1))) float gfloat;
+typedef const __attribute__((address_space(1))) uint32_t gword;
+typedef const __attribute__((address_space(1))) v4u gv4u;
+typedef const __attribute__((address_space(1))) v2u gv2u;
+
+struct Src {
+    gbyte *a, *b, *k;           // (wave-uniform) the unit's operands of group 0
+    gfloat *m4;
+    size_t b_step;              // bytes between groups of the activation plane
+    int Mp;
+};
+
+__device__ __forceinline__ v8i operand(gbyte *frag, uint32_t l) {
+    const v4u lo = *reinterpret_cast<gv4u *>(frag + l * 16);
+    const v2u hi = *reinterpret_cast<gv2u *>(frag + 1024 + l * 8);
+    v8i v;
+    v[0] = (int) lo.x; v[1] = (int) lo.y; v[2] = (int) lo.z; v[3] = (int) lo.w;
+    v[4] = (int) hi.x; v[5] = (int) hi.y;
+    // (the fp6 form reads six registers: elements 6 and 7 are left undefined)
+    return v;
+}
+
+// The wavefront's group j of n. Past the end of its share a wavefront's loads read group 0 again, from offset 0 in
+// every lane (the loop stays branch-free, so the wait counts stay exact), and nothing consumes them
+template <bool HASK>
+__device__ __forceinline__ void load_frag(Frag<HASK> &f, const Src &s, int wave, int lane, int j, int n) {
+    const int g = wave + j * kWaves;
+    // (a mask: on a condition the compiler branches around the address arithmetic, and the folds sink into the blocks behind)
+    const int keep = __builtin_amdgcn_readfirstlane((j - n) >> 31);
+    const uint32_t gk = (uint32_t) (g & keep), l = (uint32_t) (lane & keep);
+    gbyte *a = s.a + (size_t) gk * (8 * kFrag6);
+    gbyte *b = s.b + gk * s.b_step;
+    gfloat *m4 = s.m4 + (size_t) gk * s.Mp;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        f.A[i] = operand(a + i * kFrag6, l);
+        f.B[i] = operand(b + i * kFrag6, l);
+        f.m4[i] = m4[32 * i + (l & 31)];
+    }
+    if constexpr (HASK) {
+        gbyte *k = s.k + (size_t) gk * kPanelRows + 4 * (l >> 5);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) f.kw[q] = *reinterpret_cast<gword *>(k + 8 * q);
+    }
+}
+
+// What a wavefront carries from group to group: the totals of its 64 x 64 outputs and the tile whose fold is still due.
+// Without weight multipliers `acc` is the biased float accumulator of the tiled kernel; with them a group's term, which may
+// be 15 times as large, is formed on the bias by an FMA of its own and its bit pattern is added up in integers
+// (acc holds those; the bias of every term comes off at the end).
+struct State {
+    float acc[2][2][16];
+    v16f P;
+    float pm;
+    float bias;   // kBias (with weight multipliers; taken from behind the change of the rounding mode, like acc)
+};
+
+// the four tiles of one group; a tile's fold runs behind the next tile's MFMA
+__device__ __forceinline__ void group_units(const Frag<false> &f, State &st) {
+    const v16f zero = {};
+#pragma unroll
+    for (int un = 0; un < 4; ++un) {
+        const int a = un >> 1, b = un & 1;
+        const int pa = un == 0 ? 1 : (un - 1) >> 1, pb = un == 0 ? 1 : (un - 1) & 1;
+        const v16f S = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.A[a], f.B[b], zero, 2, 2, 0, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st.acc[pa][pb][r] = __builtin_fmaf(st.P[r], st.pm, st.acc[pa][pb][r]);
+        st.P = S;
+        // (a register of its own, which is not the ring's: renamed into it, the ring's newest load would be moved at the head
+        // of the loop and waited for with everything in flight)
+        asm volatile("v_mov_b32 %0, %1" : "=v"(st.pm) : "v"(f.m4[b]));
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);   // VALU: the fold of the tile before
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+// with weight multipliers: the two tiles of a row block together, which share the multipliers as floats (a group is folded
+// whole, so that the next one does not need its multipliers)
+__device__ __forceinline__ void group_units(const Frag<true> &f, State &st) {
+    const v16f zero = {};
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        v16f S[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) S[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.A[a], f.B[b], zero, 2, 2, 0, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float kf = (float) ((f.kw[4 * a + (r >> 2)] >> (8 * (r & 3))) & 0xFFu);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const float term = __builtin_fmaf(S[b][r], kf * f.m4[b], st.bias);
+                st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(int, st.acc[a][b][r]) + __builtin_bit_cast(int, term));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// the totals of this wavefront into its own part of LDS, [token][row]; FRESH: nothing is there yet
+template <bool FRESH>
+__device__ __forceinline__ void flush(State &st, int *part, int lane) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                v4i *dst = reinterpret_cast<v4i *>(part + (32 * b + (lane & 31)) * kTokStride + 32 * a + 8 * q + 4 * (lane >> 5));
+                v4i v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = __builtin_bit_cast(int, st.acc[a][b][4 * q + e]) - kBiasBits;
+                    st.acc[a][b][4 * q + e] = kBias;
+                }
+                *dst = FRESH ? v : *dst + v;
+            }
+        }
+    }
+}
+
+template <bool HASK>
+__device__ __forceinline__ void stream(const Src &s, int wave, int lane, int n, int *part) {
+    State st;
+    st.P = v16f{};
+    st.pm = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                st.acc[a][b][r] = HASK ? 0.0f : kBias;
+                asm volatile("" : "+v"(st.acc[a][b][r]));   // (behind the change of the rounding mode)
+            }
+        }
+    }
+    constexpr int kDepth = depth_of(HASK);
+    st.bias = kBias;
+    asm volatile("" : "+s"(st.bias));
+    Frag<HASK> ring[kDepth];
+#pragma unroll
+    for (int i = 0; i < kDepth; ++i) {
+        load_frag<HASK>(ring[i], s, wave, lane, i, n);
+        __builtin_amdgcn_sched_barrier(0);   // (group by group: a wait counts the loads behind the one it is for)
+    }
+    const int rounds = n / kDepth;
+    bool fresh = true;
+    for (int r = 0; r < rounds; ++r) {
+#pragma unroll
+        for (int i = 0; i < kDepth; ++i) {
+            const int j = r * kDepth + i + kDepth;
+            group_units(ring[i], st);
+            __builtin_amdgcn_sched_barrier(0);
+            load_frag<HASK>(ring[i], s, wave, lane, j, n);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!HASK && (r + 1) % (kFlushGroups / kDepth) == 0) {
+            if (fresh) flush<true>(st, part, lane);
+            else flush<false>(st, part, lane);
+            fresh = false;
+        }
+    }
+    const int rem = n - rounds * kDepth;   // the last n % kDepth groups are already here
+#pragma unroll
+    for (int i = 0; i < kDepth - 1; ++i) {
+        if (i < rem) group_units(ring[i], st);
+    }
+    if constexpr (HASK) {
+        // n terms, each with the bias's bit pattern on it
+        const int off = n * kBiasBits - kBiasBits;   // (flush takes one off)
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(int, st.acc[a][b][r]) - off);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st.acc[1][1][r] = __builtin_fmaf(st.P[r], st.pm, st.acc[1][1][r]);
+    }
+    if (fresh) flush<true>(st, part, lane);
+    else flush<false>(st, part, lane);
+}
+
+struct BlockSet {
+    const float   *s_w[kMaxFused];
+    const uint8_t *kmul[kMaxFused];
+    const int32_t *flags[kMaxFused];
+    float         *y[kMaxFused];
+    int64_t        ldy[kMaxFused];
+    int64_t        N[kMaxFused];
+    int            n_panels[kMaxFused];
+    int            first[kMaxFused];   // first panel, or row tile of 256 rows; unused slots hold the total, so none selects them
+};
+
+__global__ void __launch_bounds__(kThreads, 2)
+rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
+                 const float *__restrict__ u, int M, int Mp, int ng, int n_runs, int super_tiles, int first_tile,
+                 int n_units) {
+    __shared__ __align__(16) int s_part[kWaves][kTok * kTokStride];
+    // An XCD gets a contiguous run of the units, so that those that share a panel or a run of tokens read them from one L2.
+    int v = blockIdx.x;
+    const int per_xcd = n_units / kXcds;
+    if (v < per_xcd * kXcds) v = (v % kXcds) * per_xcd + v / kXcds;
+    int wsel, panel, t0;   // which weight, which of its panels, first token
+    if (first_tile < 0) {
+        // the whole product: panel by panel, the runs of tokens running fastest. (No unit is without rows or tokens: workgroups
+        // are dealt to the shader engines in turn, and with every second one empty the others queue on half of them. 160
+        // units and 160 empty ones, K = 5120: 18.8 us.)
+        panel = v / n_runs;
+        t0 = (v - panel * n_runs) * kTok;
+        wsel = (panel >= ts.first[1]) + (panel >= ts.first[2]);
+        panel -= wsel == 0 ? 0 : wsel == 1 ? ts.first[1] : ts.first[2];   // now of its weight
+    } else {
+        // the tiles (256 rows x 128 tokens) from first_tile on in the tiled kernel's order, eight units each
+        const int n_tok_tiles = Mp / kGemmTokens, sub = v & 7;
+        v = first_tile + (v >> 3);
+        int row_tile;
+        if (super_tiles) {
+            const int s = v >> 5, i = v & 31;
+            const int spr = n_tok_tiles >> 2;
+            const int sr = s / spr;
+            row_tile = sr * 8 + (i >> 2);
+            t0 = ((s - sr * spr) * 4 + (i & 3)) * kGemmTokens;
+        } else {
+            row_tile = v / n_tok_tiles;
+            t0 = (v - row_tile * n_tok_tiles) * kGemmTokens;
+        }
+        t0 += (sub & 1) * kTok;
+        wsel = (row_tile >= ts.first[1]) + (row_tile >= ts.first[2]);
+        row_tile -= wsel == 0 ? 0 : wsel == 1 ? ts.first[1] : ts.first[2];
+        panel = row_tile * 4 + (sub >> 1);
+    }
+    auto of_weight = [&](const auto &w) { return wsel == 0 ? w[0] : wsel == 1 ? w[1] : w[2]; };
+    if (t0 >= M || panel >= of_weight(ts.n_panels)) return;
+    const float *__restrict__ s_w = of_weight(ts.s_w);
+    const uint8_t *__restrict__ kmul = of_weight(ts.kmul);
+    const int32_t *__restrict__ flags = of_weight(ts.flags);
+    float *__restrict__ y = of_weight(ts.y);
+    const int64_t ldy = of_weight(ts.ldy);
+    const int64_t N = of_weight(ts.N);
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint8_t *w6 = reinterpret_cast<const uint8_t *>((uintptr_t) *reinterpret_cast<const unsigned long long *>(flags + 2));
+    const bool hask = flags[0] & 1;
+    Src s;
+    s.a = (gbyte *) (w6 + ((size_t) (panel >> 2) * ng * 8 + 2 * (panel & 3)) * kFrag6);
+    s.b_step = (size_t) (Mp / 32) * kFrag6;
+    s.b = (gbyte *) (act6 + (size_t) (t0 / 32) * kFrag6);
+    s.m4 = (gfloat *) (m4 + t0);
+    s.k = (gbyte *) (kmul + (size_t) panel * ng * kPanelRows);
+    s.Mp = Mp;
+    // what the epilogue needs from memory is asked for first: a thread ends with four rows of two tokens
+    const int quad = tid & 15, tok = tid >> 4;
+    const float4 sw = *reinterpret_cast<const float4 *>(s_w + panel * kPanelRows + 4 * quad);   // rows past N are stored as zero
+    float ut[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ut[i] = u[min(t0 + tok + 32 * i, M - 1)];
+
+    const int n = wave < ng ? (ng - wave + kWaves - 1) / kWaves : 0;   // groups wave, wave + 8, ...
+    // fp32 rounding toward minus infinity for the folds (MODE bits 1:0); the MFMA sums are exact in any mode
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2" ::: "memory");
+    if (hask) stream<true>(s, wave, lane, n, s_part[wave]);
+    else stream<false>(s, wave, lane, n, s_part[wave]);
+    // (the totals are in LDS when the mode goes back to round to nearest even, and the conversions below read them from there)
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0" ::: "memory");
+    __syncthreads();
+
+    // y = ((float(total) * 16) * u) * s_w (reference patch line 176)
+    const int64_t row = (int64_t) panel * kPanelRows + 4 * quad;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int t = t0 + tok + 32 * i;
+        v4i tot = *reinterpret_cast<const v4i *>(&s_part[0][(tok + 32 * i) * kTokStride + 4 * quad]);
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) tot += *reinterpret_cast<const v4i *>(&s_part[w][(tok + 32 * i) * kTokStride + 4 * quad]);
+        if (t >= M) continue;
+        const float o[4] = { (((float) tot.x * 16.0f) * ut[i]) * sw.x, (((float) tot.y * 16.0f) * ut[i]) * sw.y,
+                             (((float) tot.z * 16.0f) * ut[i]) * sw.z, (((float) tot.w * 16.0f) * ut[i]) * sw.w };
+        float *dst = y + (int64_t) t * ldy + row;
+        if (row + 3 < N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
+            typedef float v4f __attribute__((ext_vector_type(4)));
+            __builtin_nontemporal_store(v4f{ o[0], o[1], o[2], o[3] }, reinterpret_cast<v4f *>(dst));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (row + e < N) dst[e] = o[e];
+            }
+        }
+    }
+}
+
+}  // namespace
+
+namespace {
+
+hipError_t launch(const Gemm6Args &a, int super_tiles, int first_tile, int n_units, hipStream_t stream) {
+    BlockSet ts;
+    int first = 0;
+    for (int i = 0; i < kMaxFused; ++i) {
+        const int k = i < a.w.n ? i : a.w.n - 1;   // unused slots repeat the last weight (never selected)
+        const PreparedLayout &L = a.w.L[k];
+        const uint8_t *p = a.w.prepared[k];
+        ts.s_w[i] = reinterpret_cast<const float *>(p + L.off_sw);
+        ts.kmul[i] = p + L.off_kmul;
+        ts.flags[i] = reinterpret_cast<const int32_t *>(p + L.off_flags);
+        ts.y[i] = a.w.y[k];
+        ts.ldy[i] = a.w.ldy[k];
+        ts.N[i] = L.N;
+        ts.n_panels[i] = L.n_panels;
+        ts.first[i] = first;
+        if (i < a.w.n) first += first_tile < 0 ? L.n_panels : L.n_rtiles;
+    }
+    const int ng = a.w.L[0].ng;
+    const float *m4 = reinterpret_cast<const float *>(a.act6 + act6_plane_bytes(ng, a.Mp));
+    hipLaunchKernelGGL(rq_block6_kernel, dim3(n_units), dim3(kThreads), 0, stream, ts, a.act6, m4, a.u, a.M, a.Mp, ng,
+                       (a.M + kTok - 1) / kTok, super_tiles, first_tile, n_units);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_block6(const Gemm6Args &a, hipStream_t stream) {
+    int n_panels = 0;
+    for (int i = 0; i < a.w.n; ++i) n_panels += a.w.L[i].n_panels;
+    return launch(a, 0, -1, n_panels * ((a.M + kTok - 1) / kTok), stream);
+}
+
+hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_tile, int n_tiles, hipStream_t stream) {
+    return launch(a, super_tiles, first_tile, (n_tiles - first_tile) * kUnitsPerTile, stream);
+}
+
+// 33 .. 64 tokens. The skinny kernel reads two thirds of the bytes (int4 codes) but runs 16 x 16 MFMAs with three vector
+// instructions per output behind each, where this one has 32 x 32 and one, and of its form for 64 tokens a round of the chip
+// is 18 us at K = 5120. 64 tokens, whole call, skinny and here: K = 3072, N = 4096 14.9 / 13.2 us, N = 10240 20.2 / 14.0, N = 17408
+// 27.3 / 21.7; K = 5120, N = 2048 14.9 / 16.1, N = 4096 16.7 / 16.3, N = 8192 17.1 / 17.1, N = 10240 24.6 / 17.4, N = 17408 32.5 /
+// 27.8; K = 10240, N = 4096 25.9 / 25.8, N = 17408 48.4 / 45.4; K = 17408, N = 4096 34.1 / 37.8, N = 8192 42.7 / 39.1, N = 17408
+// 69.6 / 68.8. 33 tokens cost the same in both.
+bool block6_takes(int64_t n_panels, int64_t M) { return M > 32 && n_panels >= 96; }
+
+}  // namespace rq

@@ -810,14 +810,67 @@ namespace {
 // Microseconds of a launch by its plan: a round of whole tiles and, behind it, the slices of the tiles that are cut, by
 // steps of two groups. Fitted to 112 sets of two and three weights (K = 2560 to 32768, 5 to 750 tiles), in one launch and
 // in one each; it gives the ratio of the two within 7 % where that is near 1.
-double launch_price(int n_row_tiles, int64_t M, int ng, bool weight_multipliers) {
-    const Gemm6Plan pl = gemm6_plan(n_row_tiles, M, ng, 1);
+double tiled_price(const Gemm6Plan &pl, int ng, bool weight_multipliers) {
     const int steps = ng / 2;
     const int rounds = (pl.n_whole + kPlanUnits - 1) / kPlanUnits;
     const double whole = weight_multipliers ? 5.8 + 1.53 * steps : 7.4 + 0.72 * steps;
     const int slice = (steps + pl.parts - 1) / pl.parts;
     const double cut = weight_multipliers ? 11.5 + 1.56 * slice + 0.8 * (pl.parts - 1) : 12.3 + 0.85 * slice + 1.1 * (pl.parts - 1);
     return rounds * whole + (pl.parts > 1 ? cut : 0.0);
+}
+
+// The same for the kernel of small launches (rq_block6.hip), by rounds of its units and the groups of one wavefront.
+// K = 1024 / 5120 / 17408: 16 units 5.2 / 9.3 / 21.2 us, 192 units 5.6 / 10.5 / 24.7, 384 units 9.5 / 18.7 / 44 (of long rows);
+// weight groups of 64, K = 5120 / 17408, 16 units 12.2 / 29.6, 192 units 13.4 / 32.7, 384 units 24.2.
+double block_price(int64_t units, int ng, bool weight_multipliers) {
+    const double rounds = (double) ((units + kPlanUnits - 1) / kPlanUnits);
+    const int per_wave = (ng + 7) / 8;
+    return rounds * (weight_multipliers ? 5.2 + 0.75 * per_wave : 4.2 + 0.53 * per_wave);
+}
+
+// How a launch goes: the tiles in front of `first_block` through the tiled kernel by `plan`, the others through the kernel
+// of small launches.
+struct Route {
+    Gemm6Plan plan;
+    int       n_tiles, first_block;
+    double    price;
+};
+
+// The cheapest of three. Few tiles: all of them in small units, as long as those are at most two rounds of the chip (K = 5120:
+// 2 tiles 19.5 us in slices and 9.9 in units, 48 tiles 24.4 and 19.4, 96 tiles, three rounds, 27.7 and 28.6; K = 17408: 2
+// tiles 29.2 and 22.1, 48 tiles 39.2 and 47.3). Whole rounds and a few tiles over: those few in units behind the rounds (K = 5120, N = 17408, 512 tokens, 256 + 16
+// tiles: 60.8 us with the 16 in slices, 54.4 with them in 128 units). Everything else: tiles, the rest in slices.
+Route route_of(int n_row_tiles, int64_t n_panels, int64_t M, int ng, int groups_per_fold, bool weight_multipliers, bool have_slabs) {
+    Route r;
+    r.plan = gemm6_plan(n_row_tiles, M, ng, groups_per_fold);
+    r.n_tiles = r.first_block = r.plan.n_tiles;
+    if (!have_slabs) {   // a workspace without slabs: every tile whole
+        r.plan.n_whole = r.plan.n_tiles;
+        r.plan.parts = 1;
+    }
+    r.price = tiled_price(r.plan, ng, weight_multipliers);
+    if (groups_per_fold != 1) return r;   // (the small units fold groups of 64)
+    const int64_t units = n_panels * ((M + 63) / 64);
+    const double all = block_price(units, ng, weight_multipliers);
+    if (units <= 2 * kPlanUnits && all < r.price) {
+        r.plan.n_tiles = r.plan.n_whole = r.first_block = 0;
+        r.plan.parts = 1;
+        r.price = all;
+        return r;
+    }
+    const int left = r.n_tiles % kPlanUnits, rounds = r.n_tiles - left;
+    if (left > 0 && rounds > 0) {
+        Gemm6Plan whole = r.plan;
+        whole.n_tiles = whole.n_whole = rounds;
+        whole.parts = 1;
+        const double both = tiled_price(whole, ng, weight_multipliers) + 2.0 + block_price((int64_t) left * 8, ng, weight_multipliers);
+        if (left * 8 <= 2 * kPlanUnits && both < r.price) {
+            r.plan = whole;
+            r.first_block = rounds;
+            r.price = both;
+        }
+    }
+    return r;
 }
 
 }  // namespace
@@ -828,33 +881,38 @@ double launch_price(int n_row_tiles, int64_t M, int ng, bool weight_multipliers)
 // The other way round K = 5120, N = 6144 + 1024 + 1024, 512 tokens is 40 and 79 us. (3 % apart is what the prices tell.)
 bool gemm6_one_launch(const FusedWeights &w, int64_t M, bool weight_multipliers) {
     int n_row_tiles = 0;
+    int64_t n_panels = 0;
     double each = 0.0;
     for (int i = 0; i < w.n; ++i) {
         n_row_tiles += w.L[i].n_rtiles;
-        each += launch_price(w.L[i].n_rtiles, M, w.L[i].ng, weight_multipliers);
+        n_panels += w.L[i].n_panels;
+        each += route_of(w.L[i].n_rtiles, w.L[i].n_panels, M, w.L[i].ng, 1, weight_multipliers, true).price;
     }
-    return launch_price(n_row_tiles, M, w.L[0].ng, weight_multipliers) <= 1.03 * each;
+    return route_of(n_row_tiles, n_panels, M, w.L[0].ng, 1, weight_multipliers, true).price <= 1.03 * each;
 }
 
 hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
     TileSet<true> ts;
     TileSet<false> t1;
     int n_row_tiles = 0;
+    int64_t n_panels = 0;
     for (int i = 0; i < kMaxFused; ++i) {
         const int k = i < a.w.n ? i : a.w.n - 1;   // unused slots repeat the last weight (never selected)
         set_weight(ts, i, a.w, k, n_row_tiles);
         if (i == 0) set_weight(t1, 0, a.w, 0, 0);
-        if (i < a.w.n) n_row_tiles += a.w.L[k].n_rtiles;
+        if (i < a.w.n) {
+            n_row_tiles += a.w.L[k].n_rtiles;
+            n_panels += a.w.L[k].n_panels;
+        }
     }
     const int ng = a.w.L[0].ng;
     const int n_tok_tiles = a.Mp / kTileTok;
-    Gemm6Plan pl = gemm6_plan(n_row_tiles, a.M, ng, a.groups_per_fold);
-    if (pl.n_tiles != n_row_tiles * n_tok_tiles) return hipErrorInvalidValue;
-    if (a.cells == nullptr) {   // a workspace without slabs: every tile whole
-        pl.n_whole = pl.n_tiles;
-        pl.parts = 1;
-    }
+    const Route route = route_of(n_row_tiles, n_panels, a.M, ng, a.groups_per_fold, a.weight_multipliers, a.cells != nullptr);
+    const Gemm6Plan &pl = route.plan;
+    if (route.n_tiles != n_row_tiles * n_tok_tiles) return hipErrorInvalidValue;
+    if (a.w.n > 1 && a.groups_per_fold != 1) return hipErrorInvalidValue;   // (wider groups go weight by weight)
     const int super_tiles = n_tok_tiles % 4 == 0 && n_row_tiles % 8 == 0;
+    if (pl.n_tiles == 0) return launch_block6(a, stream);
     const int grid = pl.n_whole + (pl.n_tiles - pl.n_whole) * pl.parts;
     const float *m4 = reinterpret_cast<const float *>(a.act6 + act6_plane_bytes(ng, a.Mp));
 #define RQ_LAUNCH6(GS, KFMA, SET, TS)                                                                                      \
@@ -874,12 +932,13 @@ hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
         else if (a.groups_per_fold == 2) RQ_LAUNCH6(2, false, false, t1);
         else RQ_LAUNCH6(4, false, false, t1);
     } else {
-        if (a.groups_per_fold != 1) return hipErrorInvalidValue;   // (wider groups go weight by weight)
         if (a.weight_multipliers) RQ_LAUNCH6(1, true, true, ts);
         else RQ_LAUNCH6(1, false, true, ts);
     }
 #undef RQ_LAUNCH6
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || route.first_block == route.n_tiles) return e;
+    return launch_block6_tiles(a, super_tiles, route.first_block, route.n_tiles, stream);
 }
 
 }  // namespace rq

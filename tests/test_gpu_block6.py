@@ -1,0 +1,82 @@
+"""The fp6 product in units of 64 rows x 64 tokens (rq_block6.hip), bit for bit against the oracle: where a wavefront has no
+group, a few or enough to move its totals to LDS on the way; ragged rows, tokens and row strides; every kind of weight
+multiplier; one round of the chip, two, and the tiles that the tiled kernel leaves over; and 33 .. 64 tokens, which take it only
+in calls that share their activation with no other."""
+import numpy as np
+import pytest
+import torch
+
+import ruquant_amd as rq
+from ruquant_amd import synth
+from tests.gpu_util import adversarial_weights, adversarial_activations, bits_equal, first_mismatch, run_gpu
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("K,N,M,wgroup", [
+    (256, 64, 65, 0),         # four groups for eight wavefronts
+    (512, 1, 128, 64),        # one group each, one row
+    (4352, 130, 190, 0),      # eight or nine, ragged
+    (4352, 130, 190, 256),
+    (15360, 70, 66, 0),       # 30: past the 28 between two transfers
+    (32768, 65, 67, 64),      # the longest row
+    (512, 4096, 512, 0),      # 512 units: two rounds
+    (512, 4300, 2048, 0),     # 17 x 16 tiles: 16 left over behind a round, the last row tile ragged
+    (512, 8192, 1100, 256),   # 32 x 9 tiles: 32 left over, in runs of nine token tiles
+    (2560, 6200, 33, 0),      # 97 panels: 33 .. 64 tokens
+    (2560, 6200, 64, 64),
+    (17408, 6145, 41, 0)])
+def test_units_of_64_rows_and_tokens(oracle, K, N, M, wgroup):
+    type_ = rq.TYPE_W4A4 if K in (256, 512, 32768) else rq.TYPE_W4A4H
+    blocks, wf = adversarial_weights(oracle, N, K, type_, seed=N + M, wgroup=wgroup)
+    W = rq.W4A4Weight(blocks, type_, DEV)
+    x = adversarial_activations(M, K, type_, wf, seed=M)
+    want = oracle.mul_mat(type_, blocks, x, W.clip, n_rot=max(W.n_rot, 0))
+    got = run_gpu(W, x)
+    assert bits_equal(got, want), first_mismatch(got, want)
+    # rows of y that are no multiple of four floats apart, and nothing written between them
+    out = torch.full((M, N + 3), -7.0, dtype=torch.float32, device=DEV)
+    rq.mul_mat(W, torch.from_numpy(x).to(DEV), out=out[:, :N])
+    got = out.cpu().numpy()
+    assert bits_equal(got[:, :N], want), first_mismatch(got[:, :N], want)
+    assert (got[:, N:] == -7.0).all()
+
+
+def test_extreme_sums_between_two_transfers(oracle):
+    """K = 32768: 64 groups per wavefront, rows of all -8 / all 7 against tokens of q - z = +-15 with m = 255, so that the float
+    totals move by 122,400 per group, 28 groups and a tile of one more between two transfers: 3.55 M of their 4.19 M."""
+    N, K, M, type_ = 64, 32768, 80, rq.TYPE_W4A4
+    blocks = synth.random_weight_blocks(N, K, 5, type_)
+    qs = blocks["qs"].reshape(N, -1)
+    qs[0, :] = 0x88888888
+    qs[1, :] = 0x77777777
+    qs[2, ::2] = 0x88888888
+    qs[2, 1::2] = 0x77777777
+    blocks["qs"] = qs.reshape(blocks["qs"].shape)
+    x = np.ones((M, K), dtype=np.float32)
+    x[1::2] = -1.0
+    x[2::4, ::2] = -1.0
+    W = rq.W4A4Weight(blocks, type_, DEV)
+    want = oracle.mul_mat(type_, blocks, x, W.clip)
+    got = run_gpu(W, x)
+    assert bits_equal(got, want), first_mismatch(got, want)
+
+
+@pytest.mark.parametrize("M", [40, 70])
+def test_a_set_of_weights(oracle, M):
+    """Three weights, with and without multipliers, whose panels do not end with a row tile, in one launch (40 tokens) or one
+    each (70, where the two kinds go apart)."""
+    K, type_ = 1024, rq.TYPE_W4A4H
+    ws, want = [], []
+    x = None
+    for i, (N, g) in enumerate([(3000, 0), (2100, 64), (1500, 0)]):
+        blocks, wf = adversarial_weights(oracle, N, K, type_, seed=i, wgroup=g)
+        w = rq.W4A4Weight(blocks, type_, DEV)
+        if x is None:
+            x = adversarial_activations(M, K, type_, wf, seed=3)
+        ws.append(w)
+        want.append(oracle.mul_mat(type_, blocks, x, w.clip, n_rot=w.n_rot))
+    outs = rq.mul_mat_fused(ws, torch.from_numpy(x).to(DEV))
+    for o, v in zip(outs, want):
+        assert bits_equal(o.cpu().numpy(), v), first_mismatch(o.cpu().numpy(), v)
