@@ -92,6 +92,24 @@ __device__ __forceinline__ void paley_pick_stream(int s, const float *src, int s
     }
 }
 
+// The same with element i of the column at at(i), and with the signs of the transposed matrix (TR) where asked for.
+template <int P, int O, bool TR, int S = 0, class At>
+__device__ __forceinline__ void paley_pick_at(int s, At at, float (&out)[O]) {
+    if (s == S) {
+        constexpr PaleyTable<P> T = make_paley<P>();
+#pragma unroll
+        for (int o = 0; o < O; ++o) out[o] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const float c = at(i);
+#pragma unroll
+            for (int o = 0; o < O; ++o) out[o] = (TR ? T.neg[O * S + o][i] : T.neg[i][O * S + o]) ? out[o] - c : out[o] + c;
+        }
+    } else if constexpr (S + 1 < P / O) {
+        paley_pick_at<P, O, TR, S + 1>(s, at, out);
+    }
+}
+
 // The same for two columns at once (two runs of 64 columns of one slice): twice the independent sums per
 // instruction stream, which is what hides the latency of the dependent additions and of the LDS reads when a
 // wavefront has only two items.
@@ -443,6 +461,43 @@ __device__ __forceinline__ void load_row_fwht256(float *buf, const float *__rest
             for (int j = 0; j < 16; ++j) dd[j] = v[j];
         }
     }
+}
+
+// The Paley stage of a whole padded row, in place, by a workgroup of NT threads, every column by four of them: wavefront w
+// takes a quarter of the outputs (w / (NT / 256)) of 64 columns, so a column needs P / 4 registers and every wavefront of
+// the workgroup adds. (With a thread per column 256 of 512 threads had one at K = 17408, and its 68 sums took the registers
+// of two.) All of a run's columns are read before the first is written.
+template <int P, int NT, bool TR>
+__device__ __forceinline__ void paley_row(float *buf, int K, int m, int n_rot, float scale, int tid) {
+    constexpr int kCols = 256, kO = P / (NT / kCols);
+    const int ncols = K / P;   // columns of all rotation blocks of this row
+    const int pm = m + (m >> 4), lm = __ffs(m) - 1;
+    const int s = __builtin_amdgcn_readfirstlane(tid / kCols);
+    for (int c0 = 0; c0 < ncols; c0 += kCols) {
+        const int cidx = c0 + (tid & (kCols - 1));
+        const bool on = cidx < ncols;
+        const int rb = cidx >> lm, j = cidx & (m - 1);
+        const int b0 = on ? rb * n_rot + j : 0;
+        float out[kO];
+        float *col = buf + padi(b0);
+        if (pm == 272) {   // chunks of 256 (K = 17408): a compile-time stride, one address register for the column
+            paley_pick_at<P, kO, TR>(s, [&](int i) { return col[i * 272]; }, out);
+        } else if ((m & 15) == 0) {
+            paley_pick_at<P, kO, TR>(s, [&](int i) { return col[i * pm]; }, out);
+        } else {
+            paley_pick_at<P, kO, TR>(s, [&](int i) { return buf[padi(b0 + i * m)]; }, out);
+        }
+        __syncthreads();
+        if (on && pm == 272) {
+            float *dst = col + kO * s * 272;
+#pragma unroll
+            for (int o = 0; o < kO; ++o) dst[o * 272] = out[o] * scale;
+        } else if (on) {
+#pragma unroll
+            for (int o = 0; o < kO; ++o) buf[padi(b0 + (kO * s + o) * m)] = out[o] * scale;
+        }
+    }
+    __syncthreads();
 }
 
 // all Sylvester stages from stride 1 << ls0 up of every chunk of m = 1 << lm floats of a padded row, four stages per

@@ -22,20 +22,22 @@ namespace {
 // Threads per token workgroup. Small batches (the sliced variant) with a short Paley stage get 1024: there the kernel
 // is one workgroup per compute unit at most, bound by the latency of its own phases, and twice the threads halve the
 // work per phase. Long Paley stages keep their columns in registers and need the 256-register budget of 512 threads.
-template <int P, bool SLICED>
-constexpr int threads_of() { return SLICED && P < 44 ? 1024 : 512; }
+template <int P, bool SLICED, bool WIDE>
+constexpr int threads_of() { return WIDE || (SLICED && P < 44) ? 1024 : 512; }
 
 using namespace had;
 
-template <int P, bool SLICED, bool ALONE = false>
+template <int P, bool SLICED, bool WIDE = false>
 // Registers are capped so that two workgroups (p >= 44: long columns, long rows) or three fit a compute unit: the
 // stages of one token are separated by barriers, and it is the other workgroups that keep the vector ALU busy. (The
-// sliced variant serves small batches, where occupancy is not the limit.) ALONE is the plain variant for rows so long
-// that LDS holds one workgroup per compute unit anyway: the cap then only makes the p >= 60 columns spill (136 to 504
-// bytes per lane), so it goes (2048 tokens, K = 26624, p = 104: 354 -> 269 us; K = 21504, p = 84: 204 -> 193 us).
-__global__ void __launch_bounds__((threads_of<P, SLICED>()), SLICED ? (P < 44 ? 4 : 2) : ALONE ? 2 : P >= 44 ? 4 : 6)
+// sliced variant serves small batches, where occupancy is not the limit.) WIDE: rows of at least 256 columns of a long Paley
+// stage, whose columns four threads share (paley_row): 1024 threads, a fourth of the registers per column. The rotation alone,
+// K = 17408, p = 68, a thread per column with 512 threads and this: 1 token 17.9 / 10.0 us, 64 tokens 14.9 / 10.9, 256 18.0 /
+// 14.2, 2048 85.2 / 73.6; K = 27648, p = 108, where LDS holds one workgroup per compute unit, 26.7 / 18.1, 28.6 / 19.4, 34.5 /
+// 25.7, 250 / 190. (Shorter chunks leave most of the 1024 threads without a column: K = 5376 = 84 x 64, one token 9.2 / 11.0.)
+__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE>()), WIDE ? (P >= 84 ? 4 : 8) : SLICED ? (P < 44 ? 4 : 2) : P >= 44 ? 4 : 6)
 rq_rotate_quant_kernel(const RotQuantArgs a) {
-    constexpr int kNT = threads_of<P, SLICED>();
+    constexpr int kNT = threads_of<P, SLICED, WIDE>();
     extern __shared__ __align__(16) float smem[];
     __shared__ float s_red[kNT / 64];
 
@@ -78,7 +80,7 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     } else if (fused_first) {
         // long Paley stages go with long rows (several units of 16 floats per thread): all of a thread's loads go
         // out before the first butterfly
-        load_row_fwht16<kNT, (P >= 44 ? 3 : 1)>(buf, xr, K, tid);
+        load_row_fwht16<kNT, (WIDE ? 2 : P >= 44 ? 3 : 1)>(buf, xr, K, tid);
     } else {
         load_row<kNT>(buf, xr, K, tid);
     }
@@ -126,12 +128,14 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
                 }
                 __syncthreads();
                 float *tmp = buf; buf = alt; alt = tmp;
+            } else if constexpr (WIDE) {
+                paley_row<P, kNT, false>(buf, K, m, a.n_rot, a.scale, tid);
             } else {
                 for (int cidx = tid; cidx < ncols; cidx += kNT) {
                     const int rb = cidx / m, j = cidx - rb * m;
                     const int b0 = rb * a.n_rot + j;
                     float col[P];
-                    if (pm == 272) {   // chunks of 256 (K = 5120, 17408): the common case, compile-time stride
+                    if (P < 44 && pm == 272) {   // chunks of 256 (K = 5120): the common case, compile-time stride
                         float *src = buf + padi(b0);
                         load_column<P, 272>(col, src, pm);
                         paley_column<P, 0, false, 272>(col, src, pm, a.scale);
@@ -321,39 +325,37 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
 }
 
 // the kernels keep a whole row in dynamic LDS: raise the per-kernel limit (once per device, see init_activation_kernels)
-template <int P, bool SLICED, bool ALONE = false>
+template <int P, bool SLICED, bool WIDE = false>
 hipError_t allow_big_lds() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, ALONE>),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, WIDE>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 64);
 }
 
-// the plain variant has an ALONE build where the cap makes its columns spill and rows of up to RQ_MAX_K floats get that
-// long (p = 68 and 72 would need chunks of 512: past RQ_MAX_K)
-constexpr bool has_alone(int p) { return p == 60 || p >= 84; }
+constexpr bool has_wide(int p) { return p >= 44; }
 
 template <int P>
 hipError_t allow_big_lds_both() {
     hipError_t e = allow_big_lds<P, false>();
     if (e == hipSuccess && P > 1) e = allow_big_lds<P, (P > 1)>();
-    if (e == hipSuccess && has_alone(P)) e = allow_big_lds<P, false, has_alone(P)>();
+    if (e == hipSuccess && has_wide(P)) e = allow_big_lds<P, false, has_wide(P)>();
     return e;
 }
 
-template <int P, bool SLICED, bool ALONE = false>
+template <int P, bool SLICED, bool WIDE = false>
 hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
     static bool attr_set = false;   // calls that never went through rq_w4a4_prepare on this device
     if (!attr_set) {
-        hipError_t e = allow_big_lds<P, SLICED, ALONE>();
+        hipError_t e = allow_big_lds<P, SLICED, WIDE>();
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    constexpr int kNT = threads_of<P, SLICED>();
+    constexpr int kNT = threads_of<P, SLICED, WIDE>();
     // blocks past the tokens clear the split-K cells, four ints per thread
     RotQuantArgs b = a;
     b.token_blocks = a.M;
     const int grid = a.M + (int) ((a.zero_ints + (int64_t) kNT * 4 - 1) / ((int64_t) kNT * 4));
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, ALONE>), dim3(grid), dim3(kNT), lds, stream, b);
+    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, WIDE>), dim3(grid), dim3(kNT), lds, stream, b);
     return hipGetLastError();
 }
 
@@ -363,12 +365,11 @@ template <int P>
 hipError_t launch_p(const RotQuantArgs &a, hipStream_t stream) {
     const size_t row = (size_t) (a.K + (a.K >> 4) + 1) * sizeof(float);
     const size_t stats = (size_t) 2 * (a.K / kGroup + 1) * sizeof(float);
+    if (has_wide(P) && a.K / P >= 256) return launch_one<P, false, has_wide(P)>(a, row + stats, stream);
     // long Paley stages: past kTwoStepTokens tokens the plain variant (two workgroups per CU) is the faster one
     if (P > 1 && a.M <= (P >= 44 ? kTwoStepTokens : 64) && 2 * row + stats <= 160 * 1024 - 64) {
         return launch_one<P, (P > 1)>(a, 2 * row + stats, stream);
     }
-    // a second workgroup does not fit beside this one
-    if (has_alone(P) && 2 * (row + stats + 64) > 160 * 1024) return launch_one<P, false, has_alone(P)>(a, row + stats, stream);
     return launch_one<P, false>(a, row + stats, stream);
 }
 
