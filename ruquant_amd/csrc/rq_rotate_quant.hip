@@ -245,23 +245,27 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
             // fp6 fragment plane: q - z as sign and magnitude, six bits each (as fp6 E2M3 the value is (q - z) / 8);
             // this word's 48 bits are bytes 6 (w % 4) .. of the 24 bytes that lane token % 32 + 32 * (half of the group)
             // holds in the fragment of 32 tokens: bytes 0 .. 15 at lane * 16, bytes 16 .. 23 at 1024 + lane * 8
-            uint64_t bits = 0;
+            // (as a float q - z has the sign where the code wants it, and its magnitude converts without it)
+            uint32_t c[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const int d = (int) (fminf(fmaxf(rintf(f[j] * inv) + zf, 0.0f), 15.0f) - zf);
-                const uint32_t code = d < 0 ? (32u | (uint32_t) (-d)) : (uint32_t) d;
-                bits |= (uint64_t) code << (6 * j);
+                const float d = __builtin_amdgcn_fmed3f(rintf(f[j] * inv) + zf, 0.0f, 15.0f) - zf;
+                c[j] = (uint32_t) fabsf(d) | ((__builtin_bit_cast(uint32_t, d) >> 26) & 32u);
             }
+            const uint32_t lo6 = c[0] | c[1] << 6 | c[2] << 12 | c[3] << 18 | c[4] << 24 | c[5] << 30;
+            const uint32_t hi6 = c[5] >> 2 | c[6] << 4 | c[7] << 10;
+            // The four words of a half group, in the four lanes of a quad, are one lane's 24 bytes of the fragment: the first
+            // lane gathers and stores its 16-byte piece, the third the 8-byte one (three 2-byte stores per lane before).
+            const uint32_t lo_n = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) lo6, 0xF5, 0xF, 0xF, false);   // quad_perm [1, 1, 3, 3]
+            const uint32_t hi_n = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) hi6, 0xF5, 0xF, 0xF, false);
+            const uint32_t lo_2 = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) lo6, 0xAA, 0xF, 0xF, false);   // quad_perm [2, 2, 2, 2]
+            const uint32_t p1 = hi6 | lo_n << 16, p2 = lo_n >> 16 | hi_n << 16;
             if (on) {
                 const int c8 = w & 7;
                 const int lane = (t & 31) + 32 * (c8 >> 2);
                 uint8_t *frag = reinterpret_cast<uint8_t *>(a.act) + ((size_t) g * (a.Mp >> 5) + (t >> 5)) * kFrag6;
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    const int o = 6 * (c8 & 3) + 2 * i;   // byte of the lane's 24
-                    uint8_t *dst = o < 16 ? frag + lane * 16 + o : frag + 1024 + lane * 8 + (o - 16);
-                    *reinterpret_cast<uint16_t *>(dst) = (uint16_t) (bits >> (16 * i));
-                }
+                if ((c8 & 3) == 0) *reinterpret_cast<uint4 *>(frag + lane * 16) = make_uint4(lo6, p1, p2, lo_2);
+                if ((c8 & 3) == 2) *reinterpret_cast<uint2 *>(frag + 1024 + lane * 8) = make_uint2(p1, p2);
                 if (c8 == 0) a.m4[(size_t) g * a.Mp + t] = 4.0f * (float) mg;
             }
             continue;
