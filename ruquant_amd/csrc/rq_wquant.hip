@@ -45,6 +45,7 @@ struct SearchArgs {
 };
 
 __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const SearchArgs a) {
+    __shared__ float4 s_x[2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
     const int tid = threadIdx.x, r = tid & 15;
     int64_t seg = (int64_t) blockIdx.x * (kSearchThreads / 16) + (tid >> 4);
     const bool live = seg < a.segments;
@@ -53,20 +54,31 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
     const float *x = a.x + row * a.ld + (seg - row * a.per_row) * (int64_t) a.n;
     const int n = a.n;
 
+    // Elements come by the sixteen lanes of a segment together, a block of 64 to a load (n is a multiple of 64). Eight loads at
+    // once here: one after the other, this pass alone would be n / 64 trips to memory.
+    constexpr int kBatch = 8;
+    const float4 *xv = reinterpret_cast<const float4 *>(x) + r;
+    const int nv = n >> 6;
+    auto block = [&](int k) { return xv[16 * (k < nv ? k : nv - 1)]; };   // (past the end: the last again)
     float amax = 0.0f;
-    for (int i = r * 4; i < n; i += 64) {
-        const float4 v = *reinterpret_cast<const float4 *>(x + i);
-        amax = fmaxf(fmaxf(fmaxf(fmaxf(amax, fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));
+    for (int i0 = 0; i0 < nv; i0 += kBatch) {
+        float4 v[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) v[j] = block(i0 + j);
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            amax = fmaxf(fmaxf(fmaxf(fmaxf(amax, fabsf(v[j].x)), fabsf(v[j].y)), fabsf(v[j].z)), fabsf(v[j].w));
+        }
     }
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 16));
 
-    float s = 0.0f;
-    double err = INFINITY;
-    if (amax > 0.0f && r < kRatios) {
-        s = amax * (1.0f - 0.025f * (float) r) / 7.0f;
+    // (the lanes that try no ratio go through the loop too: they fetch for the others)
+    const bool tries = amax > 0.0f && r < kRatios;
+    const float s = tries ? amax * (1.0f - 0.025f * (float) r) / 7.0f : 1.0f;
+    double err = 0.0;
+    if (__any(tries)) {
         const float rs = 1.0f / s;
-        err = 0.0;
         // What bounds this loop: a lane's error sum is a chain of n additions in element order, and there are only
         // 13 lanes per segment to hide it with (6144 rows: 1.5 wavefronts per SIMD), so everything in front of the
         // addition is worked out for kRun elements at once, independent of each other, and the next run's elements
@@ -79,23 +91,27 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
         // 236 us with four runs in flight. 4096 rows, a wavefront per SIMD: 222 us with the error in double precision from the
         // start (two conversions, a subtraction, a product and a sum, of which a conversion takes four times as long as a
         // sum), 178 us with one conversion and one FMA.
-        constexpr int kRun = 8, kAhead = 4;   // (segments are multiples of 64 floats)
+        // A block goes through LDS, where every lane reads its segment's elements, and is requested three blocks before it is
+        // worked on. Search and encoding, 5120 inputs, with this and the batched first pass, before and after: 2048 rows 169 /
+        // 137 us, 4096 229 / 173 (a wavefront per SIMD), 6144 241 / 187. (Every lane read its segment for itself, four
+        // runs ahead: four times the load instructions.)
+        constexpr int kRun = 8;
         const bool normal = rs < 1e37f && rs > 2e-38f;
-        float4 ring[kAhead][2];
+        float4 ahead[2] = { block(1), block(2) };
+        s_x[0][tid] = block(0);
+        for (int k0 = 0; k0 < nv; k0 += 2) {
 #pragma unroll
-        for (int d = 0; d < kAhead; ++d) {
-            ring[d][0] = *reinterpret_cast<const float4 *>(x + kRun * d);
-            ring[d][1] = *reinterpret_cast<const float4 *>(x + kRun * d + 4);
-        }
-        for (int i0 = 0; i0 < n; i0 += kRun * kAhead) {
-            // (past the end: the first elements again, unused)
-            const float *next = x + (i0 + kRun * kAhead < n ? i0 + kRun * kAhead : 0);
+          for (int h = 0; h < 2; ++h) {
+            const int k = k0 + h;
+            if (k >= nv) break;   // (uniform)
+            s_x[h ^ 1][tid] = ahead[h];
+            ahead[h] = block(k + 3);
+            // (one wavefront: its LDS operations are carried out in order)
+            asm volatile("" ::: "memory");
 #pragma unroll
-            for (int d = 0; d < kAhead; ++d) {
-                const float xs[kRun] = { ring[d][0].x, ring[d][0].y, ring[d][0].z, ring[d][0].w,
-                                         ring[d][1].x, ring[d][1].y, ring[d][1].z, ring[d][1].w };
-                ring[d][0] = *reinterpret_cast<const float4 *>(next + kRun * d);
-                ring[d][1] = *reinterpret_cast<const float4 *>(next + kRun * d + 4);
+            for (int d = 0; d < 64 / kRun; ++d) {
+                const float4 x0 = s_x[h][(tid & 48) + 2 * d], x1 = s_x[h][(tid & 48) + 2 * d + 1];
+                const float xs[kRun] = { x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w };
                 float q[kRun], off[kRun];
 #pragma unroll
                 for (int j = 0; j < kRun; ++j) {
@@ -108,7 +124,7 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
                 float far = absmax3_raw(0.0f, off[0], off[1]);
 #pragma unroll
                 for (int j = 2; j < kRun; j += 2) far = absmax3_raw(far, off[j], off[j + 1]);
-                if (!(normal && far < 0.49999f)) {
+                if (tries && !(normal && far < 0.49999f)) {
 #pragma unroll
                     for (int j = 0; j < kRun; ++j) q[j] = fminf(fmaxf(rintf(xs[j] / s), -8.0f), 7.0f);
                 }
@@ -123,8 +139,10 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
 #pragma unroll
                 for (int j = 0; j < kRun; ++j) err = __builtin_fma(e[j], e[j], err);
             }
+          }
         }
     }
+    if (!tries) err = INFINITY;
     // first smallest error in ratio order, as the reference's `err < best_err` scan
     const int base = (tid & 63) & ~15;
     float best_s = 0.0f;
@@ -246,8 +264,12 @@ __device__ __forceinline__ int weight_mult(int32_t sum, int g) {
     return 1;
 }
 
-template <int P>
-__global__ void __launch_bounds__(512) rq_dequant_rows_kernel(const DequantArgs a) {
+// WIDE: rows of at least 256 columns of a long Paley stage, whose columns four threads share (paley_row), 1024 threads. A thread
+// per column with 512 threads and this, K = 17408, p = 68: 64 rows 16.3 / 12.0 us, 427 rows 34.3 / 23.4, 2048 rows 128 / 82;
+// K = 27648, p = 108, 2048 rows 252 / 174. (p = 44, K = 11264: 427 rows 13.3 / 14.4, so it stays.)
+template <int P, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 1024 : 512) rq_dequant_rows_kernel(const DequantArgs a) {
+    constexpr int kNT = WIDE ? 1024 : 512;
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
@@ -256,7 +278,7 @@ __global__ void __launch_bounds__(512) rq_dequant_rows_kernel(const DequantArgs 
     float *o = a.out + row * a.ldo;
     float *buf = smem;
 
-    for (int w = tid; w < nw; w += 512) {
+    for (int w = tid; w < nw; w += kNT) {
         const rq_block_w4a4 &blk = in[w >> 5];
         const int ww = w & 31;
         const uint32_t word = blk.qs[ww];
@@ -290,12 +312,14 @@ __global__ void __launch_bounds__(512) rq_dequant_rows_kernel(const DequantArgs 
 
     const int m = a.m;
     const int lm = __ffs(m) - 1;
-    fwht_row(buf, K, lm, tid, 512);
-    if constexpr (P > 1) {
+    fwht_row(buf, K, lm, tid, kNT);
+    if constexpr (WIDE) {
+        paley_row<P, kNT, true>(buf, K, m, a.n_rot, a.scale, tid);
+    } else if constexpr (P > 1) {
         const int ncols = K / P;
         const bool m16 = (m & 15) == 0;
         const int pm = m + (m >> 4);
-        for (int cidx = tid; cidx < ncols; cidx += 512) {
+        for (int cidx = tid; cidx < ncols; cidx += kNT) {
             const int rb = cidx / m, j = cidx - rb * m;
             const int b0 = rb * a.n_rot + j;
             float col[P];
@@ -311,27 +335,35 @@ __global__ void __launch_bounds__(512) rq_dequant_rows_kernel(const DequantArgs 
             }
         }
     } else {
-        for (int i = tid; i < K; i += 512) buf[padi(i)] = buf[padi(i)] * a.scale;
+        for (int i = tid; i < K; i += kNT) buf[padi(i)] = buf[padi(i)] * a.scale;
     }
     __syncthreads();
-    for (int i = tid * 4; i < K; i += 512 * 4) {
+    for (int i = tid * 4; i < K; i += kNT * 4) {
         const float *sp = buf + padi(i);
         *reinterpret_cast<float4 *>(o + i) = make_float4(sp[0], sp[1], sp[2], sp[3]);
     }
 }
 
-template <int P>
-hipError_t launch_dequant(const DequantArgs &a, int64_t rows, hipStream_t stream) {
+template <int P, bool WIDE>
+hipError_t launch_dequant_form(const DequantArgs &a, int64_t rows, hipStream_t stream) {
     const size_t lds = a.rotate ? (size_t) (a.K + (a.K >> 4) + 1) * sizeof(float) : 0;
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_dequant_rows_kernel<P>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_dequant_rows_kernel<P, WIDE>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 64);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    hipLaunchKernelGGL((rq_dequant_rows_kernel<P>), dim3((unsigned) rows), dim3(512), lds, stream, a);
+    hipLaunchKernelGGL((rq_dequant_rows_kernel<P, WIDE>), dim3((unsigned) rows), dim3(WIDE ? 1024 : 512), lds, stream, a);
     return hipGetLastError();
+}
+
+template <int P>
+hipError_t launch_dequant(const DequantArgs &a, int64_t rows, hipStream_t stream) {
+    if constexpr (P >= 60) {
+        if (a.K / P >= 256) return launch_dequant_form<P, true>(a, rows, stream);
+    }
+    return launch_dequant_form<P, false>(a, rows, stream);
 }
 
 bool factor(int64_t n, int &p, int &m) { return rq_w4a4_hadamard_factor(n, &p, &m) != 0; }
