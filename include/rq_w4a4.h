@@ -87,7 +87,8 @@ size_t rq_w4a4_prepared_bytes(int64_t K, int64_t N);
  * call ends by waiting for `stream` and reading one word of the result back: whether the tensor carries weight
  * multipliers, which the wide-batch launcher remembers per prepared address to choose between two kernels (both are
  * right for every tensor; a prepared weight that is copied to another address, or prepared under capture, runs the
- * one that is slow on tensors with multipliers). */
+ * one that is slow on tensors with multipliers). The prepared bytes hold no address of themselves: a copy works
+ * whatever becomes of the original. */
 int rq_w4a4_prepare(const void *w_blocks_dev, int64_t K, int64_t N,
                     void *prepared_dev, size_t prepared_bytes, rq_stream_t stream);
 

@@ -294,7 +294,7 @@ rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const floa
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint8_t *w6 = reinterpret_cast<const uint8_t *>((uintptr_t) *reinterpret_cast<const unsigned long long *>(flags + 2));
+    const uint8_t *w6 = plane6_of(flags);
     const bool hask = flags[0] & 1;
     Src s;
     s.a = (gbyte *) (w6 + ((size_t) (panel >> 2) * ng * 8 + 2 * (panel & 3)) * kFrag6);

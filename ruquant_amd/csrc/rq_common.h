@@ -32,7 +32,7 @@ constexpr int kGemvMaxTokens = 64;  // workspaces of up to this many tokens hold
 //   s_w   : n_panels x 64 floats (rows past N are zero).
 //   kmul  : n_panels x ng x 64 bytes, the integer weight multiplier of (row, group): 1 for legacy headers.
 //   flags : one int32; bit 0 set when any multiplier differs from 1 (kernels branch on it, uniformly). At byte 8 of
-//           the section: the device address of the fp6 plane below (0: none), which the fp6 GEMM reads from there.
+//           the section: where the fp6 plane below lies (plane6_of), which the fp6 kernels read from there.
 //   w6    : (unless RQ_GEMM_FP6=0) the same codes once more as fp6 (E2M3) MFMA fragments for wide token batches:
 //           n_rtiles x ng x 8 fragments x 1536 bytes. Fragment f of row tile R (rows 256 R + 32 f ..), group g:
 //           lane l = row % 32 + 32 * half holds inputs 64 g + 32 half .. + 31 as 32 six-bit values (sign, then the
@@ -45,10 +45,19 @@ constexpr int kFrag6 = 1536;      // bytes of one 32 x 64 fp6 MFMA fragment
 constexpr int kRowTile6 = 256;    // rows of one tile of the fp6 plane
 
 // The flag region of a prepared weight: int 0 = the flag word (bit 0: some weight multiplier differs from 1), ints 2-3 =
-// the device address of the fp6 plane; behind these 256 bytes, kFlagReplicas copies of the flag word, one per 64-byte
+// where the fp6 plane lies; behind these 256 bytes, kFlagReplicas copies of the flag word, one per 64-byte
 // line, for the one-token kernel, whose 2048 stream wavefronts would otherwise all read the one line.
 constexpr int kFlagReplicas = 32;
 constexpr size_t kFlagRegionBytes = 256 + 64 * kFlagReplicas;
+
+// Where the fp6 plane lies, as the flag region keeps it. A plane inside the prepared buffer: its distance from the flag
+// word with bit 0 set, so that prepared bytes work at any address they are copied to, whatever becomes of the
+// original. A plane in a buffer of its own (a weight prepared in place): its device address, which is a multiple of 256.
+// 0: no plane.
+__device__ __forceinline__ const uint8_t *plane6_of(const int32_t *flags) {
+    const uint64_t v = *reinterpret_cast<const unsigned long long *>(flags + 2);
+    return reinterpret_cast<const uint8_t *>((uintptr_t) ((v & ~(uint64_t) 1) + (v & 1 ? (uint64_t) (uintptr_t) flags : 0)));
+}
 
 struct PreparedLayout {
     int64_t K, N;

@@ -541,9 +541,7 @@ rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const f
     const int s_begin = sliced ? (int) ((int64_t) (ng / 2) * part / parts) : 0;
     const int s_end = sliced ? (int) ((int64_t) (ng / 2) * (part + 1) / parts) : ng / 2;
     const int tid = threadIdx.x;
-    // the fp6 plane's address stands beside the flag word (it is inside the prepared buffer, or, for a weight that was
-    // prepared in place, a buffer of its own)
-    const uint8_t *w6 = reinterpret_cast<const uint8_t *>((uintptr_t) *reinterpret_cast<const unsigned long long *>(flags + 2));
+    const uint8_t *w6 = plane6_of(flags);
     // (read up here, in front of the assembly statements: behind them the compiler takes the word as possibly overwritten
     // and fetches it with a vector load, whose wait stands for a trip to memory between the set-up and the first group, 0.4
     // to 1 us of every launch)

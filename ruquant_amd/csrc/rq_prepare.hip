@@ -86,13 +86,12 @@ __global__ void __launch_bounds__(256) rq_prepare6_kernel(const rq_block_w4a4 *_
     *reinterpret_cast<uint2 *>(dst + 1024 + lane * 8) = make_uint2(out[4], out[5]);
 }
 
-// the flag word of a prepared weight and, beside it, the device address of its fp6 plane (0: none), which the fp6
-// GEMM reads from here: the plane may live inside the prepared buffer or, for a weight prepared in place, elsewhere
-__global__ void rq_finish_flags_kernel(int32_t *flags, const int32_t *from, const uint8_t *plane6) {
+// the flag word of a prepared weight and, beside it, where its fp6 plane lies (plane6_of)
+__global__ void rq_finish_flags_kernel(int32_t *flags, const int32_t *from, unsigned long long plane6) {
     const int32_t f = from ? from[0] : flags[0];
     if (threadIdx.x == 0) {
         flags[0] = f;
-        *reinterpret_cast<unsigned long long *>(flags + 2) = (unsigned long long) (uintptr_t) plane6;
+        *reinterpret_cast<unsigned long long *>(flags + 2) = plane6;
     }
     if (threadIdx.x < kFlagReplicas) flags[64 + 16 * threadIdx.x] = f;   // (the copies: a 64-byte line each)
 }
@@ -116,7 +115,7 @@ hipError_t launch_prepare(const void *blocks, const PreparedLayout &L, uint8_t *
                            prepared + L.off_w6);
     }
     hipLaunchKernelGGL(rq_finish_flags_kernel, dim3(1), dim3(64), 0, stream, flags, (const int32_t *) nullptr,
-                       L.off_w6 != 0 ? prepared + L.off_w6 : (const uint8_t *) nullptr);
+                       L.off_w6 != 0 ? (unsigned long long) (L.off_w6 - L.off_flags) | 1 : 0ull);
     return hipGetLastError();
 }
 
@@ -169,7 +168,8 @@ hipError_t launch_prepare_inplace(void *blocks, const PreparedLayout &L, uint8_t
     e = hipMemcpyAsync(base + L.off_kmul, side_kmul, (size_t) L.n_panels * L.ng * kPanelRows, hipMemcpyDeviceToDevice, stream);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(rq_finish_flags_kernel, dim3(1), dim3(64), 0, stream,
-                       reinterpret_cast<int32_t *>(base + L.off_flags), side_flags, plane6);
+                       reinterpret_cast<int32_t *>(base + L.off_flags), side_flags,
+                       (unsigned long long) (uintptr_t) plane6);
     return hipGetLastError();
 }
 

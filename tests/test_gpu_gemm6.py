@@ -132,6 +132,26 @@ def test_weight_multipliers_at_an_address_the_library_has_not_seen(oracle):
     assert bits_equal(got, want), first_mismatch(got, want)
 
 
+@pytest.mark.parametrize("in_place", [False, True], ids=["one_buffer", "plane_apart"])
+@pytest.mark.parametrize("N,M", [(6200, 40), (8300, 40), (570, 200), (570, 1100), (300, 3)])
+def test_a_moved_weight_needs_nothing_of_its_original(oracle, N, M, in_place):
+    """Prepared bytes copied to another address, the original overwritten: every kernel that reads the fp6 plane (small
+    units, tiles, K slices) or the int4 panels gives the same bits. (Of a weight prepared in place the plane is a buffer of
+    its own, which the caller keeps.)"""
+    K, type_ = 2560, rq.TYPE_W4A4
+    blocks, wf = adversarial_weights(oracle, N, K, type_, seed=M)
+    W = rq.W4A4Weight(blocks, type_, DEV, in_place=in_place)
+    x = adversarial_activations(M, K, type_, wf, seed=M)
+    want = oracle.mul_mat(type_, blocks, x, W.clip)
+    original = W.prepared
+    moved = torch.empty(original.numel() + 4096, dtype=torch.uint8, device=DEV)[2048:2048 + original.numel()]
+    moved.copy_(original)
+    original.fill_(0x5A)
+    W.prepared = moved
+    got = run_gpu(W, x)
+    assert bits_equal(got, want), first_mismatch(got, want)
+
+
 @pytest.mark.parametrize("M", [65, 128, 129, 300])
 def test_token_counts_around_the_tile(oracle, M):
     """One and a few token tiles, partly filled, K = 5120 (every tile cut along K: few tiles, long rows)."""
@@ -245,14 +265,13 @@ def test_sets_of_weights(oracle, K, M, Ns, wgroups, moved, launches):
     """Sets whose tiles are cut, whole and in super-tiles that straddle weights, against the oracle, with outputs of their
     own row strides."""
     type_ = rq.TYPE_W4A4
-    ws, bl, kept = [], [], []
+    ws, bl = [], []
     for i, (N, g) in enumerate(zip(Ns, wgroups)):
         b, wf = adversarial_weights(oracle, N, K, type_, seed=60 + i, wgroup=g)
         w = rq.W4A4Weight(b, type_, DEV)
         if moved:
             copy = torch.empty(w.prepared.numel() + 4096, dtype=torch.uint8, device=DEV)[2048:2048 + w.prepared.numel()]
             copy.copy_(w.prepared)
-            kept.append(w.prepared)   # (the copy's fp6 plane is the original's)
             w.prepared = copy
         bl.append(b)
         ws.append(w)
