@@ -35,7 +35,7 @@ constexpr int kUnitsPerTile = 8;               // 4 panels x 2 runs of 64 tokens
 constexpr int depth_of(bool hask) { return hask ? 2 : 4; }
 constexpr int kTokStride = kPanelRows + 4;     // ints between tokens of a wavefront's totals in LDS
 constexpr float kBias = 12582912.0f;           // 1.5 x 2^23
-constexpr int kBiasBits = 0x4B400000;
+constexpr uint32_t kBiasBits = 0x4B400000;
 constexpr int kFlushGroups = 28;               // (and the tile of one more that is folded late): less than 2^22
 
 template <bool HASK>
@@ -97,7 +97,9 @@ __device__ __forceinline__ void load_frag(Frag<HASK> &f, const Src &s, int wave,
 // What a wavefront carries from group to group: the totals of its 64 x 64 outputs and the tile whose fold is still due.
 // Without weight multipliers `acc` is the biased float accumulator of the tiled kernel; with them a group's term, which may
 // be 15 times as large, is formed on the bias by an FMA of its own and its bit pattern is added up in integers
-// (acc holds those; the bias of every term comes off at the end).
+// (acc holds those; the bias of every term comes off at the end). The sum of the patterns passes 2^32 from the fourth group on:
+// unsigned, modulo 2^32, which gives the total back, since that is small: at most 64 groups of a wavefront x 15 x 122,400 =
+// 117.5 M, and 940 M over the eight.
 struct State {
     float acc[2][2][16];
     v16f P;
@@ -139,7 +141,7 @@ __device__ __forceinline__ void group_units(const Frag<true> &f, State &st) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const float term = __builtin_fmaf(S[b][r], kf * f.m4[b], st.bias);
-                st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(int, st.acc[a][b][r]) + __builtin_bit_cast(int, term));
+                st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, st.acc[a][b][r]) + __builtin_bit_cast(uint32_t, term));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -159,7 +161,7 @@ __device__ __forceinline__ void flush(State &st, int *part, int lane) {
                 v4i v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    v[e] = __builtin_bit_cast(int, st.acc[a][b][4 * q + e]) - kBiasBits;
+                    v[e] = (int) (__builtin_bit_cast(uint32_t, st.acc[a][b][4 * q + e]) - kBiasBits);
                     st.acc[a][b][4 * q + e] = kBias;
                 }
                 *dst = FRESH ? v : *dst + v;
@@ -217,13 +219,13 @@ __device__ __forceinline__ void stream(const Src &s, int wave, int lane, int n, 
     }
     if constexpr (HASK) {
         // n terms, each with the bias's bit pattern on it
-        const int off = n * kBiasBits - kBiasBits;   // (flush takes one off)
+        const uint32_t off = (uint32_t) n * kBiasBits - kBiasBits;   // (flush takes one off)
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(int, st.acc[a][b][r]) - off);
+                for (int r = 0; r < 16; ++r) st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, st.acc[a][b][r]) - off);
             }
         }
     } else {

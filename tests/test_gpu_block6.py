@@ -63,6 +63,36 @@ def test_extreme_sums_between_two_transfers(oracle):
     assert bits_equal(got, want), first_mismatch(got, want)
 
 
+def test_extreme_sums_with_weight_multipliers(oracle):
+    """The longest row with a multiplier of 15 on every group: 64 groups per wavefront, whose terms of up to 1.836 M each are
+    added as bit patterns, modulo 2^32, the bias of every one still on it. Rows of all -8 / all 7 / both in turn against tokens
+    of q - z = +-15 with m = 255: totals of 117.5 M per wavefront and 940 M per output, both signs."""
+    K, M, panels, type_ = 32768, 40, 129, rq.TYPE_W4A4
+    rng = np.random.default_rng(3)
+    codes = rng.integers(-8, 8, size=(64, K), dtype=np.int8)
+    codes[0] = -8
+    codes[1] = 7
+    codes[2] = np.where((np.arange(K) // 64) % 2 == 0, -8, 7)
+    units = np.abs(rng.normal(0.02, 0.005, size=64)).astype(np.float32)
+    mults = rng.integers(1, 16, size=(64, K // 64), dtype=np.int32)
+    mults[:3] = 15
+    panel = rq.pack_groups(codes, units, mults)
+    W = rq.W4A4Weight(np.tile(panel, (panels, 1)), type_, DEV, keep_blocks=False)
+    x = synth.activations("outlier_channels", M, K, 9)
+    x[0] = 1.0
+    x[1] = -1.0
+    x[2] = np.where((np.arange(K) // 64) % 2 == 0, 1.0, -1.0)
+    x[39] = 0.5
+    want = oracle.mul_mat(type_, panel, x, W.clip)
+    got = run_gpu(W, x).reshape(M, panels, 64)
+    for p in (0, 1, 64, 128):
+        assert bits_equal(got[:, p], want), first_mismatch(got[:, p], want)
+    assert (got == got[:, :1]).all()
+    unit = np.float32(1.0) / np.float32(3825.0)
+    expect = (np.float32(-15 * 122400 * (K // 64)) * np.float32(16.0)) * unit * units[0]
+    assert got[0, 0, 0] == np.float32(expect)
+
+
 @pytest.mark.parametrize("M", [40, 70])
 def test_a_set_of_weights(oracle, M):
     """Three weights, with and without multipliers, whose panels do not end with a row tile, in one launch (40 tokens) or one
