@@ -245,6 +245,26 @@ int rq_w4a4_dequantize(int type, const void *blocks_dev, int64_t rows, int64_t K
  * P:2163-2172); for hosts and benchmarks that time or capture the stages separately. */
 int rq_w4a4_stage_mask(int type, int64_t K, int64_t M, int64_t n_rot);
 
+/* What rq_w4a4_mul_mat_fused (once != 0: _fused_once; n = 1: rq_w4a4_mul_mat / _once) runs for n weights of N[i] rows and
+ * M >= 1 tokens with a workspace of workspace_bytes; multipliers: bit i set when weight i carries weight multipliers and
+ * the library knows it (rq_w4a4_prepare's note). A host query for tests and benchmarks that mean one kernel: writes
+ * RQ_PLAN_FIELDS numbers to plan, those below the launches only for RQ_KERNEL_FP6 and summed over the launches. No
+ * counterpart in the reference. */
+#define RQ_PLAN_KERNEL   0   /* RQ_KERNEL_* */
+#define RQ_PLAN_LAUNCHES 1   /* product launches: 1, or one per weight */
+#define RQ_PLAN_WHOLE    2   /* tiles of 256 rows x 128 tokens that run whole */
+#define RQ_PLAN_CUT      3   /* tiles that are cut along K */
+#define RQ_PLAN_SLICES   4   /* slices of such a tile (the most of any launch; 1: none is cut) */
+#define RQ_PLAN_UNITS    5   /* units of 64 rows x 64 tokens */
+#define RQ_PLAN_FIELDS   6
+#define RQ_KERNEL_DECODE 1   /* one token, one launch */
+#define RQ_KERNEL_GEMV   2
+#define RQ_KERNEL_SKINNY 3
+#define RQ_KERNEL_FP6    4   /* the fp6 product: tiles, slices, units */
+#define RQ_KERNEL_INT8   5   /* the int8 product (RQ_GEMM_FP6=0) */
+int rq_w4a4_product_plan(int type, int n, int64_t K, const int64_t *N, int64_t M, int64_t n_rot, int multipliers, int once,
+                         size_t workspace_bytes, int64_t *plan);
+
 /* Library version, for the host binding to check: bumped whenever an entry point, an error code or the meaning of an
  * argument changes. A binding built against this header refuses a library that reports another number. (An entry point
  * that is only added leaves the number: everything an older binding calls is as it was, and a binding that needs it finds

@@ -170,17 +170,96 @@ Path path_of(int64_t M) {
     return M <= kGemvMax ? kPathGemv : kPathSkinny;
 }
 
+// How a call's workspace is used. The streaming kernels serve all the weights of a fused call in one launch when it has
+// split-K cells for all their rows (rq_w4a4_workspace_bytes with N = the padded sum); with cells for the largest weight
+// only, the products are launched one after the other. Everything else in the workspace does not depend on N.
+struct Space {
+    WorkspaceLayout W;
+    int64_t Ncells;       // rows with split-K cells
+    bool    one_launch;
+    bool    have_slabs;   // (fp6 GEMM: room to cut leftover tiles along K)
+};
+
+Space space_of(int n, int64_t K, const int64_t *N, int64_t M, size_t ws_bytes) {
+    int64_t Nmax = 0, Nsum = 0;
+    for (int i = 0; i < n; ++i) {
+        if (N[i] > Nmax) Nmax = N[i];
+        Nsum += (N[i] + kPanelRows - 1) / kPanelRows * kPanelRows;
+    }
+    Space s;
+    s.W = workspace_layout(K, Nmax, M);
+    s.Ncells = Nmax;
+    s.one_launch = false;
+    if (n > 1) {
+        const WorkspaceLayout Wsum = workspace_layout(K, Nsum, M);
+        if (ws_bytes >= Wsum.bytes_min) {
+            s.W = Wsum;
+            s.Ncells = Nsum;
+            s.one_launch = true;
+        }
+    }
+    s.have_slabs = ws_bytes >= s.W.bytes;
+    return s;
+}
+
+// What a call runs (behind the one-launch kernel of one token), from its sizes and from which weights are noted to carry
+// multipliers (mult, looked at above 32 tokens only).
+struct Choice {
+    Path path;
+    bool two_step;   // rotation and quantizer in launches of their own
+    bool small6;     // up to 64 tokens through the small units of the fp6 product
+    bool fp6;        // the activations as fp6 fragments
+    int  n_launch;   // product launches: one for all weights, or one each
+};
+
+Choice choose(int n, int64_t K, const int64_t *N, int64_t M, bool rotate, int p, int m, bool once, const bool *mult, const Space &s) {
+    const int G = env().act_group;
+    Choice c;
+    c.path = path_of(M);
+    // Skinny batches with a long Paley stage: one workgroup per token would leave most of the chip idle for tens of
+    // microseconds, so the rotation runs spread over workgroups (ranges out) and a second small kernel quantizes.
+    // (up to 40 tokens: from there on the one-workgroup-per-token kernel has enough tokens to fill the chip: K = 17408,
+    // 64 tokens: 17.9 us against 21.2 us)
+    // (the second kernel reads ranges per run of 64: activation groups of 64 only)
+    c.two_step = c.path == kPathSkinny && G == kGroup && rotate && p >= 44 && (m & 63) == 0 && M <= kTwoStepTokens;
+    // 33 .. 64 tokens of a call that shares its activation with no other: the small units of the fp6 product where they are
+    // the faster ones (block6_takes); they read the activations as the fp6 GEMM does
+    c.small6 = false;
+    if (c.path == kPathSkinny && once && G == kGroup && gemm_fp6_enabled() && !c.two_step) {
+        int64_t panels = 0;
+        for (int i = 0; i < n; ++i) panels += (N[i] + kPanelRows - 1) / kPanelRows;
+        c.small6 = block6_takes(panels, M);
+    }
+    c.fp6 = c.small6 || (c.path == kPathGemm && gemm_fp6_enabled());
+    bool one = s.one_launch;
+    if (c.path == kPathGemm) {
+        // (the fp6 GEMM's slabs do not depend on N, so it needs no room beyond the largest weight's. It runs weights with and
+        // without multipliers through different kernels: a set that has both kinds goes weight by weight. K = 5120, 2048
+        // tokens, N = 6144 + 1024 + 1024: the three launches leave 128, 64 and 64 tiles over to be cut along K, one launch is
+        // two whole rounds of tiles)
+        one = c.fp6 && G == kGroup;
+        for (int i = 1; i < n && one; ++i) one = mult[i] == mult[0];
+        if (one && n > 1 && s.have_slabs) {   // (without room for slabs no tile is cut, and one launch never has more rounds)
+            FusedWeights fw;
+            memset(&fw, 0, sizeof fw);
+            fw.n = n;
+            for (int i = 0; i < n; ++i) fw.L[i] = prepared_layout(K, N[i]);
+            one = gemm6_one_launch(fw, M, mult[0]);
+        }
+    }
+    c.n_launch = one ? 1 : n;
+    return c;
+}
+
 // once: no stage-2 call will use what this call leaves in the workspace
 int run_products(int type, int n, const void *const *prepared, int64_t K, const int64_t *N, const float *x,
                  int64_t ldx, int64_t M, float *const *y, const int64_t *ldy, float clip, int64_t n_rot, void *ws,
                  size_t ws_bytes, hipStream_t stream, int stages = 3, bool once = false) {
     if (n < 1 || n > 3 || !prepared || !N || !y || !ldy || !x || !ws) return RQ_E_ARGUMENT;
-    int64_t Nmax = 0;
     for (int i = 0; i < n; ++i) {
         if (!shape_ok(type, K, N[i], M)) return RQ_E_UNSUPPORTED;
         if (!prepared[i] || !y[i] || ldy[i] < N[i]) return RQ_E_ARGUMENT;
         if ((reinterpret_cast<uintptr_t>(prepared[i]) & 255) != 0) return RQ_E_WORKSPACE;
-        if (N[i] > Nmax) Nmax = N[i];
     }
     if (!(clip > 0.0f) || !isfinite(clip)) return RQ_E_ARGUMENT;
     if (ldx < K || (ldx * 4) % 16 != 0 || (reinterpret_cast<uintptr_t>(x) & 15) != 0) return RQ_E_ARGUMENT;
@@ -188,23 +267,9 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     if (!rotation_of(type, K, n_rot, p, m)) return RQ_E_ARGUMENT;
     if (M == 0) return 0;
 
-    // The streaming kernels serve all the weights of a fused call in one launch when the workspace has split-K cells
-    // for all their rows (rq_w4a4_workspace_bytes with N = the padded sum); with cells for the largest weight only,
-    // the products are launched one after the other. Everything else in the workspace does not depend on N.
-    int64_t Nsum = 0;
-    for (int i = 0; i < n; ++i) Nsum += (N[i] + kPanelRows - 1) / kPanelRows * kPanelRows;
-    WorkspaceLayout W = workspace_layout(K, Nmax, M);
-    bool one_launch = false;
-    if (n > 1) {
-        const WorkspaceLayout Wsum = workspace_layout(K, Nsum, M);
-        if (ws_bytes >= Wsum.bytes_min) {
-            W = Wsum;
-            one_launch = true;
-        }
-    }
-    const int64_t Ncells = one_launch ? Nsum : Nmax;
+    const Space sp = space_of(n, K, N, M, ws_bytes);
+    const WorkspaceLayout &W = sp.W;
     if (ws_bytes < W.bytes_min || (reinterpret_cast<uintptr_t>(ws) & 255) != 0) return RQ_E_WORKSPACE;
-    const bool have_slabs = ws_bytes >= W.bytes;   // (fp6 GEMM: room to cut leftover tiles along K)
     uint8_t *wsb = reinterpret_cast<uint8_t *>(ws);
 
     // Activation groups of 128 / 256 (RQ_ACT_GROUP) change where the per-group floor falls. The GEMV and the skinny
@@ -235,7 +300,11 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         d.compute_units = device_compute_units();
         return (int) launch_decode(d, stream);
     }
-    const Path path = path_of(M);
+    bool mult[kMaxFused] = {};
+    for (int i = 0; i < n && M > 32; ++i) mult[i] = multipliers_noted(prepared[i]);
+    const Choice ch = choose(n, K, N, M, type == RQ_TYPE_W4A4H, p, m, once, mult, sp);
+    const Path path = ch.path;
+    const bool two_step = ch.two_step, small6 = ch.small6, fp6 = ch.fp6;
     const bool gemm = path != kPathGemv;   // the int8 digit planes feed both MFMA kernels
     RotQuantArgs q;
     memset(&q, 0, sizeof q);
@@ -250,30 +319,15 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     q.scale = 1.0f / sqrtf((float) q.n_rot);
     q.clip = clip;
     q.G = G;   // (the GEMV path takes ranges per run of 64 whatever G is, and folds them itself: set below)
-    // Skinny batches with a long Paley stage: one workgroup per token would leave most of the chip idle for tens of
-    // microseconds, so the rotation runs spread over workgroups (ranges out) and a second small kernel quantizes.
-    // (up to 40 tokens: from there on the one-workgroup-per-token kernel has enough tokens to fill the chip: K = 17408,
-    // 64 tokens: 17.9 us against 21.2 us)
-    // (the second kernel reads ranges per run of 64: activation groups of 64 only)
-    const bool two_step = path == kPathSkinny && G == kGroup && q.rotate && p >= 44 && (m & 63) == 0 && M <= kTwoStepTokens;
     q.mode = gemm && !two_step ? kActI8 : kActStats;
     q.u = reinterpret_cast<float *>(wsb + W.off_u);
     q.act = reinterpret_cast<uint32_t *>(wsb + W.off_i8);
-    // 33 .. 64 tokens of a call that shares its activation with no other: the small units of the fp6 product where they are
-    // the faster ones (block6_takes); they read the activations as the fp6 GEMM does
-    bool small6 = false;
-    if (path == kPathSkinny && once && G == kGroup && gemm_fp6_enabled() && !two_step) {
-        int64_t panels = 0;
-        for (int i = 0; i < n; ++i) panels += (N[i] + kPanelRows - 1) / kPanelRows;
-        small6 = block6_takes(panels, M);
-    }
     // token stride of the digit planes: the GEMM pads to its tile; the skinny kernel wants them dense (a padded
     // plane would put all of its reads on the few L2 channels that the used 256 bytes of every 2 KB map to)
     const int act_mp = path == kPathSkinny && !small6 ? (int) ((M + 15) / 16 * 16) : (int) W.Mp;
     q.Mp = act_mp;
     // the skinny path: one plane of q - z and the multipliers beside it (half the activation bytes per group, which
     // count against the weight bytes a compute unit can have in flight)
-    const bool fp6 = small6 || (path == kPathGemm && gemm_fp6_enabled());
     const bool single = path == kPathSkinny && !small6;
     q.single = fp6 ? 2 : single;
     q.m4 = reinterpret_cast<float *>(wsb + W.off_i8 + act6_plane_bytes((int) (K / kGroup), W.Mp));
@@ -323,7 +377,7 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
         // only the token slots this call can touch: [min(M, 8)][padded rows] cells of two ints
         const int64_t slots = M < kGemvTokens ? M : kGemvTokens;
-        q.zero_ints = 2 * slots * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
+        q.zero_ints = 2 * slots * (int64_t) ((sp.Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
     } else if (path == kPathSkinny && !small6) {
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
         // A stage-2 call may follow with any weight of at most N rows, whose plan cuts other panels than this call's:
@@ -332,11 +386,10 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         // compute unit holds one or two; 34.5 us, 33.7 with the cells of the 16 cut panels alone.)
         int64_t cells = 0;
         if (!once) {
-            cells = M * (int64_t) ((Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
+            cells = M * (int64_t) ((sp.Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);
         } else {
-            const int n_launch = one_launch ? 1 : n;
-            for (int l = 0; l < n_launch; ++l) {
-                const int64_t c = skinny_cells(skinny_args(weights_of(l, n_launch)));
+            for (int l = 0; l < ch.n_launch; ++l) {
+                const int64_t c = skinny_cells(skinny_args(weights_of(l, ch.n_launch)));
                 if (c > cells) cells = c;
             }
         }
@@ -358,18 +411,8 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
     if (!(stages & 2)) return 0;
 
     // launches: one for all weights, or one per weight
-    // (the fp6 GEMM's slabs do not depend on N, so it needs no room beyond the largest weight's. It runs weights with and
-    // without multipliers through different kernels: a set that has both kinds goes weight by weight. K = 5120, 2048
-    // tokens, N = 6144 + 1024 + 1024: the three launches leave 128, 64 and 64 tiles over to be cut along K, one launch is
-    // two whole rounds of tiles)
-    bool fuse_gemm = fp6 && G == kGroup;
-    for (int i = 1; i < n && fuse_gemm; ++i) fuse_gemm = multipliers_noted(prepared[i]) == multipliers_noted(prepared[0]);
-    // (without room for slabs no tile is cut, and one launch never has more rounds)
-    if (fuse_gemm && n > 1 && have_slabs && !small6) fuse_gemm = gemm6_one_launch(weights_of(0, 1), M, multipliers_noted(prepared[0]));
-    if (small6) fuse_gemm = one_launch;
-    const int n_launch = (fp6 || path == kPathGemm ? fuse_gemm : one_launch) ? 1 : n;
-    for (int l = 0; l < n_launch; ++l) {
-        const FusedWeights fw = weights_of(l, n_launch);
+    for (int l = 0; l < ch.n_launch; ++l) {
+        const FusedWeights fw = weights_of(l, ch.n_launch);
         if (path == kPathSkinny && !small6) {
             const SkinnyArgs g = skinny_args(fw);
             e = launch_skinny(g, stream);
@@ -382,8 +425,8 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
             g.M = (int) M;
             g.Mp = (int) W.Mp;
             g.groups_per_fold = G / kGroup;
-            g.cells = have_slabs ? wsb + W.off_tot : nullptr;
-            g.weight_multipliers = multipliers_noted(fw.prepared[0]);
+            g.cells = sp.have_slabs ? wsb + W.off_tot : nullptr;
+            g.weight_multipliers = mult[l];   // (one launch: of all alike, or looked at by neither kernel)
             e = small6 ? launch_block6(g, stream) : launch_gemm6(g, stream);
             if (e != hipSuccess) return (int) e;
         } else if (gemm) {
@@ -598,6 +641,46 @@ int rq_w4a4_stage_mask(int type, int64_t K, int64_t M, int64_t n_rot) {
     // one token that the single-launch kernel takes: everything happens in stage 2
     if (M == 1 && env().decode_fused && decode_takes((int) K, type == RQ_TYPE_W4A4H, p, m, env().act_group)) return 2;
     return 3;
+}
+
+int rq_w4a4_product_plan(int type, int n, int64_t K, const int64_t *N, int64_t M, int64_t n_rot, int multipliers, int once,
+                         size_t workspace_bytes, int64_t *plan) {
+    if (n < 1 || n > 3 || !N || !plan) return RQ_E_ARGUMENT;
+    for (int i = 0; i < n; ++i) {
+        if (!shape_ok(type, K, N[i], M) || M < 1) return RQ_E_UNSUPPORTED;
+    }
+    int p, m;
+    if (!rotation_of(type, K, n_rot, p, m)) return RQ_E_ARGUMENT;
+    const Space sp = space_of(n, K, N, M, workspace_bytes);
+    if (workspace_bytes < sp.W.bytes_min) return RQ_E_WORKSPACE;
+    bool mult[kMaxFused];
+    for (int i = 0; i < kMaxFused; ++i) mult[i] = (multipliers >> i) & 1;
+    memset(plan, 0, RQ_PLAN_FIELDS * sizeof *plan);
+    if (M == 1 && env().decode_fused && decode_takes((int) K, type == RQ_TYPE_W4A4H, p, m, env().act_group)) {
+        plan[RQ_PLAN_KERNEL] = RQ_KERNEL_DECODE;
+        plan[RQ_PLAN_LAUNCHES] = 1;
+        return 0;
+    }
+    const Choice ch = choose(n, K, N, M, type == RQ_TYPE_W4A4H, p, m, once != 0, mult, sp);
+    plan[RQ_PLAN_LAUNCHES] = ch.n_launch;
+    plan[RQ_PLAN_KERNEL] = ch.fp6 ? RQ_KERNEL_FP6 : ch.path == kPathGemm ? RQ_KERNEL_INT8 : ch.path == kPathSkinny ? RQ_KERNEL_SKINNY : RQ_KERNEL_GEMV;
+    if (!ch.fp6) return 0;
+    for (int l = 0; l < ch.n_launch; ++l) {
+        FusedWeights fw;
+        memset(&fw, 0, sizeof fw);
+        fw.n = ch.n_launch == 1 ? n : 1;
+        for (int j = 0; j < fw.n; ++j) fw.L[j] = prepared_layout(K, N[ch.n_launch == 1 ? j : l]);
+        if (ch.small6) {
+            for (int j = 0; j < fw.n; ++j) plan[RQ_PLAN_UNITS] += fw.L[j].n_panels;
+            continue;
+        }
+        const Gemm6Route r = gemm6_route(fw, M, env().act_group / kGroup, mult[l], sp.have_slabs);
+        plan[RQ_PLAN_WHOLE] += r.plan.n_whole;
+        plan[RQ_PLAN_CUT] += r.plan.n_tiles - r.plan.n_whole;
+        if (r.plan.parts > plan[RQ_PLAN_SLICES]) plan[RQ_PLAN_SLICES] = r.plan.parts;
+        plan[RQ_PLAN_UNITS] += r.units;
+    }
+    return 0;
 }
 
 int rq_w4a4_mul_mat_fused(int type, int n, const void *const *prepared_dev, int64_t K, const int64_t *N,

@@ -310,6 +310,16 @@ struct Gemm6Plan {
     size_t cell_bytes;
 };
 Gemm6Plan gemm6_plan(int n_row_tiles, int64_t M, int ng, int groups_per_fold);
+// How a launch over these weights goes: the tiles in front of `first_block` through the tiled kernel by `plan`, the others
+// (of n_tiles; first_block == 0: the whole product) through the kernel of small launches, in `units` workgroups. Price in
+// microseconds. have_slabs: the workspace has room for K slices.
+struct Gemm6Route {
+    Gemm6Plan plan;
+    int       n_tiles, first_block;
+    int64_t   units;
+    double    price;
+};
+Gemm6Route gemm6_route(const FusedWeights &w, int64_t M, int groups_per_fold, bool weight_multipliers, bool have_slabs);
 // whether one launch over all these weights (activation groups of 64) is not slower than one each
 bool gemm6_one_launch(const FusedWeights &w, int64_t M, bool weight_multipliers);
 

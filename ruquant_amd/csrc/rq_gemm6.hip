@@ -826,22 +826,24 @@ double block_price(int64_t units, int ng, bool weight_multipliers) {
     return rounds * (weight_multipliers ? 5.2 + 0.75 * per_wave : 4.2 + 0.53 * per_wave);
 }
 
-// How a launch goes: the tiles in front of `first_block` through the tiled kernel by `plan`, the others through the kernel
-// of small launches.
-struct Route {
-    Gemm6Plan plan;
-    int       n_tiles, first_block;
-    double    price;
-};
+}  // namespace
 
 // The cheapest of three. Few tiles: all of them in small units, as long as those are at most two rounds of the chip (K = 5120:
 // 2 tiles 19.5 us in slices and 9.9 in units, 48 tiles 24.4 and 19.4, 96 tiles, three rounds, 27.7 and 28.6; K = 17408: 2
 // tiles 29.2 and 22.1, 48 tiles 39.2 and 47.3). Whole rounds and a few tiles over: those few in units behind the rounds (K = 5120, N = 17408, 512 tokens, 256 + 16
 // tiles: 60.8 us with the 16 in slices, 54.4 with them in 128 units). Everything else: tiles, the rest in slices.
-Route route_of(int n_row_tiles, int64_t n_panels, int64_t M, int ng, int groups_per_fold, bool weight_multipliers, bool have_slabs) {
-    Route r;
+Gemm6Route gemm6_route(const FusedWeights &w, int64_t M, int groups_per_fold, bool weight_multipliers, bool have_slabs) {
+    int n_row_tiles = 0;
+    int64_t n_panels = 0;
+    for (int i = 0; i < w.n; ++i) {
+        n_row_tiles += w.L[i].n_rtiles;
+        n_panels += w.L[i].n_panels;
+    }
+    const int ng = w.L[0].ng;
+    Gemm6Route r;
     r.plan = gemm6_plan(n_row_tiles, M, ng, groups_per_fold);
     r.n_tiles = r.first_block = r.plan.n_tiles;
+    r.units = 0;
     if (!have_slabs) {   // a workspace without slabs: every tile whole
         r.plan.n_whole = r.plan.n_tiles;
         r.plan.parts = 1;
@@ -853,6 +855,7 @@ Route route_of(int n_row_tiles, int64_t n_panels, int64_t M, int ng, int groups_
     if (units <= 2 * kPlanUnits && all < r.price) {
         r.plan.n_tiles = r.plan.n_whole = r.first_block = 0;
         r.plan.parts = 1;
+        r.units = units;
         r.price = all;
         return r;
     }
@@ -865,47 +868,41 @@ Route route_of(int n_row_tiles, int64_t n_panels, int64_t M, int ng, int groups_
         if (left * 8 <= 2 * kPlanUnits && both < r.price) {
             r.plan = whole;
             r.first_block = rounds;
+            r.units = (int64_t) left * 8;
             r.price = both;
         }
     }
     return r;
 }
 
-}  // namespace
-
 // One launch has at most the rounds of all the separate ones, but what it has left over may be too many tiles to cut (more
 // than half a round), where each weight's own tiles can be. With long rows that is the greater loss: K = 17408,
 // N = 4134 + 2216, 525 tokens (85 + 45 tiles) 123.4 us in one launch, 116.4 in two; K = 32768, 66 + 82 tiles 204 and 196.
 // The other way round K = 5120, N = 6144 + 1024 + 1024, 512 tokens is 40 and 79 us. (3 % apart is what the prices tell.)
 bool gemm6_one_launch(const FusedWeights &w, int64_t M, bool weight_multipliers) {
-    int n_row_tiles = 0;
-    int64_t n_panels = 0;
     double each = 0.0;
     for (int i = 0; i < w.n; ++i) {
-        n_row_tiles += w.L[i].n_rtiles;
-        n_panels += w.L[i].n_panels;
-        each += route_of(w.L[i].n_rtiles, w.L[i].n_panels, M, w.L[i].ng, 1, weight_multipliers, true).price;
+        FusedWeights one = {};
+        one.n = 1;
+        one.L[0] = w.L[i];
+        each += gemm6_route(one, M, 1, weight_multipliers, true).price;
     }
-    return route_of(n_row_tiles, n_panels, M, w.L[0].ng, 1, weight_multipliers, true).price <= 1.03 * each;
+    return gemm6_route(w, M, 1, weight_multipliers, true).price <= 1.03 * each;
 }
 
 hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
     TileSet<true> ts;
     TileSet<false> t1;
     int n_row_tiles = 0;
-    int64_t n_panels = 0;
     for (int i = 0; i < kMaxFused; ++i) {
         const int k = i < a.w.n ? i : a.w.n - 1;   // unused slots repeat the last weight (never selected)
         set_weight(ts, i, a.w, k, n_row_tiles);
         if (i == 0) set_weight(t1, 0, a.w, 0, 0);
-        if (i < a.w.n) {
-            n_row_tiles += a.w.L[k].n_rtiles;
-            n_panels += a.w.L[k].n_panels;
-        }
+        if (i < a.w.n) n_row_tiles += a.w.L[k].n_rtiles;
     }
     const int ng = a.w.L[0].ng;
     const int n_tok_tiles = a.Mp / kTileTok;
-    const Route route = route_of(n_row_tiles, n_panels, a.M, ng, a.groups_per_fold, a.weight_multipliers, a.cells != nullptr);
+    const Gemm6Route route = gemm6_route(a.w, a.M, a.groups_per_fold, a.weight_multipliers, a.cells != nullptr);
     const Gemm6Plan &pl = route.plan;
     if (route.n_tiles != n_row_tiles * n_tok_tiles) return hipErrorInvalidValue;
     if (a.w.n > 1 && a.groups_per_fold != 1) return hipErrorInvalidValue;   // (wider groups go weight by weight)

@@ -77,6 +77,8 @@ PROTOTYPES = {
     "rq_w4a4_dequantize": (ctypes.c_int, [ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
                                           ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "rq_w4a4_stage_mask": (ctypes.c_int, [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]),
+    "rq_w4a4_product_plan": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int64, c_i64p, ctypes.c_int64,
+                                            ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_size_t, c_i64p]),
     "rq_w4a4_quantize_act": (ctypes.c_int, [ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
                                             ctypes.c_int64, ctypes.c_float, ctypes.c_int64, ctypes.c_void_p,
                                             ctypes.c_void_p]),
