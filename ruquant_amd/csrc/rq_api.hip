@@ -224,11 +224,17 @@ Choice choose(int n, int64_t K, const int64_t *N, int64_t M, bool rotate, int p,
     c.two_step = c.path == kPathSkinny && G == kGroup && rotate && p >= 44 && (m & 63) == 0 && M <= kTwoStepTokens;
     // 33 .. 64 tokens of a call that shares its activation with no other: the small units of the fp6 product where they are
     // the faster ones (block6_takes); they read the activations as the fp6 GEMM does
-    c.small6 = false;
-    if (c.path == kPathSkinny && once && G == kGroup && gemm_fp6_enabled() && !c.two_step) {
-        int64_t panels = 0;
-        for (int i = 0; i < n; ++i) panels += (N[i] + kPanelRows - 1) / kPanelRows;
-        c.small6 = block6_takes(panels, M);
+    // (they share the activations, so all of a call's launches go that way or none)
+    c.small6 = c.path == kPathSkinny && once && G == kGroup && gemm_fp6_enabled() && !c.two_step;
+    int64_t panels = 0;
+    bool any = false;
+    for (int i = 0; i < n && c.small6; ++i) {
+        panels += (N[i] + kPanelRows - 1) / kPanelRows;
+        any |= mult[i];
+        if (s.one_launch && i < n - 1) continue;
+        c.small6 = block6_takes(panels, M, (int) (K / kGroup), any);
+        panels = 0;
+        any = false;
     }
     c.fp6 = c.small6 || (c.path == kPathGemm && gemm_fp6_enabled());
     bool one = s.one_launch;

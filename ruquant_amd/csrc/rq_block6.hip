@@ -386,11 +386,28 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 }
 
 // 33 .. 64 tokens. The skinny kernel reads two thirds of the bytes (int4 codes) but runs 16 x 16 MFMAs with three vector
-// instructions per output behind each, where this one has 32 x 32 and one, and of its form for 64 tokens a round of the chip
-// is 18 us at K = 5120. 64 tokens, whole call, skinny and here: K = 3072, N = 4096 14.9 / 13.2 us, N = 10240 20.2 / 14.0, N = 17408
-// 27.3 / 21.7; K = 5120, N = 2048 14.9 / 16.1, N = 4096 16.7 / 16.3, N = 8192 17.1 / 17.1, N = 10240 24.6 / 17.4, N = 17408 32.5 /
-// 27.8; K = 10240, N = 4096 25.9 / 25.8, N = 17408 48.4 / 45.4; K = 17408, N = 4096 34.1 / 37.8, N = 8192 42.7 / 39.1, N = 17408
-// 69.6 / 68.8. 33 tokens cost the same in both.
-bool block6_takes(int64_t n_panels, int64_t M) { return M > 32 && n_panels >= 96; }
+// instructions per output behind each, where this one has 32 x 32 and one. So this one is faster on weights that the
+// memory-side cache holds and loses on weights that come from memory, as those of a whole model do: a unit's 3 KB a group
+// then arrive at 20 KB per microsecond, whatever the other compute units do. The line lies where it is faster from the cache
+// and at most 6 % slower from memory. (64 tokens, whole call in us, skinny / here; in front from the cache, behind from memory.)
+// - Up to 128 panels (half the chip: the skinny kernel has two workgroups of 32 tokens a panel): K = 5120, N = 8192 14.8 / 15.0,
+//   16.1 / 19.6; K = 17408, N = 8192 47.6 / 39.4, 38.4 / 46.6. The skinny kernel.
+// - 129 to 256 panels, a round of units, and two of the skinny kernel's: N = 12288, K = 1024 15.6 / 9.5, 16.3 / 10.9; K = 5120
+//   24.4 / 16.4, 25.6 / 20.5; K = 10240 32.0 / 24.6, 32.8 / 32.9; K = 17408 48.1 / 35.5, 48.4 / 50.7; K = 32768 81 / 85 in both.
+//   Here up to K = 17408.
+// - More: N = 17408 (272), K = 3072 25.7 / 20.0, 27.1 / 24.3; K = 5120 30.7 / 25.9, 31.8 / 32.5; K = 10240 44.5 / 41.1, 45.3 / 53.7;
+//   K = 17408 63.0 / 61.7, 63.6 / 83.1; K = 32768 100 / 147. N = 24576 (384), K = 10240 55.7 / 42.2, 56.7 / 55.8; N = 34816 (544)
+//   73.7 / 65.7, 74.5 / 79.8. Here up to K = 5120, and up to K = 10240 where the last round is at least half full.
+// - Weight multipliers cost the skinny kernel more: up to 128 panels K = 1024, N = 8192 9.8 / 10.3, K = 5120 18.3 / 17.9, 20.0 / 21.3;
+//   N = 12288, K = 5120 29.7 / 18.9, 31.2 / 22.4, K = 32768 128 / 91, 128 / 95; N = 17408, K = 17408 86 / 71, 87 / 91, K = 32768
+//   145 / 160. Here from 129 panels up, beyond a round of units up to K = 17408.
+// 33 tokens are within a tenth of 64 on both sides.
+bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers) {
+    if (M <= 32 || n_panels <= kPlanUnits / 2) return false;
+    if (n_panels <= kPlanUnits) return ng <= 272 || weight_multipliers;
+    if (weight_multipliers) return ng <= 272;
+    const int64_t last = n_panels % kPlanUnits;
+    return ng <= 80 || (ng <= 160 && (last == 0 || last >= kPlanUnits / 2));
+}
 
 }  // namespace rq

@@ -9,6 +9,7 @@ import torch
 import ruquant_amd as rq
 from ruquant_amd import synth
 from tests.gpu_util import adversarial_weights, adversarial_activations, bits_equal, first_mismatch, run_gpu
+from tests.plan_util import FP6, SKINNY, plan
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -24,9 +25,13 @@ DEV = "cuda:0"
     (512, 4096, 512, 0),      # 512 units: two rounds
     (512, 4300, 2048, 0),     # 17 x 16 tiles: 16 left over behind a round, the last row tile ragged
     (512, 8192, 1100, 256),   # 32 x 9 tiles: 32 left over, in runs of nine token tiles
-    (2560, 6200, 33, 0),      # 97 panels: 33 .. 64 tokens
+    (2560, 6200, 33, 0),      # 97 panels: the skinny kernel
     (2560, 6200, 64, 64),
-    (17408, 6145, 41, 0)])
+    (17408, 6145, 41, 0),
+    (2560, 8300, 33, 0),      # 130 panels: 33 .. 64 tokens in units
+    (2560, 8300, 64, 64),
+    (17408, 8257, 41, 0),
+    (512, 16500, 57, 0)])     # 258: two rounds
 def test_units_of_64_rows_and_tokens(oracle, K, N, M, wgroup):
     type_ = rq.TYPE_W4A4 if K in (256, 512, 32768) else rq.TYPE_W4A4H
     blocks, wf = adversarial_weights(oracle, N, K, type_, seed=N + M, wgroup=wgroup)
@@ -68,6 +73,7 @@ def test_extreme_sums_with_weight_multipliers(oracle):
     added as bit patterns, modulo 2^32, the bias of every one still on it. Rows of all -8 / all 7 / both in turn against tokens
     of q - z = +-15 with m = 255: totals of 117.5 M per wavefront and 940 M per output, both signs."""
     K, M, panels, type_ = 32768, 40, 129, rq.TYPE_W4A4
+    assert plan(type_, K, 64 * panels, M, multipliers=1)["units"] == panels
     rng = np.random.default_rng(3)
     codes = rng.integers(-8, 8, size=(64, K), dtype=np.int8)
     codes[0] = -8
@@ -93,14 +99,18 @@ def test_extreme_sums_with_weight_multipliers(oracle):
     assert got[0, 0, 0] == np.float32(expect)
 
 
-@pytest.mark.parametrize("M", [40, 70])
-def test_a_set_of_weights(oracle, M):
-    """Three weights, with and without multipliers, whose panels do not end with a row tile, in one launch (40 tokens) or one
-    each (70, where the two kinds go apart)."""
+@pytest.mark.parametrize("M,Ns", [(40, (3000, 2100, 1500)), (70, (3000, 2100, 1500)), (40, (4000, 2100, 2500))],
+                         ids=["skinny", "70_tokens", "40_tokens"])
+def test_a_set_of_weights(oracle, M, Ns):
+    """Three weights, with and without multipliers, whose panels do not end with a row tile, in one launch (40 tokens, 136
+    panels) or one each (70, where the two kinds go apart); 104 panels at 40 tokens are the skinny kernel's."""
     K, type_ = 1024, rq.TYPE_W4A4H
     ws, want = [], []
     x = None
-    for i, (N, g) in enumerate([(3000, 0), (2100, 64), (1500, 0)]):
+    p = plan(type_, K, Ns, M, multipliers=2)
+    assert (p["kernel"], p["launches"]) == ((SKINNY, 1) if sum(Ns) == 6600 and M == 40 else (FP6, 1 if M == 40 else 3))
+    assert p["whole"] == p["cut"] == 0
+    for i, (N, g) in enumerate(zip(Ns, (0, 64, 0))):
         blocks, wf = adversarial_weights(oracle, N, K, type_, seed=i, wgroup=g)
         w = rq.W4A4Weight(blocks, type_, DEV)
         if x is None:

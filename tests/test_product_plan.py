@@ -15,6 +15,37 @@ def test_kernel_by_token_count(M, kernel):
     assert p["kernel"] == kernel and p["launches"] == 1
 
 
+@pytest.mark.parametrize("K,N,multipliers,kernel", [
+    (5120, 8192, 0, SKINNY), (5120, 8193, 0, FP6), (17408, 12288, 0, FP6), (18432, 12288, 0, SKINNY), (32768, 17408, 0, SKINNY),
+    (5120, 17408, 0, FP6), (5376, 17408, 0, SKINNY), (10240, 17408, 0, SKINNY), (10240, 24576, 0, FP6), (10240, 34816, 0, SKINNY),
+    (12288, 24576, 0, SKINNY), (17408, 17408, 0, SKINNY), (5120, 34816, 0, FP6),
+    (1024, 8192, 1, SKINNY), (1024, 8256, 1, FP6), (32768, 12288, 1, FP6), (17408, 17408, 1, FP6), (32768, 17408, 1, SKINNY)])
+@pytest.mark.parametrize("M", [33, 64])
+def test_33_to_64_tokens(K, N, multipliers, kernel, M):
+    """Units of the fp6 product only where they are no slower on weights that come from memory either (6 % at most)."""
+    p = plan(W4A4, K, N, M, multipliers)
+    assert p["kernel"] == kernel and p["launches"] == 1
+    assert p["units"] == (-(-N // 64) if kernel == FP6 else 0) and p["whole"] == p["cut"] == 0
+    # a call whose activations others may use keeps the form that all weights can read
+    assert plan(W4A4, K, N, M, multipliers, once=False)["kernel"] == SKINNY
+    assert plan(W4A4, K, N, 32, multipliers)["kernel"] == SKINNY
+
+
+def test_33_to_64_tokens_launch_by_launch():
+    """With room for the largest weight only, every weight's own launch has to be one that the units are faster for."""
+    Ns = (6144, 6144, 6144)
+    room = rq.load_library().rq_w4a4_workspace_bytes(W4A4, 5120, 6144, 64)
+    assert plan(W4A4, 5120, Ns, 64)["kernel"] == FP6 and plan(W4A4, 5120, Ns, 64)["launches"] == 1
+    p = plan(W4A4, 5120, Ns, 64, workspace=room)
+    assert p["kernel"] == SKINNY and p["launches"] == 3
+    Ns = (12288, 9000, 6144)
+    room = rq.load_library().rq_w4a4_workspace_bytes(W4A4, 1024, 12288, 64)
+    assert plan(W4A4, 1024, Ns, 64, workspace=room)["kernel"] == SKINNY
+    Ns = (12288, 9000, 8256)
+    p = plan(W4A4, 1024, Ns, 64, workspace=room)
+    assert p["kernel"] == FP6 and p["launches"] == 3 and p["units"] == 192 + 141 + 129
+
+
 def test_every_tile_is_counted_once():
     """Tiles whole, cut, or in units (eight a tile where whole tiles run beside them)."""
     for N, M in [(17408, 65), (17408, 2048), (6100, 1500), (3000, 700), (256, 5000)]:
