@@ -830,8 +830,15 @@ double block_price(int64_t units, int ng, bool weight_multipliers) {
 
 // The cheapest of three. Few tiles: all of them in small units, as long as those are at most two rounds of the chip (K = 5120:
 // 2 tiles 19.5 us in slices and 9.9 in units, 48 tiles 24.4 and 19.4, 96 tiles, three rounds, 27.7 and 28.6; K = 17408: 2
-// tiles 29.2 and 22.1, 48 tiles 39.2 and 47.3). Whole rounds and a few tiles over: those few in units behind the rounds (K = 5120, N = 17408, 512 tokens, 256 + 16
-// tiles: 60.8 us with the 16 in slices, 54.4 with them in 128 units). Everything else: tiles, the rest in slices.
+// tiles 29.2 and 22.1, 48 tiles 39.2 and 47.3). Whole rounds and a few tiles over: those few in units behind the rounds
+// (K = 5120, N = 17408, 512 tokens, 256 + 16 tiles: 60.8 us with the 16 in slices, 54.4 with them in 128 units). Everything
+// else: tiles, the rest in slices.
+// The prices are of weights in the memory-side cache. From memory a unit gets its rows at 20 KB per microsecond, whatever the
+// others do, while K slices spread a tile's over compute units, so units end where the rows are long: without multipliers
+// at K = 17408 in one round and K = 6144 in two (with them the fold is slow enough to hide it). Whole call in us, slices / units,
+// from the cache, then from memory. One round, 128 tokens: K = 17408, N = 1000 39.4 / 32.4, 40.6 / 42.1, N = 6000 42.0 / 33.4,
+// 47.4 / 44.0; K = 22528, N = 1000 44.0 / 39.5, 45.1 / 51.7; K = 32768 51.5 / 52.5, 52.7 / 69.7. Two: K = 5120, N = 3000, 400 tokens
+// 31.4 / 26.2, 32.8 / 30.9; K = 10240 40.5 / 41.0, 41.7 / 48.8, N = 6000, 256 tokens 38.3 / 38.5, 39.7 / 48.3.
 Gemm6Route gemm6_route(const FusedWeights &w, int64_t M, int groups_per_fold, bool weight_multipliers, bool have_slabs) {
     int n_row_tiles = 0;
     int64_t n_panels = 0;
@@ -852,7 +859,8 @@ Gemm6Route gemm6_route(const FusedWeights &w, int64_t M, int groups_per_fold, bo
     if (groups_per_fold != 1) return r;   // (the small units fold groups of 64)
     const int64_t units = n_panels * ((M + 63) / 64);
     const double all = block_price(units, ng, weight_multipliers);
-    if (units <= 2 * kPlanUnits && all < r.price) {
+    const bool short_rows = weight_multipliers || ng <= (units <= kPlanUnits ? 272 : 96);
+    if (units <= 2 * kPlanUnits && short_rows && all < r.price) {
         r.plan.n_tiles = r.plan.n_whole = r.first_block = 0;
         r.plan.parts = 1;
         r.units = units;

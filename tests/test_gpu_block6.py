@@ -48,10 +48,14 @@ def test_units_of_64_rows_and_tokens(oracle, K, N, M, wgroup):
     assert (got[:, N:] == -7.0).all()
 
 
-def test_extreme_sums_between_two_transfers(oracle):
-    """K = 32768: 64 groups per wavefront, rows of all -8 / all 7 against tokens of q - z = +-15 with m = 255, so that the float
-    totals move by 122,400 per group, 28 groups and a tile of one more between two transfers: 3.55 M of their 4.19 M."""
-    N, K, M, type_ = 64, 32768, 80, rq.TYPE_W4A4
+@pytest.mark.parametrize("K", [17408, 32768])
+def test_extreme_sums_between_two_transfers(oracle, K):
+    """K = 17408, the longest row without multipliers that goes in units: 34 groups per wavefront, rows of all -8 / all 7 against
+    tokens of q - z = +-15 with m = 255, so that the float totals move by 122,400 per group, 28 groups and a tile of one more
+    between two transfers: 3.55 M of their 4.19 M. (The same at K = 32768 in K slices.)"""
+    N, M, type_ = 64, 80, rq.TYPE_W4A4
+    p = plan(type_, K, N, M)
+    assert (p["units"], p["cut"]) == ((2, 0) if K == 17408 else (0, 1))
     blocks = synth.random_weight_blocks(N, K, 5, type_)
     qs = blocks["qs"].reshape(N, -1)
     qs[0, :] = 0x88888888

@@ -46,6 +46,16 @@ def test_33_to_64_tokens_launch_by_launch():
     assert p["kernel"] == FP6 and p["launches"] == 3 and p["units"] == 192 + 141 + 129
 
 
+@pytest.mark.parametrize("K,N,M,multipliers,units", [
+    (17408, 1000, 128, 0, True), (17664, 1000, 128, 0, False), (32768, 256, 1536, 0, False), (32768, 3000, 65, 0, False),
+    (5120, 3000, 400, 0, True), (6144, 3000, 400, 0, True), (8192, 3000, 400, 0, False), (10240, 6000, 256, 0, False),
+    (22528, 1000, 128, 1, True), (32768, 6000, 128, 1, True), (5120, 6000, 200, 1, True)])
+def test_long_rows_above_64_tokens(K, N, M, multipliers, units):
+    """Few tiles of long rows without multipliers are cut along K: units get weights from memory too slowly."""
+    p = plan(W4A4, K, N, M, multipliers)
+    assert (p["units"] > 0) == units and (p["cut"] > 0) == (not units) and p["whole"] == 0
+
+
 def test_every_tile_is_counted_once():
     """Tiles whole, cut, or in units (eight a tile where whole tiles run beside them)."""
     for N, M in [(17408, 65), (17408, 2048), (6100, 1500), (3000, 700), (256, 5000)]:
