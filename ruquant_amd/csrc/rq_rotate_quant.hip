@@ -21,21 +21,21 @@ namespace {
 
 // Threads per token workgroup. Small batches (the sliced variant) with a short Paley stage get 1024: there the kernel
 // is one workgroup per compute unit at most, bound by the latency of its own phases, and twice the threads halve the
-// work per phase. Long Paley stages keep their columns in registers and need the 256-register budget of 512 threads.
+// work per phase. Long Paley stages that keep a column in one thread's registers need the 256-register budget of 512
+// threads; those whose columns four threads share (WIDE) get 1024.
 template <int P, bool SLICED, bool WIDE>
 constexpr int threads_of() { return WIDE || (SLICED && P < 44) ? 1024 : 512; }
 
 using namespace had;
 
-template <int P, bool SLICED, bool WIDE = false>
+template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
 // Registers are capped so that two workgroups (p >= 44: long columns, long rows) or three fit a compute unit: the
 // stages of one token are separated by barriers, and it is the other workgroups that keep the vector ALU busy. (The
-// sliced variant serves small batches, where occupancy is not the limit.) WIDE: rows of at least 256 columns of a long Paley
-// stage, whose columns four threads share (paley_row): 1024 threads, a fourth of the registers per column. The rotation alone,
-// K = 17408, p = 68, a thread per column with 512 threads and this: 1 token 17.9 / 10.0 us, 64 tokens 14.9 / 10.9, 256 18.0 /
-// 14.2, 2048 85.2 / 73.6; K = 27648, p = 108, where LDS holds one workgroup per compute unit, 26.7 / 18.1, 28.6 / 19.4, 34.5 /
-// 25.7, 250 / 190. (Shorter chunks leave most of the 1024 threads without a column: K = 5376 = 84 x 64, one token 9.2 / 11.0.)
-__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE>()), WIDE ? (P >= 84 ? 4 : 8) : SLICED ? (P < 44 ? 4 : 2) : P >= 44 ? 4 : 6)
+// sliced variant serves small batches, where occupancy is not the limit.) WIDE: 1024 threads, the columns of a long Paley stage
+// by four threads each (paley_row), a fourth of the registers per column; see takes_wide for where. ALONE is the plain
+// variant for rows so long that LDS holds one workgroup per compute unit anyway: the cap then only makes the p >= 60 columns
+// spill (136 to 504 bytes per lane), so it goes (2048 tokens, K = 21504, p = 84: 204 -> 193 us).
+__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE>()), WIDE ? (P >= 84 ? 4 : 8) : SLICED ? (P < 44 ? 4 : 2) : ALONE ? 2 : P >= 44 ? 4 : 6)
 rq_rotate_quant_kernel(const RotQuantArgs a) {
     constexpr int kNT = threads_of<P, SLICED, WIDE>();
     extern __shared__ __align__(16) float smem[];
@@ -135,7 +135,7 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
                     const int rb = cidx / m, j = cidx - rb * m;
                     const int b0 = rb * a.n_rot + j;
                     float col[P];
-                    if (P < 44 && pm == 272) {   // chunks of 256 (K = 5120): the common case, compile-time stride
+                    if (P < 68 && pm == 272) {   // chunks of 256 (K = 5120): the common case, compile-time stride
                         float *src = buf + padi(b0);
                         load_column<P, 272>(col, src, pm);
                         paley_column<P, 0, false, 272>(col, src, pm, a.scale);
@@ -329,27 +329,30 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
 }
 
 // the kernels keep a whole row in dynamic LDS: raise the per-kernel limit (once per device, see init_activation_kernels)
-template <int P, bool SLICED, bool WIDE = false>
+template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
 hipError_t allow_big_lds() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, WIDE>),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 64);
 }
 
 constexpr bool has_wide(int p) { return p >= 44; }
+// the plain variant has an ALONE build where the cap makes its columns spill and rows past takes_wide get that long
+constexpr bool has_alone(int p) { return p == 60 || p >= 84; }
 
 template <int P>
 hipError_t allow_big_lds_both() {
     hipError_t e = allow_big_lds<P, false>();
     if (e == hipSuccess && P > 1) e = allow_big_lds<P, (P > 1)>();
     if (e == hipSuccess && has_wide(P)) e = allow_big_lds<P, false, has_wide(P)>();
+    if (e == hipSuccess && has_alone(P)) e = allow_big_lds<P, false, false, has_alone(P)>();
     return e;
 }
 
-template <int P, bool SLICED, bool WIDE = false>
+template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
 hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
     static bool attr_set = false;   // calls that never went through rq_w4a4_prepare on this device
     if (!attr_set) {
-        hipError_t e = allow_big_lds<P, SLICED, WIDE>();
+        hipError_t e = allow_big_lds<P, SLICED, WIDE, ALONE>();
         if (e != hipSuccess) return e;
         attr_set = true;
     }
@@ -359,8 +362,32 @@ hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
     b.token_blocks = a.M;
     const int grid = a.M + (int) ((a.zero_ints + (int64_t) kNT * 4 - 1) / ((int64_t) kNT * 4));
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, WIDE>), dim3(grid), dim3(kNT), lds, stream, b);
+    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE>), dim3(grid), dim3(kNT), lds, stream, b);
     return hipGetLastError();
+}
+
+// Whether the columns of a long Paley stage go to four threads each. They read every column four times out of LDS and take
+// 256 columns in a run, so it pays where a thread per column leaves threads without one, and where that form's registers
+// spill. The rotation alone / with the quantizer, in us, a thread per column -> four:
+// - 256 columns, half of 512 threads: K = 11264 (p = 44) 1 token 10.4 -> 6.9, 2048 41.2 -> 40.6; K = 17408 (68) 17.9 -> 10.0, 64
+//   tokens 14.9 -> 10.9, 2048 78.9 -> 75.0; K = 27648 (108) 26.7 -> 18.1, 28.4 -> 19.6, 251 -> 196. Always.
+// - Fewer leave most of 1024 threads without a column (K = 5376 = 84 x 64, one token 9.2 -> 11.0). Never.
+// - More, whole runs or not: K = 19712 (44 x 448) 64 tokens 10.8 -> 12.1 / 14.2 -> 15.0; K = 19200 (60 x 320) 13.3 -> 15.5 / 16.8
+//   -> 18.2; K = 32256 (84 x 384) 2048 tokens 208 -> 229 / 228 -> 240; K = 29952 (104 x 288) 256 -> 283 / 272 -> 292. Not, but:
+//   - where the other form is the sliced one, which works on two rows of LDS (up to 40 tokens): K = 16896 (44 x 384), one token 15.0
+//     -> 10.4 / 18.6 -> 13.5;
+//   - p = 68 and 72, whose plain form spills with two workgroups to a compute unit, from 129 tokens up: K = 30464 (68 x 448)
+//     128 tokens 21.0 -> 22.1 / 24.6 -> 24.0, 256 27.8 -> 24.7 / 30.8 -> 24.1, 2048 203 -> 188 / 230 -> 195; K = 20736 (72 x 288) 128
+//     tokens 19.2 -> 20.3, 2048 182 -> 175 / 194 -> 177;
+//   - two whole runs in chunks of 256 or more when the quantizer follows, which has twice the threads: K = 22528 (44 x 512) 64
+//     tokens 13.7 -> 14.2 / 17.4 -> 16.9, K = 30720 (60 x 512) 19.0 -> 19.8 / 23.7 -> 23.3.
+template <int P>
+bool takes_wide(const RotQuantArgs &a, bool sliced) {
+    const int columns = a.K / P;
+    if (!has_wide(P) || columns < 256) return false;
+    if (columns == 256 || sliced) return true;
+    if (P == 68 || P == 72) return a.M > 128;
+    return columns == 512 && a.m >= 256 && a.mode != kActRotateOnly;
 }
 
 // LDS: one padded row (two when the Paley stage is sliced over more threads) plus the group ranges. Slicing buys
@@ -369,11 +396,12 @@ template <int P>
 hipError_t launch_p(const RotQuantArgs &a, hipStream_t stream) {
     const size_t row = (size_t) (a.K + (a.K >> 4) + 1) * sizeof(float);
     const size_t stats = (size_t) 2 * (a.K / kGroup + 1) * sizeof(float);
-    if (has_wide(P) && a.K / P >= 256) return launch_one<P, false, has_wide(P)>(a, row + stats, stream);
     // long Paley stages: past kTwoStepTokens tokens the plain variant (two workgroups per CU) is the faster one
-    if (P > 1 && a.M <= (P >= 44 ? kTwoStepTokens : 64) && 2 * row + stats <= 160 * 1024 - 64) {
-        return launch_one<P, (P > 1)>(a, 2 * row + stats, stream);
-    }
+    const bool sliced = P > 1 && a.M <= (P >= 44 ? kTwoStepTokens : 64) && 2 * row + stats <= 160 * 1024 - 64;
+    if (takes_wide<P>(a, sliced)) return launch_one<P, false, has_wide(P)>(a, row + stats, stream);
+    if (sliced) return launch_one<P, (P > 1)>(a, 2 * row + stats, stream);
+    // a second workgroup does not fit beside this one
+    if (has_alone(P) && 2 * (row + stats + 64) > 160 * 1024) return launch_one<P, false, false, has_alone(P)>(a, row + stats, stream);
     return launch_one<P, false>(a, row + stats, stream);
 }
 
