@@ -264,9 +264,7 @@ __device__ __forceinline__ int weight_mult(int32_t sum, int g) {
     return 1;
 }
 
-// WIDE: rows of at least 256 columns of a long Paley stage, whose columns four threads share (paley_row), 1024 threads. A thread
-// per column with 512 threads and this, K = 17408, p = 68: 64 rows 16.3 / 12.0 us, 427 rows 34.3 / 23.4, 2048 rows 128 / 82;
-// K = 27648, p = 108, 2048 rows 252 / 174. (p = 44, K = 11264: 427 rows 13.3 / 14.4, so it stays.)
+// WIDE: the columns of a long Paley stage by four threads each (paley_row), 1024 threads; see launch_dequant for where.
 template <int P, bool WIDE>
 __global__ void __launch_bounds__(WIDE ? 1024 : 512) rq_dequant_rows_kernel(const DequantArgs a) {
     constexpr int kNT = WIDE ? 1024 : 512;
@@ -358,10 +356,17 @@ hipError_t launch_dequant_form(const DequantArgs &a, int64_t rows, hipStream_t s
     return hipGetLastError();
 }
 
+// Four threads per column where a thread each leaves half of 512 threads without one, 256 columns: K = 17408, p = 68, 64 rows
+// 16.3 -> 12.0 us, 427 rows 34.3 -> 23.4, 2048 rows 128 -> 82; K = 27648, p = 108, 2048 rows 252 -> 174 (p = 44, K = 11264: 427 rows
+// 13.3 -> 14.4, so it stays). With more columns the fourfold reads of LDS cost more than the idle threads: 600 rows of K = 29952
+// (104 x 288, chunks of 8 / 32) 91.7 -> 108.7 / 96.7 -> 101.9, K = 32256 (84 x 384) 77.9 -> 81.5, (72 x 448, chunks of 8) 63.0 ->
+// 76.7, K = 27648 (72 x 384) 63.1 -> 66.2; but for two whole runs in chunks of 256 or more, whose strides are constants: K = 30720 (60 x
+// 512) 68.5 -> 65.2, 60.1 -> 55.8 in two chunks of 256.
 template <int P>
 hipError_t launch_dequant(const DequantArgs &a, int64_t rows, hipStream_t stream) {
     if constexpr (P >= 60) {
-        if (a.K / P >= 256) return launch_dequant_form<P, true>(a, rows, stream);
+        const int columns = a.K / P;
+        if (columns == 256 || (columns == 512 && a.m >= 256)) return launch_dequant_form<P, true>(a, rows, stream);
     }
     return launch_dequant_form<P, false>(a, rows, stream);
 }
