@@ -44,8 +44,11 @@ struct SearchArgs {
     float *scale;      // [segments]
 };
 
+// ONE: segments of 64 (a scale per 64 inputs), one block each: nothing to fetch ahead and no eight loads to batch. (With the
+// general form's, which fetch the one block again: 4096 x 17408, search and encoding, 450 us against 402.)
+template <bool ONE>
 __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const SearchArgs a) {
-    __shared__ float4 s_x[2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
+    __shared__ float4 s_x[ONE ? 1 : 2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
     const int tid = threadIdx.x, r = tid & 15;
     int64_t seg = (int64_t) blockIdx.x * (kSearchThreads / 16) + (tid >> 4);
     const bool live = seg < a.segments;
@@ -56,9 +59,9 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
 
     // Elements come by the sixteen lanes of a segment together, a block of 64 to a load (n is a multiple of 64). Eight loads at
     // once here: one after the other, this pass alone would be n / 64 trips to memory.
-    constexpr int kBatch = 8;
+    constexpr int kBatch = ONE ? 1 : 8;
     const float4 *xv = reinterpret_cast<const float4 *>(x) + r;
-    const int nv = n >> 6;
+    const int nv = ONE ? 1 : n >> 6;
     auto block = [&](int k) { return xv[16 * (k < nv ? k : nv - 1)]; };   // (past the end: the last again)
     float amax = 0.0f;
     for (int i0 = 0; i0 < nv; i0 += kBatch) {
@@ -97,15 +100,21 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
         // runs ahead: four times the load instructions.)
         constexpr int kRun = 8;
         const bool normal = rs < 1e37f && rs > 2e-38f;
-        float4 ahead[2] = { block(1), block(2) };
+        float4 ahead[2];
+        if constexpr (!ONE) {
+            ahead[0] = block(1);
+            ahead[1] = block(2);
+        }
         s_x[0][tid] = block(0);
         for (int k0 = 0; k0 < nv; k0 += 2) {
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
+          for (int h = 0; h < (ONE ? 1 : 2); ++h) {
             const int k = k0 + h;
             if (k >= nv) break;   // (uniform)
-            s_x[h ^ 1][tid] = ahead[h];
-            ahead[h] = block(k + 3);
+            if constexpr (!ONE) {
+                s_x[h ^ 1][tid] = ahead[h];
+                ahead[h] = block(k + 3);
+            }
             // (one wavefront: its LDS operations are carried out in order)
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -456,8 +465,9 @@ int rq_w4a4_quantize_weights(int type, const float *w_dev, int64_t ldw, int64_t 
     s.n = (int) (K / per_row);
     s.scale = reinterpret_cast<float *>(base + ws.off_scale);
     const int64_t per_wg = kSearchThreads / 16;
-    hipLaunchKernelGGL(rq_wsearch_kernel, dim3((unsigned) ((s.segments + per_wg - 1) / per_wg)), dim3(kSearchThreads), 0,
-                       st, s);
+    const dim3 grid((unsigned) ((s.segments + per_wg - 1) / per_wg));
+    if (s.n == 64) hipLaunchKernelGGL((rq_wsearch_kernel<true>), grid, dim3(kSearchThreads), 0, st, s);
+    else hipLaunchKernelGGL((rq_wsearch_kernel<false>), grid, dim3(kSearchThreads), 0, st, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int) e;
 
