@@ -267,19 +267,9 @@ rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const floa
         panel -= wsel == 0 ? 0 : wsel == 1 ? ts.first[1] : ts.first[2];   // now of its weight
     } else {
         // the tiles (256 rows x 128 tokens) from first_tile on in the tiled kernel's order, eight units each
-        const int n_tok_tiles = Mp / kGemmTokens, sub = v & 7;
-        v = first_tile + (v >> 3);
+        const int sub = v & 7;
         int row_tile;
-        if (super_tiles) {
-            const int s = v >> 5, i = v & 31;
-            const int spr = n_tok_tiles >> 2;
-            const int sr = s / spr;
-            row_tile = sr * 8 + (i >> 2);
-            t0 = ((s - sr * spr) * 4 + (i & 3)) * kGemmTokens;
-        } else {
-            row_tile = v / n_tok_tiles;
-            t0 = (v - row_tile * n_tok_tiles) * kGemmTokens;
-        }
+        gemm6_tile(first_tile + (v >> 3), Mp / kGemmTokens, super_tiles, row_tile, t0);
         t0 += (sub & 1) * kTok;
         wsel = (row_tile >= ts.first[1]) + (row_tile >= ts.first[2]);
         row_tile -= wsel == 0 ? 0 : wsel == 1 ? ts.first[1] : ts.first[2];

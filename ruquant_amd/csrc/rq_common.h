@@ -305,6 +305,21 @@ bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers);
 // K each, which meet in cell_bytes of workspace: kGemm6CounterBytes of arrival counters (one int per cut tile: zero on
 // entry, left zero), then one slab of partial totals per slice (needs no clearing).
 
+// Tile v of such a launch, in the order in which both kernels of the fp6 product count: super-tiles of 8 row tiles x 4
+// token tiles, or the token tiles running fastest where the launch is not made of whole super-tiles.
+__device__ __forceinline__ void gemm6_tile(int v, int n_tok_tiles, int super_tiles, int &row_tile, int &t0) {
+    if (super_tiles) {
+        const int s = v >> 5, i = v & 31;
+        const int spr = n_tok_tiles >> 2;
+        const int sr = s / spr;
+        row_tile = sr * 8 + (i >> 2);
+        t0 = ((s - sr * spr) * 4 + (i & 3)) * kGemmTokens;
+    } else {
+        row_tile = v / n_tok_tiles;
+        t0 = (v - row_tile * n_tok_tiles) * kGemmTokens;
+    }
+}
+
 struct Gemm6Plan {
     int    n_tiles, n_whole, parts;
     size_t cell_bytes;

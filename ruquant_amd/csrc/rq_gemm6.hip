@@ -508,16 +508,7 @@ rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const f
             v = n_whole + j / parts;
             part = j - (j / parts) * parts;
         }
-        if (super_tiles) {
-            const int s = v >> 5, i = v & 31;
-            const int spr = n_tok_tiles >> 2;
-            const int sr = s / spr;
-            row_tile = sr * 8 + (i >> 2);
-            t0 = ((s - sr * spr) * 4 + (i & 3)) * kTileTok;
-        } else {
-            row_tile = v / n_tok_tiles;
-            t0 = (v - row_tile * n_tok_tiles) * kTileTok;
-        }
+        gemm6_tile(v, n_tok_tiles, super_tiles, row_tile, t0);
         slot = v - n_whole;
     }
     int wsel = 0;

@@ -15,27 +15,29 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("K,N,M,wgroup", [
-    (256, 64, 65, 0),         # four groups for eight wavefronts
-    (512, 1, 128, 64),        # one group each, one row
-    (4352, 130, 190, 0),      # eight or nine, ragged
-    (4352, 130, 190, 256),
-    (15360, 70, 66, 0),       # 30: past the 28 between two transfers
-    (32768, 65, 67, 64),      # the longest row
-    (512, 4096, 512, 0),      # 512 units: two rounds
-    (512, 4300, 2048, 0),     # 17 x 16 tiles: 16 left over behind a round, the last row tile ragged
-    (512, 8192, 1100, 256),   # 32 x 9 tiles: 32 left over, in runs of nine token tiles
-    (2560, 6200, 33, 0),      # 97 panels: the skinny kernel
-    (2560, 6200, 64, 64),
-    (17408, 6145, 41, 0),
-    (2560, 8300, 33, 0),      # 130 panels: 33 .. 64 tokens in units
-    (2560, 8300, 64, 64),
-    (17408, 8257, 41, 0),
-    (512, 16500, 57, 0)])     # 258: two rounds
-def test_units_of_64_rows_and_tokens(oracle, K, N, M, wgroup):
+@pytest.mark.parametrize("K,N,M,wgroup,units", [
+    (256, 64, 65, 0, 2),             # four groups for eight wavefronts
+    (512, 1, 128, 64, 2),            # one group each, one row
+    (4352, 130, 190, 0, 9),          # eight or nine, ragged
+    (4352, 130, 190, 256, 9),
+    (15360, 70, 66, 0, 4),           # 30: past the 28 between two transfers
+    (32768, 65, 67, 64, 0),          # the longest row: by price one tile in slices
+    (17408, 70, 67, 64, 4),          # 34, with multipliers
+    (512, 4096, 512, 0, 512),        # 512 units: two rounds
+    (512, 4300, 2048, 0, 128),       # 17 x 16 tiles: 16 left over behind a round, the last row tile ragged
+    (512, 8192, 1100, 256, 256),     # 32 x 9 tiles: 32 left over, in runs of nine token tiles
+    (2560, 6200, 33, 0, 0),          # 97 panels: the skinny kernel
+    (2560, 6200, 64, 64, 0),
+    (17408, 6145, 41, 0, 0),
+    (2560, 8300, 33, 0, 130),        # 130 panels: 33 .. 64 tokens in units
+    (2560, 8300, 64, 64, 130),
+    (17408, 8257, 41, 0, 130),
+    (512, 16500, 57, 0, 258)])       # two rounds
+def test_units_of_64_rows_and_tokens(oracle, K, N, M, wgroup, units):
     type_ = rq.TYPE_W4A4 if K in (256, 512, 32768) else rq.TYPE_W4A4H
     blocks, wf = adversarial_weights(oracle, N, K, type_, seed=N + M, wgroup=wgroup)
     W = rq.W4A4Weight(blocks, type_, DEV)
+    assert plan(type_, K, N, M, wgroup != 0)["units"] == units
     x = adversarial_activations(M, K, type_, wf, seed=M)
     want = oracle.mul_mat(type_, blocks, x, W.clip, n_rot=max(W.n_rot, 0))
     got = run_gpu(W, x)

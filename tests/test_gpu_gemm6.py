@@ -1,6 +1,6 @@
-"""The wide-batch product kernel on the fp6 MFMA (rq_gemm6.hip): launches made of whole tiles and of tiles cut along
-K, compared bit for bit with the oracle; and the int8 MFMA kernel it replaced, which RQ_GEMM_FP6=0 still selects, in a
-child process (the variable is read once per process)."""
+"""Wide batches through the fp6 MFMA kernels, compared bit for bit with the oracle, by whichever of tiles, K slices and units the
+router takes (test_gpu_tiles.py and test_gpu_block6.py mean one of them each); and the int8 MFMA kernel they replaced, which
+RQ_GEMM_FP6=0 still selects, in a child process (the variable is read once per process)."""
 import ctypes
 import os
 import subprocess
@@ -30,9 +30,8 @@ def test_prepared_weight_carries_the_fp6_plane():
 @pytest.mark.parametrize("type_,wgroup", [(rq.TYPE_W4A4H, 0), (rq.TYPE_W4A4, 64), (rq.TYPE_W4A4, 256)],
                          ids=["w4a4h", "w4a4_wgroup64", "w4a4_wgroup256"])
 def test_leftover_tiles_cut_along_k_uneven_slices(oracle, type_, wgroup):
-    """8 row tiles x 33 token tiles = 264 tiles: 256 run whole, the last 8 (one row tile, eight token tiles) are cut
-    into five slices of 6 or 7 steps of the row's 34 (K = 4352 = 68 x 64: an odd step count in most slices), which
-    meet through their slabs. Ragged rows and tokens, with and without weight multipliers."""
+    """8 row tiles x 33 token tiles = 264 tiles: 256 run whole, the last 8 (one row tile, eight token tiles) as 64 units.
+    Ragged rows and tokens, with and without weight multipliers, K = 4352 = 68 x 64."""
     N, K, M = 2000, 4352, 4200
     blocks, wf = adversarial_weights(oracle, N, K, type_, wgroup=wgroup)
     W = rq.W4A4Weight(blocks, type_, DEV)
@@ -40,7 +39,7 @@ def test_leftover_tiles_cut_along_k_uneven_slices(oracle, type_, wgroup):
     got = run_gpu(W, x)
     want = oracle.mul_mat(type_, blocks, x, W.clip, n_rot=max(W.n_rot, 0))
     assert bits_equal(got, want), first_mismatch(got, want)
-    # twice on the same workspace: the arrival counters are left zero
+    # twice
     got2 = run_gpu(W, x)
     assert bits_equal(got2, want), first_mismatch(got2, want)
 
@@ -48,7 +47,7 @@ def test_leftover_tiles_cut_along_k_uneven_slices(oracle, type_, wgroup):
 def test_slices_longest_row_extreme_sums(oracle):
     """K = 32768 with every tile cut along K (1 row tile x 12 token tiles: 13 slices of 19 or 20 steps each), inputs
     that drive the sums to their ends: rows of all -8 / all +7 codes against tokens that quantize to q - z = +-15 with
-    m = 255 in all 512 groups. Within a slice the biased fp32 accumulator moves by 122400 per group for 32 groups
+    m = 255 in all 512 groups (without weight multipliers such rows do not go in units). Within a slice the biased fp32 accumulator moves by 122400 per group for 32 groups
     between two transfers to the int32 total (3.9 M of the 4.19 M its window allows), in both directions."""
     N, K, M, type_ = 256, 32768, 1536, rq.TYPE_W4A4
     blocks = synth.random_weight_blocks(N, K, 5, type_, clip=0.9)
@@ -78,9 +77,9 @@ def test_slices_longest_row_extreme_sums(oracle):
 @pytest.mark.parametrize("per", [256, 64])
 def test_weight_multipliers_extreme_sums(oracle, per):
     """The same extremes on a tensor with weight multipliers (rq.pack_groups, one per block or per 64 inputs): rows of
-    all -8 / all +7 codes with multiplier 15 everywhere against q - z = +-15 with m = 255. A group then moves the
-    biased accumulator by 15 x 122400 = 1.836 M, so the kernel for such tensors transfers it to the int32 total after
-    every second group (3.67 M of the 4.19 M of its window); whole tiles and K slices, both signs."""
+    all -8 / all +7 codes with multiplier 15 everywhere against q - z = +-15 with m = 255, both signs: 95 units, whose
+    sums of bit patterns take 15 x 122400 = 1.836 M per group. (The tiled kernel, which transfers its float totals after
+    every second group, has the same rows in test_gpu_tiles.py.)"""
     N, K, M, type_ = 300, 4352, 1200, rq.TYPE_W4A4
     rng = np.random.default_rng(17)
     codes = rng.integers(-8, 8, size=(N, K), dtype=np.int8)
@@ -154,7 +153,7 @@ def test_a_moved_weight_needs_nothing_of_its_original(oracle, N, M, in_place):
 
 @pytest.mark.parametrize("M", [65, 128, 129, 300])
 def test_token_counts_around_the_tile(oracle, M):
-    """One and a few token tiles, partly filled, K = 5120 (every tile cut along K: few tiles, long rows)."""
+    """One and a few runs of 64 tokens, partly filled, K = 5120, few rows: units."""
     N, K, type_ = 520, 5120, rq.TYPE_W4A4H
     blocks, wf = adversarial_weights(oracle, N, K, type_)
     W = rq.W4A4Weight(blocks, type_, DEV)
@@ -166,7 +165,7 @@ def test_token_counts_around_the_tile(oracle, M):
 
 def test_workspace_without_slabs_runs_every_tile_whole(oracle):
     """A workspace that ends in front of the slabs of the K slices (what the static entry point has for wide batches)
-    gives the same bits: the launch then runs every tile whole."""
+    gives the same bits; these few rows go in units either way."""
     N, K, M, type_ = 520, 2560, 200, rq.TYPE_W4A4H
     blocks, wf = adversarial_weights(oracle, N, K, type_)
     W = rq.W4A4Weight(blocks, type_, DEV)
@@ -200,8 +199,8 @@ def test_int8_gemm_under_rq_gemm_fp6_0():
 @pytest.mark.parametrize("M,slabs", [(65, True), (200, True), (200, False), (4700, True)])
 def test_several_weights_in_one_launch(oracle, M, slabs, wgroup):
     """Three weights of one kind whose row tiles (2 + 1 + 4, ragged) are counted through in one launch, rows too short to
-    be cut along K: one and two token tiles, a workspace without slabs, and a whole round with tiles left over (7 x 37
-    tiles). Outputs with row strides of their own; what lies beside them stays."""
+    be cut along K: units at 65 and 200 tokens, a workspace without slabs, and a whole round with three tiles left over to the
+    units (7 x 37 tiles). Outputs with row strides of their own; what lies beside them stays."""
     K, type_ = 512, rq.TYPE_W4A4
     ws, bl = [], []
     for i, N in enumerate([384, 98, 1000]):
@@ -255,15 +254,15 @@ def test_one_launch_only_where_it_is_not_slower(K, Ns, M, launches):
 
 
 @pytest.mark.parametrize("K,M,Ns,wgroups,moved,launches", [
-    (2560, 512, (500, 200, 1200), (0, 0, 0), False, 1),        # 2 + 1 + 5 row tiles: super-tiles over weights, all cut
-    (512, 4096, (500, 200, 1200), (256, 256, 256), False, 1),  # the same, one whole round
+    (2560, 512, (500, 200, 1200), (0, 0, 0), False, 1),        # units over weights
+    (512, 4096, (500, 200, 1200), (256, 256, 256), False, 1),  # 2 + 1 + 5 row tiles: super-tiles over weights, one whole round
     (2560, 200, (1000, 700), (64, 64), False, 1),              # two weights: the third slot selects nothing
     (2560, 200, (384, 98, 1000), (64, 0, 64), False, 3),       # with and without multipliers: a launch each
-    (2560, 200, (384, 98, 1000), (64, 256, 0), True, 1)],      # copies the launcher knows nothing of: folds per tile
-    ids=["super_tiles_cut", "super_tiles_whole", "two_weights", "both_kinds", "unknown_addresses"])
+    (2560, 200, (384, 98, 1000), (64, 256, 0), True, 1)],      # copies the launcher knows nothing of: units read the flags
+    ids=["units", "super_tiles_whole", "two_weights", "both_kinds", "unknown_addresses"])
 def test_sets_of_weights(oracle, K, M, Ns, wgroups, moved, launches):
-    """Sets whose tiles are cut, whole and in super-tiles that straddle weights, against the oracle, with outputs of their
-    own row strides."""
+    """Sets in units and in whole super-tiles that straddle weights, against the oracle, with outputs of their own row
+    strides (slices of sets: test_gpu_tiles.py)."""
     type_ = rq.TYPE_W4A4
     ws, bl = [], []
     for i, (N, g) in enumerate(zip(Ns, wgroups)):

@@ -624,7 +624,8 @@ def test_split_k_cells_in_a_dirty_workspace(oracle, M, Ns, one_launch):
     """Up to 64 tokens the panels beyond whole rounds of the chip meet in cells of the workspace, and the call clears
     the cells of those panels only: two such panels, one, none, or all the panels of a small weight; the weights of a call in one
     launch, or (cells for the largest alone) in launches that take turns on the same cells. The workspace holds other
-    bytes before each call."""
+    bytes before each call. (33 and 64 tokens of so many panels go in units and need no cells; the calls that keep the skinny
+    kernel there are in test_gpu_tiles.py.)"""
     K, type_ = 1024, rq.TYPE_W4A4
     ws, bl = [], []
     for i, N in enumerate(Ns):
