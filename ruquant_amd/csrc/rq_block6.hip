@@ -10,10 +10,11 @@
 // Arithmetic and operands are the tiled kernel's: one v_mfma_f32_32x32x64_f8f6f4 on fp6 fragments per 32 x 32 outputs and
 // group, and the floor as one FMA rounded toward minus infinity (see there for why both are exact; reference patch lines
 // 148-177). The fragments go from memory (L2, after the first reader) straight into registers, four groups of a wavefront
-// in flight (non-temporal hints and deeper or shallower rings change nothing). Measured: 4.2 us + 0.52 us per group of a
-// wavefront (K = 5120: ten of them, 9.3 us; the tiled kernel 19.5), of which the loads, 6 KB per group through the
-// compute unit's 64 bytes per cycle, take 0.32 and the vector ALU and the MFMAs 0.33. Beyond two rounds of the chip the tiled
-// kernel's twofold reuse out of LDS wins.
+// in flight (non-temporal hints and deeper or shallower rings change nothing). Measured, with the weights in the memory-side
+// cache: 4.2 us + 0.52 us per group of a wavefront (K = 5120: ten of them, 9.3 us; the tiled kernel 19.5). Eight groups are 48 KB
+// through the compute unit's 64 bytes per cycle, 0.32 us; 112 vector instructions each, 0.37 us of the SIMDs' time, and four
+// MFMAs, 0.11 (counters: 1.144 M vector instructions and 1.31 M MFMA cycles for 128 units of 80 groups). From memory the weights'
+// 24 KB are the longest, 1.0 to 1.2 us. Beyond two rounds of the chip the tiled kernel's twofold reuse out of LDS wins.
 #include "rq_common.h"
 
 #pragma clang fp contract(off)
@@ -388,12 +389,14 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 // - More: N = 17408 (272), K = 3072 25.7 / 20.0, 27.1 / 24.3; K = 5120 30.7 / 25.9, 31.8 / 32.5; K = 10240 44.5 / 41.1, 45.3 / 53.7;
 //   K = 17408 63.0 / 61.7, 63.6 / 83.1; K = 32768 100 / 147. N = 24576 (384), K = 10240 55.7 / 42.2, 56.7 / 55.8; N = 34816 (544)
 //   73.7 / 65.7, 74.5 / 79.8. Here up to K = 5120, and up to K = 10240 where the last round is at least half full.
-// - Weight multipliers cost the skinny kernel more: up to 128 panels K = 1024, N = 8192 9.8 / 10.3, K = 5120 18.3 / 17.9, 20.0 / 21.3;
-//   N = 12288, K = 5120 29.7 / 18.9, 31.2 / 22.4, K = 32768 128 / 91, 128 / 95; N = 17408, K = 17408 86 / 71, 87 / 91, K = 32768
-//   145 / 160. Here from 129 panels up, beyond a round of units up to K = 17408.
+// - Weight multipliers cost the skinny kernel more: 96 to 128 panels, N = 8192, K = 1024 9.8 / 10.3, K = 3072 N = 6144 14.1 / 13.8,
+//   15.3 / 15.8, K = 5120 18.3 / 17.9, 20.0 / 21.3, K = 10240 33.9 / 26.6, 34.9 / 33.4, K = 17408 58.2 / 45.9, 48.4 / 50.7 (and 8 % more
+//   at 33 tokens); N = 12288, K = 5120 29.7 / 18.9, 31.2 / 22.4, K = 32768 128 / 91, 128 / 95; N = 17408, K = 17408 86 / 71, 87 / 91,
+//   K = 32768 145 / 160. Here from K = 3072 to 10240 with 96 panels, any length in one round of units, up to K = 17408 beyond.
 // 33 tokens are within a tenth of 64 on both sides.
 bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers) {
-    if (M <= 32 || n_panels <= kPlanUnits / 2) return false;
+    if (M <= 32) return false;
+    if (n_panels <= kPlanUnits / 2) return weight_multipliers && n_panels >= 96 && ng >= 48 && ng <= 160;
     if (n_panels <= kPlanUnits) return ng <= 272 || weight_multipliers;
     if (weight_multipliers) return ng <= 272;
     const int64_t last = n_panels % kPlanUnits;

@@ -28,6 +28,7 @@ DEV = "cuda:0"
     (512, 8192, 1100, 256, 256),     # 32 x 9 tiles: 32 left over, in runs of nine token tiles
     (2560, 6200, 33, 0, 0),          # 97 panels: the skinny kernel
     (2560, 6200, 64, 64, 0),
+    (3072, 6200, 40, 64, 97),        # with multipliers there too
     (17408, 6145, 41, 0, 0),
     (2560, 8300, 33, 0, 130),        # 130 panels: 33 .. 64 tokens in units
     (2560, 8300, 64, 64, 130),

@@ -19,7 +19,8 @@ def test_kernel_by_token_count(M, kernel):
     (5120, 8192, 0, SKINNY), (5120, 8193, 0, FP6), (17408, 12288, 0, FP6), (18432, 12288, 0, SKINNY), (32768, 17408, 0, SKINNY),
     (5120, 17408, 0, FP6), (5376, 17408, 0, SKINNY), (10240, 17408, 0, SKINNY), (10240, 24576, 0, FP6), (10240, 34816, 0, SKINNY),
     (12288, 24576, 0, SKINNY), (17408, 17408, 0, SKINNY), (5120, 34816, 0, FP6),
-    (1024, 8192, 1, SKINNY), (1024, 8256, 1, FP6), (32768, 12288, 1, FP6), (17408, 17408, 1, FP6), (32768, 17408, 1, SKINNY)])
+    (1024, 8192, 1, SKINNY), (2816, 8192, 1, SKINNY), (3072, 6080, 1, SKINNY), (3072, 6081, 1, FP6), (10240, 8192, 1, FP6),
+    (10496, 8192, 1, SKINNY), (10240, 8192, 0, SKINNY), (1024, 8256, 1, FP6), (32768, 12288, 1, FP6), (17408, 17408, 1, FP6), (32768, 17408, 1, SKINNY)])
 @pytest.mark.parametrize("M", [33, 64])
 def test_33_to_64_tokens(K, N, multipliers, kernel, M):
     """Units of the fp6 product only where they are no slower on weights that come from memory either (6 % at most)."""
