@@ -126,8 +126,10 @@ int rq_w4a4_mul_mat(int type, const void *prepared_dev, int64_t K, int64_t N,
 
 /* rq_w4a4_mul_mat for a caller that will not run stage 2 of rq_w4a4_mul_mat_stages on this workspace afterwards: same
  * arguments and results. rq_w4a4_mul_mat clears the split-K cells of all N rows, so that a later stage-2 call finds them
- * clear whichever of them its plan uses; this call clears only those that it uses itself (5 to 64 tokens; K = 5120,
- * N = 17408 at 64 tokens: 0.5 instead of 8.9 MB). No counterpart in the reference. */
+ * clear whichever of them its plan uses, and keeps the activations in the form that a product of any weight reads. This
+ * call clears only the cells that it uses itself (5 to 64 tokens), and at 33 to 64 tokens of enough rows (some
+ * thousands, by row length and multipliers) it runs a kernel with an activation form of its own and no cells (K = 5120, N = 17408 at 64
+ * tokens: 27.3 instead of 34.5 us). No counterpart in the reference. */
 int rq_w4a4_mul_mat_once(int type, const void *prepared_dev, int64_t K, int64_t N,
                          const float *x_dev, int64_t ldx, int64_t M,
                          float *y_dev, int64_t ldy,

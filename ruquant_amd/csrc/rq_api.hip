@@ -158,8 +158,8 @@ bool rotation_of(int type, int64_t K, int64_t n_rot, int &p, int &m) {
     return hadamard_factor(n_rot, p, m);
 }
 
-// Measured crossovers: up to four tokens the dot-product GEMV, from five the skinny MFMA kernel, from 65 the tiled
-// MFMA GEMM. (Four tokens, K = 5120, whole call on the GEMV against the skinny kernel: N = 1024 9.1 against 11.4 us,
+// Measured crossovers: up to four tokens the dot-product GEMV, from five the skinny MFMA kernel, from 65 the fp6
+// product (from 33 for some calls, block6_takes). (Four tokens, K = 5120, whole call on the GEMV against the skinny kernel: N = 1024 9.1 against 11.4 us,
 // N = 5120 11.8 against 12.3, N = 8192 and 17408 the same, N = 34816 26.2 against 25.5: the GEMV's activation side is
 // one launch, the skinny kernel's two. Five tokens: 13.7 against 12.3 us at N = 5120, 22.7 against 18.0 at N = 17408.
 // The choice depends on the token count only, so that a quantized activation can be shared between weights.)
@@ -218,8 +218,9 @@ Choice choose(int n, int64_t K, const int64_t *N, int64_t M, bool rotate, int p,
     c.path = path_of(M);
     // Skinny batches with a long Paley stage: one workgroup per token would leave most of the chip idle for tens of
     // microseconds, so the rotation runs spread over workgroups (ranges out) and a second small kernel quantizes.
-    // (up to 40 tokens: from there on the one-workgroup-per-token kernel has enough tokens to fill the chip: K = 17408,
-    // 64 tokens: 17.9 us against 21.2 us)
+    // (up to 40 tokens, where the two meet: K = 17408 5 tokens 9.7 us, 16 10.1, 24 12.4, 40 13.4, in one launch 13.5 to 13.9 for any
+    // of them. Orders without a slab kernel, all but 68, rotate a token per workgroup either way, and the second launch costs
+    // them 1.3 to 2.7 us: K = 15360, 16 tokens 13.4 against 11.6, K = 18432 15.6 / 14.3, K = 21504 18.1 / 16.5.)
     // (the second kernel reads ranges per run of 64: activation groups of 64 only)
     c.two_step = c.path == kPathSkinny && G == kGroup && rotate && p >= 44 && (m & 63) == 0 && M <= kTwoStepTokens;
     // 33 .. 64 tokens of a call that shares its activation with no other: the small units of the fp6 product where they are
@@ -388,8 +389,9 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
         q.zero_ptr = reinterpret_cast<int32_t *>(wsb + W.off_tot);
         // A stage-2 call may follow with any weight of at most N rows, whose plan cuts other panels than this call's:
         // cells for all rows. A call that is said to be the workspace's only one clears the cells of the panels that it
-        // cuts itself. (One 64-token call, K = 5120, N = 17408: all cells are 8.9 MB, cleared by workgroups of which a
-        // compute unit holds one or two; 34.5 us, 33.7 with the cells of the 16 cut panels alone.)
+        // cuts itself. (64 tokens through this kernel, K = 5120, N = 17408: all cells are 8.9 MB, cleared by workgroups of which
+        // a compute unit holds one or two; 34.5 us, 33.7 with the cells of the 16 cut panels alone. Such calls now go in
+        // units, which have no cells; what is left here is smaller.)
         int64_t cells = 0;
         if (!once) {
             cells = M * (int64_t) ((sp.Ncells + kPanelRows - 1) / kPanelRows * kPanelRows);

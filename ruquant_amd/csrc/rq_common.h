@@ -110,7 +110,7 @@ inline size_t act6_plane_bytes(int ng, int64_t Mp) { return (size_t) ng * (size_
 //            the K slice it consumes itself.
 //            MFMA paths: two int8 digit planes of m (q - z), [g][digit][quarter][Mp][16 bytes], in the byte order
 //            the weight unpack produces (for M <= 64 they follow the fp32 form, which the skinny path may use as
-//            an intermediate). The fp6 GEMM (M >= 65) takes one plane of q - z as fp6 MFMA fragments instead,
+//            an intermediate). The fp6 product (M >= 65, and from 33 tokens where block6_takes) takes one plane of q - z as fp6 MFMA fragments instead,
 //            [g][Mp / 32][1536 bytes] (lane = token % 32 + 32 * half, as in the weight plane), followed by the
 //            group multipliers as floats 4 m, [g][Mp].
 //   cells  : split-K cells [8 or 64 tokens][n_panels * 64], 64 bits each: arrival count above bit 48, exact sum
