@@ -850,7 +850,8 @@ Gemm6Route gemm6_route(const FusedWeights &w, int64_t M, int groups_per_fold, bo
     if (groups_per_fold != 1) return r;   // (the small units fold groups of 64)
     const int64_t units = n_panels * ((M + 63) / 64);
     const double all = block_price(units, ng, weight_multipliers);
-    const bool short_rows = weight_multipliers || ng <= (units <= kPlanUnits ? 272 : 96);
+    // (a workspace without slabs: the choice is between units and whole tiles, K = 32768 200 us)
+    const bool short_rows = weight_multipliers || !have_slabs || ng <= (units <= kPlanUnits ? 272 : 96);
     if (units <= 2 * kPlanUnits && short_rows && all < r.price) {
         r.plan.n_tiles = r.plan.n_whole = r.first_block = 0;
         r.plan.parts = 1;

@@ -132,6 +132,14 @@ def test_tiles_left_over_to_the_units(oracle, K, Ns, M, multipliers, whole, unit
     check(oracle, bl, ws, tokens(M, K, M), sample_of(M), repeats=1)
 
 
+def test_without_slabs_long_rows_go_in_units(oracle):
+    K, N, M = 32768, 200, 100
+    assert plan(rq.TYPE_W4A4, K, N, M)["cut"] == 1 and plan(rq.TYPE_W4A4, K, N, M, slabs=False)["units"] == 8
+    b = weights(N, K, 8, 0)
+    w = rq.W4A4Weight(b, rq.TYPE_W4A4, DEV, keep_blocks=False)
+    check(oracle, [b], [w], tokens(M, K, 4), sample_of(M), workspace=rq.fused_workspace_bytes([w], M) - 256)
+
+
 @pytest.mark.parametrize("N,M,units", [(8300, 40, 130), (8300, 64, 130), (6200, 64, 0)])
 def test_static_workspace_at_33_to_64_tokens(oracle, N, M, units):
     """rq_w4a4_mul_mat_static from 129 panels up (units) and below (the skinny kernel), the two in turn on the one array."""

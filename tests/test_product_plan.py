@@ -55,6 +55,8 @@ def test_long_rows_above_64_tokens(K, N, M, multipliers, units):
     """Few tiles of long rows without multipliers are cut along K: units get weights from memory too slowly."""
     p = plan(W4A4, K, N, M, multipliers)
     assert (p["units"] > 0) == units and (p["cut"] > 0) == (not units) and p["whole"] == 0
+    # without room for slices the other choice is whole tiles, a workgroup each: units
+    assert plan(W4A4, K, N, M, multipliers, slabs=False)["units"] > 0
 
 
 def test_every_tile_is_counted_once():
