@@ -18,9 +18,9 @@
 // groups (3,916,800 < 2^22) its offset from the start is moved into an int32 total (two integer instructions per
 // value: the float's bit pattern minus the bit pattern of 1.5 x 2^23 is that offset) and it starts again.
 //
-// Tensors with integer weight multipliers k (uniform branch on the prepared flag) fold
-// floor(k m S / 16) in integers instead. Activation groups of 128 / 256 (RQ_ACT_GROUP) chain the 2 or 4 MFMAs of a
-// group through the accumulator operand before the one fold.
+// Tensors with integer weight multipliers k (uniform branch on the prepared flag) fold 4 m k instead of 4 m, on the bias itself,
+// and add the bit patterns up in integers. Activation groups of 128 / 256 (RQ_ACT_GROUP) chain the 2 or 4 MFMAs of a
+// group through the accumulator operand before the one fold (and multipliers in integers).
 //
 // Data movement: a workgroup of eight wavefronts owns 256 rows x 128 tokens; wavefront (wr, wc) owns rows 64 wr .. and
 // tokens 64 wc .. as 2 x 2 MFMA tiles of 32 x 32. Operands go from global memory straight into LDS
@@ -28,6 +28,13 @@
 // rq_w4a4_prepare writes and the activation plane of the quantizer are stored as MFMA fragments (32 rows or tokens x
 // 64 inputs = 1536 bytes: a 16-byte and an 8-byte piece per lane, each piece contiguous across the lanes), so a
 // stage is filled by whole 1 KiB runs and read back without bank conflicts.
+//
+// What bounds it: the issue of vector instructions (per MFMA 16 FMAs of four cycles each and 14 cycles of the MFMA that none of
+// them hides: 400,000 of the 526,000 cycles at K = 10240, N = 16384, 2048 tokens) and, above that, the clock, which the matrix
+// cores, the vector ALU and LDS together pull down to 1.87 GHz (2.2 for MFMAs and FMAs alone). 16 MFMAs of a SIMD, a step, take
+// 0.72 us, without LDS reads and fetches 0.53; a tile costs 9.4 us besides its steps. K = 5120, N = 17408, 2048 tokens 183.6 ->
+// 171 us and K = 17408, N = 5120 160 -> 147.5 since a wavefront waits for its operands where it uses them and every read of the
+// ring has a fixed base; with weight multipliers (K = 5120, N = 8192) 139 -> 128, in the same kernel.
 #include "rq_common.h"
 
 #include <string.h>
@@ -49,18 +56,21 @@ constexpr int kTileTok = 128;                  // tokens of a workgroup's tile
 constexpr int kCellsA = 8 * kFrag6 / 16;       // 768 cells: eight weight fragments of one group
 constexpr int kCellsB = 4 * kFrag6 / 16;       // 384 cells: four activation fragments of one group
 constexpr int kCellsM = kTileTok * 4 / 16;     // 32 cells: the 128 tokens' multipliers of one group (4 m as float)
-// One ring stage = two groups: [A g0][A g1][B g0][B g1][m g0][m g1][k g0][k g1] = 2400 cells of 16 bytes = 37.5 KiB
 constexpr int kCellsK = kTileRows / 16;         // 16 cells: the 256 rows' weight multipliers of one group (a byte each)
-constexpr int kOffA = 0, kOffB = 2 * kCellsA, kOffM = kOffB + 2 * kCellsB, kOffK = kOffM + 2 * kCellsM;
-constexpr int kStageCellsPlain = kOffK;                 // without the rows' weight multipliers
-constexpr int kStageCellsK = kOffK + 2 * kCellsK;       // with them
+// A ring stage is two groups. The stages of the two operands stand apart, those of the activations first, each [B g0][B g1][m g0]
+// [m g1][k g0][k g1], behind them those of the weights, [A g0][A g1]: a lane's reads then reach every stage from few base
+// registers (an instruction's offset is 64 KB): one for the activations' 16-byte pieces, one for their 8-byte pieces, one for
+// the multipliers, and two each for the weights'.
 constexpr int kRing = 4;
-static_assert(kStageCellsPlain == 2368 && kStageCellsK == 2400, "stage size");
-// Each wavefront moves four whole 1 KiB runs per step (cells 0 .. 2047: the weights and the first 512 activation
-// cells) and 44 lanes' worth of a fifth (cells 2048 .. 2399: the rest of the activations, the tokens' multipliers and the
-// rows' weight multipliers).
-constexpr int kTailCell = 2048;
-static_assert(kTailCell + 8 * 40 == kStageCellsPlain && kTailCell + 8 * 44 == kStageCellsK, "tail split");
+constexpr int kStageA = 2 * kCellsA * 16;
+constexpr int kOffM = 2 * kCellsB * 16, kOffK = kOffM + 2 * kCellsM * 16;   // in a stage of the activations
+constexpr int kStageB = kOffK + 1024;                                       // (k is 512 bytes, moved by a whole wavefront)
+constexpr int kOffA = kRing * kStageB;
+constexpr int kRingBytes = kOffA + kRing * kStageA;
+// Each wavefront moves five runs of 1 KiB per step: three of the weights' 24, one of the activations' first eight, and of the
+// rest of their stage wavefronts 0 .. 3 the last four, 4 the tokens' multipliers, 5 the rows'; 6 and 7 the same as 4 and 5 (so
+// that every wavefront has the same number of loads in flight).
+static_assert(kStageA == 24 * 1024 && kOffM == 12 * 1024 && kStageB == 14 * 1024, "split of a step's loads");
 constexpr int kLoadsPerStep = 5;
 
 constexpr int kXposeStride = 36;               // floats between tokens of a wavefront's output block in LDS (32 rows + 4)
@@ -69,17 +79,6 @@ constexpr int kBiasBits = 0x4B400000;
 constexpr int kFlushSteps = 16;                // 32 groups
 constexpr int kRsrcWord3 = 0x00020000;         // last word of a raw buffer descriptor on this target (32-bit data format)
 constexpr int kDeviceScope = 16;               // cache policy of a buffer access: the sc1 bit
-
-// WITHK: the stage of the kernel form that folds with weight multipliers from LDS. (Two layouts, because the 512
-// bytes shift the stages' LDS offsets, and with them the plain kernel's loop needs base registers it does not have.)
-// (SET is a tag that keeps the helpers of two kernels apart: a helper that both call no longer has constant LDS addresses
-// when the compiler simplifies it ahead of inlining, and the plain loop then spills 113 registers instead of 9.)
-template <bool WITHK, bool SET>
-struct StageT {
-    static constexpr int kCells = WITHK ? kStageCellsK : kStageCellsPlain;
-    static constexpr int kTailLanes = WITHK ? 44 : 40;   // lanes of a wavefront's fifth load
-    uint4 cell[kCells];
-};
 
 // 64 lanes x 16 bytes from base + lane offset to 1 KiB of LDS at `lds` (wave-uniform; the hardware adds lane * 16).
 // Assembly, so that the count of outstanding loads stays under this file's control (the s_waitcnt of step()).
@@ -91,25 +90,13 @@ __device__ __forceinline__ const uint8_t *uniform(const uint8_t *p) {
                      (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (b >> 32)) << 32));
 }
 
-__device__ __forceinline__ void load_run(const uint8_t *base, uint32_t lane_off, uint4 *lds) {
-    const uint32_t lds_addr = (uint32_t) (uintptr_t) (lds_void *) lds;
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+// (OFF: a constant part of the LDS address, added on the way into M0)
+template <int OFF>
+__device__ __forceinline__ void load_run(const uint8_t *base, uint32_t lane_off, uint32_t lds) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
-                 : "v"(lane_off), "s"(base), "s"(lds_addr)
-                 : "memory", "m0");
-}
-
-// the same from per-lane addresses, for the lanes of `mask` only (the others move nothing). The execution mask is
-// switched inside the statement: a branch around the load would cut the step into several basic blocks, and the
-// compiler then sinks the folds of one step behind the barrier of the next (their inputs, 128 registers, spill).
-__device__ __forceinline__ void load_cells(const uint8_t *gptr, uint4 *lds, uint64_t mask) {
-    const uint32_t lds_addr = (uint32_t) (uintptr_t) (lds_void *) lds;
-    uint64_t saved;
-    asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 %0, exec\n\ts_mov_b64 exec, %3\n\t"
-                 "global_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, %0"
-                 : "=&s"(saved)
-                 : "v"(gptr), "s"(lds_addr), "s"(mask)
-                 : "memory", "m0");
+                 : "v"(lane_off), "s"(base), "s"(lds), "n"(OFF)
+                 : "memory", "m0", "scc");
 }
 
 __device__ __forceinline__ void load_to_lds_dword(const float *gptr, float *lds) {
@@ -121,48 +108,75 @@ __device__ __forceinline__ void load_to_lds_dword(const float *gptr, float *lds)
 }
 
 struct Ctx {
-    // the four whole runs this wavefront moves per step: address of step 0 and advance per step (wave-uniform)
-    const uint8_t *run_src[4];
-    size_t run_step[4];
-    const uint8_t *tail_src; // this lane's cell of the fifth load, current step
-    uint32_t tail_step;      // its advance per step (bytes: under 4 GiB for any batch the workspace can hold)
+    // what this wavefront moves per step (wave-uniform): three runs of the weights, 8 KB apart, one of the activations, a fifth
+    // with lane offsets of its own; and where to, in the first stage
+    const uint8_t *a_src, *b_src, *t_src;
+    uint32_t b_step, t_step;       // their advance per step (bytes: under 4 GiB for any batch the workspace can hold)
+    uint32_t t_off;
+    uint32_t lds_run, lds_t;
+    // this lane's places in the first stage of the ring: 16- and 8-byte pieces of the activations, the tokens' and the rows'
+    // multipliers, and the pieces of the weights in stages 0 and 2
+    uint32_t b16, b8, m, k, a16[2], a8[2];
     const uint8_t *k_src;    // weight multipliers of this wavefront's panel, row offset of the lane's first quad
     int wave, wr, wc, lane;
     int n_steps;             // steps (two groups each) of this workgroup
     int g0;                  // its first group
 };
 
-// fetch of step `st` (two groups) into stage s, then advance the sources; past the last step they stay where they
+// fetch of step `st` (two groups) into stage S, then advance the sources; past the last step they stay where they
 // are (the last step is fetched again, into cells nobody reads), so every step issues the same number of loads.
 // In pieces, so that the loop can deal them out between its MFMAs: five loads issued back to back by all eight
 // wavefronts right behind the barrier queue up in front of the memory pipeline, and a wavefront that waits to issue a
-// load issues no MFMA either.
-template <class Stage>
-__device__ __forceinline__ void fetch_run(Ctx &c, Stage &s, int st, int i) {
-    load_run(c.run_src[i], (uint32_t) c.lane * 16, &s.cell[(i * 8 + c.wave) * 64]);
-    c.run_src[i] = uniform(c.run_src[i] + (st + 1 < c.n_steps ? c.run_step[i] : 0));
+// load issues no MFMA either. Piece 0 .. 2 the weights, 3 and 4 the activations' stage.
+template <int S, int PIECE>
+__device__ __forceinline__ void fetch_piece(Ctx &c, int st) {
+    const bool more = st + 1 < c.n_steps;
+    if constexpr (PIECE < 3) {
+        load_run<kOffA + S * kStageA + PIECE * 8192>(uniform(c.a_src + PIECE * 8192), (uint32_t) c.lane * 16, c.lds_run);
+        if (PIECE == 2) c.a_src = uniform(c.a_src + (more ? kStageA : 0));
+    } else if constexpr (PIECE == 3) {
+        load_run<S * kStageB>(c.b_src, (uint32_t) c.lane * 16, c.lds_run);
+        c.b_src = uniform(c.b_src + (more ? c.b_step : 0));
+    } else {
+        load_run<S * kStageB>(c.t_src, c.t_off, c.lds_t);
+        c.t_src = uniform(c.t_src + (more ? c.t_step : 0));
+    }
 }
-template <class Stage>
-__device__ __forceinline__ void fetch_tail(Ctx &c, Stage &s, int st) {
-    load_cells(c.tail_src, &s.cell[kTailCell + c.wave * Stage::kTailLanes], ((uint64_t) 1 << Stage::kTailLanes) - 1);
-    c.tail_src += st + 1 < c.n_steps ? c.tail_step : 0;
-}
-template <class Stage>
-__device__ __forceinline__ void fetch(Ctx &c, Stage &s, int st) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fetch_run(c, s, st, i);
-    fetch_tail(c, s, st);
+template <int S>
+__device__ __forceinline__ void fetch(Ctx &c, int st) {
+    fetch_piece<S, 0>(c, st);
+    fetch_piece<S, 1>(c, st);
+    fetch_piece<S, 2>(c, st);
+    fetch_piece<S, 3>(c, st);
+    fetch_piece<S, 4>(c, st);
 }
 
-template <class Stage>
-__device__ __forceinline__ v8i fragment(const Stage &s, int cell0, int lane) {
-    const uint4 p0 = s.cell[cell0 + lane];
-    const uint2 p1 = *(reinterpret_cast<const uint2 *>(&s.cell[cell0 + 64]) + lane);
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+template <class T>
+__device__ __forceinline__ const __attribute__((address_space(3))) T *lds_at(uint32_t addr, int off) {
+    return reinterpret_cast<const __attribute__((address_space(3))) T *>((const __attribute__((address_space(3))) uint8_t *) addr + off);
+}
+// The two pieces of a fragment straight into the six registers of the operand. (The 8-byte piece by a volatile read: two
+// ordinary ones become one ds_read2st64_b64, whose results have to be moved into the operands' registers, and a wavefront
+// waits for its reads where the moves stand, right behind them, instead of in front of the MFMA a group later.)
+__device__ __forceinline__ v8i fragment(uint32_t p16, uint32_t p8, int off) {
+    const v4u lo = *lds_at<v4u>(p16, off);
+    const v2u hi = *reinterpret_cast<const volatile __attribute__((address_space(3))) v2u *>(lds_at<v2u>(p8, off));
     v8i v;
-    v[0] = (int) p0.x; v[1] = (int) p0.y; v[2] = (int) p0.z; v[3] = (int) p0.w;
-    v[4] = (int) p1.x; v[5] = (int) p1.y;
+    v[0] = (int) lo.x; v[1] = (int) lo.y; v[2] = (int) lo.z; v[3] = (int) lo.w;
+    v[4] = (int) hi.x; v[5] = (int) hi.y;
     // (the fp6 form reads six registers: elements 6 and 7 are left undefined)
     return v;
+}
+__device__ __forceinline__ v8i read_a(const Ctx &c, int stage, int gi, int i) {
+    return fragment(c.a16[stage >> 1], c.a8[stage >> 1], (stage & 1) * kStageA + gi * (kCellsA * 16) + i * kFrag6);
+}
+__device__ __forceinline__ v8i read_b(const Ctx &c, int stage, int gi, int i) {
+    return fragment(c.b16, c.b8, stage * kStageB + gi * (kCellsB * 16) + i * kFrag6);
+}
+__device__ __forceinline__ float read_m(const Ctx &c, int stage, int gi, int i) {
+    return *lds_at<float>(c.m, stage * kStageB + gi * (kCellsM * 16) + i * 128);
 }
 
 // fast path: acc += floor(m S / 16) for the 16 outputs of one tile (round toward minus infinity is set)
@@ -171,27 +185,22 @@ __device__ __forceinline__ void fold_fast(const v16f &S, float m4, float (&acc)[
     for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf(S[r], m4, acc[r]);
 }
 
-// weight multipliers (reference patch lines 169-173): acc += floor(k m S / 16), the same single FMA with 4 m k in
-// place of 4 m (k <= 15, so a group moves the accumulator by at most 15 x 122,400: flush after every second group).
-// kw: the multipliers of the lane's sixteen rows, four bytes per register.
-__device__ __forceinline__ void fold_km(const v16f &S, float m4, const uint32_t (&kw)[4], float (&acc)[16]) {
+// weight multipliers (reference patch lines 169-173): floor(k m S / 16) by the same FMA with 4 m k in place of 4 m, on the bias
+// itself: a term may be 15 times as large, so its bit pattern is added up in integers, and the bias of every term comes off at
+// the end. (The sum of the patterns passes 2^32 from the fourth group on: unsigned, modulo 2^32, which gives the total back, since
+// that is small: at most 512 groups x 15 x 122,400 = 940 M.)
+__device__ __forceinline__ void fold_km(const v16f &S, float m4, const float (&kf)[16], float bias, float (&acc)[16]) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        const float kf = (float) ((kw[r >> 2] >> (8 * (r & 3))) & 0xFFu);
-        acc[r] = __builtin_fmaf(S[r], kf * m4, acc[r]);
+        const float term = __builtin_fmaf(S[r], kf[r] * m4, bias);
+        acc[r] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, acc[r]) + __builtin_bit_cast(uint32_t, term));
+        asm volatile("" : "+v"(acc[r]));   // (formed here, not sunk into the blocks behind)
     }
 }
 // the sixteen multipliers a lane needs for row block a (rows 32 a + 8 q + 4 (lane / 32) + 0 .. 3, q = 0 .. 3) of group gi
-template <class Stage>
-__device__ __forceinline__ void read_kw(const Ctx &c, const Stage &s, int gi, int a, uint32_t (&kw)[4]) {
-    // (the lane's part of the address is worked out here each time: kept across the loop, the eight addresses that the
-    // compiler forms from it, one per stage and group, are registers the loop does not have, and their reloads from
-    // scratch wait for every load in flight)
-    uint32_t h = (uint32_t) c.lane >> 5;
-    asm volatile("" : "+v"(h));
-    const uint32_t *k = reinterpret_cast<const uint32_t *>(&s.cell[kOffK + gi * kCellsK]) + 16 * c.wr + 8 * a + h;
+__device__ __forceinline__ void read_kw(const Ctx &c, int stage, int gi, int a, uint32_t (&kw)[4]) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) kw[q] = k[2 * q];
+    for (int q = 0; q < 4; ++q) kw[q] = *lds_at<uint32_t>(c.k, stage * kStageB + gi * (kCellsK * 16) + 32 * a + 8 * q);
 }
 
 // the same in integers, from multipliers in global memory (the forms for activation groups of 128 / 256)
@@ -207,8 +216,8 @@ __device__ __forceinline__ void fold_k(const v16f &S, float m4, const int (&kk)[
 // One step (two groups of 64 inputs) of one wavefront: 64 rows x 64 tokens as 2 x 2 tiles. GS = runs of 64 per
 // activation group (1, 2, 4). A unit = one tile x one activation group's runs inside this step: its MFMAs chain through
 // the accumulator operand; the fold of unit i runs behind the MFMAs of unit i + 1.
-template <bool HASK, int GS, class Stage>
-__device__ __forceinline__ void compute(const Ctx &c, const Stage &s, int st, float (&acc)[2][2][16],
+template <bool HASK, int GS, int S0>
+__device__ __forceinline__ void compute(const Ctx &c, int st, float (&acc)[2][2][16],
                                         int32_t (&tot)[2][2][16], v16f (&carry)[2][2]) {
     constexpr int kRuns = GS == 1 ? 1 : 2;        // runs of a unit inside one step
     constexpr int kUnits = GS == 1 ? 8 : 4;
@@ -218,9 +227,9 @@ __device__ __forceinline__ void compute(const Ctx &c, const Stage &s, int st, fl
     for (int gi = 0; gi < 2; ++gi) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            A[gi][i] = fragment(s, kOffA + gi * kCellsA + (2 * c.wr + i) * (kFrag6 / 16), c.lane);
-            B[gi][i] = fragment(s, kOffB + gi * kCellsB + (2 * c.wc + i) * (kFrag6 / 16), c.lane);
-            m4[gi][i] = reinterpret_cast<const float *>(&s.cell[kOffM + gi * kCellsM])[64 * c.wc + 32 * i + (c.lane & 31)];
+            A[gi][i] = read_a(c, S0, gi, i);
+            B[gi][i] = read_b(c, S0, gi, i);
+            m4[gi][i] = read_m(c, S0, gi, i);
         }
     }
     // with groups of 256 a unit spans two steps: the even step leaves its half in `carry`, the odd step folds
@@ -273,15 +282,15 @@ __device__ __forceinline__ void compute(const Ctx &c, const Stage &s, int st, fl
     }
 }
 
-template <bool HASK, int GS, class Stage>
-__device__ __forceinline__ void step(Ctx &c, const Stage &cur, Stage &refill, int st, float (&acc)[2][2][16],
+template <bool HASK, int GS, int S>
+__device__ __forceinline__ void step(Ctx &c, int st, float (&acc)[2][2][16],
                                      int32_t (&tot)[2][2][16], v16f (&carry)[2][2]) {
     // the loads of steps st + 1 and st + 2 may still be in flight
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoadsPerStep) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    fetch(c, refill, st + 3);
-    compute<HASK, GS>(c, cur, st, acc, tot, carry);
+    fetch<(S + 3) % kRing>(c, st + 3);
+    compute<HASK, GS, S>(c, st, acc, tot, carry);
 }
 
 __device__ __forceinline__ void flush(float (&acc)[2][2][16], int32_t (&tot)[2][2][16]) {
@@ -298,158 +307,194 @@ __device__ __forceinline__ void flush(float (&acc)[2][2][16], int32_t (&tot)[2][
     }
 }
 
-template <bool HASK, int GS, class Stage>
-__device__ __forceinline__ void body(Ctx &c, Stage &s0, Stage &s1, Stage &s2, Stage &s3,
-                                     float (&acc)[2][2][16], int32_t (&tot)[2][2][16]) {
+template <bool HASK, int GS>
+__device__ __forceinline__ void body(Ctx &c, int32_t (&tot)[2][2][16]) {
     v16f carry[2][2] = {};
-    fetch(c, s0, 0);
-    fetch(c, s1, 1);
-    fetch(c, s2, 2);
+    float acc[2][2][16];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[a][b][r] = kBias;
+                tot[a][b][r] = 0;
+            }
+        }
+    }
+    fetch<0>(c, 0);
+    fetch<1>(c, 1);
+    fetch<2>(c, 2);
     for (int st = 0; st < c.n_steps; st += kRing) {
         // (K is a multiple of 256: the number of steps is even, so steps come in pairs)
-        step<HASK, GS>(c, s0, s3, st, acc, tot, carry);
-        step<HASK, GS>(c, s1, s0, st + 1, acc, tot, carry);
+        step<HASK, GS, 0>(c, st, acc, tot, carry);
+        step<HASK, GS, 1>(c, st + 1, acc, tot, carry);
         if (st + 2 < c.n_steps) {
-            step<HASK, GS>(c, s2, s1, st + 2, acc, tot, carry);
-            step<HASK, GS>(c, s3, s2, st + 3, acc, tot, carry);
+            step<HASK, GS, 2>(c, st + 2, acc, tot, carry);
+            step<HASK, GS, 3>(c, st + 3, acc, tot, carry);
         }
         if (!HASK && ((st / kRing + 1) % (kFlushSteps / kRing)) == 0) flush(acc, tot);
     }
+    flush(acc, tot);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the refetches of the last steps
 }
 
 // ---- groups of 64 (the common case): the same steps with the LDS reads taken out of the critical path.
-// The operands of a group are read from LDS while the previous group is being computed: the reads of a step's second
-// group are issued in front of the first group's MFMAs, and the wait for the next stage (vmcnt + barrier) sits between
-// the two groups, so that the next step's first group can be read behind the second group's MFMAs. (With all reads at
-// the top of a step every wavefront waited for 12 KiB from LDS at the same moment, right behind the barrier: a
-// quarter of the step.)
+// The operands of a group are read from LDS while the group before is being computed, a piece behind each of its MFMAs
+// (fragment pairs in the order in which the next group's MFMAs take them), and the wait for the next stage (vmcnt + barrier)
+// sits between the two groups of a step, so that the next step's first group can be read behind the second group's MFMAs.
 struct Operands {
     v8i A[2], B[2];
     float m4[2];
 };
 
-template <class Stage>
-__device__ __forceinline__ void read_operands(const Ctx &c, const Stage &s, int gi, Operands &o) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        o.A[i] = fragment(s, kOffA + gi * kCellsA + (2 * c.wr + i) * (kFrag6 / 16), c.lane);
-        o.B[i] = fragment(s, kOffB + gi * kCellsB + (2 * c.wc + i) * (kFrag6 / 16), c.lane);
-        o.m4[i] = reinterpret_cast<const float *>(&s.cell[kOffM + gi * kCellsM])[64 * c.wc + 32 * i + (c.lane & 31)];
+__device__ __forceinline__ void read_piece(const Ctx &c, int stage, int gi, int piece, Operands &o) {
+    if (piece == 0) {
+        o.A[0] = read_a(c, stage, gi, 0);
+        o.B[0] = read_b(c, stage, gi, 0);
+    } else if (piece == 1) {
+        o.B[1] = read_b(c, stage, gi, 1);
+    } else if (piece == 2) {
+        o.A[1] = read_a(c, stage, gi, 1);
+        o.m4[0] = read_m(c, stage, gi, 0);
+        o.m4[1] = read_m(c, stage, gi, 1);
     }
 }
 
+// What a wavefront carries from group to group: the accumulators (without weight multipliers the biased floats above, with them
+// the sums of bit patterns), the tile whose fold is still due, always (1, 1), its tokens' multipliers, and its rows'.
+template <bool HASK>
+struct State {
+    float acc[2][2][16];
+    v16f P;
+    float pm;
+    float kf[HASK ? 16 : 1];
+    uint32_t kw[HASK ? 2 : 1][2][4];   // bytes of both groups of a step: [group][row block]
+    float bias;
+};
+
 // the four tiles of one group; the fold of a tile runs behind the MFMA of the next one, the last tile's result is
-// handed to the next group (P, pm, and the tile it belongs to is always (1, 1))
-// (with weight multipliers: `sk`, `gi` = the stage and the group in it that `o` was read from, `sp`, `gp` = those of
-// the group before it, whose last tile is folded behind this group's first MFMA; the multipliers of a fold's rows are
-// read from LDS in front of the MFMA that the fold stands behind)
-// KFMA: the one-FMA fold with multipliers from LDS; otherwise (a kernel that is launched when nothing says the tensor
-// has weight multipliers, and must still be right when it has) the integer fold with multipliers from global memory.
-template <bool HASK, bool KFMA, class Stage, class Between>
-__device__ __forceinline__ void group_units(const Ctx &c, const Operands &o, int g, const Stage &sp, int gp, const Stage &sk, int gi,
-                                            v16f &P, float &pm, float (&acc)[2][2][16], int32_t (&tot)[2][2][16], Between between) {
+// handed to the next group. With weight multipliers the two tiles of a row block share its multipliers, converted once.
+template <bool HASK, class Between>
+__device__ __forceinline__ void group_units(const Operands &o, int gi, State<HASK> &s, Between between) {
     const v16f zero = {};
 #pragma unroll
     for (int un = 0; un < 4; ++un) {
         const int a = un >> 1, b = un & 1;
         const int pa = un == 0 ? 1 : (un - 1) >> 1, pb = un == 0 ? 1 : (un - 1) & 1;
-        uint32_t kw[4];
-        if (HASK && KFMA) read_kw(c, un == 0 ? sp : sk, un == 0 ? gp : gi, pa, kw);
-        // The wavefront asks for issue priority while it hands over its MFMA. The two statements also pin the order
-        // MFMA, load, fold: without them the compiler moves the load (an assembly statement) in front of the MFMA,
-        // which then waits behind the load's issue (M=2048: 185.5 -> 180 us; with the priority left at 0 in both
-        // statements, 181 us).
-        __builtin_amdgcn_s_setprio(1);
+        // (The two statements around the MFMA pin the order MFMA, load, fold: without them the compiler moves the load in front of
+        // the MFMA, which then waits behind the load's issue. A raised issue priority for the MFMA costs 1.5 %.)
+        __builtin_amdgcn_sched_barrier(0);
         const v16f S = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(o.A[a], o.B[b], zero, 2, 2, 0, 0, 0, 0);
-        __builtin_amdgcn_s_setprio(0);
-        between(un);   // (a piece of the next stages' fetch: behind the MFMA, in front of the previous tile's fold)
-        if (!HASK) {
-            fold_fast(P, pm, acc[pa][pb]);
-        } else if (KFMA) {
-            fold_km(P, pm, kw, acc[pa][pb]);   // (a workgroup's first fold adds nothing: P and pm start as zero)
-        } else {
-            const int pg = un == 0 ? g - 1 : g;
-            int k16[16];
+        __builtin_amdgcn_sched_barrier(0);
+        between(un);   // (pieces of the next operands' reads and of the next stages' fetch: behind the MFMA, in front of the fold)
+        if constexpr (HASK) {
+            if (b == 1) {   // (the fold below is the first one of row block a)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t k4 = *reinterpret_cast<const uint32_t *>(c.k_src + (size_t) (pg < 0 ? 0 : pg) * kPanelRows + 32 * pa + 8 * q);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) k16[4 * q + i] = (k4 >> (8 * i)) & 0xFF;
+                for (int r = 0; r < 16; ++r) s.kf[r] = (float) ((s.kw[gi][a][r >> 2] >> (8 * (r & 3))) & 0xFFu);
             }
-            fold_k(P, pm, k16, tot[pa][pb]);
+            fold_km(s.P, s.pm, s.kf, s.bias, s.acc[pa][pb]);   // (a workgroup's first fold adds nothing but the bias)
+        } else {
+            fold_fast(s.P, s.pm, s.acc[pa][pb]);
         }
-        P = S;
-        pm = o.m4[b];
+        s.P = S;
+        s.pm = o.m4[b];
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                // MFMA
         if (!HASK) __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);    // VALU: the fold
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-template <bool HASK, bool KFMA, class Stage>
-__device__ __forceinline__ void body64(Ctx &c, Stage &s0, Stage &s1, Stage &s2, Stage &s3, float (&acc)[2][2][16],
-                                       int32_t (&tot)[2][2][16]) {
-    Stage *ring[kRing] = { &s0, &s1, &s2, &s3 };
-    Operands X, Y;
-    v16f P = {};
-    float pm = 0.0f;
-    // stages 0 and 1 whole, of stage 2 the first three runs: its other two loads and everything after them is dealt
-    // out between the MFMAs of the loop (three runs of step st + 3 behind the barrier of step st, the fourth run and the
-    // fifth load in the first half of step st + 1)
-    fetch(c, s0, 0);
-    fetch(c, s1, 1);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) fetch_run(c, s2, 2, i);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoadsPerStep - 2) : "memory");
+// step st, whose stage is S
+template <bool HASK, int S>
+__device__ __forceinline__ void step64(Ctx &c, int st, Operands &X, Operands &Y, State<HASK> &state) {
+    constexpr int kNext = (S + 1) % kRing, kPrev = (S + 3) % kRing;
+    group_units<HASK>(X, 0, state, [&](int un) {
+        read_piece(c, S, 1, un, Y);
+        // (both groups' multipliers in this half: behind the barrier their stage belongs to a later step)
+        if constexpr (HASK) read_kw(c, S, un & 1, un >> 1, state.kw[un & 1][un >> 1]);
+        if (un == 0) fetch_piece<kPrev, 3>(c, st + 3);
+        if (un == 2) fetch_piece<kPrev, 4>(c, st + 3);
+    });
+    // Stage st + 1 is whole once every wavefront has seen its own loads of it arrive (those of steps st + 2 and st + 3
+    // may still be in flight). This step's stage has been read by then, a wavefront's last reads of it included, and is free
+    // for step st + 4: a load is three steps ahead of its use.
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * kLoadsPerStep) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    read_operands(c, s0, 0, X);
-    for (int st0 = 0; st0 < c.n_steps; st0 += kRing) {
+    group_units<HASK>(Y, 1, state, [&](int un) {
+        read_piece(c, kNext, 0, un, X);   // (past the last step: stale cells, never used)
+        if (un == 0) fetch_piece<S, 0>(c, st + 4);
+        if (un == 1) fetch_piece<S, 1>(c, st + 4);
+        if (un == 2) fetch_piece<S, 2>(c, st + 4);
+    });
+}
+
+template <bool HASK>
+__device__ __forceinline__ void body64(Ctx &c, int32_t (&tot)[2][2][16]) {
+    Operands X, Y;
+    State<HASK> s;
+    s.P = v16f{};
+    s.pm = 0.0f;
+    s.bias = kBias;
+    asm volatile("" : "+s"(s.bias));
 #pragma unroll
-        for (int j = 0; j < kRing; ++j) {
-            const int st = st0 + j;
-            if (j > 0 && st >= c.n_steps) break;   // (wave-uniform)
-            const Stage &cur = *ring[j];
-            const Stage &next = *ring[(j + 1) % kRing];
-            Stage &refill2 = *ring[(j + 2) % kRing];
-            Stage &refill3 = *ring[(j + 3) % kRing];
-            read_operands(c, cur, 1, Y);
-            __builtin_amdgcn_sched_barrier(0);
-            group_units<HASK, KFMA>(c, X, c.g0 + 2 * st, *ring[(j + 3) % kRing], 1, cur, 0, P, pm, acc, tot, [&](int un) {
-                if (un == 0) fetch_run(c, refill2, st + 2, 3);
-                if (un == 2) fetch_tail(c, refill2, st + 2);
-            });
-            // stage st + 1 is whole once every wavefront has seen its own loads of it arrive (those of step st + 2
-            // may still be in flight); stage st - 1 is then free for step st + 3
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoadsPerStep) : "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            read_operands(c, next, 0, X);   // (past the last step: stale cells, never used)
-            __builtin_amdgcn_sched_barrier(0);
-            group_units<HASK, KFMA>(c, Y, c.g0 + 2 * st + 1, cur, 0, cur, 1, P, pm, acc, tot, [&](int un) {
-                if (un < 3) fetch_run(c, refill3, st + 3, un);
-            });
-            if (HASK && KFMA) flush(acc, tot);   // (every accumulator has taken two groups' terms since the last one)
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s.acc[a][b][r] = HASK ? 0.0f : kBias;
+                tot[a][b][r] = 0;
+            }
         }
-        if (!HASK && ((st0 / kRing + 1) % (kFlushSteps / kRing)) == 0) flush(acc, tot);
+    }
+    if constexpr (HASK) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s.kf[r] = 0.0f;
+    }
+    // stages 0 to 2 whole, of stage 3 the weights: its other two loads and everything after them is dealt
+    // out between the MFMAs of the loop (three runs of step st + 4 behind the barrier of step st, the fourth and the
+    // fifth in the first half of step st + 1)
+    fetch<0>(c, 0);
+    fetch<1>(c, 1);
+    fetch<2>(c, 2);
+    fetch_piece<3, 0>(c, 3);
+    fetch_piece<3, 1>(c, 3);
+    fetch_piece<3, 2>(c, 3);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kLoadsPerStep - 2) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) read_piece(c, 0, 0, i, X);
+    for (int st = 0; st < c.n_steps; st += kRing) {
+        step64<HASK, 0>(c, st, X, Y, s);
+        if (st + 1 >= c.n_steps) break;   // (wave-uniform)
+        step64<HASK, 1>(c, st + 1, X, Y, s);
+        if (st + 2 >= c.n_steps) break;
+        step64<HASK, 2>(c, st + 2, X, Y, s);
+        if (st + 3 >= c.n_steps) break;
+        step64<HASK, 3>(c, st + 3, X, Y, s);
+        if (!HASK && ((st / kRing + 1) % (kFlushSteps / kRing)) == 0) flush(s.acc, tot);
     }
     // the last tile of the last group
-    if (!HASK) {
-        fold_fast(P, pm, acc[1][1]);
-    } else if (KFMA) {
-        uint32_t kw[4];
-        read_kw(c, *ring[(c.n_steps - 1) % kRing], 1, 1, kw);
-        fold_km(P, pm, kw, acc[1][1]);
-    } else {
-        int k16[16];
+    if constexpr (HASK) {
+        fold_km(s.P, s.pm, s.kf, s.bias, s.acc[1][1]);
+        // a bias for every group (and, in tile (1, 1), one of the first fold)
+        const uint32_t off = 2 * (uint32_t) c.n_steps * (uint32_t) kBiasBits;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t k4 = *reinterpret_cast<const uint32_t *>(c.k_src + (size_t) (c.g0 + 2 * c.n_steps - 1) * kPanelRows + 32 + 8 * q);
+        for (int a = 0; a < 2; ++a) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) k16[4 * q + i] = (k4 >> (8 * i)) & 0xFF;
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    tot[a][b][r] = (int32_t) (__builtin_bit_cast(uint32_t, s.acc[a][b][r]) - off - (a & b ? (uint32_t) kBiasBits : 0u));
+                }
+            }
         }
-        fold_k(P, pm, k16, tot[1][1]);
+    } else {
+        fold_fast(s.P, s.pm, s.acc[1][1]);
+        flush(s.acc, tot);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the refetches of the last steps
 }
@@ -472,18 +517,15 @@ struct TileSet {
     int            first[kN];   // unused slots hold the total, so no tile selects them
 };
 
-// KFMA (activation groups of 64 only): the form of the kernel for tensors with weight multipliers; see group_units
-// SET: a launch over several weights (a form of its own: the loop has no register to spare for the selection, and a single
-// weight's launch would pay 1 % for it)
-template <int GS, bool KFMA, bool SET>
+// SET: a launch over several weights (a form of its own: a single weight's launch would pay 1 % for the selection)
+template <int GS, bool SET>
 __global__ void __launch_bounds__(kThreads)
 rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
                 const float *__restrict__ u, int M, int Mp, int ng, int n_tok_tiles, int n_tiles, int super_tiles,
                 int n_whole, int parts, int *__restrict__ counters, unsigned long long *__restrict__ slabs) {
-    using Stage = StageT<KFMA, SET>;
-    __shared__ Stage ring[kRing];
-    Stage &s0 = ring[0], &s1 = ring[1], &s2 = ring[2], &s3 = ring[3];
-    static_assert(8 * 32 * kXposeStride * 4 <= sizeof(Stage), "the epilogue's output blocks fit one stage");
+    __shared__ __align__(16) uint8_t ring[kRingBytes];
+    constexpr int kXpose = kRingBytes - 8 * 32 * kXposeStride * 4;   // the epilogue's output blocks
+    static_assert(kXpose >= kOffA, "fit the weights' stages");
     // the epilogue's operands, fetched ahead of the first groups: the scales of the tile's 256 rows, then the units of
     // its 128 tokens
     __shared__ __align__(16) float s_pre[kTileRows + kTileTok + 4];   // (+ a word for the arrival count of a slice)
@@ -547,38 +589,42 @@ rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const f
     const uint8_t *w_tile = w6 + (size_t) row_tile * ng * (kCellsA * 16);   // this tile's rows, group 0
     const size_t a_step = (size_t) (Mp / 32) * kFrag6;                       // bytes between groups of the activation plane
     const uint8_t *a_tile = act6 + (size_t) (t0 / 32) * kFrag6;              // this tile's tokens, group 0
+    // (the weights of a step's two groups are 24 runs of 1 KiB one behind the other, the activations' 6 and 6: a wavefront takes
+    // runs w, w + 8, w + 16 of the one and run w of the other)
+    c.a_src = uniform(w_tile + (size_t) s_begin * kStageA + c.wave * 1024);
+    c.b_step = (uint32_t) (2 * a_step);
+    c.b_src = uniform(a_tile + (size_t) (c.wave / 6) * a_step + (size_t) (c.wave % 6) * 1024 + (size_t) s_begin * c.b_step);
+    if (c.wave < 4) {          // the last 4 KB of the second group's activations
+        c.t_step = c.b_step;
+        c.t_off = (uint32_t) c.lane * 16;
+        c.t_src = a_tile + a_step + (size_t) (2 + c.wave) * 1024 + (size_t) s_begin * c.t_step;
+    } else if (!(c.wave & 1)) { // the tokens' multipliers of the two groups, half a wavefront each
+        c.t_step = (uint32_t) (2 * Mp * sizeof(float));
+        c.t_off = (uint32_t) (c.lane >> 5) * (uint32_t) (Mp * sizeof(float)) + (uint32_t) (c.lane & 31) * 16;
+        c.t_src = reinterpret_cast<const uint8_t *>(m4 + t0) + (size_t) s_begin * c.t_step;
+    } else {                    // the weight multipliers of the tile's 256 rows (a byte per row: 64 bytes per panel of 64 rows), a
+                                // quarter of a wavefront a group; the other half fetches them once more, into cells nobody reads
+        const int x = c.lane & 15, pnl = min(row_tile * 4 + (x >> 2), n_panels - 1) - row_tile * 4;
+        c.t_step = 2 * kPanelRows;
+        c.t_off = (uint32_t) ((pnl * ng + ((c.lane >> 4) & 1)) * kPanelRows + (x & 3) * 16);
+        c.t_src = kmul + (size_t) row_tile * 4 * ng * kPanelRows + (size_t) s_begin * c.t_step;
+    }
+    c.t_src = uniform(c.t_src);
+    const uint32_t lds0 = (uint32_t) (uintptr_t) (lds_void *) ring;
+    c.lds_run = lds0 + c.wave * 1024;
+    c.lds_t = lds0 + (c.wave < 4 ? 8192 + c.wave * 1024 : c.wave & 1 ? kOffK : kOffM);
+    c.b16 = lds0 + 2 * c.wc * kFrag6 + 16 * c.lane;
+    c.b8 = lds0 + 2 * c.wc * kFrag6 + 1024 + 8 * c.lane;
+    c.m = lds0 + kOffM + 256 * c.wc + 4 * (c.lane & 31);
+    c.k = lds0 + kOffK + 64 * c.wr + 4 * (c.lane >> 5);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // run L of the stage: runs 0 .. 23 are the weights of the step's two groups (12 each), 24 .. 35 the activations
-        // (6 each; the last four belong to the fifth load)
-        const int L = i * 8 + c.wave;
-        if (L < 24) {
-            c.run_step[i] = (size_t) 2 * kCellsA * 16;
-            c.run_src[i] = uniform(w_tile + (size_t) (L / 12) * (kCellsA * 16) + (size_t) (L % 12) * 1024 + s_begin * c.run_step[i]);
-        } else {
-            c.run_step[i] = 2 * a_step;
-            c.run_src[i] = uniform(a_tile + (size_t) ((L - 24) / 6) * a_step + (size_t) ((L - 24) % 6) * 1024 + s_begin * c.run_step[i]);
-        }
+    for (int i = 0; i < 2; ++i) {
+        c.a16[i] = lds0 + kOffA + 2 * i * kStageA + 2 * c.wr * kFrag6 + 16 * c.lane;
+        c.a8[i] = lds0 + kOffA + 2 * i * kStageA + 2 * c.wr * kFrag6 + 1024 + 8 * c.lane;
+        // (registers of their own: without these statements the compiler forms an address per stage)
+        asm volatile("" : "+v"(c.a16[i]), "+v"(c.a8[i]));
     }
-    {
-        // fifth load: cells 2048 .. 2303 are the last 256 cells of the second group's activations, cells 2304 .. 2367
-        // the tokens' multipliers of the two groups, cells 2368 .. 2399 the weight multipliers of the tile's 256 rows
-        // for the two groups (a byte per row: 64 bytes per panel of 64 rows)
-        const int cell = kTailCell + c.wave * Stage::kTailLanes + (c.lane < Stage::kTailLanes ? c.lane : 0);
-        if (cell < kOffM) {
-            c.tail_step = (uint32_t) (2 * a_step);
-            c.tail_src = a_tile + a_step + (size_t) (cell - (kOffB + kCellsB)) * 16 + (size_t) s_begin * c.tail_step;
-        } else if (cell < kOffK) {
-            const int gi = (cell - kOffM) / kCellsM, off = (cell - kOffM) % kCellsM;
-            c.tail_step = (uint32_t) (2 * Mp * sizeof(float));
-            c.tail_src = reinterpret_cast<const uint8_t *>(m4 + (size_t) gi * Mp + t0) + (size_t) off * 16 + (size_t) s_begin * c.tail_step;
-        } else {
-            const int gi = (cell - kOffK) / kCellsK, x = (cell - kOffK) % kCellsK;
-            const int pnl = min(row_tile * 4 + (x >> 2), n_panels - 1);
-            c.tail_step = 2 * kPanelRows;
-            c.tail_src = kmul + ((size_t) pnl * ng + gi) * kPanelRows + (size_t) (x & 3) * 16 + (size_t) s_begin * c.tail_step;
-        }
-    }
+    asm volatile("" : "+v"(c.b16), "+v"(c.b8), "+v"(c.m), "+v"(c.k));
     const int panel = min(row_tile * 4 + c.wr, n_panels - 1);
     c.k_src = kmul + (size_t) panel * ng * kPanelRows + 4 * (c.lane >> 5);
 
@@ -590,29 +636,16 @@ rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const f
         load_to_lds_dword(u + (t < M ? t : M - 1), &s_pre[kTileRows + 64 * (c.wave - 4)]);
     }
 
-    float acc[2][2][16];
     int32_t tot[2][2][16];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[a][b][r] = kBias;
-                tot[a][b][r] = 0;
-            }
-        }
-    }
     // fp32 rounding toward minus infinity for the folds (MODE bits 1:0); the MFMA sums are exact in any mode
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2" ::: "memory");
-    if (KFMA || hask) {   // (the form for weight multipliers takes every tensor that way: multipliers of 1 where there are none)
-        if constexpr (GS == 1) body64<true, KFMA>(c, s0, s1, s2, s3, acc, tot);
-        else body<true, GS>(c, s0, s1, s2, s3, acc, tot);
+    if (hask) {
+        if constexpr (GS == 1) body64<true>(c, tot);
+        else body<true, GS>(c, tot);
     } else {
-        if constexpr (GS == 1) body64<false, KFMA>(c, s0, s1, s2, s3, acc, tot);
-        else body<false, GS>(c, s0, s1, s2, s3, acc, tot);
+        if constexpr (GS == 1) body64<false>(c, tot);
+        else body<false, GS>(c, tot);
     }
-    flush(acc, tot);
     // Back to round to nearest even for the epilogue. The compiler does not know that fp32 arithmetic reads MODE, so
     // the totals pass through a statement on either side of the change: the one in front keeps the last folds (which
     // the totals depend on) from being scheduled behind it, the one behind keeps the conversions below from being
@@ -699,7 +732,7 @@ rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const f
     // wavefront turns its four 32 x 32 blocks through LDS one after the other (4.5 KiB per wavefront, all eight inside
     // the last ring stage, which no fetch is aimed at when the loop ends) and writes 128 contiguous bytes per token.
     __syncthreads();   // every wavefront is done reading the ring
-    float *xp = reinterpret_cast<float *>(&s3.cell[0]) + c.wave * (32 * kXposeStride);
+    float *xp = reinterpret_cast<float *>(ring + kXpose) + c.wave * (32 * kXposeStride);
     const int h = c.lane >> 5;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
@@ -910,25 +943,21 @@ hipError_t launch_gemm6(const Gemm6Args &a, hipStream_t stream) {
     if (pl.n_tiles == 0) return launch_block6(a, stream);
     const int grid = pl.n_whole + (pl.n_tiles - pl.n_whole) * pl.parts;
     const float *m4 = reinterpret_cast<const float *>(a.act6 + act6_plane_bytes(ng, a.Mp));
-#define RQ_LAUNCH6(GS, KFMA, SET, TS)                                                                                      \
-    hipLaunchKernelGGL((rq_gemm6_kernel<GS, KFMA, SET>), dim3(grid), dim3(kThreads), 0, stream, TS, a.act6, m4, a.u, a.M,  \
+#define RQ_LAUNCH6(GS, SET, TS)                                                                                            \
+    hipLaunchKernelGGL((rq_gemm6_kernel<GS, SET>), dim3(grid), dim3(kThreads), 0, stream, TS, a.act6, m4, a.u, a.M,  \
                        a.Mp, ng, n_tok_tiles, pl.n_tiles, super_tiles, pl.n_whole, pl.parts,                         \
                        reinterpret_cast<int *>(a.cells),                                                             \
                        reinterpret_cast<unsigned long long *>(reinterpret_cast<uint8_t *>(a.cells) + kGemm6CounterBytes))
-    // (a.weight_multipliers: what the host knows about the tensor; only a choice between two kernels that are both
-    // right for every tensor)
     // (The kernels lie in the code object in the order in which they stand here. Behind the 57 KB of the H68 rotation a
     // launch starts with a cold instruction cache, and how much of it the two share depends on the place: with the sets'
     // kernels first, K = 17408, N = 5120 takes 60.1 us at 256 tokens and 77.9 at 512, with the single weights' first 58.7
     // and 76.9; each kernel by itself takes the same time either way.)
     if (a.w.n == 1) {
-        if (a.groups_per_fold == 1 && a.weight_multipliers) RQ_LAUNCH6(1, true, false, t1);
-        else if (a.groups_per_fold == 1) RQ_LAUNCH6(1, false, false, t1);
-        else if (a.groups_per_fold == 2) RQ_LAUNCH6(2, false, false, t1);
-        else RQ_LAUNCH6(4, false, false, t1);
+        if (a.groups_per_fold == 1) RQ_LAUNCH6(1, false, t1);
+        else if (a.groups_per_fold == 2) RQ_LAUNCH6(2, false, t1);
+        else RQ_LAUNCH6(4, false, t1);
     } else {
-        if (a.weight_multipliers) RQ_LAUNCH6(1, true, true, ts);
-        else RQ_LAUNCH6(1, false, true, ts);
+        RQ_LAUNCH6(1, true, ts);
     }
 #undef RQ_LAUNCH6
     const hipError_t e = hipGetLastError();

@@ -76,7 +76,10 @@ def sample_of(M):
     (5120, 8300, 256, 0, 66, 3),       # two, in turn
     (2560, 9300, 330, 0, 111, 2),
     (32768, 256, 1536, 0, 12, 13),     # the longest row: 19 and 20 steps, the float totals at 3.9 M of the 4.19 M of their window
-    (1024, 8192, 1000, 256, 0, 1)],    # a round of whole tiles in super-tiles, nothing left over
+    (1024, 8192, 1000, 256, 0, 1),     # a round of whole tiles in super-tiles, nothing left over
+    (256, 4300, 700, 102, 0, 1),      # fewer steps (2) than stages of the ring
+    (512, 4300, 700, 102, 0, 1),      # as many
+    (768, 4300, 700, 102, 0, 1)],     # a step and a half of them
     ids=lambda v: str(v))
 def test_whole_tiles_and_slices(oracle, K, N, M, whole, cut, slices, multipliers):
     p = plan(rq.TYPE_W4A4, K, N, M, multipliers)
