@@ -1,11 +1,13 @@
 // Weight-side quantizer and the dequantizers of the four block types, on the GPU: what ggml calls from_float_ref and
 // to_float for W4A4 / W4A4H / A4 / A4H (reference patch lines 2507-2580, 2681-2710, 2738-2773).
 //
-// A converter quantizes whole tensors; the reference does it a row at a time on the host. Here the row (or the weight
-// group) is the unit of parallelism, and the results are bit-identical because the only order-sensitive quantity, the
-// double-precision error sum of the scale search, is accumulated by one lane in the reference's element order:
-//   * search kernel: sixteen lanes per segment (a row, a block of 256 or a group of 64); thirteen of them each try one
-//     clip ratio over the whole segment, sequentially, and a scan in ratio order keeps the first smallest error;
+// A converter quantizes whole tensors; the reference does it a row at a time on the host. The one quantity whose order of
+// operations matters is the double-precision error sum of the scale search, and of it only which of the thirteen clip ratios
+// has the smallest is kept. So the sums are taken in fp32 first, over all lanes and in any order, with a bound on what that
+// can change; where the smallest two are further apart than the bound allows, the reference's sums are too, and the search is
+// over. Where they are not (a row in a hundred), the same again in double precision, and only where that cannot tell either
+// (ties, infinities, NaNs, scales out of range) do lanes add up the reference's sums in its element order:
+//   * search kernels: a workgroup per row, or sixteen lanes per weight group of 256 or 64;
 //   * encode kernel: a workgroup per row turns the chosen scale(s) into codes, row sum / multiplier headers and
 //     blocks;
 //   * dequantize kernel: a workgroup per row decodes blocks into the padded LDS row and, for the rotated types, runs
@@ -44,15 +46,278 @@ struct SearchArgs {
     float *scale;      // [segments]
 };
 
-// ONE: segments of 64 (a scale per 64 inputs), one block each: nothing to fetch ahead and no eight loads to batch. (With the
-// general form's, which fetch the one block again: 4096 x 17408, search and encoding, 450 us against 402.)
-template <bool ONE>
-__global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const SearchArgs a) {
-    __shared__ float4 s_x[ONE ? 1 : 2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
+// What the fp32 sums may be off by, relative to the exact sum of the reference's squares. The quotient t = x * (1 / s) differs
+// from x / s by less than 8e-6 (|x / s| is at most 10), so a code differs from the reference's only where x / s is that near
+// to a half-way point; its error then is (0.5 +- 9e-6) s either way, and the square off by 7.2e-5 of itself. The errors
+// themselves and their squares are rounded as the reference's or once (6e-8), and a thread adds up at most 128 of them and 12
+// sums: 8.5e-6. Together below 8.2e-5; the reference's own rounding (32768 additions in double precision, 4e-12) is nothing to
+// that. Two sums can have their order changed only if they are within (1 + 8.2e-5) / (1 - 8.2e-5) of each other.
+constexpr float kApart = 1.0f + 1.7e-4f;
+// The double-precision sums of the second look have the reference's terms and at most 400 roundings, the reference's own sums at
+// most 32768: 3.7e-12 and 4.5e-14.
+constexpr double kApart64 = 1.0 + 1e-11;
+// (below this the squares may be denormal, which the bound does not cover)
+constexpr float kLeast = 1e-30f;
+
+__device__ __forceinline__ float ratio_scale(float amax, int r) { return amax * (1.0f - 0.025f * (float) r) / 7.0f; }
+// what stands in place of a scale that these sums leave open, for rq_wsearch_kernel
+constexpr float kOpen = -1.0f;
+__device__ __forceinline__ bool reciprocal_holds(float rs) { return rs < 1e37f && rs > 2e-38f; }
+
+// the sums of the squared errors of one element under all ratios (rs: reciprocals of the scales)
+__device__ __forceinline__ void add_errors(float x, const float (&sc)[kRatios], const float (&rs)[kRatios], float (&acc)[kRatios]) {
+#pragma unroll
+    for (int r = 0; r < kRatios; ++r) {
+        float q = rintf(x * rs[r]);
+        if (r > 2) q = __builtin_amdgcn_fmed3f(q, -8.0f, 7.0f);   // (|x / s| is at most 7 / 0.95 before that)
+        const float e = q * sc[r] - x;
+        acc[r] = __builtin_fmaf(e, e, acc[r]);
+    }
+}
+
+// v plus the value of lane `ctrl` of the same row of sixteen
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+// the sum over a row of sixteen lanes, in all of them
+__device__ __forceinline__ float row_sum(float v) {
+    v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+    v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    v = dpp_add<0x141>(v);   // row_half_mirror
+    return dpp_add<0x140>(v);   // row_mirror
+}
+
+// whether the smallest of the sums is the smallest in the reference's sums too (not with a NaN or an infinity among them)
+__device__ __forceinline__ bool settled(const float (&sum)[kRatios], float &least) {
+    float second = INFINITY, all = sum[0];
+    least = sum[0];
+#pragma unroll
+    for (int r = 1; r < kRatios; ++r) {
+        second = __builtin_amdgcn_fmed3f(least, second, sum[r]);
+        least = fminf(least, sum[r]);
+        all += sum[r];
+    }
+    return second > least * kApart && least > kLeast && all < INFINITY;
+}
+
+// Weight groups of 256 (V = 4) or 64 (V = 1): sixteen lanes per group, V blocks of 64 elements in their registers.
+// What bounds it: vector instructions, six per element and ratio. Search and encoding of 4096 x 17408, groups of 64, with a lane per
+// ratio and the sums in order from the start 402 us, this way 306 (search 250); groups of 256 299 and 217 (134).
+template <int V>
+__global__ void __launch_bounds__(kSearchThreads, 4) rq_wsearch_groups_kernel(const SearchArgs a) {
     const int tid = threadIdx.x, r = tid & 15;
     int64_t seg = (int64_t) blockIdx.x * (kSearchThreads / 16) + (tid >> 4);
     const bool live = seg < a.segments;
-    if (!live) seg = a.segments - 1;   // idle lanes follow a live segment so that the shuffles below stay uniform
+    if (!live) seg = a.segments - 1;   // idle lanes follow a live segment
+    const int64_t row = seg / a.per_row;
+    const float *x = a.x + row * a.ld + (seg - row * a.per_row) * (int64_t) a.n;
+    float4 v[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) v[k] = reinterpret_cast<const float4 *>(x)[16 * k + r];
+    float amax = 0.0f;
+#pragma unroll
+    for (int k = 0; k < V; ++k) amax = fmaxf(fmaxf(fmaxf(fmaxf(amax, fabsf(v[k].x)), fabsf(v[k].y)), fabsf(v[k].z)), fabsf(v[k].w));
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 16));
+
+    const bool tries = amax > 0.0f && r < kRatios;
+    const float s = tries ? ratio_scale(amax, r) : 1.0f;
+    // lane r's scale to all lanes of the group (row_newbcast)
+    const float inv = 1.0f / s;
+    float sc[kRatios], rs[kRatios], sum[kRatios];
+#define RQ_FROM_LANE(R)                                                                                                      \
+    sc[R] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x150 + R, 0xF, 0xF, false)); \
+    rs[R] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, inv), 0x150 + R, 0xF, 0xF, false));
+    RQ_FROM_LANE(0) RQ_FROM_LANE(1) RQ_FROM_LANE(2) RQ_FROM_LANE(3) RQ_FROM_LANE(4) RQ_FROM_LANE(5) RQ_FROM_LANE(6)
+    RQ_FROM_LANE(7) RQ_FROM_LANE(8) RQ_FROM_LANE(9) RQ_FROM_LANE(10) RQ_FROM_LANE(11) RQ_FROM_LANE(12)
+#undef RQ_FROM_LANE
+#pragma unroll
+    for (int i = 0; i < kRatios; ++i) sum[i] = 0.0f;
+    float4 w = v[0];
+#pragma unroll 1
+    for (int k = 0; k < V; ++k) {
+        // (read again: kept, the registers of the four blocks let the compiler mix their sums, and spill)
+        const float4 next = reinterpret_cast<const float4 *>(x)[16 * (k + 1 < V ? k + 1 : k) + r];
+        add_errors(w.x, sc, rs, sum);
+        add_errors(w.y, sc, rs, sum);
+        add_errors(w.z, sc, rs, sum);
+        add_errors(w.w, sc, rs, sum);
+        w = next;
+    }
+#pragma unroll
+    for (int i = 0; i < kRatios; ++i) sum[i] = row_sum(sum[i]);
+    float least;
+    // (the largest and the smallest reciprocal)
+    bool sure = settled(sum, least) && reciprocal_holds(rs[0]) && reciprocal_holds(rs[kRatios - 1]);
+    float scale = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kRatios; ++i) scale = sum[i] == least ? sc[i] : scale;
+    if (!(amax > 0.0f)) {   // (a group of zeros or of NaNs)
+        scale = 0.0f;
+        sure = true;
+    }
+    if (live && r == 0) a.scale[seg] = sure ? scale : kOpen;
+}
+
+// Few groups go to the search in order at once: its one launch is as long as the two that spare it. Search and encoding, 1024
+// inputs, in order / this way, groups of 64: 1024 rows 12.1 / 13.8 us, 2048 17.5 / 18.2, of 256: 1024 13.7 / 17.2, 2048 16.6 / 19.7,
+// 4096 28.4 / 26.9.
+constexpr int64_t kFewFloats = 3 << 20;
+
+// Rows: a workgroup each, which reads its row twice (the second time out of the caches).
+// What bounds it: vector instructions, six per element and ratio (four of them of two cycles, beside a second wavefront).
+// Search and encoding, 5120 inputs, with four rows per wavefront, a lane per ratio and the sums in order from the start: 2048 rows
+// 137 us, 4096 173, 6144 187; this way 39, 63, 85 (search of 4096: 45). 17408 inputs, 1800 rows 441 and 97.
+constexpr int kRowThreads = 256;
+__global__ void __launch_bounds__(kRowThreads) rq_wsearch_rows_kernel(const SearchArgs a) {
+    __shared__ float s_sum[kRowThreads / 16][kRatios];   // per row of sixteen lanes
+    __shared__ float s_sc[kRatios], s_rs[kRatios], s_all[kRatios];
+    __shared__ float s_max[kRowThreads / 64];
+    __shared__ double s_err[kRowThreads / 64];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const float *x = a.x + (int64_t) blockIdx.x * a.ld;
+    const float4 *xv = reinterpret_cast<const float4 *>(x);
+    const int nv = a.n >> 2;   // (a multiple of 64: whole wavefronts have an element or none)
+    float amax = 0.0f;
+    constexpr int kBatch = 5;
+    for (int i0 = tid; i0 < nv; i0 += kBatch * kRowThreads) {
+        float4 v[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int i = i0 + k * kRowThreads;
+            v[k] = xv[i < nv ? i : i0];
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) amax = fmaxf(fmaxf(fmaxf(fmaxf(amax, fabsf(v[k].x)), fabsf(v[k].y)), fabsf(v[k].z)), fabsf(v[k].w));
+    }
+    amax = wave_max(amax);
+    if ((tid & 63) == 0) s_max[wave] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+    if (!(amax > 0.0f)) {   // (a row of zeros or of NaNs)
+        if (tid == 0) a.scale[blockIdx.x] = 0.0f;
+        return;
+    }
+    if (tid < kRatios) {
+        const float s = ratio_scale(amax, tid);
+        s_sc[tid] = s;
+        s_rs[tid] = 1.0f / s;
+    }
+    __syncthreads();
+    // (the same in all threads: scalar registers)
+    float sc[kRatios], rs[kRatios], sum[kRatios];
+#pragma unroll
+    for (int r = 0; r < kRatios; ++r) {
+        sc[r] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s_sc[r])));
+        rs[r] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s_rs[r])));
+        sum[r] = 0.0f;
+    }
+    float4 v = xv[tid < nv ? tid : 0];
+    for (int i = tid; i < nv; i += kRowThreads) {
+        const float4 next = xv[i + kRowThreads < nv ? i + kRowThreads : i];
+        add_errors(v.x, sc, rs, sum);
+        add_errors(v.y, sc, rs, sum);
+        add_errors(v.z, sc, rs, sum);
+        add_errors(v.w, sc, rs, sum);
+        v = next;
+    }
+#pragma unroll
+    for (int r = 0; r < kRatios; ++r) {
+        const float t = row_sum(sum[r]);
+        if ((tid & 15) == 0) s_sum[tid >> 4][r] = t;
+    }
+    __syncthreads();
+    if (tid < kRatios) {
+        float t = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kRowThreads / 16; ++k) t += s_sum[k][tid];
+        s_all[tid] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRatios; ++r) sum[r] = s_all[r];
+    float least;
+    const bool normal = reciprocal_holds(rs[0]) && reciprocal_holds(rs[kRatios - 1]);
+    if (settled(sum, least) && normal) {
+        float scale = 0.0f;
+#pragma unroll
+        for (int r = 0; r < kRatios; ++r) scale = sum[r] == least ? sc[r] : scale;
+        if (tid == 0) a.scale[blockIdx.x] = scale;
+        return;
+    }
+
+    // The second look, at the ratios that the first could not tell from the smallest: the reference's terms, added up in
+    // double precision by all threads.
+    bool finite = normal;
+#pragma unroll
+    for (int r = 0; r < kRatios; ++r) finite = finite && sum[r] < INFINITY;
+    if (finite && least > kLeast) {
+        double err64[2] = { INFINITY, INFINITY };   // the smallest and the second smallest
+        int arg = 0;
+        for (int r = 0; r < kRatios; ++r) {
+            if (s_all[r] > least * kApart) continue;   // (uniform)
+            const float s = s_sc[r], inv = s_rs[r];
+            double err = 0.0;
+            for (int i = tid; i < nv; i += kRowThreads) {
+                const float4 w = xv[i];
+                const float xs[4] = { w.x, w.y, w.z, w.w };
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float t = xs[j] * inv;
+                    float q = rintf(t);
+                    if (!(fabsf(t - q) < 0.49999f)) q = rintf(xs[j] / s);
+                    const double e = (double) (fminf(fmaxf(q, -8.0f), 7.0f) * s - xs[j]);
+                    err = __builtin_fma(e, e, err);
+                }
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) err += __shfl_xor(err, off, 64);
+            __syncthreads();
+            if ((tid & 63) == 0) s_err[wave] = err;
+            __syncthreads();
+            err = (s_err[0] + s_err[1]) + (s_err[2] + s_err[3]);
+            if (err < err64[0]) {
+                err64[1] = err64[0];
+                err64[0] = err;
+                arg = r;
+            } else if (err < err64[1]) {
+                err64[1] = err;
+            }
+        }
+        if (err64[1] > err64[0] * kApart64) {
+            if (tid == 0) a.scale[blockIdx.x] = s_sc[arg];
+            return;
+        }
+    }
+    if (tid == 0) a.scale[blockIdx.x] = kOpen;
+}
+
+// The reference's search, for the segments that the kernels above left open: sixteen lanes per segment, thirteen of them try one
+// ratio each over the whole segment in element order, and a scan in ratio order keeps the first smallest error. A wavefront looks
+// through CHUNK segments and takes the open ones four at a time.
+// ONE: segments of 64 (a scale per 64 inputs), one block each: nothing to fetch ahead and no eight loads to batch. (With the
+// general form's, which fetch the one block again: 4096 x 17408, search and encoding, 450 us against 402.)
+// (ALL: every segment, whatever stands in place of its scale)
+template <bool ONE, int CHUNK, bool ALL = false>
+__global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const SearchArgs a) {
+    __shared__ float4 s_x[ONE ? 1 : 2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
+    const int tid = threadIdx.x, r = tid & 15;
+    const int64_t seg0 = (int64_t) blockIdx.x * CHUNK;
+    const bool mine = tid < CHUNK && seg0 + tid < a.segments;
+    uint64_t open = __ballot(mine && (ALL || a.scale[seg0 + (mine ? tid : 0)] < 0.0f));
+  while (open != 0) {
+    // the first four; a row of lanes without one follows the first
+    int64_t seg = seg0 + __builtin_ctzll(open);
+    bool live = false;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (open != 0 && k == tid >> 4) {
+            seg = seg0 + __builtin_ctzll(open);
+            live = true;
+        }
+        open &= open - 1;   // (zero stays zero)
+    }
     const int64_t row = seg / a.per_row;
     const float *x = a.x + row * a.ld + (seg - row * a.per_row) * (int64_t) a.n;
     const int n = a.n;
@@ -78,7 +343,7 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
 
     // (the lanes that try no ratio go through the loop too: they fetch for the others)
     const bool tries = amax > 0.0f && r < kRatios;
-    const float s = tries ? amax * (1.0f - 0.025f * (float) r) / 7.0f : 1.0f;
+    const float s = tries ? ratio_scale(amax, r) : 1.0f;
     double err = 0.0;
     if (__any(tries)) {
         const float rs = 1.0f / s;
@@ -90,16 +355,10 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
         // at most 10: two roundings of half a unit in the last place, 1 / s included), so rint agrees unless t is
         // within 1e-5 of a half-way point; those elements (one in 50,000), infinities, NaNs and scales whose
         // reciprocal is not a normal number take the division.
-        // 6144 x 5120: 577 us with a division per element and four elements at a time, 332 us with this in runs of eight,
-        // 236 us with four runs in flight. 4096 rows, a wavefront per SIMD: 222 us with the error in double precision from the
-        // start (two conversions, a subtraction, a product and a sum, of which a conversion takes four times as long as a
-        // sum), 178 us with one conversion and one FMA.
         // A block goes through LDS, where every lane reads its segment's elements, and is requested three blocks before it is
-        // worked on. Search and encoding, 5120 inputs, with this and the batched first pass, before and after: 2048 rows 169 /
-        // 137 us, 4096 229 / 173 (a wavefront per SIMD), 6144 241 / 187. (Every lane read its segment for itself, four
-        // runs ahead: four times the load instructions.)
+        // worked on.
         constexpr int kRun = 8;
-        const bool normal = rs < 1e37f && rs > 2e-38f;
+        const bool normal = reciprocal_holds(rs);
         float4 ahead[2];
         if constexpr (!ONE) {
             ahead[0] = block(1);
@@ -166,6 +425,7 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
         }
     }
     if (live && r == 0) a.scale[seg] = best_s;
+  }
 }
 
 struct EncodeArgs {
@@ -464,10 +724,21 @@ int rq_w4a4_quantize_weights(int type, const float *w_dev, int64_t ldw, int64_t 
     s.segments = N * per_row;
     s.n = (int) (K / per_row);
     s.scale = reinterpret_cast<float *>(base + ws.off_scale);
-    const int64_t per_wg = kSearchThreads / 16;
-    const dim3 grid((unsigned) ((s.segments + per_wg - 1) / per_wg));
-    if (s.n == 64) hipLaunchKernelGGL((rq_wsearch_kernel<true>), grid, dim3(kSearchThreads), 0, st, s);
-    else hipLaunchKernelGGL((rq_wsearch_kernel<false>), grid, dim3(kSearchThreads), 0, st, s);
+    auto blocks_of = [&](int64_t per) { return dim3((unsigned) ((s.segments + per - 1) / per)); };
+    // (the kernels that decide nearly all of them, then the one for what they leave open)
+    if (s.n <= 256 && N * K <= kFewFloats) {
+        if (s.n == 64) hipLaunchKernelGGL((rq_wsearch_kernel<true, 4, true>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
+        else hipLaunchKernelGGL((rq_wsearch_kernel<false, 4, true>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
+    } else if (s.n == 64) {
+        hipLaunchKernelGGL((rq_wsearch_groups_kernel<1>), blocks_of(kSearchThreads / 16), dim3(kSearchThreads), 0, st, s);
+        hipLaunchKernelGGL((rq_wsearch_kernel<true, 64>), blocks_of(64), dim3(kSearchThreads), 0, st, s);
+    } else if (s.n == 256) {
+        hipLaunchKernelGGL((rq_wsearch_groups_kernel<4>), blocks_of(kSearchThreads / 16), dim3(kSearchThreads), 0, st, s);
+        hipLaunchKernelGGL((rq_wsearch_kernel<false, 64>), blocks_of(64), dim3(kSearchThreads), 0, st, s);
+    } else {
+        hipLaunchKernelGGL(rq_wsearch_rows_kernel, dim3((unsigned) N), dim3(kRowThreads), 0, st, s);
+        hipLaunchKernelGGL((rq_wsearch_kernel<false, 4>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int) e;
 

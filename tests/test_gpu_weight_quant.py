@@ -298,3 +298,24 @@ def test_conversions_keep_their_second_stream():
         t.join()
     assert len(ok) == 20 and all(ok)
     assert [len(s) for s in seen] == [1, 1] and seen[0][0] is not seen[1][0]
+
+
+@pytest.mark.parametrize("wgroup", [0, 256, 64])
+def test_scales_that_the_first_look_leaves_open(oracle, wgroup):
+    """Enough segments that some (one in a hundred or fewer) have two ratios whose errors are too near for the fp32 sums, and rows
+    that those sums do not cover: sums of zero, denormal ones, infinite ones, infinities, NaNs, scales out of range; the last
+    wavefront is not full. Every byte as from the reference's sums in its order."""
+    N, K = 3202, 1024
+    w = tensor(N, K, 11 + wgroup)
+    rng = np.random.default_rng(wgroup)
+    for r, scale in enumerate([1e-38, 1e-30, 1e-20, 1e18, 1e37]):
+        w[10 * r + 1] = (rng.standard_normal(K) * scale).astype(f32)
+    w[60], w[61], w[62] = 0.0, 0.0, 0.0
+    w[60, ::64] = 0.3                     # one element of every group
+    w[61, ::64] = np.float32(1e-44)
+    w[62, 5] = -2.0
+    w[70, 3], w[71, ::64], w[72, :] = np.inf, np.nan, np.nan
+    w[N - 1] = np.where(np.arange(K) % 2 == 0, 0.7, -0.7)
+    got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4, wgroup=wgroup)
+    want = oracle.quantize_rows_w(w, wgroup=wgroup)
+    assert blocks_equal(got, want), block_diff(got, want)
