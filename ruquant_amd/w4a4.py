@@ -283,19 +283,15 @@ def _pinned(nbytes):
     return torch.empty(nbytes, dtype=torch.uint8, device="cpu", pin_memory=True)
 
 
-def _stages(nbytes):
-    return [_pinned(nbytes) for _ in range(_STAGES)]
-
-
 # A stream's first work costs 0.2 ms, and 2.9 ms while it gets a hardware queue of its own (a few per process), so a
 # conversion in several runs does not take another of torch's streams each time but keeps the one that its thread used
-# beside the same current stream. (Not one for all: copies wait for the work in front of them on the current stream,
+# beside the same current stream. (Not one for all: its runs wait for the work in front of them on the current stream,
 # and would make another stream's conversion wait for it too.)
 _copiers = threading.local()
 _COPIERS = 8   # per thread, the latest ones
 
 
-def _copier(current):
+def _second_stream(current):
     kept = _copiers.__dict__.setdefault("streams", {})
     key = (current.device_index, current.cuda_stream)
     stream = kept.pop(key, None)
@@ -321,40 +317,6 @@ def _copy_bytes(pinned, src):
         np.copyto(pinned[:src.size].numpy(), src)
 
 
-def _fetch(dev, parts):
-    """Bytes of the device tensor `dev` as a new numpy array; parts: (first byte, one past the last byte, event behind
-    which they are ready), in the order in which they become ready."""
-    host = np.empty(dev.numel(), dtype=np.uint8)
-    to = torch.from_numpy(host)
-    if len(parts) == 1 and dev.numel() <= _STAGE_BYTES:
-        stage = _pinned(dev.numel())
-        stage.copy_(dev, non_blocking=True)
-        torch.cuda.current_stream().synchronize()
-        to.copy_(stage)
-        return host
-    copier = _copier(torch.cuda.current_stream(dev.device))
-    runs = [(a0 + a, a0 + b, ready) for a0, b0, ready in parts for a, b in _chunks(b0 - a0, _STAGE_BYTES)]
-    stages = _stages(max(b - a for a, b, _ in runs))
-    done = [None] * len(runs)
-
-    def land(i):
-        a, b, _ = runs[i]
-        done[i].synchronize()
-        to[a:b].copy_(stages[i % _STAGES][:b - a])
-
-    with torch.cuda.stream(copier):
-        for i, (a, b, ready) in enumerate(runs):
-            if i >= _STAGES:
-                land(i - _STAGES)
-            copier.wait_event(ready)
-            stages[i % _STAGES][:b - a].copy_(dev[a:b], non_blocking=True)
-            done[i] = torch.cuda.Event()
-            done[i].record()
-    for i in range(max(0, len(runs) - _STAGES), len(runs)):
-        land(i)
-    return host
-
-
 def quantize_weights(w, type_, n_rot=None, wgroup=0):
     """w[N, K] fp32 on the GPU -> [N, K/256] weight blocks (numpy, host): the type's from_float_ref for whole
     tensors (quantize_row_w4a4_ref / quantize_row_w4a4h_ref, patch lines 2681-2710). wgroup 0 / 256 / 64 is the
@@ -363,28 +325,64 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
     assert w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and w.stride(1) == 1
     N, K = w.shape
     n_rot = int(n_rot or K)
-    # With one scale per row the search has a wavefront for four rows: 4096 rows are one per SIMD, and as many more take
-    # as long again, so a tensor goes through in runs of that many and a run's blocks travel while the next one is
-    # searched. (Weight groups fill the GPU with any number of rows: the same runs serve.)
-    runs = [(a, min(a + 4096, N)) for a in range(0, N, 4096)]
-    nbytes = L.rq_w4a4_quantize_weights_workspace_bytes(int(type_), K, min(N, 4096), int(wgroup))
+    # Runs of rows whose blocks fit one buffer, in turn on two streams, the conversion and its copy behind one another: a run is
+    # converted while the one before travels, and the link, which is what takes long, starts with the first one's blocks and
+    # goes from copy to copy without a pause. (6144 x 5120: rows in runs of 4096, all launched in front of the first copy, left
+    # it idle for 130 us at first: 637 us, this way 585.) Up to one and a half buffers' worth is one run: 1500 x 5120 215 us in
+    # one, 275 in two.
+    row = (K // 256) * 144
+    runs = [(0, N)] if 2 * N * row <= 3 * _STAGE_BYTES else _chunks(N, max(1, _STAGE_BYTES // row))
+    nbytes = L.rq_w4a4_quantize_weights_workspace_bytes(int(type_), K, max(b - a for a, b in runs), int(wgroup))
     if nbytes == 0:
         raise RqError("unsupported weight shape or group: K=%d N=%d wgroup=%d" % (K, N, wgroup))
-    ws = _device_bytes(nbytes, w.device)
-    row = (K // 256) * 144
     out = torch.empty(N * row, dtype=torch.uint8, device=w.device)
     ldw = w.stride(0) if N > 1 else K
-    parts = []
+
+    def convert(a, b, ws):
+        rc = L.rq_w4a4_quantize_weights(int(type_), w.data_ptr() + 4 * ldw * a, ldw, b - a, K, n_rot, int(wgroup),
+                                        out.data_ptr() + row * a, ws.data_ptr(), ws.numel(), _stream_ptr())
+        _check(rc, "rq_w4a4_quantize_weights")
+
     with torch.cuda.device(w.device):
         _refuse_capture()
-        for a, b in runs:
-            rc = L.rq_w4a4_quantize_weights(int(type_), w.data_ptr() + 4 * ldw * a, ldw, b - a, K, n_rot, int(wgroup),
-                                            out.data_ptr() + row * a, ws.data_ptr(), ws.numel(), _stream_ptr())
-            _check(rc, "rq_w4a4_quantize_weights")
-            ready = torch.cuda.Event()
-            ready.record()
-            parts.append((row * a, row * b, ready))
-        return _fetch(out, parts).view(BLOCK_DTYPE).reshape(N, K // 256)
+        current = torch.cuda.current_stream()
+        if len(runs) == 1:
+            convert(0, N, _device_bytes(nbytes, w.device))
+            stage = _pinned(N * row)
+            stage.copy_(out, non_blocking=True)
+            host = np.empty(N * row, dtype=np.uint8)
+            current.synchronize()
+            torch.from_numpy(host).copy_(stage)
+            return host.view(BLOCK_DTYPE).reshape(N, K // 256)
+        other = _second_stream(current)
+        other.wait_stream(current)   # (w, and the memory of out and the workspaces)
+        ws = [_device_bytes(nbytes, w.device) for _ in range(2)]
+        host = np.empty(N * row, dtype=np.uint8)
+        to = torch.from_numpy(host)
+        stages, done = [], []
+
+        def land(i):
+            a, b = runs[i]
+            done[i].synchronize()
+            to[row * a:row * b].copy_(stages[i % _STAGES][:row * (b - a)])
+
+        try:
+            for i, (a, b) in enumerate(runs):
+                with torch.cuda.stream(other if i & 1 else current):
+                    convert(a, b, ws[i & 1])
+                    if i >= _STAGES:
+                        land(i - _STAGES)
+                    else:
+                        stages.append(_pinned(row * max(d - c for c, d in runs)))
+                    stages[i % _STAGES][:row * (b - a)].copy_(out[row * a:row * b], non_blocking=True)
+                    done.append(torch.cuda.Event())
+                    done[i].record()
+            for i in range(max(0, len(runs) - _STAGES), len(runs)):
+                land(i)
+        except BaseException:
+            current.wait_stream(other)   # (the memory given back here may still be in use there)
+            raise
+        return host.view(BLOCK_DTYPE).reshape(N, K // 256)
 
 
 def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
@@ -412,27 +410,31 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
             rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr(), rows, K, int(n_rot), out.data_ptr(), K, _stream_ptr())
             _check(rc, "rq_w4a4_dequantize")
             return out
-        # a run of rows is decoded while the next one travels
+        # runs of rows, in turn on two streams: one is decoded while the next one travels
         current = torch.cuda.current_stream()
-        copier = _copier(current)
-        copier.wait_stream(current)   # (the memory of `raw` may still be in use by work in front of this call)
+        other = _second_stream(current)
+        other.wait_stream(current)   # (the memory of `raw` may still be in use by work in front of this call)
         runs = _chunks(rows, max(1, _STAGE_BYTES // row))   # (a row too long for the library is refused by it)
         host = blocks.view(np.uint8).reshape(-1)
-        stages = _stages(row * max(b - a for a, b in runs))
-        sent = [None] * _STAGES
-        for i, (a, b) in enumerate(runs):
-            n, k = row * (b - a), i % _STAGES
-            if sent[k] is not None:
-                sent[k].synchronize()
-            _copy_bytes(stages[k], host[row * a:row * b])
-            with torch.cuda.stream(copier):
-                raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
-                sent[k] = torch.cuda.Event()
-                sent[k].record()
-            current.wait_event(sent[k])
-            rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot),
-                                      out.data_ptr() + 4 * K * a, K, _stream_ptr())
-            _check(rc, "rq_w4a4_dequantize")
+        stages, sent = [], []
+        try:
+            for i, (a, b) in enumerate(runs):
+                n, k = row * (b - a), i % _STAGES
+                if i < _STAGES:
+                    stages.append(_pinned(row * max(d - c for c, d in runs)))
+                else:
+                    sent[i - _STAGES].synchronize()
+                _copy_bytes(stages[k], host[row * a:row * b])
+                with torch.cuda.stream(other if i & 1 else current):
+                    raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
+                    if i + _STAGES < len(runs):
+                        sent.append(torch.cuda.Event())
+                        sent[i].record()
+                    rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot),
+                                              out.data_ptr() + 4 * K * a, K, _stream_ptr())
+                _check(rc, "rq_w4a4_dequantize")
+        finally:
+            current.wait_stream(other)   # (what comes behind this call, also on an error the reuse of the memory)
     return out
 
 

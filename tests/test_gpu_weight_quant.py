@@ -203,8 +203,8 @@ def test_conversions_in_several_runs(oracle):
 
 @pytest.mark.parametrize("type_,wgroup", [(rq.TYPE_W4A4H, 0), (rq.TYPE_W4A4, 64)])
 def test_blocks_fetched_in_more_runs_than_buffers(type_, wgroup):
-    """9000 rows of 4096: three runs of rows, seven copies (20.7 MB) through three buffers, which are used again while the
-    next run is searched. The bytes are those of one call of the C entry point."""
+    """9000 rows of 4096: five runs of rows (20.7 MB) through three buffers, in turn on two streams. The bytes are those of one
+    call of the C entry point."""
     N, K = 9000, 4096
     g = torch.Generator(device=DEV)
     g.manual_seed(4)
@@ -220,10 +220,10 @@ def test_blocks_fetched_in_more_runs_than_buffers(type_, wgroup):
         assert blocks_equal(got, want), block_diff(got, want)
 
 
-@pytest.mark.parametrize("rows", [1, 3639, 3640, 3641])
+@pytest.mark.parametrize("rows", [1, 3639, 3640, 3641, 5461, 5462])
 def test_conversions_around_one_buffer(oracle, rows):
-    """A tensor whose blocks fit one pinned buffer (3640 rows of 8 blocks, 4 MiB) goes through without the second stream;
-    the last that fits and the first that does not; a read-only array and a writable one."""
+    """A tensor whose blocks fit one pinned buffer (3640 rows of 8 blocks, 4 MiB; 5461 on the way to the host) goes through
+    without the second stream; the last that fits and the first that does not; a read-only array and a writable one."""
     w = tensor(rows, 2048, 5)
     got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4)
     want = oracle.quantize_rows_w(w)
