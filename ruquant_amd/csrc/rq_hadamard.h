@@ -215,6 +215,14 @@ __device__ __forceinline__ void minmax8_raw(const float (&v)[8], float &lo, floa
     lo = min3_raw(min3_raw(lo, v[0], v[1]), min3_raw(v[2], v[3], v[4]), min3_raw(v[5], v[6], v[7]));
     hi = max3_raw(max3_raw(hi, v[0], v[1]), max3_raw(v[2], v[3], v[4]), max3_raw(v[5], v[6], v[7]));
 }
+// max / min over aligned runs of two, four or eight lanes, the same value in all of them
+template <bool MAX>
+__device__ __forceinline__ float group248_reduce(float v, int lanes) {
+    RQ_DPP_MINMAX(v, "quad_perm:[1,0,3,2]")
+    if (lanes > 2) RQ_DPP_MINMAX(v, "quad_perm:[2,3,0,1]")
+    if (lanes > 4) RQ_DPP_MINMAX(v, "row_half_mirror")
+    return v;
+}
 // max / min over aligned runs of eight lanes, the same value in all eight
 template <bool MAX>
 __device__ __forceinline__ float group8_reduce(float v) {

@@ -28,6 +28,83 @@ constexpr int threads_of() { return WIDE || (SLICED && P < 44) ? 1024 : 512; }
 
 using namespace had;
 
+// a group's multiplier, the reciprocal of its step and its zero point, from its range (reference lines 2662-2668)
+__device__ __forceinline__ void group_params(float lo, float hi, float R, float u, int &mg, float &inv, float &zf) {
+    mg = (int) fminf(fmaxf(ceilf(((hi - lo) * 255.0f) / R), 1.0f), 255.0f);
+    inv = 1.0f / ((float) mg * u);
+    zf = fminf(fmaxf(rintf(-lo * inv), 0.0f), 15.0f);
+}
+
+// The quantizer of the fp6 form: the token's rotated row in LDS -> its lanes of the fragments (q - z as fp6 E2M3, whose value is
+// (q - z) / 8) and its groups' multipliers. A thread has half a group of 64, the 32 values of one lane of a fragment:
+// v_cvt_scalef32_2xpk16_fp6_f32 converts and packs them in one instruction (they are representable, so nothing is rounded).
+// What bounds the kernel at thousands of tokens is the issue of vector instructions; with eight values to a thread, each group's
+// parameters worked out eight times and the codes put together bit by bit, the quantizer was XXX. 2048 tokens, K = 5120 XXX -> XXX us,
+// K = 17408 XXX -> XXX.
+template <int kNT>
+__device__ __forceinline__ void quantize_fp6(const RotQuantArgs &a, const float *buf, float *g_lo, float *g_hi, float *s_red, int t,
+                                             int tid) {
+    typedef float v16f __attribute__((ext_vector_type(16)));
+    typedef unsigned v6u __attribute__((ext_vector_type(6)));
+    const int nh = a.K >> 5;                                     // halves of groups of 64
+    const int lanes = a.G >> 5, ll = __ffs(lanes) - 1;           // of an activation group: 2, 4 or 8 (RQ_ACT_GROUP)
+    float rmax = 0.0f;
+    for (int h0 = 0; h0 < nh; h0 += kNT) {
+        const int h = h0 + tid;
+        const bool on = h < nh;
+        float mn = 0.0f, mx = 0.0f;
+        if (on) {
+            const float *sp = buf + padi(32 * h);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v8[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v8[j] = sp[8 * q + j + (q >> 1)];   // (a float of padding behind the first 16)
+                had::minmax8_raw(v8, mn, mx);
+            }
+        }
+        mn = had::group248_reduce<false>(mn, lanes);
+        mx = had::group248_reduce<true>(mx, lanes);
+        const float lo = mn * a.clip, hi = mx * a.clip;
+        if (on) {
+            if ((tid & (lanes - 1)) == 0) {
+                g_lo[h >> ll] = lo;
+                g_hi[h >> ll] = hi;
+            }
+            rmax = fmaxf(rmax, hi - lo);
+        }
+    }
+    rmax = wave_max(rmax);
+    if ((tid & 63) == 0) s_red[tid >> 6] = rmax;
+    __syncthreads();
+    float R = s_red[0];
+#pragma unroll
+    for (int i = 1; i < kNT / 64; ++i) R = fmaxf(R, s_red[i]);
+    if (R == 0.0f) R = 2.0f;
+    const float u = R / 3825.0f;  // 15 * 255
+    if (tid == 0 && a.u != nullptr) a.u[t] = u;
+    for (int h = tid; h < nh; h += kNT) {
+        int mg;
+        float inv, zf;
+        group_params(g_lo[h >> ll], g_hi[h >> ll], R, u, mg, inv, zf);
+        // q - z = clamp(rint(x / step) + z, 0, 15) - z: integers, exact however they are ordered
+        const float least = 0.0f - zf, most = 15.0f - zf;
+        const float *sp = buf + padi(32 * h);
+        v16f even, odd;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            even[j] = __builtin_amdgcn_fmed3f(rintf(sp[2 * j + (j >> 3)] * inv), least, most);
+            odd[j] = __builtin_amdgcn_fmed3f(rintf(sp[2 * j + 1 + (j >> 3)] * inv), least, most);
+        }
+        const v6u c = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(even, odd, 8.0f);   // even values first, divided by 8
+        const int g = h >> 1, lane = (t & 31) + 32 * (h & 1);
+        uint8_t *frag = reinterpret_cast<uint8_t *>(a.act) + ((size_t) g * (a.Mp >> 5) + (t >> 5)) * kFrag6;
+        *reinterpret_cast<uint4 *>(frag + lane * 16) = make_uint4(c[0], c[1], c[2], c[3]);
+        *reinterpret_cast<uint2 *>(frag + 1024 + lane * 8) = make_uint2(c[4], c[5]);
+        if ((h & 1) == 0) a.m4[(size_t) g * a.Mp + t] = 4.0f * (float) mg;
+    }
+}
+
 template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
 // Registers are capped so that two workgroups (p >= 44: long columns, long rows) or three fit a compute unit: the
 // stages of one token are separated by barriers, and it is the other workgroups that keep the vector ALU busy. (The
@@ -166,6 +243,11 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
         return;
     }
 
+    if (a.mode == kActI8 && a.single == 2) {
+        quantize_fp6<kNT>(a, buf, g_lo, g_hi, s_red, t, tid);
+        return;
+    }
+
     // ---- group ranges [min(x,0), max(x,0)] * clip and the token's widest range (reference lines 2646-2654)
     const int nw = K >> 3;  // code words of this token: a thread per word, lpg lanes per activation group
     const int lpg = a.G >> 3, lgl = __ffs(lpg) - 1;   // 8, 16 or 32 lanes: groups of 64, 128 or 256 (RQ_ACT_GROUP)
@@ -235,41 +317,12 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
         const int wc = on ? w : 0;
         const int g = wc >> 3;                     // 64-wide group: where the digits go
         const float lo = g_lo[wc >> lgl], hi = g_hi[wc >> lgl];
-        const int mg = (int) fminf(fmaxf(ceilf(((hi - lo) * 255.0f) / R), 1.0f), 255.0f);
-        const float inv = 1.0f / ((float) mg * u);
-        const float zf = fminf(fmaxf(rintf(-lo * inv), 0.0f), 15.0f);
+        int mg;
+        float inv, zf;
+        group_params(lo, hi, R, u, mg, inv, zf);
         const int z = (int) zf;
         const float *sp = buf + padi(8 * wc);
         const float f[8] = { sp[0], sp[1], sp[2], sp[3], sp[4], sp[5], sp[6], sp[7] };
-        if (a.mode == kActI8 && a.single == 2) {
-            // fp6 fragment plane: q - z as sign and magnitude, six bits each (as fp6 E2M3 the value is (q - z) / 8);
-            // this word's 48 bits are bytes 6 (w % 4) .. of the 24 bytes that lane token % 32 + 32 * (half of the group)
-            // holds in the fragment of 32 tokens: bytes 0 .. 15 at lane * 16, bytes 16 .. 23 at 1024 + lane * 8
-            // (as a float q - z has the sign where the code wants it, and its magnitude converts without it)
-            uint32_t c[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float d = __builtin_amdgcn_fmed3f(rintf(f[j] * inv) + zf, 0.0f, 15.0f) - zf;
-                c[j] = (uint32_t) fabsf(d) | ((__builtin_bit_cast(uint32_t, d) >> 26) & 32u);
-            }
-            const uint32_t lo6 = c[0] | c[1] << 6 | c[2] << 12 | c[3] << 18 | c[4] << 24 | c[5] << 30;
-            const uint32_t hi6 = c[5] >> 2 | c[6] << 4 | c[7] << 10;
-            // The four words of a half group, in the four lanes of a quad, are one lane's 24 bytes of the fragment: the first
-            // lane gathers and stores its 16-byte piece, the third the 8-byte one (three 2-byte stores per lane before).
-            const uint32_t lo_n = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) lo6, 0xF5, 0xF, 0xF, false);   // quad_perm [1, 1, 3, 3]
-            const uint32_t hi_n = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) hi6, 0xF5, 0xF, 0xF, false);
-            const uint32_t lo_2 = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) lo6, 0xAA, 0xF, 0xF, false);   // quad_perm [2, 2, 2, 2]
-            const uint32_t p1 = hi6 | lo_n << 16, p2 = lo_n >> 16 | hi_n << 16;
-            if (on) {
-                const int c8 = w & 7;
-                const int lane = (t & 31) + 32 * (c8 >> 2);
-                uint8_t *frag = reinterpret_cast<uint8_t *>(a.act) + ((size_t) g * (a.Mp >> 5) + (t >> 5)) * kFrag6;
-                if ((c8 & 3) == 0) *reinterpret_cast<uint4 *>(frag + lane * 16) = make_uint4(lo6, p1, p2, lo_2);
-                if ((c8 & 3) == 2) *reinterpret_cast<uint2 *>(frag + 1024 + lane * 8) = make_uint2(p1, p2);
-                if (c8 == 0) a.m4[(size_t) g * a.Mp + t] = 4.0f * (float) mg;
-            }
-            continue;
-        }
         if (a.mode == kActI8 && a.single) {
             uint32_t even, odd;
             qz_of_word(f, inv, zf, even, odd);
