@@ -38,9 +38,9 @@ __device__ __forceinline__ void group_params(float lo, float hi, float R, float 
 // The quantizer of the fp6 form: the token's rotated row in LDS -> its lanes of the fragments (q - z as fp6 E2M3, whose value is
 // (q - z) / 8) and its groups' multipliers. A thread has half a group of 64, the 32 values of one lane of a fragment:
 // v_cvt_scalef32_2xpk16_fp6_f32 converts and packs them in one instruction (they are representable, so nothing is rounded).
-// What bounds the kernel at thousands of tokens is the issue of vector instructions; with eight values to a thread, each group's
-// parameters worked out eight times and the codes put together bit by bit, the quantizer was XXX. 2048 tokens, K = 5120 XXX -> XXX us,
-// K = 17408 XXX -> XXX.
+// What bounds the kernel at thousands of tokens is the issue of vector instructions: with eight values to a thread each group's
+// parameters were worked out eight times and the codes put together bit by bit. Activation stage, 2048 tokens: K = 5120 24.2 -> 22 us,
+// K = 17408 92 -> 77.
 template <int kNT>
 __device__ __forceinline__ void quantize_fp6(const RotQuantArgs &a, const float *buf, float *g_lo, float *g_hi, float *s_red, int t,
                                              int tid) {
