@@ -15,6 +15,13 @@
 // through the compute unit's 64 bytes per cycle, 0.32 us; 112 vector instructions each, 0.37 us of the SIMDs' time, and four
 // MFMAs, 0.11 (counters: 1.144 M vector instructions and 1.31 M MFMA cycles for 128 units of 80 groups). From memory the weights'
 // 24 KB are the longest, 1.0 to 1.2 us. Beyond two rounds of the chip the tiled kernel's twofold reuse out of LDS wins.
+//
+// A last round that leaves half of the compute units without a unit, or three quarters, cuts its units in pieces, two of 32 rows x
+// 64 tokens or four of 32 x 32, with the whole K as before: a compute unit's share of the loads (which bind it, from memory by the
+// weights' rows) and of the vector instructions is halved, and nothing has to meet in memory. Product kernel in us, whole units
+// -> pieces, weights from the memory-side cache, then from memory: K = 5120, 32 units 9.2 -> 5.9, 10.9 -> 7.2; 94 units 9.7 -> 8.2,
+// 13.4 -> 11.2; K = 17408, 32 units 22.1 -> 12.6, 32.0 -> 17.7; 94 units 23.6 -> 19.1, 32.3 -> 25.7; K = 10240, 128 units 15.6 -> 13.1,
+// 20.4 -> 16.6; behind a round, 64 tokens, 256 + 16 units, whole call 27.3 -> 23.8.
 #include "rq_common.h"
 
 #pragma clang fp contract(off)
@@ -32,18 +39,20 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 8, kThreads = kWaves * 64;
 constexpr int kTok = 64;                       // tokens of a unit
 constexpr int kUnitsPerTile = 8;               // 4 panels x 2 runs of 64 tokens of a tile of 256 x 128
-// groups of a wavefront whose operands are on their way (with weight multipliers the registers end there)
+// groups of a wavefront whose operands are on their way (with weight multipliers the registers end there; pieces with 3 and 7 are
+// 1 % slower at K = 5120)
 constexpr int depth_of(bool hask) { return hask ? 2 : 4; }
 constexpr int kTokStride = kPanelRows + 4;     // ints between tokens of a wavefront's totals in LDS
 constexpr float kBias = 12582912.0f;           // 1.5 x 2^23
 constexpr uint32_t kBiasBits = 0x4B400000;
 constexpr int kFlushGroups = 28;               // (and the tile of one more that is folded late): less than 2^22
 
-template <bool HASK>
+// RA, RB: fragments of 32 rows and of 32 tokens that the workgroup's unit or piece of one has
+template <bool HASK, int RA, int RB>
 struct Frag {
-    v8i A[2], B[2];       // this lane's parts of the two fragments of rows and the two of tokens (six registers each)
-    float m4[2];          // 4 m of this lane's two tokens
-    uint32_t kw[HASK ? 8 : 1];   // weight multipliers of the lane's rows (32 a + 8 q + 4 (lane / 32) + 0 .. 3), a byte each
+    v8i A[RA], B[RB];     // this lane's parts of the fragments of rows and of tokens (six registers each)
+    float m4[RB];         // 4 m of this lane's tokens
+    uint32_t kw[HASK ? 4 * RA : 1];   // weight multipliers of the lane's rows (32 a + 8 q + 4 (lane / 32) + 0 .. 3), a byte each
 };
 
 // (global memory, said so: the plane's address comes out of memory, and the loads the compiler makes for a pointer of unknown
@@ -55,7 +64,7 @@ typedef const __attribute__((address_space(1))) v4u gv4u;
 typedef const __attribute__((address_space(1))) v2u gv2u;
 
 struct Src {
-    gbyte *a, *b, *k;           // (wave-uniform) the unit's operands of group 0
+    gbyte *a, *b, *k;           // (wave-uniform) the unit's or piece's operands of group 0
     gfloat *m4;
     size_t b_step;              // bytes between groups of the activation plane
     int Mp;
@@ -73,8 +82,8 @@ __device__ __forceinline__ v8i operand(gbyte *frag, uint32_t l) {
 
 // The wavefront's group j of n. Past the end of its share a wavefront's loads read group 0 again, from offset 0 in
 // every lane (the loop stays branch-free, so the wait counts stay exact), and nothing consumes them
-template <bool HASK>
-__device__ __forceinline__ void load_frag(Frag<HASK> &f, const Src &s, int wave, int lane, int j, int n) {
+template <bool HASK, int RA, int RB>
+__device__ __forceinline__ void load_frag(Frag<HASK, RA, RB> &f, const Src &s, int wave, int lane, int j, int n) {
     const int g = wave + j * kWaves;
     // (a mask: on a condition the compiler branches around the address arithmetic, and the folds sink into the blocks behind)
     const int keep = __builtin_amdgcn_readfirstlane((j - n) >> 31);
@@ -84,14 +93,16 @@ __device__ __forceinline__ void load_frag(Frag<HASK> &f, const Src &s, int wave,
     gfloat *m4 = s.m4 + (size_t) gk * s.Mp;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        f.A[i] = operand(a + i * kFrag6, l);
-        f.B[i] = operand(b + i * kFrag6, l);
-        f.m4[i] = m4[32 * i + (l & 31)];
+        if (i < RA) f.A[i] = operand(a + i * kFrag6, l);
+        if (i < RB) {
+            f.B[i] = operand(b + i * kFrag6, l);
+            f.m4[i] = m4[32 * i + (l & 31)];
+        }
     }
     if constexpr (HASK) {
         gbyte *k = s.k + (size_t) gk * kPanelRows + 4 * (l >> 5);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) f.kw[q] = *reinterpret_cast<gword *>(k + 8 * q);
+        for (int q = 0; q < 4 * RA; ++q) f.kw[q] = *reinterpret_cast<gword *>(k + 8 * q);
     }
 }
 
@@ -101,20 +112,22 @@ __device__ __forceinline__ void load_frag(Frag<HASK> &f, const Src &s, int wave,
 // (acc holds those; the bias of every term comes off at the end). The sum of the patterns passes 2^32 from the fourth group on:
 // unsigned, modulo 2^32, which gives the total back, since that is small: at most 64 groups of a wavefront x 15 x 122,400 =
 // 117.5 M, and 940 M over the eight.
+template <int RA, int RB>
 struct State {
-    float acc[2][2][16];
+    float acc[RA][RB][16];
     v16f P;
     float pm;
     float bias;   // kBias (with weight multipliers; taken from behind the change of the rounding mode, like acc)
 };
 
-// the four tiles of one group; a tile's fold runs behind the next tile's MFMA
-__device__ __forceinline__ void group_units(const Frag<false> &f, State &st) {
+// the tiles of one group; a tile's fold runs behind the next tile's MFMA
+template <int RA, int RB>
+__device__ __forceinline__ void group_units(const Frag<false, RA, RB> &f, State<RA, RB> &st) {
     const v16f zero = {};
 #pragma unroll
-    for (int un = 0; un < 4; ++un) {
-        const int a = un >> 1, b = un & 1;
-        const int pa = un == 0 ? 1 : (un - 1) >> 1, pb = un == 0 ? 1 : (un - 1) & 1;
+    for (int un = 0; un < RA * RB; ++un) {
+        const int a = un / RB, b = un % RB;
+        const int pu = (un + RA * RB - 1) % (RA * RB), pa = pu / RB, pb = pu % RB;
         const v16f S = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.A[a], f.B[b], zero, 2, 2, 0, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 16; ++r) st.acc[pa][pb][r] = __builtin_fmaf(st.P[r], st.pm, st.acc[pa][pb][r]);
@@ -129,18 +142,19 @@ __device__ __forceinline__ void group_units(const Frag<false> &f, State &st) {
 }
 // with weight multipliers: the two tiles of a row block together, which share the multipliers as floats (a group is folded
 // whole, so that the next one does not need its multipliers)
-__device__ __forceinline__ void group_units(const Frag<true> &f, State &st) {
+template <int RA, int RB>
+__device__ __forceinline__ void group_units(const Frag<true, RA, RB> &f, State<RA, RB> &st) {
     const v16f zero = {};
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        v16f S[2];
+    for (int a = 0; a < RA; ++a) {
+        v16f S[RB];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) S[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.A[a], f.B[b], zero, 2, 2, 0, 0, 0, 0);
+        for (int b = 0; b < RB; ++b) S[b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.A[a], f.B[b], zero, 2, 2, 0, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const float kf = (float) ((f.kw[4 * a + (r >> 2)] >> (8 * (r & 3))) & 0xFFu);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
+            for (int b = 0; b < RB; ++b) {
                 const float term = __builtin_fmaf(S[b][r], kf * f.m4[b], st.bias);
                 st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, st.acc[a][b][r]) + __builtin_bit_cast(uint32_t, term));
             }
@@ -150,12 +164,12 @@ __device__ __forceinline__ void group_units(const Frag<true> &f, State &st) {
 }
 
 // the totals of this wavefront into its own part of LDS, [token][row]; FRESH: nothing is there yet
-template <bool FRESH>
-__device__ __forceinline__ void flush(State &st, int *part, int lane) {
+template <bool FRESH, int RA, int RB>
+__device__ __forceinline__ void flush(State<RA, RB> &st, int *part, int lane) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < RB; ++b) {
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
+        for (int a = 0; a < RA; ++a) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 v4i *dst = reinterpret_cast<v4i *>(part + (32 * b + (lane & 31)) * kTokStride + 32 * a + 8 * q + 4 * (lane >> 5));
@@ -171,15 +185,15 @@ __device__ __forceinline__ void flush(State &st, int *part, int lane) {
     }
 }
 
-template <bool HASK>
+template <bool HASK, int RA, int RB>
 __device__ __forceinline__ void stream(const Src &s, int wave, int lane, int n, int *part) {
-    State st;
+    State<RA, RB> st;
     st.P = v16f{};
     st.pm = 0.0f;
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
+    for (int a = 0; a < RA; ++a) {
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < RB; ++b) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 st.acc[a][b][r] = HASK ? 0.0f : kBias;
@@ -190,10 +204,10 @@ __device__ __forceinline__ void stream(const Src &s, int wave, int lane, int n, 
     constexpr int kDepth = depth_of(HASK);
     st.bias = kBias;
     asm volatile("" : "+s"(st.bias));
-    Frag<HASK> ring[kDepth];
+    Frag<HASK, RA, RB> ring[kDepth];
 #pragma unroll
     for (int i = 0; i < kDepth; ++i) {
-        load_frag<HASK>(ring[i], s, wave, lane, i, n);
+        load_frag<HASK, RA, RB>(ring[i], s, wave, lane, i, n);
         __builtin_amdgcn_sched_barrier(0);   // (group by group: a wait counts the loads behind the one it is for)
     }
     const int rounds = n / kDepth;
@@ -204,7 +218,7 @@ __device__ __forceinline__ void stream(const Src &s, int wave, int lane, int n, 
             const int j = r * kDepth + i + kDepth;
             group_units(ring[i], st);
             __builtin_amdgcn_sched_barrier(0);
-            load_frag<HASK>(ring[i], s, wave, lane, j, n);
+            load_frag<HASK, RA, RB>(ring[i], s, wave, lane, j, n);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (!HASK && (r + 1) % (kFlushGroups / kDepth) == 0) {
@@ -222,16 +236,16 @@ __device__ __forceinline__ void stream(const Src &s, int wave, int lane, int n, 
         // n terms, each with the bias's bit pattern on it
         const uint32_t off = (uint32_t) n * kBiasBits - kBiasBits;   // (flush takes one off)
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
+        for (int a = 0; a < RA; ++a) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
+            for (int b = 0; b < RB; ++b) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) st.acc[a][b][r] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, st.acc[a][b][r]) - off);
             }
         }
     } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) st.acc[1][1][r] = __builtin_fmaf(st.P[r], st.pm, st.acc[1][1][r]);
+        for (int r = 0; r < 16; ++r) st.acc[RA - 1][RB - 1][r] = __builtin_fmaf(st.P[r], st.pm, st.acc[RA - 1][RB - 1][r]);
     }
     if (fresh) flush<true>(st, part, lane);
     else flush<false>(st, part, lane);
@@ -248,15 +262,26 @@ struct BlockSet {
     int            first[kMaxFused];   // first panel, or row tile of 256 rows; unused slots hold the total, so none selects them
 };
 
+// CUT: the launch has units in pieces.
+template <bool CUT>
 __global__ void __launch_bounds__(kThreads, 2)
 rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const float *__restrict__ m4,
                  const float *__restrict__ u, int M, int Mp, int ng, int n_runs, int super_tiles, int first_tile,
-                 int n_units) {
+                 int n_whole, int n_cut, int pieces) {
     __shared__ __align__(16) int s_part[kWaves][kTok * kTokStride];
+    // The first n_whole workgroups have a unit each, the others a piece of one of the n_cut units behind those.
     // An XCD gets a contiguous run of the units, so that those that share a panel or a run of tokens read them from one L2.
-    int v = blockIdx.x;
-    const int per_xcd = n_units / kXcds;
+    const bool whole = !CUT || (int) blockIdx.x < n_whole;
+    int v = whole ? blockIdx.x : blockIdx.x - n_whole;
+    const int per_xcd = (whole ? n_whole : n_cut * pieces) / kXcds;
     if (v < per_xcd * kXcds) v = (v % kXcds) * per_xcd + v / kXcds;
+    int ra = 0, rb = 0;   // (of a piece) which 32 of the unit's rows, and in quarters which 32 of its tokens
+    const bool quarter = pieces == 4;
+    if (!whole) {
+        rb = quarter ? v & 1 : 0;
+        ra = (v >> (quarter ? 1 : 0)) & 1;
+        v = n_whole + (v >> (quarter ? 2 : 1));
+    }
     int wsel, panel, t0;   // which weight, which of its panels, first token
     if (first_tile < 0) {
         // the whole product: panel by panel, the runs of tokens running fastest. (No unit is without rows or tokens: workgroups
@@ -284,17 +309,19 @@ rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const floa
     float *__restrict__ y = of_weight(ts.y);
     const int64_t ldy = of_weight(ts.ldy);
     const int64_t N = of_weight(ts.N);
+    // (a piece without rows or tokens)
+    if (t0 + 32 * rb >= M || (int64_t) panel * kPanelRows + 32 * ra >= N) return;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint8_t *w6 = plane6_of(flags);
     const bool hask = flags[0] & 1;
     Src s;
-    s.a = (gbyte *) (w6 + ((size_t) (panel >> 2) * ng * 8 + 2 * (panel & 3)) * kFrag6);
+    s.a = (gbyte *) (w6 + ((size_t) (panel >> 2) * ng * 8 + 2 * (panel & 3) + ra) * kFrag6);
     s.b_step = (size_t) (Mp / 32) * kFrag6;
-    s.b = (gbyte *) (act6 + (size_t) (t0 / 32) * kFrag6);
-    s.m4 = (gfloat *) (m4 + t0);
-    s.k = (gbyte *) (kmul + (size_t) panel * ng * kPanelRows);
+    s.b = (gbyte *) (act6 + (size_t) (t0 / 32 + rb) * kFrag6);
+    s.m4 = (gfloat *) (m4 + t0 + 32 * rb);
+    s.k = (gbyte *) (kmul + (size_t) panel * ng * kPanelRows + 32 * ra);
     s.Mp = Mp;
     // what the epilogue needs from memory is asked for first: a thread ends with four rows of two tokens
     const int quad = tid & 15, tok = tid >> 4;
@@ -306,8 +333,17 @@ rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const floa
     const int n = wave < ng ? (ng - wave + kWaves - 1) / kWaves : 0;   // groups wave, wave + 8, ...
     // fp32 rounding toward minus infinity for the folds (MODE bits 1:0); the MFMA sums are exact in any mode
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 2" ::: "memory");
-    if (hask) stream<true>(s, wave, lane, n, s_part[wave]);
-    else stream<false>(s, wave, lane, n, s_part[wave]);
+    int *part = s_part[wave] + 32 * rb * kTokStride + 32 * ra;
+    if (whole) {
+        if (hask) stream<true, 2, 2>(s, wave, lane, n, part);
+        else stream<false, 2, 2>(s, wave, lane, n, part);
+    } else if (quarter) {
+        if (hask) stream<true, 1, 1>(s, wave, lane, n, part);
+        else stream<false, 1, 1>(s, wave, lane, n, part);
+    } else {
+        if (hask) stream<true, 1, 2>(s, wave, lane, n, part);
+        else stream<false, 1, 2>(s, wave, lane, n, part);
+    }
     // (the totals are in LDS when the mode goes back to round to nearest even, and the conversions below read them from there)
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0" ::: "memory");
     __syncthreads();
@@ -316,6 +352,7 @@ rq_block6_kernel(const BlockSet ts, const uint8_t *__restrict__ act6, const floa
     const int64_t row = (int64_t) panel * kPanelRows + 4 * quad;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
+        if (!whole && ((quad >> 3) != ra || (quarter && i != rb))) continue;
         const int t = t0 + tok + 32 * i;
         v4i tot = *reinterpret_cast<const v4i *>(&s_part[0][(tok + 32 * i) * kTokStride + 4 * quad]);
 #pragma unroll
@@ -359,8 +396,17 @@ hipError_t launch(const Gemm6Args &a, int super_tiles, int first_tile, int n_uni
     }
     const int ng = a.w.L[0].ng;
     const float *m4 = reinterpret_cast<const float *>(a.act6 + act6_plane_bytes(ng, a.Mp));
-    hipLaunchKernelGGL(rq_block6_kernel, dim3(n_units), dim3(kThreads), 0, stream, ts, a.act6, m4, a.u, a.M, a.Mp, ng,
-                       (a.M + kTok - 1) / kTok, super_tiles, first_tile, n_units);
+    // units of the last round in four pieces where the chip has room for them, in two, or whole (160 units are no faster in pieces,
+    // which would be a second round)
+    const int last = n_units % kPlanUnits;
+    const int pieces = last <= kPlanUnits / 4 ? 4 : last <= kPlanUnits / 2 ? 2 : 1;
+    const int n_cut = pieces > 1 ? last : 0, n_whole = n_units - n_cut;
+#define RQ_LAUNCH_BLOCK6(CUT)                                                                                              \
+    hipLaunchKernelGGL(rq_block6_kernel<CUT>, dim3(n_whole + n_cut * pieces), dim3(kThreads), 0, stream, ts, a.act6, m4,   \
+                       a.u, a.M, a.Mp, ng, (a.M + kTok - 1) / kTok, super_tiles, first_tile, n_whole, n_cut, pieces)
+    if (n_cut > 0) RQ_LAUNCH_BLOCK6(true);
+    else RQ_LAUNCH_BLOCK6(false);
+#undef RQ_LAUNCH_BLOCK6
     return hipGetLastError();
 }
 
@@ -381,7 +427,10 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 // memory-side cache holds and loses on weights that come from memory, as those of a whole model do: a unit's 3 KB a group
 // then arrive at 20 KB per microsecond, whatever the other compute units do. The line lies where it is faster from the cache
 // and at most 6 % slower from memory. (64 tokens, whole call in us, skinny / here; in front from the cache, behind from memory.)
-// - Up to 128 panels (half the chip: the skinny kernel has two workgroups of 32 tokens a panel): K = 5120, N = 8192 14.8 / 15.0,
+// - Up to 64 panels, a unit in four pieces: K = 1024, N = 4096 8.8 / 8.1, 9.4 / 8.9 (40 tokens); K = 5120, N = 1024 11.6 / 10.4,
+//   12.6 / 12.2, N = 4096 14.1 / 10.4, 15.6 / 13.5; K = 10240 21.6 / 14.2, 23.4 / 18.8; K = 17408, N = 1024 20.2 / 18.6, 22.0 / 25.1,
+//   N = 4096 27.3 / 19.7, 28.6 / 27.0; K = 32768, N = 1024 28.7 / 30.3, 28.6 / 40.0. Here up to K = 10240.
+// - 65 to 128 panels (half the chip: the skinny kernel has two workgroups of 32 tokens a panel): K = 5120, N = 8192 14.8 / 15.0,
 //   16.1 / 19.6; K = 17408, N = 8192 47.6 / 39.4, 38.4 / 46.6. The skinny kernel.
 // - 129 to 256 panels, a round of units, and two of the skinny kernel's: N = 12288, K = 1024 15.6 / 9.5, 16.3 / 10.9; K = 5120
 //   24.4 / 16.4, 25.6 / 20.5; K = 10240 32.0 / 24.6, 32.8 / 32.9; K = 17408 48.1 / 35.5, 48.4 / 50.7; K = 32768 81 / 85 in both.
@@ -396,6 +445,7 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 // 33 tokens are within a tenth of 64 on both sides.
 bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers) {
     if (M <= 32) return false;
+    if (n_panels <= kPlanUnits / 4) return ng <= 160;
     if (n_panels <= kPlanUnits / 2) return weight_multipliers && n_panels >= 96 && ng >= 48 && ng <= 160;
     if (n_panels <= kPlanUnits) return ng <= 272 || weight_multipliers;
     if (weight_multipliers) return ng <= 272;

@@ -33,7 +33,13 @@ DEV = "cuda:0"
     (2560, 8300, 33, 0, 130),        # 130 panels: 33 .. 64 tokens in units
     (2560, 8300, 64, 64, 130),
     (17408, 8257, 41, 0, 130),
-    (512, 16500, 57, 0, 258)])       # two rounds
+    (512, 16500, 57, 0, 258),        # two rounds
+    (10240, 4096, 64, 0, 64),        # units in four pieces: as many as that takes
+    (1024, 70, 33, 0, 2),            # ... without rows, and with one token
+    (1280, 2050, 70, 64, 66),        # one more: in two pieces, the last panel's second without rows
+    (1280, 4070, 128, 0, 128),       # as many as that takes
+    (512, 4100, 97, 256, 130),       # one more: whole
+    (11264, 70, 40, 0, 0)])          # few panels of longer rows: the skinny kernel
 def test_units_of_64_rows_and_tokens(oracle, K, N, M, wgroup, units):
     type_ = rq.TYPE_W4A4 if K in (256, 512, 32768) else rq.TYPE_W4A4H
     blocks, wf = adversarial_weights(oracle, N, K, type_, seed=N + M, wgroup=wgroup)
