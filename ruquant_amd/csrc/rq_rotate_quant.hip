@@ -22,9 +22,9 @@ namespace {
 // Threads per token workgroup. Small batches (the sliced variant) with a short Paley stage get 1024: there the kernel
 // is one workgroup per compute unit at most, bound by the latency of its own phases, and twice the threads halve the
 // work per phase. Long Paley stages that keep a column in one thread's registers need the 256-register budget of 512
-// threads; those whose columns four threads share (WIDE) get 1024.
-template <int P, bool SLICED, bool WIDE>
-constexpr int threads_of() { return WIDE || (SLICED && P < 44) ? 1024 : 512; }
+// threads; those whose columns four threads share (WIDE) get 1024. Many tokens of short rows (FEW, takes_few) get 256.
+template <int P, bool SLICED, bool WIDE, bool FEW>
+constexpr int threads_of() { return FEW ? 256 : WIDE || (SLICED && P < 44) ? 1024 : 512; }
 
 using namespace had;
 
@@ -105,16 +105,17 @@ __device__ __forceinline__ void quantize_fp6(const RotQuantArgs &a, const float 
     }
 }
 
-template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
+template <int P, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
 // Registers are capped so that two workgroups (p >= 44: long columns, long rows) or three fit a compute unit: the
 // stages of one token are separated by barriers, and it is the other workgroups that keep the vector ALU busy. (The
 // sliced variant serves small batches, where occupancy is not the limit.) WIDE: 1024 threads, the columns of a long Paley stage
 // by four threads each (paley_row), a fourth of the registers per column; see takes_wide for where. ALONE is the plain
 // variant for rows so long that LDS holds one workgroup per compute unit anyway: the cap then only makes the p >= 60 columns
-// spill (136 to 504 bytes per lane), so it goes (2048 tokens, K = 21504, p = 84: 204 -> 193 us).
-__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE>()), WIDE ? (P >= 84 ? 4 : 8) : SLICED ? (P < 44 ? 4 : 2) : ALONE ? 2 : P >= 44 ? 4 : 6)
+// spill (136 to 504 bytes per lane), so it goes (2048 tokens, K = 21504, p = 84: 204 -> 193 us). FEW: five workgroups of 256 threads, with
+// the registers that p = 20 needs (six make it spill: K = 5120, 2048 tokens 19.8 us, five 18.3).
+__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE, FEW>()), FEW ? 5 : WIDE ? (P >= 84 ? 4 : 8) : SLICED ? (P < 44 ? 4 : 2) : ALONE ? 2 : P >= 44 ? 4 : 6)
 rq_rotate_quant_kernel(const RotQuantArgs a) {
-    constexpr int kNT = threads_of<P, SLICED, WIDE>();
+    constexpr int kNT = threads_of<P, SLICED, WIDE, FEW>();
     extern __shared__ __align__(16) float smem[];
     __shared__ float s_red[kNT / 64];
 
@@ -382,9 +383,9 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
 }
 
 // the kernels keep a whole row in dynamic LDS: raise the per-kernel limit (once per device, see init_activation_kernels)
-template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
+template <int P, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
 hipError_t allow_big_lds() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE>),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE, FEW>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 64);
 }
 
@@ -397,25 +398,26 @@ hipError_t allow_big_lds_both() {
     hipError_t e = allow_big_lds<P, false>();
     if (e == hipSuccess && P > 1) e = allow_big_lds<P, (P > 1)>();
     if (e == hipSuccess && has_wide(P)) e = allow_big_lds<P, false, has_wide(P)>();
+    if (e == hipSuccess && P < 44) e = allow_big_lds<P, false, false, false, (P < 44)>();
     if (e == hipSuccess && has_alone(P)) e = allow_big_lds<P, false, false, has_alone(P)>();
     return e;
 }
 
-template <int P, bool SLICED, bool WIDE = false, bool ALONE = false>
+template <int P, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
 hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
     static bool attr_set = false;   // calls that never went through rq_w4a4_prepare on this device
     if (!attr_set) {
-        hipError_t e = allow_big_lds<P, SLICED, WIDE, ALONE>();
+        hipError_t e = allow_big_lds<P, SLICED, WIDE, ALONE, FEW>();
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    constexpr int kNT = threads_of<P, SLICED, WIDE>();
+    constexpr int kNT = threads_of<P, SLICED, WIDE, FEW>();
     // blocks past the tokens clear the split-K cells, four ints per thread
     RotQuantArgs b = a;
     b.token_blocks = a.M;
     const int grid = a.M + (int) ((a.zero_ints + (int64_t) kNT * 4 - 1) / ((int64_t) kNT * 4));
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE>), dim3(grid), dim3(kNT), lds, stream, b);
+    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE, FEW>), dim3(grid), dim3(kNT), lds, stream, b);
     return hipGetLastError();
 }
 
@@ -443,6 +445,16 @@ bool takes_wide(const RotQuantArgs &a, bool sliced) {
     return columns == 512 && a.m >= 256 && a.mode != kActRotateOnly;
 }
 
+// Whether a token gets 256 threads: rows of at most 5120 floats give most of 512 nothing to do in most phases (320 threads load,
+// 256 have a column, 160 quantize), and five tokens instead of three share a compute unit. Activation stage in us, 512 threads ->
+// 256: 700 tokens K = 1024 5.0 -> 4.8, 4096 7.6 -> 7.6, 5120 9.6 -> 8.2; 2048 tokens K = 1024 9.7 -> 6.4, 1536 10.3 -> 6.6, 3072 13.1 ->
+// 9.5, 4096 15.9 -> 13.2, 5120 21.9 -> 18.3, 6144 21.3 -> 22.1, 8192 27.2 -> 30.2. Up to two tokens per compute unit each has as many
+// as it can use (400 tokens, K = 4096 6.3 -> 6.6), but p = 20, which spills with 512, 7.3 -> 7.1 (256 tokens 6.5 -> 6.3).
+template <int P>
+bool takes_few(const RotQuantArgs &a) {
+    return P < 44 && a.K <= 5120 && (a.M > 2 * kPlanUnits || P == 20);
+}
+
 // LDS: one padded row (two when the Paley stage is sliced over more threads) plus the group ranges. Slicing buys
 // parallelism inside a token and costs occupancy, so it is for small batches only.
 template <int P>
@@ -455,6 +467,7 @@ hipError_t launch_p(const RotQuantArgs &a, hipStream_t stream) {
     if (sliced) return launch_one<P, (P > 1)>(a, 2 * row + stats, stream);
     // a second workgroup does not fit beside this one
     if (has_alone(P) && 2 * (row + stats + 64) > 160 * 1024) return launch_one<P, false, false, has_alone(P)>(a, row + stats, stream);
+    if (takes_few<P>(a)) return launch_one<P, false, false, false, (P < 44)>(a, row + stats, stream);
     return launch_one<P, false>(a, row + stats, stream);
 }
 
