@@ -243,8 +243,9 @@ __device__ __forceinline__ int padi(int i) { return i + (i >> 4); }
 // One pass of the Sylvester transform: R = 2^LR elements `1 << ls` apart go through LR butterfly stages in
 // registers (strides 1 << ls, 2 << ls, ...; lower index gets a + b, upper a - b, as reference lines 2454-2464).
 // Successive passes run in ascending stride order, so every element sees the reference's stage order.
-template <int LR>
-__device__ __forceinline__ void fwht_pass(float *buf, int K, int lm, int ls, int tid, int nt) {
+// SCALED: every value is multiplied by `scale` on its way out.
+template <int LR, bool SCALED = false>
+__device__ __forceinline__ void fwht_pass(float *buf, int K, int lm, int ls, int tid, int nt, float scale = 1.0f) {
     constexpr int R = 1 << LR;
     const int units = K >> LR;
     for (int u = tid; u < units; u += nt) {
@@ -266,7 +267,7 @@ __device__ __forceinline__ void fwht_pass(float *buf, int K, int lm, int ls, int
             }
         }
 #pragma unroll
-        for (int j = 0; j < R; ++j) buf[padi(base + (j << ls))] = v[j];
+        for (int j = 0; j < R; ++j) buf[padi(base + (j << ls))] = SCALED ? v[j] * scale : v[j];
     }
 }
 
@@ -509,10 +510,23 @@ __device__ __forceinline__ void paley_row(float *buf, int K, int m, int n_rot, f
 }
 
 // all Sylvester stages from stride 1 << ls0 up of every chunk of m = 1 << lm floats of a padded row, four stages per
-// trip through LDS
-__device__ __forceinline__ void fwht_row(float *buf, int K, int lm, int tid, int nt, int ls0 = 0) {
+// trip through LDS. SCALED: the row times `scale`, in the last of the trips.
+template <bool SCALED = false>
+__device__ __forceinline__ void fwht_row(float *buf, int K, int lm, int tid, int nt, int ls0 = 0, float scale = 1.0f) {
+    if (SCALED && ls0 >= lm) {
+        for (int i = tid; i < K; i += nt) buf[padi(i)] = buf[padi(i)] * scale;
+        __syncthreads();
+    }
     for (int ls = ls0; ls < lm;) {
         const int lr = lm - ls < 4 ? lm - ls : 4;
+        if (SCALED && ls + lr == lm) {
+            if (lr == 4) fwht_pass<4, true>(buf, K, lm, ls, tid, nt, scale);
+            else if (lr == 3) fwht_pass<3, true>(buf, K, lm, ls, tid, nt, scale);
+            else if (lr == 2) fwht_pass<2, true>(buf, K, lm, ls, tid, nt, scale);
+            else fwht_pass<1, true>(buf, K, lm, ls, tid, nt, scale);
+            __syncthreads();
+            break;
+        }
         if (lr == 4) fwht_pass<4>(buf, K, lm, ls, tid, nt);
         else if (lr == 3) fwht_pass<3>(buf, K, lm, ls, tid, nt);
         else if (lr == 2) fwht_pass<2>(buf, K, lm, ls, tid, nt);

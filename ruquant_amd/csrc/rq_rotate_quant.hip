@@ -151,8 +151,10 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     // (small batches, bound by the latency of its phases) the next four ride too, between lanes, when the chunks are
     // made of blocks of 256 floats; large batches are bound by vector-ALU time, where the LDS pass is the cheaper
     // one (2048 tokens at K = 17408: 105 us against 128 us with the stages between lanes).
+    // Without a Paley stage that holds up to a token per compute unit: together with the scale in the last trip, activation stage
+    // at 16 / 200 tokens, K = 1024 4.1 -> 3.9 / 4.4 -> 4.1 us, 4096 5.3 -> 4.7 / 5.5 -> 4.9, 8192 7.8 -> 6.8 / 7.9 -> 6.8.
     const bool fused_first = a.rotate && (a.m & 15) == 0;
-    const bool fused_256 = SLICED && a.rotate && (a.m & 255) == 0;
+    const bool fused_256 = (SLICED || (P == 1 && a.M <= kPlanUnits)) && a.rotate && (a.m & 255) == 0;
     if (fused_256) {
         load_row_fwht256<kNT, (P >= 44 ? 3 : 1)>(buf, xr, K, tid);
     } else if (fused_first) {
@@ -167,7 +169,9 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     if (a.rotate) {
         const int m = a.m;
         const int lm = __ffs(m) - 1;
-        fwht_row(buf, K, lm, tid, kNT, fused_256 ? 8 : fused_first ? 4 : 0);
+        const int ls0 = fused_256 ? 8 : fused_first ? 4 : 0;
+        if constexpr (P > 1) fwht_row(buf, K, lm, tid, kNT, ls0);
+        else fwht_row<true>(buf, K, lm, tid, kNT, ls0, a.scale);   // (no Paley stage: the scale in its place)
         if constexpr (P > 1) {
             // Paley across the P chunks of every rotation block (reference lines 2466-2482), then the scale
             const int ncols = K / P;  // columns of all rotation blocks of this token
@@ -229,9 +233,6 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
                 }
                 __syncthreads();
             }
-        } else {
-            for (int i = tid; i < K; i += kNT) buf[padi(i)] = buf[padi(i)] * a.scale;
-            __syncthreads();
         }
     }
 
