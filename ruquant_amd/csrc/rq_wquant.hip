@@ -5,8 +5,9 @@
 // operations matters is the double-precision error sum of the scale search, and of it only which of the thirteen clip ratios
 // has the smallest is kept. So the sums are taken in fp32 first, over all lanes and in any order, with a bound on what that
 // can change; where the smallest two are further apart than the bound allows, the reference's sums are too, and the search is
-// over. Where they are not (a row in a hundred), the same again in double precision, and only where that cannot tell either
-// (ties, infinities, NaNs, scales out of range) do lanes add up the reference's sums in its element order:
+// over. Where they are not (a row in a hundred of gaussian weights), the same again in double precision, and only where that cannot
+// tell either (ties, infinities, NaNs, scales out of range) do lanes add up the reference's sums in its element order. A tensor that
+// lies on an int4 grid (one that was dequantized) has a ratio without any error: settled at once.
 //   * search kernels: a workgroup per row, or sixteen lanes per weight group of 256 or 64;
 //   * encode kernel: a workgroup per row turns the chosen scale(s) into codes, row sum / multiplier headers and
 //     blocks;
@@ -49,18 +50,20 @@ struct SearchArgs {
 // What the fp32 sums may be off by, relative to the exact sum of the reference's squares. The quotient t = x * (1 / s) differs
 // from x / s by less than 8e-6 (|x / s| is at most 10), so a code differs from the reference's only where x / s is that near
 // to a half-way point; its error then is (0.5 +- 9e-6) s either way, and the square off by 7.2e-5 of itself. The errors
-// themselves and their squares are rounded as the reference's or once (6e-8), and a thread adds up at most 128 of them and 12
-// sums: 8.5e-6. Together below 8.2e-5; the reference's own rounding (32768 additions in double precision, 4e-12) is nothing to
-// that. Two sums can have their order changed only if they are within (1 + 8.2e-5) / (1 - 8.2e-5) of each other.
+// themselves and their squares are rounded as the reference's or once (6e-8), and a sum goes through at most 148 additions: 128
+// elements of a thread, four steps over its row of sixteen lanes, sixteen such rows: 8.9e-6. Together below 8.2e-5; the reference's
+// own rounding (32768 additions in double precision, 4e-12) is nothing to that. Two sums can have their order changed only if they
+// are within (1 + 8.2e-5) / (1 - 8.2e-5) of each other.
 constexpr float kApart = 1.0f + 1.7e-4f;
+// ... and squares below the normal numbers lose at most half of the smallest denormal each, 32768 of them 2.3e-41, in either sum. (A
+// sum of zero, of a row that lies on the grid of one of the ratios, is told from the others by this alone.)
+constexpr float kUnderflow = 1e-40f;
 // The double-precision sums of the second look have the reference's terms and at most 400 roundings, the reference's own sums at
-// most 32768: 3.7e-12 and 4.5e-14.
+// most 32768: 3.7e-12 and 4.5e-14. (No square of a difference of floats underflows there: a sum is zero where every term is.)
 constexpr double kApart64 = 1.0 + 1e-11;
-// (below this the squares may be denormal, which the bound does not cover)
-constexpr float kLeast = 1e-30f;
 
 __device__ __forceinline__ float ratio_scale(float amax, int r) { return amax * (1.0f - 0.025f * (float) r) / 7.0f; }
-// what stands in place of a scale that these sums leave open, for rq_wsearch_kernel
+// what stands in place of a scale that these sums leave open, for rq_wsearch_open_kernel
 constexpr float kOpen = -1.0f;
 __device__ __forceinline__ bool reciprocal_holds(float rs) { return rs < 1e37f && rs > 2e-38f; }
 
@@ -88,6 +91,8 @@ __device__ __forceinline__ float row_sum(float v) {
     return dpp_add<0x140>(v);   // row_mirror
 }
 
+// a sum above this is larger than the smallest one in the reference's sums too
+__device__ __forceinline__ float bound_of(float least) { return __builtin_fmaf(least, kApart, kUnderflow); }
 // whether the smallest of the sums is the smallest in the reference's sums too (not with a NaN or an infinity among them)
 __device__ __forceinline__ bool settled(const float (&sum)[kRatios], float &least) {
     float second = INFINITY, all = sum[0];
@@ -98,12 +103,13 @@ __device__ __forceinline__ bool settled(const float (&sum)[kRatios], float &leas
         least = fminf(least, sum[r]);
         all += sum[r];
     }
-    return second > least * kApart && least > kLeast && all < INFINITY;
+    return second > bound_of(least) && all < INFINITY;
 }
 
 // Weight groups of 256 (V = 4) or 64 (V = 1): sixteen lanes per group, V blocks of 64 elements in their registers.
 // What bounds it: vector instructions, six per element and ratio. Search and encoding of 4096 x 17408, groups of 64, with a lane per
-// ratio and the sums in order from the start 402 us, this way 306 (search 250); groups of 256 299 and 217 (134).
+// ratio and the sums in order from the start 402 us, this way 306 (search 250); groups of 256 299 and 217 (134). 6144 x 5120 on a
+// grid, groups of 64: in order 329 us, this way 129 (430 while a sum of zero was left to the search in order); of 256 298, 91 (423).
 template <int V>
 __global__ void __launch_bounds__(kSearchThreads, 4) rq_wsearch_groups_kernel(const SearchArgs a) {
     const int tid = threadIdx.x, r = tid & 15;
@@ -157,18 +163,46 @@ __global__ void __launch_bounds__(kSearchThreads, 4) rq_wsearch_groups_kernel(co
         scale = 0.0f;
         sure = true;
     }
+    // Two ratios without an error, or one and squares that underflow (a group with one value, negative, beside zeros is on the grid
+    // of the first ratio and of the sixth): the first whose errors are all zero, as the reference's sum then is, and of no ratio
+    // before it. (No quotient at a half-way point has an error of zero, so its code is the reference's.)
+    if (!sure && least == 0.0f && reciprocal_holds(rs[0]) && reciprocal_holds(rs[kRatios - 1])) {
+#pragma unroll 1
+        for (int i = 0; i < kRatios && !sure; ++i) {   // (the same for all lanes of the group)
+            const float si = __shfl(s, i, 16), ri = __shfl(inv, i, 16);
+            float worst = 0.0f;
+#pragma unroll 1
+            for (int k = 0; k < V; ++k) {
+                const float4 y = reinterpret_cast<const float4 *>(x)[16 * k + r];
+                const float ys[4] = { y.x, y.y, y.z, y.w };
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    worst = fmaxf(worst, fabsf(__builtin_amdgcn_fmed3f(rintf(ys[j] * ri), -8.0f, 7.0f) * si - ys[j]));
+                }
+            }
+#pragma unroll
+            for (int off = 8; off > 0; off >>= 1) worst = fmaxf(worst, __shfl_xor(worst, off, 16));
+            if (worst == 0.0f) {
+                scale = si;
+                sure = true;
+            }
+        }
+    }
     if (live && r == 0) a.scale[seg] = sure ? scale : kOpen;
 }
 
-// Few groups go to the search in order at once: its one launch is as long as the two that spare it. Search and encoding, 1024
-// inputs, in order / this way, groups of 64: 1024 rows 12.1 / 13.8 us, 2048 17.5 / 18.2, of 256: 1024 13.7 / 17.2, 2048 16.6 / 19.7,
-// 4096 28.4 / 26.9.
-constexpr int64_t kFewFloats = 3 << 20;
+// Few groups go to the search in order at once: its one launch is as long as the two that spare it. Search and encoding of K = 256 /
+// 1024 / 5120 gaussian inputs in us, in order -> this way: groups of 256 (at K = 256 whole rows), 3.2 Mi floats 31.4 -> 32.7 / 24.4 ->
+// 25.6 / 23.8 -> 25.4, 4.6 Mi 41.2 -> 42.1 / 29.3 -> 30.5 / 28.7 -> 30.0, 6 Mi 50.0 -> 49.2 / 34.8 -> 35.3 / 34.1 -> 33.5; of 64, 2.6 Mi
+// 26.9 -> 27.5 / 21.1 -> 21.5 / 20.9 -> 21.7, 3.2 Mi 31.5 -> 31.3 / 24.6 -> 24.5 / 23.9 -> 24.0, 4.6 Mi 42.8 -> 42.1 / 34.2 -> 33.0 / 32.4 ->
+// 31.3. (Tensors on a grid are faster this way from the first row on: in order their quotients lie at half-way points, and lanes divide.)
+constexpr int64_t few_floats(int n) { return n == 64 ? 7 << 19 : 5 << 20; }
 
 // Rows: a workgroup each, which reads its row twice (the second time out of the caches).
 // What bounds it: vector instructions, six per element and ratio (four of them of two cycles, beside a second wavefront).
 // Search and encoding, 5120 inputs, with four rows per wavefront, a lane per ratio and the sums in order from the start: 2048 rows
-// 137 us, 4096 173, 6144 187; this way 39, 63, 85 (search of 4096: 45). 17408 inputs, 1800 rows 441 and 97.
+// 137 us, 4096 173, 6144 187; this way 39, 63, 85 (search of 4096: 45). 17408 inputs, 1800 rows 441 and 97. 6144 x 5120 on a grid:
+// in order 441, this way 86 (495 while a sum of zero was left open).
 constexpr int kRowThreads = 256;
 __global__ void __launch_bounds__(kRowThreads) rq_wsearch_rows_kernel(const SearchArgs a) {
     __shared__ float s_sum[kRowThreads / 16][kRatios];   // per row of sixteen lanes
@@ -252,11 +286,11 @@ __global__ void __launch_bounds__(kRowThreads) rq_wsearch_rows_kernel(const Sear
     bool finite = normal;
 #pragma unroll
     for (int r = 0; r < kRatios; ++r) finite = finite && sum[r] < INFINITY;
-    if (finite && least > kLeast) {
+    if (finite) {
         double err64[2] = { INFINITY, INFINITY };   // the smallest and the second smallest
         int arg = 0;
         for (int r = 0; r < kRatios; ++r) {
-            if (s_all[r] > least * kApart) continue;   // (uniform)
+            if (s_all[r] > bound_of(least)) continue;   // (uniform)
             const float s = s_sc[r], inv = s_rs[r];
             double err = 0.0;
             for (int i = tid; i < nv; i += kRowThreads) {
@@ -285,7 +319,7 @@ __global__ void __launch_bounds__(kRowThreads) rq_wsearch_rows_kernel(const Sear
                 err64[1] = err;
             }
         }
-        if (err64[1] > err64[0] * kApart64) {
+        if (err64[1] > err64[0] * kApart64 || err64[0] == 0.0) {   // (of ratios without any error the first)
             if (tid == 0) a.scale[blockIdx.x] = s_sc[arg];
             return;
         }
@@ -293,31 +327,14 @@ __global__ void __launch_bounds__(kRowThreads) rq_wsearch_rows_kernel(const Sear
     if (tid == 0) a.scale[blockIdx.x] = kOpen;
 }
 
-// The reference's search, for the segments that the kernels above left open: sixteen lanes per segment, thirteen of them try one
-// ratio each over the whole segment in element order, and a scan in ratio order keeps the first smallest error. A wavefront looks
-// through CHUNK segments and takes the open ones four at a time.
+// The reference's search: sixteen lanes per segment, thirteen of them try one ratio each over the whole segment in element order, and
+// a scan in ratio order keeps the first smallest error. (Lanes that are not live follow a live segment, so that the shuffles stay
+// uniform.)
 // ONE: segments of 64 (a scale per 64 inputs), one block each: nothing to fetch ahead and no eight loads to batch. (With the
 // general form's, which fetch the one block again: 4096 x 17408, search and encoding, 450 us against 402.)
-// (ALL: every segment, whatever stands in place of its scale)
-template <bool ONE, int CHUNK, bool ALL = false>
-__global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const SearchArgs a) {
-    __shared__ float4 s_x[ONE ? 1 : 2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
+template <bool ONE>
+__device__ __forceinline__ void search_in_order(const SearchArgs &a, int64_t seg, bool live, float4 (&s_x)[ONE ? 1 : 2][kSearchThreads]) {
     const int tid = threadIdx.x, r = tid & 15;
-    const int64_t seg0 = (int64_t) blockIdx.x * CHUNK;
-    const bool mine = tid < CHUNK && seg0 + tid < a.segments;
-    uint64_t open = __ballot(mine && (ALL || a.scale[seg0 + (mine ? tid : 0)] < 0.0f));
-  while (open != 0) {
-    // the first four; a row of lanes without one follows the first
-    int64_t seg = seg0 + __builtin_ctzll(open);
-    bool live = false;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (open != 0 && k == tid >> 4) {
-            seg = seg0 + __builtin_ctzll(open);
-            live = true;
-        }
-        open &= open - 1;   // (zero stays zero)
-    }
     const int64_t row = seg / a.per_row;
     const float *x = a.x + row * a.ld + (seg - row * a.per_row) * (int64_t) a.n;
     const int n = a.n;
@@ -425,7 +442,40 @@ __global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const Search
         }
     }
     if (live && r == 0) a.scale[seg] = best_s;
-  }
+}
+
+// every segment
+template <bool ONE>
+__global__ void __launch_bounds__(kSearchThreads) rq_wsearch_kernel(const SearchArgs a) {
+    __shared__ float4 s_x[ONE ? 1 : 2][kSearchThreads];   // two blocks of 64 elements of each of the four segments
+    const int64_t seg = (int64_t) blockIdx.x * (kSearchThreads / 16) + (threadIdx.x >> 4);
+    const bool live = seg < a.segments;
+    search_in_order<ONE>(a, live ? seg : a.segments - 1, live, s_x);
+}
+
+// The segments that the kernels above left open: a wavefront looks through CHUNK segments and takes the open ones four at a time. (A
+// wavefront for 64 groups: with 16 the look alone costs gaussian tensors 2 to 3 %, 6144 x 5120, groups of 64, 134.8 -> 139.1 us.)
+template <bool ONE, int CHUNK>
+__global__ void __launch_bounds__(kSearchThreads) rq_wsearch_open_kernel(const SearchArgs a) {
+    __shared__ float4 s_x[ONE ? 1 : 2][kSearchThreads];
+    const int tid = threadIdx.x;
+    const int64_t seg0 = (int64_t) blockIdx.x * CHUNK;
+    const bool mine = tid < CHUNK && seg0 + tid < a.segments;
+    uint64_t open = __ballot(mine && a.scale[seg0 + (mine ? tid : 0)] < 0.0f);
+    while (open != 0) {
+        // the first four; a row of lanes without one follows the first
+        int64_t seg = seg0 + __builtin_ctzll(open);
+        bool live = false;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (open != 0 && k == tid >> 4) {
+                seg = seg0 + __builtin_ctzll(open);
+                live = true;
+            }
+            open &= open - 1;   // (zero stays zero)
+        }
+        search_in_order<ONE>(a, seg, live, s_x);
+    }
 }
 
 struct EncodeArgs {
@@ -726,18 +776,18 @@ int rq_w4a4_quantize_weights(int type, const float *w_dev, int64_t ldw, int64_t 
     s.scale = reinterpret_cast<float *>(base + ws.off_scale);
     auto blocks_of = [&](int64_t per) { return dim3((unsigned) ((s.segments + per - 1) / per)); };
     // (the kernels that decide nearly all of them, then the one for what they leave open)
-    if (s.n <= 256 && N * K <= kFewFloats) {
-        if (s.n == 64) hipLaunchKernelGGL((rq_wsearch_kernel<true, 4, true>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
-        else hipLaunchKernelGGL((rq_wsearch_kernel<false, 4, true>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
+    if (s.n <= 256 && N * K <= few_floats(s.n)) {
+        if (s.n == 64) hipLaunchKernelGGL(rq_wsearch_kernel<true>, blocks_of(kSearchThreads / 16), dim3(kSearchThreads), 0, st, s);
+        else hipLaunchKernelGGL(rq_wsearch_kernel<false>, blocks_of(kSearchThreads / 16), dim3(kSearchThreads), 0, st, s);
     } else if (s.n == 64) {
         hipLaunchKernelGGL((rq_wsearch_groups_kernel<1>), blocks_of(kSearchThreads / 16), dim3(kSearchThreads), 0, st, s);
-        hipLaunchKernelGGL((rq_wsearch_kernel<true, 64>), blocks_of(64), dim3(kSearchThreads), 0, st, s);
+        hipLaunchKernelGGL((rq_wsearch_open_kernel<true, 64>), blocks_of(64), dim3(kSearchThreads), 0, st, s);
     } else if (s.n == 256) {
         hipLaunchKernelGGL((rq_wsearch_groups_kernel<4>), blocks_of(kSearchThreads / 16), dim3(kSearchThreads), 0, st, s);
-        hipLaunchKernelGGL((rq_wsearch_kernel<false, 64>), blocks_of(64), dim3(kSearchThreads), 0, st, s);
+        hipLaunchKernelGGL((rq_wsearch_open_kernel<false, 64>), blocks_of(64), dim3(kSearchThreads), 0, st, s);
     } else {
         hipLaunchKernelGGL(rq_wsearch_rows_kernel, dim3((unsigned) N), dim3(kRowThreads), 0, st, s);
-        hipLaunchKernelGGL((rq_wsearch_kernel<false, 4>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
+        hipLaunchKernelGGL((rq_wsearch_open_kernel<false, 4>), blocks_of(4), dim3(kSearchThreads), 0, st, s);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int) e;

@@ -163,8 +163,15 @@ def test_full_size_tensor_sampled_rows(oracle):
     assert blocks_equal(blocks[sample], want), block_diff(blocks[sample], want)
 
 
-@pytest.mark.parametrize("K,wgroup", [(256, 0), (1536, 0), (1536, 64), (1280, 256)])
-def test_search_at_rounding_boundaries_and_extreme_scales(oracle, K, wgroup):
+def repeated(rows, N):
+    return np.tile(rows, (-(-N // len(rows)),) + (1,) * (rows.ndim - 1))[:N]
+
+
+# (groups of 256 and 64, and rows of 256, are searched in element order up to 5 or 3.5 Mi floats and by fp32 sums above that; more
+# segments than a multiple of four leave lanes of the last wavefront without one)
+@pytest.mark.parametrize("K,wgroup,N", [(256, 0, 12), (1536, 0, 12), (1536, 64, 12), (1280, 256, 12),
+                                        (256, 0, 20501), (1536, 64, 2731), (1280, 256, 4101)])
+def test_search_at_rounding_boundaries_and_extreme_scales(oracle, K, wgroup, N):
     """The clip search takes the correctly rounded quotient only where x * (1 / s) is near a half-way point or 1 / s is
     no normal number: rows full of exact ties and of values one step beside them, rows of denormals, of the largest
     floats, with an infinity, and ordinary ones."""
@@ -183,9 +190,63 @@ def test_search_at_rounding_boundaries_and_extreme_scales(oracle, K, wgroup):
     w[9] = (rng.standard_normal(K) * 1e37).astype(f32)
     w[10, 5] = np.inf
     w[11] = rng.standard_normal(K).astype(f32)
-    got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4, wgroup=wgroup)
-    want = oracle.quantize_rows_w(w, wgroup=wgroup)
+    got = rq.quantize_weights(torch.from_numpy(repeated(w, N)).to(DEV), rq.TYPE_W4A4, wgroup=wgroup)
+    want = repeated(oracle.quantize_rows_w(w, wgroup=wgroup), N)
     assert blocks_equal(got, want), block_diff(got, want)
+
+
+def grid_rows(kind, N, K, rng):
+    """Rows on an int4 grid: `seven` with 7 as the largest code (the first ratio reproduces them), `eight` with -8 (the sixth does),
+    `ternary`, and `negative` from {-1, 0} (both do)."""
+    c = rng.integers(-7, 8, size=(N, K)).astype(f32)
+    if kind == "seven":
+        c[:, ::64] = 7.0
+    elif kind == "eight":
+        c[:, ::64] = -8.0
+    elif kind == "ternary":
+        c = np.sign(c)
+    else:
+        c = -(c > 0).astype(f32)
+    return c * np.abs(rng.normal(0.02, 0.005, size=(N, 1))).astype(f32)
+
+
+@pytest.mark.parametrize("K,wgroup,N", [(256, 0, 20501), (1280, 0, 48), (1280, 256, 4101), (1536, 64, 2731)])
+def test_tensors_on_the_grid(oracle, K, wgroup, N):
+    """Ratios without any error, one or two of them, and such rows where squares underflow in fp32: scaled down, or with an element so
+    small that only the reference's sums see it."""
+    rng = np.random.default_rng(K + wgroup)
+    kinds = [grid_rows(kind, 3, K, rng) for kind in ("seven", "eight", "ternary", "negative")]
+    w = np.concatenate(kinds + [k * f32(1e-15) for k in kinds] + [k * f32(1e-25) for k in kinds] + kinds)
+    w[36:, 1::64] = f32(1e-24)
+    got = rq.quantize_weights(torch.from_numpy(repeated(w, N)).to(DEV), rq.TYPE_W4A4, wgroup=wgroup)
+    want = repeated(oracle.quantize_rows_w(w, wgroup=wgroup), N)
+    assert blocks_equal(got, want), block_diff(got, want)
+
+
+@pytest.mark.parametrize("K,N,wgroup", [(256, 32768, 0), (5120, 4096, 0), (5120, 4096, 256), (5120, 4096, 64)])
+def test_tensors_on_the_grid_need_no_search_in_order(K, N, wgroup):
+    """Converting a dequantized tensor again takes about as long as converting any other one (three to seven times as long where
+    every segment goes to the search in element order behind the fp32 sums)."""
+    L = rq.load_library()
+    ws = torch.empty(L.rq_w4a4_quantize_weights_workspace_bytes(rq.TYPE_W4A4, K, N, wgroup), dtype=torch.uint8, device=DEV)
+    out = torch.empty(N * (K // 256) * 144, dtype=torch.uint8, device=DEV)
+    rng = np.random.default_rng(3)
+    us = []
+    for w in (rng.normal(0, 0.02, size=(N, K)).astype(f32), grid_rows("seven", N, K, rng), grid_rows("ternary", N, K, rng)):
+        w = torch.from_numpy(w).to(DEV)
+        times = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(10):
+                assert L.rq_w4a4_quantize_weights(rq.TYPE_W4A4, w.data_ptr(), K, N, K, K, wgroup, out.data_ptr(),
+                                                  ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1) * 100)
+        us.append(min(times))
+    print("K=%d N=%d wgroup=%d: %.0f us, on the grid %.0f, %.0f" % ((K, N, wgroup) + tuple(us)), flush=True)
+    assert max(us[1:]) < 2 * us[0]
 
 
 def test_conversions_in_several_runs(oracle):
@@ -305,7 +366,7 @@ def test_scales_that_the_first_look_leaves_open(oracle, wgroup):
     """Enough segments that some (one in a hundred or fewer) have two ratios whose errors are too near for the fp32 sums, and rows
     that those sums do not cover: sums of zero, denormal ones, infinite ones, infinities, NaNs, scales out of range; the last
     wavefront is not full. Every byte as from the reference's sums in its order."""
-    N, K = 3202, 1024
+    N, K = 5202, 1024
     w = tensor(N, K, 11 + wgroup)
     rng = np.random.default_rng(wgroup)
     for r, scale in enumerate([1e-38, 1e-30, 1e-20, 1e18, 1e37]):
