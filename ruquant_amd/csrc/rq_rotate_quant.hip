@@ -450,10 +450,22 @@ bool takes_wide(const RotQuantArgs &a, bool sliced) {
 // 256 have a column, 160 quantize), and five tokens instead of three share a compute unit. Activation stage in us, 512 threads ->
 // 256: 700 tokens K = 1024 5.0 -> 4.8, 4096 7.6 -> 7.6, 5120 9.6 -> 8.2; 2048 tokens K = 1024 9.7 -> 6.4, 1536 10.3 -> 6.6, 3072 13.1 ->
 // 9.5, 4096 15.9 -> 13.2, 5120 21.9 -> 18.3, 6144 21.3 -> 22.1, 8192 27.2 -> 30.2. Up to two tokens per compute unit each has as many
-// as it can use (400 tokens, K = 4096 6.3 -> 6.6), but p = 20, which spills with 512, 7.3 -> 7.1 (256 tokens 6.5 -> 6.3).
+// as it can use (400 tokens, K = 4096 6.3 -> 6.6), but for p = 20, which spills with 512:
+// - in front of the fp6 product, whose quantizer has a thread per 32 values: K = 5120 400 tokens 7.3 -> 7.1, 256 6.5 -> 6.3. Always.
+// - the other quantizers have one per 8 and use all 512: A4H blocks, 65 / 257 / 512 tokens, K = 2560 5.33 -> 5.71 / 5.76 -> 5.95 / 6.31 ->
+//   6.34, K = 5120 6.17 -> 7.07 / 7.07 -> 7.73 / 7.98 -> 8.24. Not, but in rows too short for that (K = 1280 4.89 -> 4.81 / 5.30 -> 5.05 /
+//   5.69 -> 5.28) and in chunks too short for the columns' fixed strides (rotation blocks of 20, K = 5120 6.07 -> 6.13 / 7.4 -> 6.9 / 8.1
+//   -> 7.2).
+// - the rotation alone, K = 5120, 65 / 257 / 400 / 512 tokens: 4.5 -> 5.0 / 5.6 -> 5.8 / 6.4 -> 6.5 / 6.9 -> 6.9, in blocks of 2560 4.6 ->
+//   4.9 / 5.7 -> 5.7 / 6.6 -> 6.3 / 7.1 -> 6.6, of 320 3.9 -> 4.0 / 4.9 -> 4.6 / 5.7 -> 5.3 / 6.2 -> 5.7: those short ones, blocks of 320,
+//   and from one and a half tokens per compute unit up.
 template <int P>
 bool takes_few(const RotQuantArgs &a) {
-    return P < 44 && a.K <= 5120 && (a.M > 2 * kPlanUnits || P == 20);
+    if (P >= 44 || a.K > 5120) return false;
+    if (a.M > 2 * kPlanUnits) return true;
+    if (P != 20) return false;
+    if (a.mode == kActI8 && a.single == 2) return true;
+    return a.K <= 1280 || a.m < 16 || (a.mode == kActRotateOnly && (a.m == 16 || 2 * a.M > 3 * kPlanUnits));
 }
 
 // LDS: one padded row (two when the Paley stage is sliced over more threads) plus the group ranges. Slicing buys
