@@ -510,13 +510,9 @@ __device__ __forceinline__ void paley_row(float *buf, int K, int m, int n_rot, f
 }
 
 // all Sylvester stages from stride 1 << ls0 up of every chunk of m = 1 << lm floats of a padded row, four stages per
-// trip through LDS. SCALED: the row times `scale`, in the last of the trips.
+// trip through LDS. SCALED: the row times `scale`, in the last of the trips (there is one: ls0 < lm).
 template <bool SCALED = false>
 __device__ __forceinline__ void fwht_row(float *buf, int K, int lm, int tid, int nt, int ls0 = 0, float scale = 1.0f) {
-    if (SCALED && ls0 >= lm) {
-        for (int i = tid; i < K; i += nt) buf[padi(i)] = buf[padi(i)] * scale;
-        __syncthreads();
-    }
     for (int ls = ls0; ls < lm;) {
         const int lr = lm - ls < 4 ? lm - ls : 4;
         if (SCALED && ls + lr == lm) {

@@ -155,7 +155,8 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     // at 16 / 200 tokens, K = 1024 4.1 -> 3.9 / 4.4 -> 4.1 us, 4096 5.3 -> 4.7 / 5.5 -> 4.9, 8192 7.8 -> 6.8 / 7.9 -> 6.8.
     const bool fused_first = a.rotate && (a.m & 15) == 0;
     const bool fused_256 = (SLICED || (P == 1 && a.M <= kPlanUnits)) && a.rotate && (a.m & 255) == 0;
-    if (fused_256) {
+    // (out of the other rows' way: in front of them this code costs a call without a rotation 0.1 us: 2 tokens, K = 2048 2.58 -> 2.68)
+    if (SLICED ? fused_256 : __builtin_expect(fused_256, 0)) {
         load_row_fwht256<kNT, (P >= 44 ? 3 : 1)>(buf, xr, K, tid);
     } else if (fused_first) {
         // long Paley stages go with long rows (several units of 16 floats per thread): all of a thread's loads go
@@ -171,7 +172,11 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
         const int lm = __ffs(m) - 1;
         const int ls0 = fused_256 ? 8 : fused_first ? 4 : 0;
         if constexpr (P > 1) fwht_row(buf, K, lm, tid, kNT, ls0);
-        else fwht_row<true>(buf, K, lm, tid, kNT, ls0, a.scale);   // (no Paley stage: the scale in its place)
+        else if (ls0 < lm) fwht_row<true>(buf, K, lm, tid, kNT, ls0, a.scale);   // (no Paley stage: the scale in its place)
+        else {   // (every stage was on the load: a pass for the scale, here, where blocks of 16 reach it 0.1 us earlier)
+            for (int i = tid; i < K; i += kNT) buf[padi(i)] = buf[padi(i)] * a.scale;
+            __syncthreads();
+        }
         if constexpr (P > 1) {
             // Paley across the P chunks of every rotation block (reference lines 2466-2482), then the scale
             const int ncols = K / P;  // columns of all rotation blocks of this token
@@ -245,7 +250,8 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
         return;
     }
 
-    if (a.mode == kActI8 && a.single == 2) {
+    // (behind the other forms: laid out in front of them it makes the plain form of p = 20, whose columns spill, 4.5 % slower in all)
+    if (__builtin_expect(a.mode == kActI8 && a.single == 2, 0)) {
         quantize_fp6<kNT>(a, buf, g_lo, g_hi, s_red, t, tid);
         return;
     }
