@@ -233,7 +233,7 @@ Choice choose(int n, int64_t K, const int64_t *N, int64_t M, bool rotate, int p,
         panels += (N[i] + kPanelRows - 1) / kPanelRows;
         any |= mult[i];
         if (s.one_launch && i < n - 1) continue;
-        c.small6 = block6_takes(panels, M, (int) (K / kGroup), any);
+        c.small6 = block6_takes(panels, M, (int) (K / kGroup), any, rotate);
         panels = 0;
         any = false;
     }

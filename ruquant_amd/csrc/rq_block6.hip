@@ -429,7 +429,14 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 // and at most 6 % slower from memory. (64 tokens, whole call in us, skinny / here; in front from the cache, behind from memory.)
 // - Up to 64 panels, a unit in four pieces: K = 1024, N = 4096 8.8 / 8.1, 9.4 / 8.9 (40 tokens); K = 5120, N = 1024 11.6 / 10.4,
 //   12.6 / 12.2, N = 4096 14.1 / 10.4, 15.6 / 13.5; K = 10240 21.6 / 14.2, 23.4 / 18.8; K = 17408, N = 1024 20.2 / 18.6, 22.0 / 25.1,
-//   N = 4096 27.3 / 19.7, 28.6 / 27.0; K = 32768, N = 1024 28.7 / 30.3, 28.6 / 40.0. Here up to K = 10240.
+//   N = 4096 27.3 / 19.7, 28.6 / 27.0; K = 32768, N = 1024 28.7 / 30.3, 28.6 / 40.0. Here up to K = 10240, but for a few panels of
+//   rows that long, where the skinny kernel has slices along K instead and the fp6 quantizer, a thread per 32 values, takes longer
+//   (33 / 64 tokens, here as a part of the skinny kernel's time, cache; memory): K = 5632 at most 1.01; K = 6144 N = 256 1.01 / 1.00;
+//   1.05 / 1.05, N = 512 1.00 / 1.00; 1.07 / 1.05, N = 768 0.98 / 0.95; 1.02 / 1.00, N = 1024 0.99 / 0.95; 1.03 / 1.00; K = 8192
+//   N = 256 0.99 / 0.97; 1.03 / 1.02, N = 512 0.96 / 0.93; 1.02 / 0.99. Without a rotation, whose launch hides some of that: K = 6144
+//   N = 512 0.99 / 1.00; 1.08 / 1.07, K = 8192 N = 256 1.09 / 1.05; 1.12 / 1.11, N = 1024 1.03 / 0.95; 1.05 / 1.00, N = 1536 0.94 / 0.90; 1.03 /
+//   1.02, K = 9216 N = 512 1.04 / 1.03; 1.09 / 1.05, N = 1536 0.91 / 0.87; 0.97 / 0.94. K = 10240 is the skinny kernel's second step: N = 256
+//   1.01 / 0.91; 1.06 / 0.96 (48 tokens 0.99; 1.02), N = 512 0.99 / 0.88; 1.04 / 0.91, N = 768 0.96 / 0.85; 0.97 / 0.86.
 // - 65 to 128 panels (half the chip: the skinny kernel has two workgroups of 32 tokens a panel): K = 5120, N = 8192 14.8 / 15.0,
 //   16.1 / 19.6; K = 17408, N = 8192 47.6 / 39.4, 38.4 / 46.6. The skinny kernel.
 // - 129 to 256 panels, a round of units, and two of the skinny kernel's: N = 12288, K = 1024 15.6 / 9.5, 16.3 / 10.9; K = 5120
@@ -443,9 +450,13 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 //   at 33 tokens); N = 12288, K = 5120 29.7 / 18.9, 31.2 / 22.4, K = 32768 128 / 91, 128 / 95; N = 17408, K = 17408 86 / 71, 87 / 91,
 //   K = 32768 145 / 160. Here from K = 3072 to 10240 with 96 panels, any length in one round of units, up to K = 17408 beyond.
 // 33 tokens are within a tenth of 64 on both sides.
-bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers) {
+bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers, bool rotate) {
     if (M <= 32) return false;
-    if (n_panels <= kPlanUnits / 4) return ng <= 160;
+    if (n_panels <= kPlanUnits / 4) {
+        if (ng < 96) return true;
+        if (ng <= 144) return n_panels > (!rotate ? 16 : ng < 128 ? 12 : 0);
+        return ng <= 160 && (n_panels > 8 || M > 40);
+    }
     if (n_panels <= kPlanUnits / 2) return weight_multipliers && n_panels >= 96 && ng >= 48 && ng <= 160;
     if (n_panels <= kPlanUnits) return ng <= 272 || weight_multipliers;
     if (weight_multipliers) return ng <= 272;

@@ -300,7 +300,7 @@ hipError_t launch_block6(const Gemm6Args &a, hipStream_t stream);
 // that for the tiles (256 rows x 128 tokens) first_tile .. n_tiles - 1 of the tiled launch, in its order, alone
 hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_tile, int n_tiles, hipStream_t stream);
 // whether up to 64 tokens are faster that way than through the skinny kernel, by the panels of one launch
-bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers);
+bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers, bool rotate);
 // How a launch of the fp6 form is cut: n_whole tiles (256 rows x 128 tokens) run whole, the rest in `parts` slices of
 // K each, which meet in cell_bytes of workspace: kGemm6CounterBytes of arrival counters (one int per cut tile: zero on
 // entry, left zero), then one slab of partial totals per slice (needs no clearing).

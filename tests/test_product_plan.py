@@ -32,6 +32,17 @@ def test_33_to_64_tokens(K, N, multipliers, kernel, M):
     assert plan(W4A4, K, N, 32, multipliers)["kernel"] == SKINNY
 
 
+@pytest.mark.parametrize("type_,K,N,M,kernel", [
+    (W4A4H, 5632, 64, 64, FP6), (W4A4H, 6144, 64, 33, SKINNY), (W4A4H, 6144, 768, 64, SKINNY), (W4A4H, 6144, 769, 64, FP6),
+    (W4A4H, 8192, 64, 33, FP6), (W4A4, 5888, 512, 33, FP6), (W4A4, 6144, 1024, 48, SKINNY), (W4A4, 8192, 1024, 64, SKINNY),
+    (W4A4, 8192, 1025, 33, FP6), (W4A4, 9216, 64, 64, SKINNY), (W4A4, 9216, 1025, 64, FP6), (W4A4, 10240, 512, 40, SKINNY),
+    (W4A4H, 10240, 512, 40, SKINNY), (W4A4H, 10240, 512, 41, FP6), (W4A4, 10240, 513, 33, FP6), (W4A4, 10496, 4096, 64, SKINNY)])
+@pytest.mark.parametrize("multipliers", [0, 1])
+def test_33_to_64_tokens_of_few_panels(type_, K, N, M, multipliers, kernel):
+    """A few panels of rows from K = 6144 up: where the units were up to 13 % slower than the skinny kernel."""
+    assert plan(type_, K, N, M, multipliers)["kernel"] == kernel
+
+
 def test_33_to_64_tokens_launch_by_launch():
     """With room for the largest weight only, every weight's own launch has to be one that the units are faster for."""
     Ns = (6144, 6144, 6144)
