@@ -355,8 +355,9 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
             torch.from_numpy(host).copy_(stage)
             return host.view(BLOCK_DTYPE).reshape(N, K // 256)
         other = _second_stream(current)
-        other.wait_stream(current)   # (w, and the memory of out and the workspaces)
         ws = [_device_bytes(nbytes, w.device) for _ in range(2)]
+        # (for w, and behind the allocations: their memory may still be in use by work in front of this call, another thread's too)
+        other.wait_stream(current)
         host = np.empty(N * row, dtype=np.uint8)
         to = torch.from_numpy(host)
         stages, done = [], []
@@ -413,7 +414,7 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
         # runs of rows, in turn on two streams: one is decoded while the next one travels
         current = torch.cuda.current_stream()
         other = _second_stream(current)
-        other.wait_stream(current)   # (the memory of `raw` may still be in use by work in front of this call)
+        other.wait_stream(current)   # (the memory of `raw` and `out` may still be in use by work in front of this call)
         runs = _chunks(rows, max(1, _STAGE_BYTES // row))   # (a row too long for the library is refused by it)
         host = blocks.view(np.uint8).reshape(-1)
         stages, sent = [], []

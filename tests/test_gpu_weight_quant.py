@@ -361,6 +361,27 @@ def test_conversions_keep_their_second_stream():
     assert [len(s) for s in seen] == [1, 1] and seen[0][0] is not seen[1][0]
 
 
+def test_second_stream_waits_behind_the_allocations(monkeypatch):
+    """Device memory that a conversion takes may still be in use by work that another thread queued on the same stream meanwhile:
+    the second stream waits for the first behind the last allocation."""
+    order = []
+    real_bytes, real_wait = w4a4._device_bytes, torch.cuda.Stream.wait_stream
+
+    def device_bytes(*args):
+        order.append("allocates")
+        return real_bytes(*args)
+
+    def wait_stream(self, other):
+        order.append("waits")
+        return real_wait(self, other)
+
+    w = torch.randn((9000, 4096), dtype=torch.float32, device=DEV)
+    monkeypatch.setattr(w4a4, "_device_bytes", device_bytes)
+    monkeypatch.setattr(torch.cuda.Stream, "wait_stream", wait_stream)
+    rq.quantize_weights(w, rq.TYPE_W4A4)
+    assert order == ["allocates", "allocates", "waits"]
+
+
 @pytest.mark.parametrize("wgroup", [0, 256, 64])
 def test_scales_that_the_first_look_leaves_open(oracle, wgroup):
     """Enough segments that some (one in a hundred or fewer) have two ratios whose errors are too near for the fp32 sums, and rows
