@@ -85,10 +85,10 @@ size_t rq_w4a4_prepared_bytes(int64_t K, int64_t N);
 /* Replaces rq_repack_once (P:2046-2075), out of place: reads N rows of K/256 blocks at w_blocks_dev, writes
  * prepared_dev (256-byte aligned, rq_w4a4_prepared_bytes). The input is not modified. Outside graph capture the
  * call ends by waiting for `stream` and reading one word of the result back: whether the tensor carries weight
- * multipliers, which the wide-batch launcher remembers per prepared address to choose between two kernels (both are
- * right for every tensor; a prepared weight that is copied to another address, or prepared under capture, runs the
- * one that is slow on tensors with multipliers). The prepared bytes hold no address of themselves: a copy works
- * whatever becomes of the original. */
+ * multipliers, which the library remembers per prepared address to choose the cheaper way to cut a product of more than
+ * 32 tokens into launches and workgroups (rq_w4a4_product_plan). The kernels read the tensor's own flag, so a prepared
+ * weight that is copied to another address, or prepared under capture, runs the same ones and is planned as one without
+ * multipliers. The prepared bytes hold no address of themselves: a copy works whatever becomes of the original. */
 int rq_w4a4_prepare(const void *w_blocks_dev, int64_t K, int64_t N,
                     void *prepared_dev, size_t prepared_bytes, rq_stream_t stream);
 
@@ -127,9 +127,9 @@ int rq_w4a4_mul_mat(int type, const void *prepared_dev, int64_t K, int64_t N,
 /* rq_w4a4_mul_mat for a caller that will not run stage 2 of rq_w4a4_mul_mat_stages on this workspace afterwards: same
  * arguments and results. rq_w4a4_mul_mat clears the split-K cells of all N rows, so that a later stage-2 call finds them
  * clear whichever of them its plan uses, and keeps the activations in the form that a product of any weight reads. This
- * call clears only the cells that it uses itself (5 to 64 tokens), and at 33 to 64 tokens of enough rows (some
- * thousands, by row length and multipliers) it runs a kernel with an activation form of its own and no cells (K = 5120, N = 17408 at 64
- * tokens: 27.3 instead of 34.5 us). No counterpart in the reference. */
+ * call clears only the cells that it uses itself (5 to 64 tokens), and at 33 to 64 tokens, by the weights' rows, row length and
+ * multipliers (rq_w4a4_product_plan), it may run a kernel with an activation form of its own and no cells (K = 5120, N = 17408 at
+ * 64 tokens: 29.5 instead of 34.8 us, weights from memory). No counterpart in the reference. */
 int rq_w4a4_mul_mat_once(int type, const void *prepared_dev, int64_t K, int64_t N,
                          const float *x_dev, int64_t ldx, int64_t M,
                          float *y_dev, int64_t ldy,

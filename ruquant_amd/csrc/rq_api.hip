@@ -77,9 +77,8 @@ bool gemm_fp6_enabled() { return env().gemm_fp6 != 0; }
 
 namespace {
 
-// Which prepared weights carry weight multipliers, for the weights this process has prepared: what the wide-batch
-// launcher chooses its kernel by. Only a hint: both kernels are right for every tensor (one is slow on tensors with
-// multipliers, the other a few percent slower on tensors without), so an address the table does not know, or knows
+// Which prepared weights carry weight multipliers, for the weights this process has prepared: what the routes above 32 tokens
+// are priced by. Only a hint: the kernels read each weight's own flag, so an address the table does not know, or knows
 // from a buffer that has since been reused, costs time at most.
 std::mutex g_notes_mutex;
 std::unordered_map<const void *, bool> g_notes;
@@ -240,10 +239,14 @@ Choice choose(int n, int64_t K, const int64_t *N, int64_t M, bool rotate, int p,
     c.fp6 = c.small6 || (c.path == kPathGemm && gemm_fp6_enabled());
     bool one = s.one_launch;
     if (c.path == kPathGemm) {
-        // (the fp6 GEMM's slabs do not depend on N, so it needs no room beyond the largest weight's. It runs weights with and
-        // without multipliers through different kernels: a set that has both kinds goes weight by weight. K = 5120, 2048
-        // tokens, N = 6144 + 1024 + 1024: the three launches leave 128, 64 and 64 tiles over to be cut along K, one launch is
-        // two whole rounds of tiles)
+        // (The fp6 GEMM's slabs do not depend on N, so it needs no room beyond the largest weight's. K = 5120, 2048 tokens,
+        // N = 6144 + 1024 + 1024: three launches leave 128, 64 and 64 tiles over, one launch is two whole rounds of tiles. A set that has
+        // weights with and without multipliers goes weight by weight: one launch would run it, each tile by its weight's flag, but the
+        // prices are of launches of one kind, and an XCD gets a run of neighbouring tiles, which of large weights is of one kind: the
+        // slow one's XCDs are the last to end. One with multipliers, us, weight by weight / in one launch, cut as without any: K = 5120,
+        // 2 x 17408 rows, 100 / 300 / 512 / 2048 tokens 66 / 70, 99 / 129, 132 / 150, 474 / 540; K = 17408, 2 x 5120 67 / 61, 114 / 119,
+        // 142 / 203, 467 / 489. Sets of few tiles are the other way round: N = 6144 + 1024 + 1024, a small one with multipliers 34 / 24,
+        // 48 / 50, 56 / 52, 136 / 115, the large one 36 / 24, 52 / 50, 69 / 53, 170 / 139.)
         one = c.fp6 && G == kGroup;
         for (int i = 1; i < n && one; ++i) one = mult[i] == mult[0];
         if (one && n > 1 && s.have_slabs) {   // (without room for slabs no tile is cut, and one launch never has more rounds)
@@ -434,7 +437,7 @@ int run_products(int type, int n, const void *const *prepared, int64_t K, const 
             g.Mp = (int) W.Mp;
             g.groups_per_fold = G / kGroup;
             g.cells = sp.have_slabs ? wsb + W.off_tot : nullptr;
-            g.weight_multipliers = mult[l];   // (one launch: of all alike, or looked at by neither kernel)
+            g.weight_multipliers = mult[l];   // (for the tiled kernel's route, where one launch has weights of one kind; the units have none)
             e = small6 ? launch_block6(g, stream) : launch_gemm6(g, stream);
             if (e != hipSuccess) return (int) e;
         } else if (gemm) {

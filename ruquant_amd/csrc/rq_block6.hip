@@ -444,7 +444,9 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 //   Here up to K = 17408.
 // - More: N = 17408 (272), K = 3072 25.7 / 20.0, 27.1 / 24.3; K = 5120 30.7 / 25.9, 31.8 / 32.5; K = 10240 44.5 / 41.1, 45.3 / 53.7;
 //   K = 17408 63.0 / 61.7, 63.6 / 83.1; K = 32768 100 / 147. N = 24576 (384), K = 10240 55.7 / 42.2, 56.7 / 55.8; N = 34816 (544)
-//   73.7 / 65.7, 74.5 / 79.8. Here up to K = 5120, and up to K = 10240 where the last round is at least half full.
+//   73.7 / 65.7, 74.5 / 79.8. Here up to K = 5120, and up to K = 10240 where the last round is at least half full. (All in whole units.
+//   With the 16 units of a second round in four pieces N = 17408, K = 5120 is 23.7 from the cache and 29.5 from memory, and longer rows might
+//   win too: the line is from before.)
 // - Weight multipliers cost the skinny kernel more: 96 to 128 panels, N = 8192, K = 1024 9.8 / 10.3, K = 3072 N = 6144 14.1 / 13.8,
 //   15.3 / 15.8, K = 5120 18.3 / 17.9, 20.0 / 21.3, K = 10240 33.9 / 26.6, 34.9 / 33.4, K = 17408 58.2 / 45.9, 48.4 / 50.7 (and 8 % more
 //   at 33 tokens); N = 12288, K = 5120 29.7 / 18.9, 31.2 / 22.4, K = 32768 128 / 91, 128 / 95; N = 17408, K = 17408 86 / 71, 87 / 91,

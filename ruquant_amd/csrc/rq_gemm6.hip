@@ -29,12 +29,15 @@
 // 64 inputs = 1536 bytes: a 16-byte and an 8-byte piece per lane, each piece contiguous across the lanes), so a
 // stage is filled by whole 1 KiB runs and read back without bank conflicts.
 //
-// What bounds it: the issue of vector instructions (per MFMA 16 FMAs of four cycles each and 14 cycles of the MFMA that none of
-// them hides: 400,000 of the 526,000 cycles at K = 10240, N = 16384, 2048 tokens) and, above that, the clock, which the matrix
-// cores, the vector ALU and LDS together pull down to 1.87 GHz (2.2 for MFMAs and FMAs alone). 16 MFMAs of a SIMD, a step, take
-// 0.72 us, without LDS reads and fetches 0.53; a tile costs 9.4 us besides its steps. K = 5120, N = 17408, 2048 tokens 183.6 ->
-// 171 us and K = 17408, N = 5120 160 -> 147.5 since a wavefront waits for its operands where it uses them and every read of the
-// ring has a fixed base; with weight multipliers (K = 5120, N = 8192) 139 -> 128, in the same kernel.
+// What bounds it: the issue of vector instructions, 16 FMAs of four cycles and three others per MFMA. Counters at K = 10240,
+// N = 16384, 2048 tokens (four whole rounds): the vector ALU issues in 393,000 of the 515,000 cycles, and in 98,000 more a matrix
+// core works without it (its 32 cycles per MFMA share 13 with a vector instruction). Above that, the clock, which the matrix cores, the
+// vector ALU and LDS together pull down: 1.9 GHz there, 2.0 at K = 5120 and N = 17408, 2.3 in a launch of one round. With weight
+// multipliers the vector ALU issues in 98 % of the cycles. 16 MFMAs of a SIMD, a step, take 0.72 us (in a timing-only build without LDS
+// reads and fetches 0.53); a tile costs 9.4 us besides its steps. Product kernels in us since a wavefront waits for its operands where
+// it uses them and every read of the ring has a fixed base, weights from the memory-side cache, then from memory: K = 5120,
+// N = 17408, 2048 tokens 179.5 -> 170, 192 -> 181 (on another card 190 -> 187); K = 17408, N = 5120 156 -> 147, 170 -> 155; N = 17408, 300
+// tokens 102 -> 90, 112 -> 105; with weight multipliers, K = 5120, N = 8192 140 -> 127, 141 -> 129.
 #include "rq_common.h"
 
 #include <string.h>
@@ -80,8 +83,6 @@ constexpr int kFlushSteps = 16;                // 32 groups
 constexpr int kRsrcWord3 = 0x00020000;         // last word of a raw buffer descriptor on this target (32-bit data format)
 constexpr int kDeviceScope = 16;               // cache policy of a buffer access: the sc1 bit
 
-// 64 lanes x 16 bytes from base + lane offset to 1 KiB of LDS at `lds` (wave-uniform; the hardware adds lane * 16).
-// Assembly, so that the count of outstanding loads stays under this file's control (the s_waitcnt of step()).
 // a wave-uniform address, said so explicitly: the compiler then keeps it in scalar registers
 __device__ __forceinline__ const uint8_t *uniform(const uint8_t *p) {
     const uint64_t b = (uint64_t) (uintptr_t) p;
@@ -90,7 +91,8 @@ __device__ __forceinline__ const uint8_t *uniform(const uint8_t *p) {
                      (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (b >> 32)) << 32));
 }
 
-// (OFF: a constant part of the LDS address, added on the way into M0)
+// 64 lanes x 16 bytes from base + lane offset to 1 KiB of LDS at `lds` + OFF (wave-uniform; the hardware adds lane * 16). OFF is added
+// on the way into M0. Assembly, so that the count of outstanding loads stays under this file's control (the s_waitcnt of the steps).
 template <int OFF>
 __device__ __forceinline__ void load_run(const uint8_t *base, uint32_t lane_off, uint32_t lds) {
     asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -729,8 +731,10 @@ rq_gemm6_kernel(const TileSet<SET> ts, const uint8_t *__restrict__ act6, const f
     // epilogue (reference patch line 176): y = ((float(total) * 16) * u) * s_w. In the MFMA result a lane holds one
     // token (column) and, per tile, rows 8 q + 4 (lane / 32) + 0 .. 3 for q = 0 .. 3: stored as they are, a wavefront's
     // stores would be 32-byte pieces of 32 different rows of y (a third of the kernel's time went there). So every
-    // wavefront turns its four 32 x 32 blocks through LDS one after the other (4.5 KiB per wavefront, all eight inside
-    // the last ring stage, which no fetch is aimed at when the loop ends) and writes 128 contiguous bytes per token.
+    // wavefront turns its four 32 x 32 blocks through LDS one after the other and writes 128 contiguous bytes per token. The
+    // eight wavefronts' 36 KiB lie over the weights of the last stage and half of those of the one before, at which the refetches
+    // of the last steps are aimed: every wavefront has waited for all its loads (the vmcnt(0) that ends body and body64)
+    // before it comes to this barrier, and that wait may not go.
     __syncthreads();   // every wavefront is done reading the ring
     float *xp = reinterpret_cast<float *>(ring + kXpose) + c.wave * (32 * kXposeStride);
     const int h = c.lane >> 5;
@@ -841,9 +845,11 @@ double tiled_price(const Gemm6Plan &pl, int ng, bool weight_multipliers) {
     return rounds * whole + (pl.parts > 1 ? cut : 0.0);
 }
 
-// The same for the kernel of small launches (rq_block6.hip), by rounds of its units and the groups of one wavefront.
-// K = 1024 / 5120 / 17408: 16 units 5.2 / 9.3 / 21.2 us, 192 units 5.6 / 10.5 / 24.7, 384 units 9.5 / 18.7 / 44 (of long rows);
-// weight groups of 64, K = 5120 / 17408, 16 units 12.2 / 29.6, 192 units 13.4 / 32.7, 384 units 24.2.
+// The same for the kernel of small launches (rq_block6.hip), by rounds of its units and the groups of one wavefront: of whole units.
+// K = 1024 / 5120 / 17408: 192 units 5.1 / 10.4 / 25.9 us, with weight groups of 64, K = 5120 / 17408, 13.6 / 35.7. A last round that goes
+// in pieces takes less than it is priced: 16 units 3.6 / 5.7 / 12.5, groups of 64 6.5 / 14.6 (whole 5.2 / 9.3 / 21.2, 12.2 / 29.6); 384 units 10.0 /
+// 18.4 at K = 1024 / 5120, groups of 64, K = 5120 23.4 (the second round's 128 in halves; whole 9.5 / 18.7, 24.2). So what goes to units by
+// this price is at least as fast there, and some of what goes to slices would be faster in units.
 double block_price(int64_t units, int ng, bool weight_multipliers) {
     const double rounds = (double) ((units + kPlanUnits - 1) / kPlanUnits);
     const int per_wave = (ng + 7) / 8;
@@ -853,14 +859,16 @@ double block_price(int64_t units, int ng, bool weight_multipliers) {
 }  // namespace
 
 // The cheapest of three. Few tiles: all of them in small units, as long as those are at most two rounds of the chip (K = 5120:
-// 2 tiles 19.5 us in slices and 9.9 in units, 48 tiles 24.4 and 19.4, 96 tiles, three rounds, 27.7 and 28.6; K = 17408: 2
-// tiles 29.2 and 22.1, 48 tiles 39.2 and 47.3). Whole rounds and a few tiles over: those few in units behind the rounds
-// (K = 5120, N = 17408, 512 tokens, 256 + 16 tiles: 60.8 us with the 16 in slices, 54.4 with them in 128 units). Everything
-// else: tiles, the rest in slices.
+// 2 tiles 19.5 us in slices and 9.9 in whole units, 5.7 in the pieces that they go in; 48 tiles 24.4 and 19.4, 18.4 with the second
+// round in halves; 96 tiles, three rounds, 27.7 and 28.6; K = 17408: 2 tiles 29.2 and 22.1, 12.5 in pieces, 48 tiles 39.2 and 47.3, all of it
+// in whole units). Whole rounds and a few tiles over: those few in units behind the rounds (K = 5120, N = 17408, 512 tokens, 256 + 16
+// tiles: 60.8 us with the 16 in slices, 54.4 with them in 128 whole units; 8.5 of the call's 55 now, in halves). Everything else: tiles,
+// the rest in slices.
 // The prices are of weights in the memory-side cache. From memory a unit gets its rows at 20 KB per microsecond, whatever the
 // others do, while K slices spread a tile's over compute units, so units end where the rows are long: without multipliers
-// at K = 17408 in one round and K = 6144 in two (with them the fold is slow enough to hide it). Whole call in us, slices / units,
-// from the cache, then from memory. One round, 128 tokens: K = 17408, N = 1000 39.4 / 32.4, 40.6 / 42.1, N = 6000 42.0 / 33.4,
+// at K = 17408 in one round and K = 6144 in two (with them the fold is slow enough to hide it). The lines are those of whole units: 64 and
+// fewer, in four pieces, get their rows from four compute units (K = 17408, 32 units from memory 17.7 us instead of 32.0), so that for them, and
+// for a second round of at most 128, units could go on to longer rows. Whole call in us, slices / whole units, from the cache, then from memory. One round, 128 tokens: K = 17408, N = 1000 39.4 / 32.4, 40.6 / 42.1, N = 6000 42.0 / 33.4,
 // 47.4 / 44.0; K = 22528, N = 1000 44.0 / 39.5, 45.1 / 51.7; K = 32768 51.5 / 52.5, 52.7 / 69.7. Two: K = 5120, N = 3000, 400 tokens
 // 31.4 / 26.2, 32.8 / 30.9; K = 10240 40.5 / 41.0, 41.7 / 48.8, N = 6000, 256 tokens 38.3 / 38.5, 39.7 / 48.3.
 Gemm6Route gemm6_route(const FusedWeights &w, int64_t M, int groups_per_fold, bool weight_multipliers, bool have_slabs) {

@@ -103,8 +103,8 @@ def test_without_slabs_every_tile_runs_whole(oracle, multipliers):
     (2560, (2300, 1000, 2800), 500, (0, 0, 0), True, 96, 2, 1),       # 9 + 4 + 11 row tiles in super-tiles over weights
     (2560, (2300, 1000, 2800), 500, (1, 1, 1), True, 96, 2, 1),
     (2560, (9000, 8400), 100, (1, 1), True, 69, 3, 1),                # two weights: the third slot selects nothing
-    (2560, (9000, 4000, 4400), 100, (1, 1, 0), False, 70, 3, 1),      # copies the launcher knows nothing of: folds per tile
-    (5120, (17100, 17408), 100, (1, 0), True, 67 + 68, 3, 2)],        # with and without multipliers: a launch each
+    (2560, (9000, 4000, 4400), 100, (1, 1, 0), False, 70, 3, 1),      # copies planned as weights without multipliers
+    (5120, (17100, 17408), 100, (1, 0), True, 67 + 68, 3, 2)],        # known to be of both kinds: a launch each
     ids=["super_tiles", "super_tiles_multipliers", "two_weights", "unknown_addresses", "both_kinds"])
 def test_slices_of_sets(oracle, K, Ns, M, multipliers, known, cut, slices, launches):
     p = plan(rq.TYPE_W4A4, K, Ns, M, sum(m << i for i, m in enumerate(multipliers)) if known else 0)

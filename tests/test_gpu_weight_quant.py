@@ -250,8 +250,8 @@ def test_tensors_on_the_grid_need_no_search_in_order(K, N, wgroup):
 
 
 def test_conversions_in_several_runs(oracle):
-    """Tensors that go through in several runs of rows; one row more than a run; on the way to the GPU more runs than there
-    are pinned buffers; a read-only array."""
+    """Blocks on the way to the GPU in more runs of rows than there are pinned buffers, from a read-only array. (Tensors on the way to
+    the host in one run here, in several in the tests below.)"""
     w = tensor(4097, 256, 3)
     got = rq.quantize_weights(torch.from_numpy(w).to(DEV), rq.TYPE_W4A4)
     want = oracle.quantize_rows_w(w)
