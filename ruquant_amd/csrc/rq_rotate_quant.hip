@@ -24,7 +24,7 @@ namespace {
 // work per phase. Long Paley stages that keep a column in one thread's registers need the 256-register budget of 512
 // threads; those whose columns four threads share (WIDE) get 1024. Many tokens of short rows (FEW, takes_few) get 256.
 template <int P, bool SLICED, bool WIDE, bool FEW>
-constexpr int threads_of() { return FEW ? 256 : WIDE || (SLICED && P < 44) ? 1024 : 512; }
+constexpr int threads_of() { return FEW ? 256 : WIDE || (SLICED && P > 1 && P < 44) ? 1024 : 512; }
 
 using namespace had;
 
@@ -105,15 +105,19 @@ __device__ __forceinline__ void quantize_fp6(const RotQuantArgs &a, const float 
     }
 }
 
-template <int P, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
+template <int P, bool FP6, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
 // Registers are capped so that two workgroups (p >= 44: long columns, long rows) or three fit a compute unit: the
 // stages of one token are separated by barriers, and it is the other workgroups that keep the vector ALU busy. (The
 // sliced variant serves small batches, where occupancy is not the limit.) WIDE: 1024 threads, the columns of a long Paley stage
 // by four threads each (paley_row), a fourth of the registers per column; see takes_wide for where. ALONE is the plain
 // variant for rows so long that LDS holds one workgroup per compute unit anyway: the cap then only makes the p >= 60 columns
 // spill (136 to 504 bytes per lane), so it goes (2048 tokens, K = 21504, p = 84: 204 -> 193 us). FEW: five workgroups of 256 threads, with
-// the registers that p = 20 needs (six make it spill: K = 5120, 2048 tokens 19.8 us, five 18.3).
-__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE, FEW>()), FEW ? 5 : WIDE ? (P >= 84 ? 4 : 8) : SLICED ? (P < 44 ? 4 : 2) : ALONE ? 2 : P >= 44 ? 4 : 6)
+// the registers that p = 20 needs (six make it spill: K = 5120, 2048 tokens 19.8 us, five 18.3). FP6: the quantizer in front of the fp6
+// product, in kernels of its own, and P = 0: rows without a rotation: in one kernel with the other forms these change their registers
+// and where their code lies. (Us, one kernel for all -> so: A4 blocks, 300 tokens, K = 1024 / 5120 / 17408 4.23 / 5.42 / 9.85 -> 4.08 /
+// 5.28 / 9.74; product of 4 tokens without a rotation, K = 6144 8.04 -> 7.9; rotation alone, K = 5376, 700 tokens, whose columns spill, 46.4
+// -> 42.5.)
+__global__ void __launch_bounds__((threads_of<P, SLICED, WIDE, FEW>()), FEW ? 5 : WIDE ? (P >= 84 ? 4 : 8) : SLICED && P > 1 ? (P < 44 ? 4 : 2) : ALONE ? 2 : P >= 44 ? 4 : 6)
 rq_rotate_quant_kernel(const RotQuantArgs a) {
     constexpr int kNT = threads_of<P, SLICED, WIDE, FEW>();
     extern __shared__ __align__(16) float smem[];
@@ -142,8 +146,8 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     const int ng = K / kGroup;
     const int Kp = padi(K) + 1;                  // floats of one padded row
     float *buf = smem;
-    float *alt = smem + Kp;                      // second row buffer (SLICED only)
-    float *g_lo = smem + (SLICED ? 2 * Kp : Kp);
+    float *alt = smem + Kp;                      // second row buffer (SLICED only, for its Paley stage)
+    float *g_lo = smem + (SLICED && P > 1 ? 2 * Kp : Kp);
     float *g_hi = g_lo + ng;
 
     const float *xr = a.x + (int64_t) t * a.ldx;
@@ -151,12 +155,12 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     // (small batches, bound by the latency of its phases) the next four ride too, between lanes, when the chunks are
     // made of blocks of 256 floats; large batches are bound by vector-ALU time, where the LDS pass is the cheaper
     // one (2048 tokens at K = 17408: 105 us against 128 us with the stages between lanes).
-    // Without a Paley stage that holds up to a token per compute unit: together with the scale in the last trip, activation stage
+    // Without a Paley stage (P = 1, whose sliced variant is that and nothing else) it holds up to a token per compute unit: together with the scale in the last trip, activation stage
     // at 16 / 200 tokens, K = 1024 4.1 -> 3.9 / 4.4 -> 4.1 us, 4096 5.3 -> 4.7 / 5.5 -> 4.9, 8192 7.8 -> 6.8 / 7.9 -> 6.8.
-    const bool fused_first = a.rotate && (a.m & 15) == 0;
-    const bool fused_256 = (SLICED || (P == 1 && a.M <= kPlanUnits)) && a.rotate && (a.m & 255) == 0;
-    // (out of the other rows' way: in front of them this code costs a call without a rotation 0.1 us: 2 tokens, K = 2048 2.58 -> 2.68)
-    if (SLICED ? fused_256 : __builtin_expect(fused_256, 0)) {
+    const bool rotate = P > 0 && a.rotate;
+    const bool fused_first = rotate && (a.m & 15) == 0;
+    const bool fused_256 = SLICED && rotate && (a.m & 255) == 0;
+    if (fused_256) {
         load_row_fwht256<kNT, (P >= 44 ? 3 : 1)>(buf, xr, K, tid);
     } else if (fused_first) {
         // long Paley stages go with long rows (several units of 16 floats per thread): all of a thread's loads go
@@ -167,7 +171,7 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
     }
     __syncthreads();
 
-    if (a.rotate) {
+    if (rotate) {
         const int m = a.m;
         const int lm = __ffs(m) - 1;
         const int ls0 = fused_256 ? 8 : fused_first ? 4 : 0;
@@ -241,18 +245,16 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
         }
     }
 
+    if constexpr (FP6) {
+        quantize_fp6<kNT>(a, buf, g_lo, g_hi, s_red, t, tid);
+        return;
+    }
     if (a.mode == kActRotateOnly) {
         float *o = a.out_f32 + (int64_t) t * a.ldo;
         for (int i = tid * 4; i < K; i += kNT * 4) {
             const float *sp = buf + padi(i);
             *reinterpret_cast<float4 *>(o + i) = make_float4(sp[0], sp[1], sp[2], sp[3]);
         }
-        return;
-    }
-
-    // (behind the other forms: laid out in front of them it makes the plain form of p = 20, whose columns spill, 4.5 % slower in all)
-    if (__builtin_expect(a.mode == kActI8 && a.single == 2, 0)) {
-        quantize_fp6<kNT>(a, buf, g_lo, g_hi, s_red, t, tid);
         return;
     }
 
@@ -390,9 +392,9 @@ rq_rotate_quant_kernel(const RotQuantArgs a) {
 }
 
 // the kernels keep a whole row in dynamic LDS: raise the per-kernel limit (once per device, see init_activation_kernels)
-template <int P, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
+template <int P, bool FP6, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
 hipError_t allow_big_lds() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE, FEW>),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&rq_rotate_quant_kernel<P, FP6, SLICED, WIDE, ALONE, FEW>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 64);
 }
 
@@ -400,21 +402,26 @@ constexpr bool has_wide(int p) { return p >= 44; }
 // the plain variant has an ALONE build where the cap makes its columns spill and rows past takes_wide get that long
 constexpr bool has_alone(int p) { return p == 60 || p >= 84; }
 
-template <int P>
-hipError_t allow_big_lds_both() {
-    hipError_t e = allow_big_lds<P, false>();
-    if (e == hipSuccess && P > 1) e = allow_big_lds<P, (P > 1)>();
-    if (e == hipSuccess && has_wide(P)) e = allow_big_lds<P, false, has_wide(P)>();
-    if (e == hipSuccess && P < 44) e = allow_big_lds<P, false, false, false, (P < 44)>();
-    if (e == hipSuccess && has_alone(P)) e = allow_big_lds<P, false, false, has_alone(P)>();
+template <int P, bool FP6>
+hipError_t allow_big_lds_forms() {
+    hipError_t e = allow_big_lds<P, FP6, false>();
+    if (e == hipSuccess && P > 0) e = allow_big_lds<P, FP6, (P > 0)>();
+    if (e == hipSuccess && has_wide(P)) e = allow_big_lds<P, FP6, false, has_wide(P)>();
+    if (e == hipSuccess && P < 44) e = allow_big_lds<P, FP6, false, false, false, (P < 44)>();
+    if (e == hipSuccess && has_alone(P)) e = allow_big_lds<P, FP6, false, false, has_alone(P)>();
     return e;
 }
+template <int P>
+hipError_t allow_big_lds_both() {
+    const hipError_t e = allow_big_lds_forms<P, false>();
+    return e == hipSuccess ? allow_big_lds_forms<P, true>() : e;
+}
 
-template <int P, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
+template <int P, bool FP6, bool SLICED, bool WIDE = false, bool ALONE = false, bool FEW = false>
 hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
     static bool attr_set = false;   // calls that never went through rq_w4a4_prepare on this device
     if (!attr_set) {
-        hipError_t e = allow_big_lds<P, SLICED, WIDE, ALONE, FEW>();
+        hipError_t e = allow_big_lds<P, FP6, SLICED, WIDE, ALONE, FEW>();
         if (e != hipSuccess) return e;
         attr_set = true;
     }
@@ -424,7 +431,7 @@ hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
     b.token_blocks = a.M;
     const int grid = a.M + (int) ((a.zero_ints + (int64_t) kNT * 4 - 1) / ((int64_t) kNT * 4));
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, SLICED, WIDE, ALONE, FEW>), dim3(grid), dim3(kNT), lds, stream, b);
+    hipLaunchKernelGGL((rq_rotate_quant_kernel<P, FP6, SLICED, WIDE, ALONE, FEW>), dim3(grid), dim3(kNT), lds, stream, b);
     return hipGetLastError();
 }
 
@@ -445,8 +452,9 @@ hipError_t launch_one(const RotQuantArgs &a, size_t lds, hipStream_t stream) {
 //     tokens 13.7 -> 14.2 / 17.4 -> 16.9, K = 30720 (60 x 512) 19.0 -> 19.8 / 23.7 -> 23.3.
 template <int P>
 bool takes_wide(const RotQuantArgs &a, bool sliced) {
-    const int columns = a.K / P;
-    if (!has_wide(P) || columns < 256) return false;
+    if (!has_wide(P)) return false;
+    const int columns = a.K / (P > 0 ? P : 1);
+    if (columns < 256) return false;
     if (columns == 256 || sliced) return true;
     if (P == 68 || P == 72) return a.M > 128;
     return columns == 512 && a.m >= 256 && a.mode != kActRotateOnly;
@@ -476,24 +484,30 @@ bool takes_few(const RotQuantArgs &a) {
 
 // LDS: one padded row (two when the Paley stage is sliced over more threads) plus the group ranges. Slicing buys
 // parallelism inside a token and costs occupancy, so it is for small batches only.
-template <int P>
-hipError_t launch_p(const RotQuantArgs &a, hipStream_t stream) {
+template <int P, bool FP6>
+hipError_t launch_form(const RotQuantArgs &a, hipStream_t stream) {
     const size_t row = (size_t) (a.K + (a.K >> 4) + 1) * sizeof(float);
     const size_t stats = (size_t) 2 * (a.K / kGroup + 1) * sizeof(float);
     // long Paley stages: past kTwoStepTokens tokens the plain variant (two workgroups per CU) is the faster one
     const bool sliced = P > 1 && a.M <= (P >= 44 ? kTwoStepTokens : 64) && 2 * row + stats <= 160 * 1024 - 64;
-    if (takes_wide<P>(a, sliced)) return launch_one<P, false, has_wide(P)>(a, row + stats, stream);
-    if (sliced) return launch_one<P, (P > 1)>(a, 2 * row + stats, stream);
+    if (P == 1 && a.M <= kPlanUnits && (a.m & 255) == 0) return launch_one<P, FP6, (P == 1)>(a, row + stats, stream);
+    if (takes_wide<P>(a, sliced)) return launch_one<P, FP6, false, has_wide(P)>(a, row + stats, stream);
+    if (sliced) return launch_one<P, FP6, (P > 1)>(a, 2 * row + stats, stream);
     // a second workgroup does not fit beside this one
-    if (has_alone(P) && 2 * (row + stats + 64) > 160 * 1024) return launch_one<P, false, false, has_alone(P)>(a, row + stats, stream);
-    if (takes_few<P>(a)) return launch_one<P, false, false, false, (P < 44)>(a, row + stats, stream);
-    return launch_one<P, false>(a, row + stats, stream);
+    if (has_alone(P) && 2 * (row + stats + 64) > 160 * 1024) return launch_one<P, FP6, false, false, has_alone(P)>(a, row + stats, stream);
+    if (takes_few<P>(a)) return launch_one<P, FP6, false, false, false, (P < 44)>(a, row + stats, stream);
+    return launch_one<P, FP6, false>(a, row + stats, stream);
+}
+template <int P>
+hipError_t launch_p(const RotQuantArgs &a, hipStream_t stream) {
+    return a.mode == kActI8 && a.single == 2 ? launch_form<P, true>(a, stream) : launch_form<P, false>(a, stream);
 }
 
 }  // namespace
 
 hipError_t init_rotate_quant_kernels() {
-    hipError_t e = allow_big_lds_both<1>();
+    hipError_t e = allow_big_lds_both<0>();
+    if (e == hipSuccess) e = allow_big_lds_both<1>();
     if (e == hipSuccess) e = allow_big_lds_both<12>();
     if (e == hipSuccess) e = allow_big_lds_both<20>();
     if (e == hipSuccess) e = allow_big_lds_both<44>();
@@ -508,8 +522,9 @@ hipError_t init_rotate_quant_kernels() {
 
 hipError_t launch_rotate_quant(const RotQuantArgs &a, hipStream_t stream) {
     if (a.M == 0 && a.zero_ints == 0) return hipSuccess;
-    const int p = a.rotate ? a.p : 1;
+    const int p = a.rotate ? a.p : 0;
     switch (p) {
+        case 0:   return launch_p<0>(a, stream);
         case 1:   return launch_p<1>(a, stream);
         case 12:  return launch_p<12>(a, stream);
         case 20:  return launch_p<20>(a, stream);

@@ -13,7 +13,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("K,M", [(256, 5), (512, 64), (4096, 256), (4096, 257), (1024, 513), (1536, 513), (1280, 65), (3072, 512),
-                                 (5120, 65), (5120, 513), (8192, 16), (8192, 200)])
+                                 (5120, 65), (5120, 513), (8192, 16), (8192, 200), (32768, 33)])
 def test_product(oracle, K, M):
     type_, N = rq.TYPE_W4A4H, 40
     blocks, wf = adversarial_weights(oracle, N, K, type_, seed=K + M)
