@@ -431,12 +431,15 @@ hipError_t launch_block6_tiles(const Gemm6Args &a, int super_tiles, int first_ti
 //   12.6 / 12.2, N = 4096 14.1 / 10.4, 15.6 / 13.5; K = 10240 21.6 / 14.2, 23.4 / 18.8; K = 17408, N = 1024 20.2 / 18.6, 22.0 / 25.1,
 //   N = 4096 27.3 / 19.7, 28.6 / 27.0; K = 32768, N = 1024 28.7 / 30.3, 28.6 / 40.0. Here up to K = 10240, but for a few panels of
 //   rows that long, where the skinny kernel has slices along K instead and the fp6 quantizer, a thread per 32 values, takes longer
-//   (33 / 64 tokens, here as a part of the skinny kernel's time, cache; memory): K = 5632 at most 1.01; K = 6144 N = 256 1.01 / 1.00;
-//   1.05 / 1.05, N = 512 1.00 / 1.00; 1.07 / 1.05, N = 768 0.98 / 0.95; 1.02 / 1.00, N = 1024 0.99 / 0.95; 1.03 / 1.00; K = 8192
-//   N = 256 0.99 / 0.97; 1.03 / 1.02, N = 512 0.96 / 0.93; 1.02 / 0.99. Without a rotation, whose launch hides some of that: K = 6144
-//   N = 512 0.99 / 1.00; 1.08 / 1.07, K = 8192 N = 256 1.09 / 1.05; 1.12 / 1.11, N = 1024 1.03 / 0.95; 1.05 / 1.00, N = 1536 0.94 / 0.90; 1.03 /
-//   1.02, K = 9216 N = 512 1.04 / 1.03; 1.09 / 1.05, N = 1536 0.91 / 0.87; 0.97 / 0.94. K = 10240 is the skinny kernel's second step: N = 256
-//   1.01 / 0.91; 1.06 / 0.96 (48 tokens 0.99; 1.02), N = 512 0.99 / 0.88; 1.04 / 0.91, N = 768 0.96 / 0.85; 0.97 / 0.86.
+//   (33 / 64 tokens, here as a part of the skinny kernel's time, cache; memory, weights in turn from 330 MB of codes): K = 5632 at most
+//   1.01; K = 6144 N = 256 1.01 / 1.00; 1.05 / 1.05, N = 512 1.00 / 1.00; 1.07 / 1.05, N = 1165 0.97 / 0.92; 1.01 / 0.97, N = 1344 0.94 / 0.89; 1.05 /
+//   0.97. K = 8192 N = 256 0.98 / 0.96; 0.96 / 0.95, N = 1024 0.95 / 0.89; 1.04 / 0.99, N = 2048 0.88 / 0.85; 1.03 / 0.99. K = 9216 (48 / 64
+//   tokens; up to 40 its rotation is a launch of its own and the skinny kernel follows) N = 64 1.03 / 1.03; 1.06 / 1.06, N = 1165 1.00 / 0.97; 1.08 /
+//   1.07, N = 2048 0.99 / 0.93; 1.06 / 1.04, N = 2238 0.98 / 0.91; 1.04 / 1.03. Without a rotation, whose launch hides some of that: K = 6144 N = 512
+//   0.99 / 1.00; 1.08 / 1.07, N = 1165 0.97 / 0.92; 1.01 / 0.97, K = 7168 N = 1165 0.96 / 0.92; 1.06 / 1.02, K = 8192 N = 1165 0.99 / 0.95; 1.12 / 1.08,
+//   N = 2048 0.92 / 0.88; 1.10 / 1.06, N = 2560 0.88 / 0.84; 1.04 / 1.01, K = 9216 N = 1165 0.98 / 0.94; 1.14 / 1.12, N = 2048 0.90 / 0.87; 1.11 / 1.07,
+//   N = 2560 0.84 / 0.81; 1.04 / 1.01. K = 10240 is the skinny kernel's second step: N = 256 1.01 / 0.91; 1.06 / 0.96 (48 tokens 0.99; 1.02),
+//   N = 1165 0.92 / 0.79; 1.08 / 0.92 (48 tokens 1.04), N = 1792 0.88 / 0.76; 1.08 / 0.91, N = 2048 0.84 / 0.71; 1.00 / 0.88.
 // - 65 to 128 panels (half the chip: the skinny kernel has two workgroups of 32 tokens a panel): K = 5120, N = 8192 14.8 / 15.0,
 //   16.1 / 19.6; K = 17408, N = 8192 47.6 / 39.4, 38.4 / 46.6. The skinny kernel.
 // - 129 to 256 panels, a round of units, and two of the skinny kernel's: N = 12288, K = 1024 15.6 / 9.5, 16.3 / 10.9; K = 5120
@@ -456,8 +459,9 @@ bool block6_takes(int64_t n_panels, int64_t M, int ng, bool weight_multipliers, 
     if (M <= 32) return false;
     if (n_panels <= kPlanUnits / 4) {
         if (ng < 96) return true;
-        if (ng <= 144) return n_panels > (!rotate ? 16 : ng < 128 ? 12 : 0);
-        return ng <= 160 && (n_panels > 8 || M > 40);
+        if (ng < 128) return n_panels > (rotate ? 12 : 16);
+        if (ng <= 144) return n_panels > (!rotate ? 36 : ng > 128 ? 32 : 0);
+        return ng <= 160 && (n_panels > 28 || M > 40);
     }
     if (n_panels <= kPlanUnits / 2) return weight_multipliers && n_panels >= 96 && ng >= 48 && ng <= 160;
     if (n_panels <= kPlanUnits) return ng <= 272 || weight_multipliers;

@@ -34,12 +34,13 @@ def test_33_to_64_tokens(K, N, multipliers, kernel, M):
 
 @pytest.mark.parametrize("type_,K,N,M,kernel", [
     (W4A4H, 5632, 64, 64, FP6), (W4A4H, 6144, 64, 33, SKINNY), (W4A4H, 6144, 768, 64, SKINNY), (W4A4H, 6144, 769, 64, FP6),
-    (W4A4H, 8192, 64, 33, FP6), (W4A4, 5888, 512, 33, FP6), (W4A4, 6144, 1024, 48, SKINNY), (W4A4, 8192, 1024, 64, SKINNY),
-    (W4A4, 8192, 1025, 33, FP6), (W4A4, 9216, 64, 64, SKINNY), (W4A4, 9216, 1025, 64, FP6), (W4A4, 10240, 512, 40, SKINNY),
-    (W4A4H, 10240, 512, 40, SKINNY), (W4A4H, 10240, 512, 41, FP6), (W4A4, 10240, 513, 33, FP6), (W4A4, 10496, 4096, 64, SKINNY)])
+    (W4A4H, 8192, 64, 33, FP6), (W4A4, 5888, 512, 33, FP6), (W4A4, 6144, 1024, 48, SKINNY), (W4A4, 7936, 1025, 33, FP6),
+    (W4A4, 8192, 2304, 64, SKINNY), (W4A4, 8192, 2305, 33, FP6), (W4A4, 9216, 64, 64, SKINNY), (W4A4, 9216, 2305, 64, FP6),
+    (W4A4H, 9216, 2048, 64, SKINNY), (W4A4H, 9216, 2049, 64, FP6), (W4A4H, 9216, 2049, 40, SKINNY), (W4A4, 10240, 1792, 40, SKINNY),
+    (W4A4H, 10240, 1792, 40, SKINNY), (W4A4H, 10240, 512, 41, FP6), (W4A4, 10240, 1793, 33, FP6), (W4A4, 10496, 4096, 64, SKINNY)])
 @pytest.mark.parametrize("multipliers", [0, 1])
 def test_33_to_64_tokens_of_few_panels(type_, K, N, M, multipliers, kernel):
-    """A few panels of rows from K = 6144 up: where the units were up to 13 % slower than the skinny kernel."""
+    """A few panels of rows from K = 6144 up: where the units were up to 14 % slower than the skinny kernel on weights from memory."""
     assert plan(type_, K, N, M, multipliers)["kernel"] == kernel
 
 
