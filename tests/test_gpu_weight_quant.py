@@ -361,6 +361,30 @@ def test_conversions_keep_their_second_stream():
     assert [len(s) for s in seen] == [1, 1] and seen[0][0] is not seen[1][0]
 
 
+def test_a_small_conversion_launches_first(monkeypatch):
+    """In one run the host makes no Stream object in front of the launch but the one that the launch needs: the GPU would wait for it."""
+    order = []
+    real_stream, real_library = torch.cuda.current_stream, rq.load_library()
+
+    class Library:
+        def __getattr__(self, name):
+            if name == "rq_w4a4_quantize_weights":
+                order.append("launches")
+            return getattr(real_library, name)
+
+    def current_stream(*args):
+        order.append("stream")
+        return real_stream(*args)
+
+    w = torch.randn((97, 1024), dtype=torch.float32, device=DEV)
+    want = rq.quantize_weights(w, rq.TYPE_W4A4, wgroup=256)
+    monkeypatch.setattr(w4a4, "load_library", Library)
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    got = rq.quantize_weights(w, rq.TYPE_W4A4, wgroup=256)
+    assert order == ["launches", "stream", "stream"]   # (the call's name is looked up, then its arguments are made)
+    assert blocks_equal(got, want)
+
+
 def test_second_stream_waits_behind_the_allocations(monkeypatch):
     """Device memory that a conversion takes may still be in use by work that another thread queued on the same stream meanwhile:
     the second stream waits for the first behind the last allocation."""
