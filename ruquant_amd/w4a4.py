@@ -388,6 +388,17 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
         return host.view(BLOCK_DTYPE).reshape(N, K // 256)
 
 
+def _decodes_slowly(K, n_rot):
+    """Whether a run of rotated rows takes more than half as long to decode as to travel (4 MiB: 75 us on the link). Long columns of few
+    (K = 5376 = 84 x 64 96 us, 9216 = 72 x 128 58, 1280 = 20 x 64 40, 27648 = 108 x 256 45; 11264 = 44 x 256 23, 17408 = 68 x 256 23) and many short
+    rows (K = 256 65, 512 39; 1024 25)."""
+    factor = hadamard_factor(n_rot) if n_rot > 0 else None
+    if factor is None:   # (refused by the library)
+        return False
+    p = factor[0]
+    return K <= 512 or (p > 1 and (p >= 104 or K <= (128 if p >= 60 else 64) * p))
+
+
 def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
     """[rows, K/256] blocks of any of the four types (numpy, host) -> [rows, K] fp32 on the GPU: the type's to_float
     (dequantize_row_w4a4 / _w4a4h / _a4 / _a4h, patch lines 2738-2773). The rotation length of the rotated types
@@ -413,10 +424,18 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
             rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr(), rows, K, int(n_rot), out.data_ptr(), K, _stream_ptr())
             _check(rc, "rq_w4a4_dequantize")
             return out
-        # runs of rows, in turn on two streams: one is decoded while the next one travels
+        # Runs of rows, in turn on two streams: one is decoded while the next one travels, and the link goes from copy to copy without
+        # a pause. But a copy waits for the run that is decoded in front of it on its stream, so where decoding takes long the
+        # copies go one behind the other on the current stream, and the runs but the last are decoded on the second. (Call by call /
+        # one call behind another in us, in turn -> apart: 5376 x 5000 587 / 611 -> 486 / 449, 9216 x 5582 807 / 843 -> 753 / 708, 256 x 200977
+        # 887 / 997 -> 782 / 735, 1280 x 40195 717 / 800 -> 740 / 703; 4096 x 12207 626 / 612 -> 684 / 642, 5120 x 6144 432 / 398 -> 461 / 422.)
+        apart = type_ in (TYPE_W4A4H, TYPE_A4H) and _decodes_slowly(K, int(n_rot))
         current = torch.cuda.current_stream()
         other = _second_stream(current)
-        other.wait_stream(current)   # (the memory of `raw` and `out` may still be in use by work in front of this call)
+        # The memory of `raw` and `out` may still be in use by work in front of this call. (Apart, what the second stream does waits for
+        # copies on the first one, and an event in front of the first copy delays it: 9216 x 865 212 us without, 262 with one.)
+        if not apart:
+            other.wait_stream(current)
         runs = _chunks(rows, max(1, _STAGE_BYTES // row))   # (a row too long for the library is refused by it)
         host = blocks.view(np.uint8).reshape(-1)
         stages, sent = [], []
@@ -428,11 +447,15 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
                 else:
                     sent[i - _STAGES].synchronize()
                 _copy_bytes(stages[k], host[row * a:row * b])
-                with torch.cuda.stream(other if i & 1 else current):
+                last = i + 1 == len(runs)
+                with torch.cuda.stream(other if i & 1 and not apart else current):
                     raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
-                    if i + _STAGES < len(runs):
+                    if i + _STAGES < len(runs) or (apart and not last):
                         sent.append(torch.cuda.Event())
                         sent[i].record()
+                if apart and not last:
+                    other.wait_event(sent[i])
+                with torch.cuda.stream(other if (not last if apart else i & 1) else current):
                     rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot),
                                               out.data_ptr() + 4 * K * a, K, _stream_ptr())
                 _check(rc, "rq_w4a4_dequantize")

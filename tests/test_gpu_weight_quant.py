@@ -281,6 +281,23 @@ def test_blocks_fetched_in_more_runs_than_buffers(type_, wgroup):
         assert blocks_equal(got, want), block_diff(got, want)
 
 
+@pytest.mark.parametrize("K,rows,apart", [(256, 100001, True), (5376, 1400, True), (5376, 6001, True), (17408, 1280, False)])
+def test_rotated_rows_in_several_runs(K, rows, apart):
+    """Rows whose runs are decoded on the second stream alone (four runs, two, five) and in turn on both: the same floats as in pieces
+    that go through in one run."""
+    assert w4a4._decodes_slowly(K, K) == apart
+    g = torch.Generator(device=DEV)
+    g.manual_seed(K)
+    blocks = rq.quantize_weights(torch.randn((rows, K), dtype=torch.float32, device=DEV, generator=g) * 0.02, rq.TYPE_W4A4H)
+    step = w4a4._STAGE_BYTES // (K // 256 * 144)
+    want = torch.cat([rq.dequantize(blocks[a:a + step], rq.TYPE_W4A4H, device=DEV) for a in range(0, rows, step)])
+    for _ in range(3):
+        got = rq.dequantize(blocks, rq.TYPE_W4A4H, device=DEV)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+        got.fill_(float("nan"))   # (the next call gets this memory)
+        del got
+
+
 @pytest.mark.parametrize("rows", [1, 3639, 3640, 3641, 5461, 5462])
 def test_conversions_around_one_buffer(oracle, rows):
     """A tensor whose blocks fit one pinned buffer (3640 rows of 8 blocks, 4 MiB; 5461 on the way to the host) goes through
