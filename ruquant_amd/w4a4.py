@@ -8,6 +8,7 @@ ggml_cuda_mul_mat_rq_w4a4_fused. A ``W4A4Weight`` plays the part of the ggml wei
 
 torch owns device memory and the stream; every computation happens inside librq_w4a4.so.
 """
+import contextlib
 import ctypes
 import threading
 
@@ -355,14 +356,26 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
             torch.cuda.current_stream().synchronize()
             to.copy_(stage)
             return host.view(BLOCK_DTYPE).reshape(N, K // 256)
+        # But the next but one run waits for the copy in front of it on its stream, and rotated rows with a scale per 64 inputs take so
+        # long that the link then stands still: those are converted one behind the other on the current stream, the copies on the
+        # second. (In turn -> apart, us: 1024 x 48828 966 -> 747, 4096 x 12207 827 to 898 -> 743 to 846, 17408 x 2872 859 -> 770, 5120 x 3000 330 ->
+        # 326; not rotated, 17408 x 804 298 -> 328; a scale per row 5120 x 6144 490 -> 513, per 256 5120 x 9765 691 to 720 -> 724.)
+        apart = wgroup == 64 and type_ == TYPE_W4A4H
         current = torch.cuda.current_stream()
         other = _second_stream(current)
-        ws = [_device_bytes(nbytes, w.device) for _ in range(2)]
+        ws = [_device_bytes(nbytes, w.device) for _ in range(1 if apart else 2)]
         # (for w, and behind the allocations: their memory may still be in use by work in front of this call, another thread's too)
-        other.wait_stream(current)
+        if not apart:   # (apart, the second stream waits for what it copies)
+            other.wait_stream(current)
         host = np.empty(N * row, dtype=np.uint8)
         to = torch.from_numpy(host)
         stages, done = [], []
+
+        def fetch(i):
+            a, b = runs[i]
+            stages[i % _STAGES][:row * (b - a)].copy_(out[row * a:row * b], non_blocking=True)
+            done.append(torch.cuda.Event())
+            done[i].record()
 
         def land(i):
             a, b = runs[i]
@@ -371,15 +384,21 @@ def quantize_weights(w, type_, n_rot=None, wgroup=0):
 
         try:
             for i, (a, b) in enumerate(runs):
-                with torch.cuda.stream(other if i & 1 else current):
-                    convert(a, b, ws[i & 1])
+                with torch.cuda.stream(other) if i & 1 and not apart else contextlib.nullcontext():
+                    convert(a, b, ws[0 if apart else i & 1])
+                    if apart:
+                        ready = torch.cuda.Event()
+                        ready.record()
                     if i >= _STAGES:
                         land(i - _STAGES)
                     else:
                         stages.append(_pinned(row * max(d - c for c, d in runs)))
-                    stages[i % _STAGES][:row * (b - a)].copy_(out[row * a:row * b], non_blocking=True)
-                    done.append(torch.cuda.Event())
-                    done[i].record()
+                    if not apart:
+                        fetch(i)
+                if apart:
+                    other.wait_event(ready)
+                    with torch.cuda.stream(other):
+                        fetch(i)
             for i in range(max(0, len(runs) - _STAGES), len(runs)):
                 land(i)
         except BaseException:
@@ -439,6 +458,12 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
         runs = _chunks(rows, max(1, _STAGE_BYTES // row))   # (a row too long for the library is refused by it)
         host = blocks.view(np.uint8).reshape(-1)
         stages, sent = [], []
+
+        def decode(a, b):
+            rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot), out.data_ptr() + 4 * K * a, K,
+                                      _stream_ptr())
+            _check(rc, "rq_w4a4_dequantize")
+
         try:
             for i, (a, b) in enumerate(runs):
                 n, k = row * (b - a), i % _STAGES
@@ -447,18 +472,18 @@ def dequantize(blocks, type_, n_rot=None, device="cuda:0"):
                 else:
                     sent[i - _STAGES].synchronize()
                 _copy_bytes(stages[k], host[row * a:row * b])
-                last = i + 1 == len(runs)
-                with torch.cuda.stream(other if i & 1 and not apart else current):
+                behind = apart and i + 1 < len(runs)   # (decoded on the second stream, behind the copy on the current one)
+                with torch.cuda.stream(other) if i & 1 and not apart else contextlib.nullcontext():
                     raw[row * a:row * b].copy_(stages[k][:n], non_blocking=True)
-                    if i + _STAGES < len(runs) or (apart and not last):
+                    if i + _STAGES < len(runs) or behind:
                         sent.append(torch.cuda.Event())
                         sent[i].record()
-                if apart and not last:
+                    if not behind:
+                        decode(a, b)
+                if behind:
                     other.wait_event(sent[i])
-                with torch.cuda.stream(other if (not last if apart else i & 1) else current):
-                    rc = L.rq_w4a4_dequantize(int(type_), raw.data_ptr() + row * a, b - a, K, int(n_rot),
-                                              out.data_ptr() + 4 * K * a, K, _stream_ptr())
-                _check(rc, "rq_w4a4_dequantize")
+                    with torch.cuda.stream(other):
+                        decode(a, b)
         finally:
             current.wait_stream(other)   # (what comes behind this call, also on an error the reuse of the memory)
     return out

@@ -262,10 +262,10 @@ def test_conversions_in_several_runs(oracle):
     assert bits_equal(got, rq.dequantize_rows(blocks))
 
 
-@pytest.mark.parametrize("type_,wgroup", [(rq.TYPE_W4A4H, 0), (rq.TYPE_W4A4, 64)])
+@pytest.mark.parametrize("type_,wgroup", [(rq.TYPE_W4A4H, 0), (rq.TYPE_W4A4, 64), (rq.TYPE_W4A4H, 64)])
 def test_blocks_fetched_in_more_runs_than_buffers(type_, wgroup):
-    """9000 rows of 4096: five runs of rows (20.7 MB) through three buffers, in turn on two streams. The bytes are those of one
-    call of the C entry point."""
+    """9000 rows of 4096: five runs of rows (20.7 MB) through three buffers, in turn on two streams or, rotated with a scale per 64
+    inputs, converted on the one and copied on the other. The bytes are those of one call of the C entry point."""
     N, K = 9000, 4096
     g = torch.Generator(device=DEV)
     g.manual_seed(4)
